@@ -38,7 +38,7 @@ constexpr int OW1 = 0, OB1 = OW1 + NH * NI, OW2 = OB1 + NH, OB2 = OW2 + NH * NH,
 constexpr int NPAR = OB3 + NO;  // 5254
 constexpr int NNORM = 2 * NI + 2 * NO;
 static_assert(NNORM == 32, "the C ABI passes the normalisation as 32 floats: mx, sx, my, sy");
-constexpr int WAVES = 4, BLOCK = 64 * WAVES, GRID = 256, NWAVES = GRID * WAVES;
+constexpr int WAVES = 4, BLOCK = 64 * WAVES, GRID = 256;
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef short s4 __attribute__((ext_vector_type(4)));
@@ -347,21 +347,28 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_forward(const float *__restrict__
   }
 }
 
-// ---- training: forward, backward and per-wave gradient partials ------------
+// ---- training: forward, backward and per-block gradient partials -----------
 // Point i of the batch is sample (mul * (base + i) + add) mod n of the data
 // set, a permutation when mul is coprime to n.  loss = mean over the batch
-// and the NO outputs of (y - t)^2.  partial[w * (NPAR + 1) + k]: gradient
-// element k summed over the tiles of wave w; element NPAR is the loss.
+// and the NO outputs of (y - t)^2.  partial[b * (NPAR + 1) + k]: gradient
+// element k summed over the tiles of block b; element NPAR is the loss.  Each
+// wave sums its tiles in FP32; the block's four waves are added in wave order
+// in FP64 from LDS, so a step writes and reads back 256 rows of doubles (11 MB)
+// and not 1024 rows of floats, one per wave (21 MB).
+constexpr int TRAIN_TILE = 4 * 16 * NH + 2 * 16 * 16;  // bf16 values of one wave's transposes
+constexpr size_t TRAIN_LDS = WAVES * (NPAR + 1) * sizeof(float);
+static_assert(TRAIN_LDS >= WAVES * TRAIN_TILE * sizeof(__bf16), "the sums' LDS also holds the transposes");
 struct Perm {
   unsigned long long mul, add, base;
 };
 
 __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X, const float *__restrict__ T,
                                                      long long n, long long batch, Perm pm,
-                                                     const float *__restrict__ P, float *__restrict__ partial) {
-  __shared__ __bf16 sh[WAVES][4 * 16 * NH + 2 * 16 * 16];
+                                                     const float *__restrict__ P, double *__restrict__ partial) {
+  // the waves' transpose tiles, then (same memory) their gradient sums
+  extern __shared__ __align__(16) char train_lds[];
   const int l = threadIdx.x & 63, c = l & 15, q = l >> 4, wv = threadIdx.x >> 6;
-  __bf16 *Tdz2 = sh[wv], *Th1 = Tdz2 + 16 * NH, *Tdz1 = Th1 + 16 * NH, *Th2 = Tdz1 + 16 * NH;
+  __bf16 *Tdz2 = reinterpret_cast<__bf16 *>(train_lds) + wv * TRAIN_TILE, *Th1 = Tdz2 + 16 * NH, *Tdz1 = Th1 + 16 * NH, *Th2 = Tdz1 + 16 * NH;
   __bf16 *Tx = Th2 + 16 * NH, *Tdy = Tx + 256;
   FwdW W;
   BwdW B;
@@ -497,7 +504,9 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
   }
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) loss += __shfl_xor(loss, off);
-  float *out = partial + (size_t)wave * (NPAR + 1);
+  __syncthreads();  // every wave is done with its transposes
+  float *sums = reinterpret_cast<float *>(train_lds);
+  float *out = sums + wv * (NPAR + 1);
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -527,28 +536,60 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
       if (4 * q + r < NO) out[OB3 + 4 * q + r] = gb3[r];
   }
   if (l == 0) out[NPAR] = loss / ((float)batch * (float)NO);
+  __syncthreads();
+  double *prow = partial + (size_t)blockIdx.x * (NPAR + 1);
+  for (int k = threadIdx.x; k <= NPAR; k += BLOCK) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) s += (double)sums[w * (NPAR + 1) + k];
+    prow[k] = s;
+  }
 }
 
-// gradient = sum of the wave partials in wave order (deterministic)
-__global__ void k_mlp_reduce(const float *__restrict__ partial, int nwaves, float *__restrict__ grad) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > NPAR) return;
+// Gradient = the block partials added in a fixed order, then (adam) Adam
+// (Kingma & Ba 2015) on the FP32 master parameters of the same element.
+// A block takes 64 elements (512 contiguous bytes of a row) and splits the
+// rows over 16 waves, so a thread has at most 16 loads, in flight together.
+// One thread per element over all 1024 rows took 250 us a step (a chain of
+// loads on 21 blocks) and Adam's own launch 6 us; this takes 5 us for both.
+constexpr int RCOL = 64, RSEG = 16;
+struct AdamStep {
+  float *P, *m1, *m2, *losses;  // losses: this step's slot (may be null)
+  float lr, c1, c2;
+};
+__global__ __launch_bounds__(RCOL * RSEG) void k_mlp_reduce(const double *__restrict__ partial, int nblk,
+                                                            float *__restrict__ grad, int adam, AdamStep ad) {
+  __shared__ double sh[RSEG][RCOL];
+  const int col = threadIdx.x % RCOL, seg = threadIdx.x / RCOL;
+  const int k = blockIdx.x * RCOL + col;
+  constexpr int STEPS = GRID / RSEG;
+  double v[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) {
+    const int b = seg + RSEG * u;
+    v[u] = b < nblk && k <= NPAR ? partial[(size_t)b * (NPAR + 1) + k] : 0.0;
+  }
   double s = 0.0;
-  for (int w = 0; w < nwaves; ++w) s += (double)partial[(size_t)w * (NPAR + 1) + k];
-  grad[k] = (float)s;
-}
-
-// Adam (Kingma & Ba 2015) on the FP32 master parameters
-__global__ void k_mlp_adam(float *__restrict__ P, const float *__restrict__ g, float *__restrict__ m1,
-                           float *__restrict__ m2, float lr, float c1, float c2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= NPAR) return;
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) s += v[u];
+  sh[seg][col] = s;
+  __syncthreads();
+  if (seg != 0 || k > NPAR) return;
+  s = 0.0;
+#pragma unroll
+  for (int w = 0; w < RSEG; ++w) s += sh[w][col];
+  const float gk = (float)s;
+  grad[k] = gk;
+  if (!adam) return;
+  if (k == NPAR) {
+    if (ad.losses) *ad.losses = gk;
+    return;
+  }
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  const float gk = g[k];
-  const float a = b1 * m1[k] + (1.0f - b1) * gk, v = b2 * m2[k] + (1.0f - b2) * gk * gk;
-  m1[k] = a;
-  m2[k] = v;
-  P[k] -= lr * (a / c1) / (sqrtf(v / c2) + eps);
+  const float a = b1 * ad.m1[k] + (1.0f - b1) * gk, w2 = b2 * ad.m2[k] + (1.0f - b2) * gk * gk;
+  ad.m1[k] = a;
+  ad.m2[k] = w2;
+  ad.P[k] -= ad.lr * (a / ad.c1) / (sqrtf(w2 / ad.c2) + eps);
 }
 
 // features and targets of the data set: X[p] = normalised (grad9, delta),
@@ -631,7 +672,10 @@ uint64_t next_prime_above(uint64_t n) {
 }  // namespace
 
 struct ghx_mlp {
-  float *P = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr, *partial = nullptr;
+  float *P = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
+  double *partial = nullptr;  // GRID rows of NPAR + 1
+  float *losses = nullptr;    // per-step losses of a training call, loss_cap entries
+  long long loss_cap = 0;
   double *mom = nullptr;
   Norm norm;
   long long step = 0;
@@ -674,7 +718,7 @@ extern "C" int ghx_mlp_create(ghx_mlp **mp, unsigned long long seed) {
   fill(OW2, NH, NH);
   fill(OW3, NO, NH);
   hipError_t e = hipMalloc(&m->P, 4 * (NPAR + 1) * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&m->partial, (size_t)NWAVES * (NPAR + 1) * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc(&m->partial, (size_t)GRID * (NPAR + 1) * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&m->mom, (size_t)GRID * 30 * sizeof(double));
   if (e != hipSuccess) {
     if (m->P) (void)hipFree(m->P);
@@ -685,6 +729,7 @@ extern "C" int ghx_mlp_create(ghx_mlp **mp, unsigned long long seed) {
   m->m1 = m->P + (NPAR + 1);
   m->m2 = m->m1 + (NPAR + 1);
   m->grad = m->m2 + (NPAR + 1);
+  MHIP(hipFuncSetAttribute((const void *)k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TRAIN_LDS));
   MHIP(hipMemset(m->P, 0, 4 * (NPAR + 1) * sizeof(float)));
   MHIP(hipMemcpy(m->P, h.data(), NPAR * sizeof(float), hipMemcpyHostToDevice));
   *mp = m;
@@ -696,6 +741,7 @@ extern "C" int ghx_mlp_destroy(ghx_mlp *m) {
   (void)hipFree(m->P);
   (void)hipFree(m->partial);
   (void)hipFree(m->mom);
+  if (m->losses) (void)hipFree(m->losses);
   delete m;
   return GHX_OK;
 }
@@ -791,12 +837,18 @@ extern "C" int ghx_mlp_forward(ghx_mlp *m, long long n, const float *X, float *Y
   return GHX_OK;
 }
 
-// gradient of the batch loss into m->grad (element NPAR = loss)
-static int grad_batch(ghx_mlp *m, long long n, const float *X, const float *T, long long batch, Perm pm) {
-  hipLaunchKernelGGL(k_mlp_train, dim3(GRID), dim3(BLOCK), 0, m->stream, X, T, n, batch, pm, m->P, m->partial);
+// gradient of the batch loss into m->grad (element NPAR = loss), and with ad
+// the optimiser step of it
+static int grad_batch(ghx_mlp *m, long long n, const float *X, const float *T, long long batch, Perm pm,
+                      const AdamStep *ad = nullptr) {
+  // a wave per 16-point tile, at most one block per CU (the kernel holds one
+  // wave per SIMD); a small batch leaves no empty rows to add
+  const long long tiles = (batch + 15) / 16, need = (tiles + WAVES - 1) / WAVES;
+  const int nblk = (int)(need < GRID ? need : GRID);
+  hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(BLOCK), TRAIN_LDS, m->stream, X, T, n, batch, pm, m->P, m->partial);
   MHIP(hipGetLastError());
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPAR + 1 + 255) / 256), dim3(256), 0, m->stream, m->partial, NWAVES,
-                     m->grad);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((NPAR + RCOL) / RCOL), dim3(RCOL * RSEG), 0, m->stream, m->partial, nblk,
+                     m->grad, ad ? 1 : 0, ad ? *ad : AdamStep{});
   MHIP(hipGetLastError());
   return GHX_OK;
 }
@@ -824,23 +876,28 @@ extern "C" int ghx_mlp_train(ghx_mlp *m, long long n, const float *X, const floa
   // consecutive batch entries over the whole data set
   uint64_t mul = n > 2 ? next_prime_above((uint64_t)(0.6180339887498949 * (double)n)) : 1;
   if (mul >= (uint64_t)n) mul = 1;
-  std::vector<float> lh(steps > 0 ? steps : 1);
+  if (losses && m->loss_cap < steps) {
+    if (m->losses) MHIP(hipFree(m->losses));
+    m->losses = nullptr;
+    m->loss_cap = 0;
+    MHIP(hipMalloc(&m->losses, (size_t)steps * sizeof(float)));
+    m->loss_cap = steps;
+  }
   unsigned long long base = 0;
   const unsigned long long add = splitmix(s) % (uint64_t)n;
   for (int it = 0; it < steps; ++it) {
     Perm pm{mul, add, base};
-    int rc = grad_batch(m, n, X, T, batch, pm);
+    const float ns = (float)(m->step + 1), c1 = 1.0f - std::pow(0.9f, ns), c2 = 1.0f - std::pow(0.999f, ns);
+    const AdamStep ad{m->P, m->m1, m->m2, losses ? m->losses + it : nullptr, lr, c1, c2};
+    int rc = grad_batch(m, n, X, T, batch, pm, &ad);
     if (rc) return rc;
     ++m->step;
-    const float c1 = 1.0f - std::pow(0.9f, (float)m->step), c2 = 1.0f - std::pow(0.999f, (float)m->step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((NPAR + 255) / 256), dim3(256), 0, m->stream, m->P, m->grad, m->m1, m->m2,
-                       lr, c1, c2);
-    MHIP(hipGetLastError());
-    if (losses) MHIP(hipMemcpyAsync(&lh[it], m->grad + NPAR, sizeof(float), hipMemcpyDeviceToHost, m->stream));
     base = (base + (unsigned long long)batch) % (unsigned long long)n;
   }
+  // the losses stay on the device until the last step
+  if (losses && steps > 0)
+    MHIP(hipMemcpyAsync(losses, m->losses, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, m->stream));
   MHIP(hipStreamSynchronize(m->stream));
-  if (losses) std::memcpy(losses, lh.data(), (size_t)steps * sizeof(float));
   return GHX_OK;
 }
 
