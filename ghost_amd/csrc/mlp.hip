@@ -111,19 +111,67 @@ DEV void load_fwd(FwdW &W, const float *__restrict__ P, int l) {
   for (int r = 0; r < 4; ++r) W.b3[r] = 4 * q + r < NO ? P[OB3 + 4 * q + r] : 0.0f;
 }
 
-DEV void load_bwd(BwdW &W, const float *__restrict__ P, int l) {
+// The training kernel's operands (load_fwd's, and W2^T and W3^T for the
+// backward products) from an LDS copy of the parameters with padded rows: W1
+// 12, W2 and W3 68 floats, so that the 16 rows of an operand's 16-byte reads
+// and the columns of the transposed ones fall on distinct banks.
+constexpr int LW1 = 0, LB1 = LW1 + NH * 12, LW2 = LB1 + NH, LB2 = LW2 + NH * 68, LW3 = LB2 + NH, LB3 = LW3 + NO * 68;
+constexpr int LPAR = LB3 + 8;
+
+DEV void stage_params(float *S, const float *__restrict__ P) {
+  constexpr int N = (NPAR + BLOCK - 1) / BLOCK;
+  float v[N];  // all loads in flight before the first store
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int k = (int)threadIdx.x + u * BLOCK;
+    v[u] = P[k < NPAR ? k : 0];
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int k = (int)threadIdx.x + u * BLOCK;
+    if (k >= NPAR) break;
+    int d;
+    if (k < OB1) d = LW1 + (k / NI) * 12 + k % NI;
+    else if (k < OW2) d = LB1 + (k - OB1);
+    else if (k < OB2) d = LW2 + ((k - OW2) / NH) * 68 + (k - OW2) % NH;
+    else if (k < OW3) d = LB2 + (k - OB2);
+    else if (k < OB3) d = LW3 + ((k - OW3) / NH) * 68 + (k - OW3) % NH;
+    else d = LB3 + (k - OB3);
+    S[d] = v[u];
+  }
+}
+
+DEV bf8 pack2(f4 lo, f4 hi);
+DEV f4 lds4(const float *p) { return *reinterpret_cast<const f4 *>(p); }
+// k-slots (s, q, 0..7) of a row of 64
+DEV bf8 slots8(const float *row, int s, int q) { return pack2(lds4(row + 32 * s + 4 * q), lds4(row + 32 * s + 16 + 4 * q)); }
+
+DEV void load_train(FwdW &W, BwdW &B, const float *S, int l) {
   const int c = l & 15, q = l >> 4;
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     const int m = 16 * b + c;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const int j = 4 * q + r;
-      W.w3t[b][r] = (__bf16)(r < 4 && j < NO ? P[OW3 + j * NH + m] : 0.0f);
-      W.w2t[b][0][r] = (__bf16)P[OW2 + uslot(0, q, r) * NH + m];
-      W.w2t[b][1][r] = (__bf16)P[OW2 + uslot(1, q, r) * NH + m];
+      const int k = 8 * q + r, j = 4 * q + r;
+      W.w1[b][r] = (__bf16)(k < NI ? S[LW1 + m * 12 + k] : 0.0f);
+      B.w3t[b][r] = (__bf16)(r < 4 && j < NO ? S[LW3 + j * 68 + m] : 0.0f);
+      B.w2t[b][0][r] = (__bf16)S[LW2 + uslot(0, q, r) * 68 + m];
+      B.w2t[b][1][r] = (__bf16)S[LW2 + uslot(1, q, r) * 68 + m];
     }
+    W.w2[b][0] = slots8(S + LW2 + m * 68, 0, q);
+    W.w2[b][1] = slots8(S + LW2 + m * 68, 1, q);
+    W.b1[b] = lds4(S + LB1 + 16 * b + 4 * q);
+    W.b2[b] = lds4(S + LB2 + 16 * b + 4 * q);
   }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const bf8 w = slots8(S + LW3 + (c < NO ? c : 0) * 68, s, q);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) W.w3[s][r] = c < NO ? w[r] : (__bf16)0.0f;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) W.b3[r] = 4 * q + r < NO ? S[LB3 + 4 * q + r] : 0.0f;
 }
 
 DEV bf8 pack2(f4 lo, f4 hi) {
@@ -355,13 +403,33 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_forward(const float *__restrict__
 // wave sums its tiles in FP32; the block's four waves are added in wave order
 // in FP64 from LDS, so a step writes and reads back 256 rows of doubles (11 MB)
 // and not 1024 rows of floats, one per wave (21 MB).
+// Sum over a row of 16 lanes, in every lane: the butterfly lane ^ 1, ^ 2, then
+// the mirrors of half rows and rows (whose quads and halves hold one value by
+// then, so these equal ^ 4 and ^ 8).
+template <int CTRL> DEV float dpp_add(float x) {
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+DEV float row16_sum(float x) {
+  x = dpp_add<0xB1>(x);   // quad_perm 1,0,3,2
+  x = dpp_add<0x4E>(x);   // quad_perm 2,3,0,1
+  x = dpp_add<0x141>(x);  // row_half_mirror
+  return dpp_add<0x140>(x);  // row_mirror
+}
+
 constexpr int TRAIN_TILE = 4 * 16 * NH + 2 * 16 * 16;  // bf16 values of one wave's transposes
 constexpr size_t TRAIN_LDS = WAVES * (NPAR + 1) * sizeof(float);
+static_assert(TRAIN_LDS >= LPAR * sizeof(float), "and, before them, the parameters");
 static_assert(TRAIN_LDS >= WAVES * TRAIN_TILE * sizeof(__bf16), "the sums' LDS also holds the transposes");
 struct Perm {
   unsigned long long mul, add, base;
 };
 
+// The kernel holds one wave per SIMD (the weights of both passes and the
+// gradient accumulators fill the registers), so latency is what it is made of:
+// 30 us at a batch of 65536, 14 us of them before and after the tiles and
+// 3.5 us per tile and wave, most of it the activations' VALU work (43 us with
+// the weights gathered from global memory by each wave, the samples loaded
+// when their tile starts and the sums over lanes through the permute unit).
 __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X, const float *__restrict__ T,
                                                      long long n, long long batch, Perm pm,
                                                      const float *__restrict__ P, double *__restrict__ partial) {
@@ -372,8 +440,11 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
   __bf16 *Tx = Th2 + 16 * NH, *Tdy = Tx + 256;
   FwdW W;
   BwdW B;
-  load_fwd(W, P, l);
-  load_bwd(B, P, l);
+  float *par = reinterpret_cast<float *>(train_lds);
+  stage_params(par, P);
+  __syncthreads();
+  load_train(W, B, par, l);
+  __syncthreads();  // the copy's memory becomes the transposes
   f4 gW2[4][4], gW3[4], gW1[4];
   f4 gb1[4], gb2[4], gb3;
 #pragma unroll
@@ -390,16 +461,39 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
   const float dscale = 2.0f / ((float)batch * (float)NO);
   const long long wave = (long long)blockIdx.x * WAVES + wv, nw = (long long)gridDim.x * WAVES;
   const long long tiles = (batch + 15) / 16;
-  for (long long t = wave; t < tiles; t += nw) {
-    const long long i = t * 16 + c;
-    const bool ok = i < batch;
-    const long long p = ok ? (long long)((pm.mul * (unsigned long long)(pm.base + i) + pm.add) % (unsigned long long)n) : 0;
-    bf8 xb;
+  // The next tile's sample is loaded while this one is worked on: the rows are
+  // scattered over the data set, and a wave has no other wave on its SIMD to
+  // hide two round trips to memory per tile (features, then targets).  The
+  // sample index moves by a fixed step mod n from tile to tile, so the 64-bit
+  // remainder is taken once.
+  const unsigned long long un = (unsigned long long)n;
+  const unsigned long long hop = (pm.mul * ((16ull * (unsigned long long)nw) % un)) % un;
+  unsigned long long at = (pm.mul * (pm.base + (unsigned long long)(wave * 16 + c)) + pm.add) % un;
+  float xn[8];
+  f4 tn;
+  auto fetch = [&](long long t) {
+    const long long p = t * 16 + c < batch ? (long long)at : 0;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const int f = 8 * q + r;
-      xb[r] = (__bf16)(ok && f < NI ? X[p * NI + f] : 0.0f);
+      xn[r] = X[p * NI + (f < NI ? f : 0)];
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 4 * q + r;
+      tn[r] = T[p * NO + (j < NO ? j : 0)];
+    }
+    at += hop;
+    if (at >= un) at -= un;
+  };
+  if (wave < tiles) fetch(wave);
+  for (long long t = wave; t < tiles; t += nw) {
+    const bool ok = t * 16 + c < batch;
+    bf8 xb;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) xb[r] = (__bf16)(ok && 8 * q + r < NI ? xn[r] : 0.0f);
+    const f4 tg = tn;
+    if (t + nw < tiles) fetch(t + nw);
     Acts a;
     forward(W, xb, a);
     f4 dy;
@@ -407,7 +501,7 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
     for (int r = 0; r < 4; ++r) {
       const int j = 4 * q + r;
       const bool v = ok && j < NO;
-      const float e = v ? a.y[r] - T[p * NO + j] : 0.0f;
+      const float e = v ? a.y[r] - tg[r] : 0.0f;
       loss += e * e;
       dy[r] = dscale * e;
     }
@@ -489,21 +583,21 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  // reduce bias sums and the loss over the 16 points of each lane group
+  // reduce bias sums and the loss over the 16 points of each lane group (DPP
+  // moves inside rows of 16 lanes: 148 of them, where shuffles through the LDS
+  // permute unit cost several us)
 #pragma unroll
-  for (int off = 1; off < 16; off <<= 1) {
+  for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int r = 0; r < 4; ++r) {
+      gb1[b][r] = row16_sum(gb1[b][r]);
+      gb2[b][r] = row16_sum(gb2[b][r]);
+    }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        gb1[b][r] += __shfl_xor(gb1[b][r], off);
-        gb2[b][r] += __shfl_xor(gb2[b][r], off);
-      }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) gb3[r] += __shfl_xor(gb3[r], off);
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) loss += __shfl_xor(loss, off);
+  for (int r = 0; r < 4; ++r) gb3[r] = row16_sum(gb3[r]);
+  loss = row16_sum(loss);
+  loss += __shfl_xor(loss, 16);
+  loss += __shfl_xor(loss, 32);
   __syncthreads();  // every wave is done with its transposes
   float *sums = reinterpret_cast<float *>(train_lds);
   float *out = sums + wv * (NPAR + 1);
