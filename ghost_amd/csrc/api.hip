@@ -681,26 +681,12 @@ static int curl3(ghx_grid *g, const void *a, const void *b, const void *c, cplx 
 
 extern "C" int ghx_energy(ghx_grid *g, const void *a, const void *b, const void *c, int kin, double *out) {
   ARGCHK(g && a && b && c && out && kin >= 0 && kin <= 2, "bad energy arguments");
-  if (kin == 1) return reduce(g, 0, a, b, c, nullptr, nullptr, nullptr, out);
-  int rc = grid_ctmp(g, 3);
-  if (rc) return rc;
-  cplx *t = g->ctmp;
-  if (kin == 0) {
-    if ((rc = curl3(g, a, b, c, t))) return rc;
-  } else {
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(a), t));
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(b), t + g->nc));
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(c), t + 2 * g->nc));
-  }
-  return reduce(g, 0, t, t + g->nc, t + 2 * g->nc, nullptr, nullptr, nullptr, out);
+  return reduce(g, kin == 1 ? 0 : (kin == 0 ? 9 : 10), a, b, c, nullptr, nullptr, nullptr, out);
 }
 
 extern "C" int ghx_helicity(ghx_grid *g, const void *a, const void *b, const void *c, double *out) {
   ARGCHK(g && a && b && c && out, "bad helicity arguments");
-  int rc = grid_ctmp(g, 3);
-  if (rc) return rc;
-  if ((rc = curl3(g, a, b, c, g->ctmp))) return rc;
-  return reduce(g, 1, a, b, c, g->ctmp, g->ctmp + g->nc, g->ctmp + 2 * g->nc, out);
+  return reduce(g, 11, a, b, c, nullptr, nullptr, nullptr, out);
 }
 
 extern "C" int ghx_cross(ghx_grid *g, const void *a, const void *b, const void *c, const void *d, const void *e,
@@ -714,55 +700,73 @@ extern "C" int ghx_divergence(ghx_grid *g, const void *a, const void *b, const v
   return reduce(g, 3, a, b, c, nullptr, nullptr, nullptr, out);
 }
 
+// The curl (kin = 0) is formed inside the z inverse, and the x inverse keeps
+// only the largest norm; row lengths without a two-for-one x kernel write the
+// real fields and reduce those.
 extern "C" int ghx_maxabs(ghx_grid *g, const void *a, const void *b, const void *c, int kin, double *out) {
   ARGCHK(g && a && b && c && out && kin >= 0 && kin <= 2, "bad maxabs arguments");
-  int rc = grid_ctmp(g, 3);
-  if (!rc) rc = grid_rtmp(g, 3);
-  if (!rc) rc = grid_work(g, ghx::reduce_work_doubles());
+  ghx_plan *p = &g->plan;
+  int rc = plan_scratch(p, 6);
+  if (!rc && kin == 1) rc = grid_ctmp(g, 3);
+  if (!rc) rc = grid_work(g, ghx::kNormBlocks + 1 > (int)ghx::reduce_work_doubles() ? ghx::kNormBlocks + 1
+                                                                                    : ghx::reduce_work_doubles());
   if (rc) return rc;
-  cplx *t = g->ctmp;
-  const void *src[3];
-  if (kin == 0) {
-    if ((rc = curl3(g, a, b, c, t))) return rc;
-    src[0] = t; src[1] = t + g->nc; src[2] = t + 2 * g->nc;
-  } else if (kin == 1) {
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(a), t));
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(b), t + g->nc));
-    HIPCHK(ghx::op_laplak3(g->gk, g->stream, C_(c), t + 2 * g->nc));
-    src[0] = t; src[1] = t + g->nc; src[2] = t + 2 * g->nc;
-  } else {
-    src[0] = a; src[1] = b; src[2] = c;
+  FieldSet in, q, pp;
+  in.p[0] = M_(a); in.p[1] = M_(b); in.p[2] = M_(c);
+  if (kin == 1)
+    for (int k = 0; k < 3; ++k) {
+      HIPCHK(ghx::op_laplak3(g->gk, g->stream, in.p[k], g->ctmp + k * g->nc));
+      in.p[k] = g->ctmp + k * g->nc;
+    }
+  const size_t slot = ghx::slot_points(g->gk);
+  for (int k = 0; k < 3; ++k) {
+    q.p[k] = p->q + k * slot;
+    pp.p[k] = p->q + (3 + k) * slot;
   }
-  double *r[3] = {g->rtmp, g->rtmp + g->nr, g->rtmp + 2 * g->nr};
-  if ((rc = do_c2r(&g->plan, 3, src, r))) return rc;
+  const double sc = (double)g->nc * sizeof(cplx), sr = (double)g->nr * sizeof(double);
+  timer_begin(p);
+  PROF(P_ZINV, 6 * sc, p->ctx.stream, ghx::zinv(p->ctx, kin == 0 ? 7 : 0, 3, in, q));
+  PROF(P_YINV, 6 * sc, p->ctx.stream, ghx::yinv(p->ctx, 3, q, pp));
   double m = 0;
-  HIPCHK(ghx::op_maxnorm(g->gk, g->stream, r[0], r[1], r[2], g->work, &m));
+  int nblk = 0;
+  const hipError_t e = ghx::xnormmax(p->ctx, pp, g->work, &nblk);
+  if (e == hipErrorNotSupported) {
+    if ((rc = grid_rtmp(g, 3))) return rc;
+    double *r[3] = {g->rtmp, g->rtmp + g->nr, g->rtmp + 2 * g->nr};
+    PROF(P_XINV, 3 * (sr + sc), p->ctx.stream, ghx::xinv(p->ctx, 3, pp, r));
+    timer_end(p);
+    HIPCHK(ghx::op_maxnorm(g->gk, g->stream, r[0], r[1], r[2], g->work, &m));
+  } else {
+    HIPCHK(e);
+    timer_end(p);
+    HIPCHK(ghx::op_max_sqrt(g->stream, g->work, nblk, &m));
+  }
   *out = m / ((double)g->gk.nx * (double)g->gk.ny * (double)g->gk.nz);
   return GHX_OK;
 }
 
+// kin = 0 and the helicity form the curl at each mode; the energy and the
+// helicity of one call come from one read of the fields (while both rows of
+// bins fit the LDS that one row was always given).
 extern "C" int ghx_spectrumc(ghx_grid *g, const void *a, const void *b, const void *c, int kin, int hel, double *Ek,
                              double *Hk) {
   ARGCHK(g && a && b && c && kin >= 0 && kin <= 2 && (hel == 0 || hel == 1), "bad spectrumc arguments");
   const int nb = g->nmax / 2 + 1;
-  int rc = grid_work(g, ghx::spectrum_work_doubles(g->gk, nb));
+  int rc = grid_work(g, ghx::spectrum_work_doubles(g->gk, 2 * nb));
   if (rc) return rc;
-  cplx *t = nullptr;
-  if (kin == 0 || hel == 1) {
-    if ((rc = grid_ctmp(g, 3))) return rc;
-    t = g->ctmp;
-    if ((rc = curl3(g, a, b, c, t))) return rc;
+  auto bins = [&](int kind, double *out) {
+    return ghx::op_spectrum(g->gk, g->stream, kind, g->Dkk, nb, C_(a), C_(b), C_(c), nullptr, nullptr, nullptr, g->work,
+                            out);
+  };
+  if (kin == 1 && Ek && hel == 1 && Hk && 2 * (size_t)nb * sizeof(double) <= 48 * 1024) {
+    std::vector<double> both(2 * (size_t)nb);
+    HIPCHK(bins(7, both.data()));
+    std::memcpy(Ek, both.data(), nb * sizeof(double));
+    std::memcpy(Hk, both.data() + nb, nb * sizeof(double));
+    return GHX_OK;
   }
-  if (kin <= 1 && Ek) {
-    if (kin == 1)
-      HIPCHK(ghx::op_spectrum(g->gk, g->stream, 0, g->Dkk, nb, C_(a), C_(b), C_(c), nullptr, nullptr, nullptr, g->work, Ek));
-    else
-      HIPCHK(ghx::op_spectrum(g->gk, g->stream, 0, g->Dkk, nb, t, t + g->nc, t + 2 * g->nc, nullptr, nullptr, nullptr,
-                              g->work, Ek));
-  }
-  if (hel == 1 && Hk)
-    HIPCHK(ghx::op_spectrum(g->gk, g->stream, 1, g->Dkk, nb, C_(a), C_(b), C_(c), t, t + g->nc, t + 2 * g->nc,
-                            g->work, Hk));
+  if (kin <= 1 && Ek) HIPCHK(bins(kin == 1 ? 0 : 5, Ek));
+  if (hel == 1 && Hk) HIPCHK(bins(8, Hk));
   return GHX_OK;
 }
 
@@ -836,12 +840,8 @@ extern "C" int ghx_heltrans(ghx_grid *g, const void *a, const void *b, const voi
   ARGCHK(g && a && b && c && d && e && f && Hk, "bad heltrans arguments");
   const int nb = g->nmax / 2 + 1;
   int rc = grid_work(g, ghx::spectrum_work_doubles(g->gk, nb));
-  if (!rc) rc = grid_ctmp(g, 3);
-  if (!rc) rc = curl3(g, a, b, c, g->ctmp);
   if (rc) return rc;
-  const cplx *t = g->ctmp;
-  HIPCHK(ghx::op_spectrum(g->gk, g->stream, 1, g->Dkk, nb, t, t + g->nc, t + 2 * g->nc, C_(d), C_(e), C_(f), g->work,
-                          Hk));
+  HIPCHK(ghx::op_spectrum(g->gk, g->stream, 6, g->Dkk, nb, C_(a), C_(b), C_(c), C_(d), C_(e), C_(f), g->work, Hk));
   return GHX_OK;
 }
 
@@ -852,12 +852,9 @@ extern "C" int ghx_crosspecc(ghx_grid *g, const void *a, const void *b, const vo
   ARGCHK(g && a && b && c && d && e && f && Ck, "bad crosspecc arguments");
   const int nb = g->nmax / 2 + 1;
   int rc = grid_work(g, ghx::spectrum_work_doubles(g->gk, nb));
-  if (!rc) rc = grid_ctmp(g, 3);
-  if (!rc) rc = curl3(g, d, e, f, g->ctmp);
   if (rc) return rc;
-  const cplx *t = g->ctmp;
-  HIPCHK(ghx::op_spectrum(g->gk, g->stream, 1, g->Dkk, nb, C_(a), C_(b), C_(c), t, t + g->nc, t + 2 * g->nc, g->work,
-                          Ck, shift + 0.501));
+  HIPCHK(ghx::op_spectrum(g->gk, g->stream, 6, g->Dkk, nb, C_(d), C_(e), C_(f), C_(a), C_(b), C_(c), g->work, Ck,
+                          shift + 0.501));
   return GHX_OK;
 }
 
@@ -1187,12 +1184,15 @@ extern "C" int ghx_hdcheck(ghx_grid *g, const void *a, const void *b, const void
                            const void *f, int hel, int chk, double *out) {
   ARGCHK(g && a && b && c && d && e && f && out, "bad hdcheck arguments");
   for (int q = 0; q < 5; ++q) out[q] = 0.0;
-  int rc = GHX_OK;
-  if (chk == 1 && (rc = ghx_divergence(g, a, b, c, &out[4]))) return rc;
-  if ((rc = ghx_energy(g, a, b, c, 1, &out[0]))) return rc;
-  if ((rc = ghx_energy(g, a, b, c, 0, &out[1]))) return rc;
-  if (hel == 1 && (rc = ghx_helicity(g, a, b, c, &out[3]))) return rc;
-  return ghx_cross(g, a, b, c, d, e, f, 1, &out[2]);
+  int rc = grid_work(g, ghx::reduce_work_doubles());
+  if (rc) return rc;
+  const cplx *v[3] = {C_(a), C_(b), C_(c)}, *fo[3] = {C_(d), C_(e), C_(f)};
+  double sum[5];
+  HIPCHK(ghx::op_hdcheck(g->gk, g->stream, v, fo, g->work, sum));
+  for (int q = 0; q < 3; ++q) out[q] = sum[q];
+  if (hel == 1) out[3] = sum[3];
+  if (chk == 1) out[4] = sum[4];
+  return GHX_OK;
 }
 
 // mhdcheck (pseudospec3D_mhd.f90:339-547) without its file output: out =
@@ -1212,9 +1212,8 @@ extern "C" int ghx_mhdcheck(ghx_grid *g, const void *a, const void *b, const voi
   double engk = 0, ens = 0, engm = 0, cur = 0;
   if ((rc = ghx_energy(g, a, b, c, 1, &engk))) return rc;
   if ((rc = ghx_energy(g, a, b, c, 0, &ens))) return rc;
-  // the magnetic field curl A lives past the three temporaries energy uses
-  if ((rc = grid_ctmp(g, 6))) return rc;
-  cplx *bm = g->ctmp + 3 * g->nc;
+  if ((rc = grid_ctmp(g, 3))) return rc;
+  cplx *bm = g->ctmp;
   if ((rc = curl3(g, ma, mb, mc, bm))) return rc;
   const cplx *b0 = bm, *b1 = bm + g->nc, *b2 = bm + 2 * g->nc;
   if ((rc = ghx_energy(g, b0, b1, b2, 1, &engm))) return rc;

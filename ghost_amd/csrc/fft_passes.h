@@ -81,6 +81,7 @@ inline size_t slot_points(const GridK &g) { return (size_t)g.nz * g.ny * p_row(g
 // (v, curl v, b = curl A, j = curl b).  mode 4 (advect3): 4 in (a, b, c, d)
 // -> 6 out (a, b, c, grad d).  mode 5 (Boussinesq): 4 in (v, th) -> 9 out
 // (v, curl v, grad th).
+// mode 7: 3 in (v) -> 3 out (curl v).
 // prune=1: the input is dealiased (zero outside tiny <= kn2 <= kmax): only
 // lines that carry kept modes are read and written (every pass below takes
 // the same flag; see the kernels for exactly what each one skips).
@@ -95,6 +96,12 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out, int prune = 0);
 // X^-1 of three P fields written interleaved: out[(row * nx + x) * 3 + f].
 hipError_t xinv3i(const FFTCtx &c, const FieldSet &in, double *out, int prune = 0);
+// X^-1 of three P fields reduced to the largest of the points' squared norms,
+// one partial maximum per block of the launch into part[0..*nblk), *nblk at
+// most kNormBlocks; hipErrorNotSupported for row lengths without a
+// two-for-one kernel.
+constexpr int kNormBlocks = 4096;
+hipError_t xnormmax(const FFTCtx &c, const FieldSet &in, double *part, int *nblk);
 // X forward: real rows -> P.
 hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &out);
 // Fused X^-1 . cross product . X on P rows: in.p[0..2] = A, in.p[3..5] = B

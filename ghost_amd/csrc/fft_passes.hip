@@ -525,6 +525,26 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
         }
         zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, tw, out.p[3 * c + dir], g, i, j0, lmask);
       }
+  } else if constexpr (MODE == 7) {
+    // v -> curl v, rotor3's components formed at each mode
+    const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j, g.ny, g.dky);
+    cplx u[3][E];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int m = 0; m < E; ++m) u[c][m] = load(in.p[c], t + T * m);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      cplx v[E];
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        const double kz = wavenum(t + T * m, g.nz, g.dkz);
+        v[m] = c == 0 ? c_sub(c_ik(ky, u[2][m]), c_ik(kz, u[1][m]))
+               : c == 1 ? c_sub(c_ik(kz, u[0][m]), c_ik(kx, u[2][m]))
+                        : c_sub(c_ik(kx, u[1][m]), c_ik(ky, u[0][m]));
+      }
+      zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, tw, out.p[c], g, i, j0, lmask);
+    }
   } else {
     // MODE 4: (a, b, c, d) -> (a, b, c, grad d).  MODE 5: (v, th) -> (v, curl v, grad th).
     using F = LineFFT<N, +1, Cfg>;
@@ -1438,6 +1458,56 @@ __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out,
   }
 }
 
+// X^-1 of three fields, kept only as the largest squared norm of the points a
+// block sees (maxabs): the three real fields are neither written nor read back.
+// Rows in a grid-stride loop, the next row's first pair loaded ahead.  At 256^3
+// 125 us for what took 141 (x inverse) and 101 us (norms of the real fields).
+template <int NX>
+__global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part, GridK g, int nxp,
+                                                      const cplx *__restrict__ twt, int kxlim) {
+  using Cfg = FFTCfg<NX>;
+  using FI = LineFFT<NX, +1>;
+  constexpr int T = Cfg::T, E = Cfg::E;
+  static_assert(T <= 64, "one row per wavefront or less");
+  extern __shared__ cplx lds[];
+  __shared__ double best[kRowBound / 64];
+  const int rpb = blockDim.x / T;
+  const int lt = threadIdx.x / T, t = threadIdx.x % T;
+  const long nrows = (long)g.nz * g.ny, hop = (long)gridDim.x * rpb;
+  cplx *buf = lds + lt * lds_line_stride(NX);
+  TwCache<NX> tw;
+  tw.load(twt, t);
+  double big = 0.0;
+  long r = (long)blockIdx.x * rpb + lt;
+  if (r < nrows) {  // whole lines only: wave-level syncs inside
+    cplx a[E], b[E], z0[E], z1[E];
+    xpair_load<NX, E, T>(a, b, in.p[0] + (size_t)r * nxp, in.p[1] + (size_t)r * nxp, t, kxlim);
+    for (; r < nrows; r += hop) {
+      const size_t off = (size_t)r * nxp;
+      xpair_make<NX, E, T>(z0, a, b, t, kxlim);
+      xpair_load<NX, E, T>(a, b, in.p[2] + off, in.p[2] + off, t, kxlim);
+      FI::run(z0, buf, t, tw);
+      xpair_make<NX, E, T>(z1, a, b, t, kxlim, false);
+      if (r + hop < nrows) {
+        const size_t no = (size_t)(r + hop) * nxp;
+        xpair_load<NX, E, T>(a, b, in.p[0] + no, in.p[1] + no, t, kxlim);
+      }
+      FI::run(z1, buf, t, tw);
+#pragma unroll
+      for (int m = 0; m < E; ++m)
+        big = fmax(big, z0[m].x * z0[m].x + z0[m].y * z0[m].y + z1[m].x * z1[m].x);
+    }
+  }
+  // (kRowBound lanes are whole waves; a narrower block leaves its missing lanes out)
+  for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+  if (threadIdx.x % 64 == 0) best[threadIdx.x / 64] = big;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < (int)(blockDim.x + 63) / 64; ++q) big = fmax(big, best[q]);
+    part[blockIdx.x] = big;
+  }
+}
+
 // X of nf real rows, two rows per transform.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, int nf, GridK g, int nxp,
@@ -1763,7 +1833,7 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, mode == 0 ? 8 : 4), max_lds());              \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, mode == 0 || mode == 7 ? 8 : 4), max_lds()); \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
     if (mode == 0) {                                                                        \
@@ -1784,6 +1854,9 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     } else if (mode == 6) {                                                                 \
       allow_lds(k_zinv<n_, 6>, lds);                                                        \
       GHX_LAUNCH_CHECK((k_zinv<n_, 6>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 6>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+    } else if (mode == 7) {                                                                 \
+      allow_lds(k_zinv<n_, 7>, lds);                                                        \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 7>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 7>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
     } else {                                                                                \
       allow_lds(k_zinv<n_, 3>, lds);                                                        \
       GHX_LAUNCH_CHECK((k_zinv<n_, 3>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 3>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
@@ -2109,6 +2182,29 @@ hipError_t xinv3i(const FFTCtx &c, const FieldSet &in, double *out, int prune) {
     return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+hipError_t xnormmax(const FFTCtx &c, const FieldSet &in, double *part, int *nblk) {
+  const GridK &g = c.gk;
+  if (g.nx % 2) return hipErrorInvalidValue;
+  if (!use_x2(g.nx)) return hipErrorNotSupported;
+  const long nrows = (long)g.nz * g.ny;
+  switch (g.nx) {
+#define GHX_CASE(n_)                                                                        \
+  case n_: {                                                                                \
+    constexpr int T = FFTCfg<n_>::T;                                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds() - kRowBound * sizeof(double)); \
+    const long nb = (nrows + s.lines - 1) / s.lines;                                        \
+    *nblk = (int)(nb < kNormBlocks ? nb : kNormBlocks);                                     \
+    GHX_LAUNCH_CHECK((k_xnorm2<n_>), s, kRowBound, T, false);                               \
+    hipLaunchKernelGGL((k_xnorm2<n_>), dim3(*nblk), dim3(s.block), s.lds, c.stream, in, part, g, p_row(g), c.tw_x, g.nxh); \
+    return hipGetLastError();                                                               \
+  }
+    GHX_X2_SIZES(GHX_CASE)
+#undef GHX_CASE
+  default:
+    return hipErrorNotSupported;
+  }
 }
 
 hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &out) {

@@ -47,14 +47,24 @@ hipError_t op_tg_real(const GridK &g, hipStream_t st, double *r1, double *r2, in
 
 // Reductions.  kind: 0 = |a|^2+|b|^2+|c|^2, 1 = Re(a d* + b e* + c f*),
 // 2 = that * kk2, 3 = |i kx a + i ky b + i kz c|^2 (divergence),
-// 4 = number of modes outside tiny <= kn2 <= kmax where (a,b,c) is non-zero.
+// 4 = number of modes outside tiny <= kn2 <= kmax where (a,b,c) is non-zero,
+// 5 = the same outside kn2 <= kmax; scalars 6 = |a|^2, 7 = kk2 |a|^2,
+// 8 = Re(a d*); of v = (a,b,c): 9 = |curl v|^2, 10 = |lap v|^2,
+// 11 = Re(v . conj(curl v)).
 // Each mode is weighted 1 on the kx=0 plane, 2 elsewhere, times 1/N^6.
 // `work` must hold reduce_work_doubles() doubles.  Result to *out (host).
 size_t reduce_work_doubles();
 hipError_t op_reduce(const GridK &g, hipStream_t st, int kind, const cplx *a, const cplx *b, const cplx *c,
                      const cplx *d, const cplx *e, const cplx *f, double *work, double *out);
+// hdcheck's sums of v and the force f: out[5] host = <v^2>, <omega^2>, <v.f>,
+// helicity, <(div v)^2>; work as for op_reduce.
+hipError_t op_hdcheck(const GridK &g, hipStream_t st, const cplx *const *v, const cplx *const *f, double *work,
+                      double *out);
 // spectrumc binning (pseudospec3D_hd.f90:1190-1415); kind 0: energy of (a,b,c),
-// kind 1: helicity Re(a d* + b e* + c f*).  nb bins; out[nb] host.
+// kind 1: Re(a d* + b e* + c f*), 2: that times kk2, 3: |a|^2, 4: Re(a d*),
+// 5: energy of curl (a,b,c), 6: curl (a,b,c) against (d,e,f), 7: energy and
+// helicity of (a,b,c) (out[2 nb], work for 2 nb bins), 8: helicity of (a,b,c).
+// nb bins; out[nb] host.
 size_t spectrum_work_doubles(const GridK &g, int nb);
 hipError_t op_spectrum(const GridK &g, hipStream_t st, int kind, double dkk, int nb, const cplx *a, const cplx *b,
                        const cplx *c, const cplx *d, const cplx *e, const cplx *f, double *work, double *out, double off = (double)0.501f);
@@ -79,6 +89,8 @@ hipError_t op_zplane(const GridK &g, hipStream_t st, int kind, const double *r1,
                      const double *r4, double fo, double bv, double scale, double *work, double *out);
 hipError_t op_spectr1d(const GridK &g, hipStream_t st, int dir, double ldir, int nb, const cplx *a, double *work,
                        double *out);
+// the largest of n partial maxima (work[0..n)) and its square root to *out (host)
+hipError_t op_max_sqrt(hipStream_t st, double *work, int n, double *out);
 // max over real points of sqrt(r1^2+r2^2+r3^2) (maxabs)
 hipError_t op_maxnorm(const GridK &g, hipStream_t st, const double *r1, const double *r2, const double *r3,
                       double *work, double *out);

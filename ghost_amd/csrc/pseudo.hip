@@ -385,84 +385,199 @@ GHX_DEV double block_sum(double v) {
 GHX_DEV double cabs2(cplx a) { return a.x * a.x + a.y * a.y; }
 GHX_DEV double cre_dot(cplx a, cplx b) { return a.x * b.x + a.y * b.y; }  // Re(a conj(b))
 
-__global__ void k_reduce(GridK g, int kind, const cplx *a, const cplx *b, const cplx *c, const cplx *d,
-                         const cplx *e, const cplx *f, double *part) {
+// Every mode (i, j, k) of the grid for one block: threads along a kz line
+// (kl = nz rounded up to a power of two, at most the block), kBlock / kl lines
+// at a time, lines in a grid-stride loop.  i and j cost one 32-bit division
+// per line instead of two 64-bit ones per mode, which had these kernels at
+// 3.8 TB/s; neighbouring lanes still read neighbouring modes.
+struct LineWalk {
+  int kl, sh, lb, nl;
+};
+__host__ __device__ inline LineWalk line_walk(const GridK &g) {
+  LineWalk w;
+  w.sh = 0;
+  while ((1 << w.sh) < g.nz && (1 << w.sh) < kBlock) ++w.sh;
+  w.kl = 1 << w.sh;
+  w.lb = kBlock / w.kl;
+  w.nl = g.nxh * g.ny;
+  return w;
+}
+template <typename F> GHX_DEV void for_modes(const GridK &g, F f) {
+  const LineWalk w = line_walk(g);
+  const int k0 = threadIdx.x & (w.kl - 1), sub = threadIdx.x >> w.sh;
+  for (int l = (int)blockIdx.x * w.lb + sub; l < w.nl; l += (int)gridDim.x * w.lb) {
+    Idx q;
+    q.i = l / g.ny;
+    q.j = l - q.i * g.ny;
+    for (q.k = k0; q.k < g.nz; q.k += w.kl) f(q, (size_t)l * g.nz + q.k);
+  }
+}
+
+// the curl of (a, b, c) at one mode, as rotor3 forms its components
+struct Vec3 {
+  cplx x, y, z;
+};
+GHX_DEV Vec3 curl_at(const GridK &g, const Idx &q, cplx a, cplx b, cplx c) {
+  const double kx = wavenum(q.i, g.nx, g.dkx), ky = wavenum(q.j, g.ny, g.dky), kz = wavenum(q.k, g.nz, g.dkz);
+  return Vec3{c_sub(c_ik(ky, c), c_ik(kz, b)), c_sub(c_ik(kz, a), c_ik(kx, c)), c_sub(c_ik(kx, b), c_ik(ky, a))};
+}
+GHX_DEV double div2_at(const GridK &g, const Idx &q, cplx a, cplx b, cplx c) {
+  const double kx = wavenum(q.i, g.nx, g.dkx), ky = wavenum(q.j, g.ny, g.dky), kz = wavenum(q.k, g.nz, g.dkz);
+  return cabs2(c_add(c_add(c_ik(kx, a), c_ik(ky, b)), c_ik(kz, c)));
+}
+
+// The kinds of op_reduce (pseudo.h).  Curls and Laplacians are formed at each
+// mode from the three components read anyway: a pass over three fields, where
+// three temporaries written and read back cost nine more.
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_reduce(GridK g, const cplx *a, const cplx *b, const cplx *c,
+                                                   const cplx *d, const cplx *e, const cplx *f, double *part) {
   double acc = 0.0;
   const double tmp = g.inv_n6;
-  GRID_STRIDE(m, ncplx(g)) {
-    Idx q = decompose(m, g);
+  for_modes(g, [&](const Idx &q, size_t m) {
     const double w = q.i == 0 ? 1.0 : 2.0;
     double s;
-    if (kind == 0) {
+    if constexpr (KIND == 0) {
       s = cabs2(a[m]) + cabs2(b[m]) + cabs2(c[m]);
-    } else if (kind == 1 || kind == 2) {
+    } else if constexpr (KIND == 1 || KIND == 2) {
       s = cre_dot(a[m], d[m]) + cre_dot(b[m], e[m]) + cre_dot(c[m], f[m]);
-      if (kind == 2) s *= kk2_at(g, q);
-    } else if (kind == 3) {
-      double kx = wavenum(q.i, g.nx, g.dkx), ky = wavenum(q.j, g.ny, g.dky), kz = wavenum(q.k, g.nz, g.dkz);
-      cplx dv = c_add(c_add(c_ik(kx, a[m]), c_ik(ky, b[m])), c_ik(kz, c[m]));
-      s = cabs2(dv);
-    } else if (kind >= 6) {
+      if constexpr (KIND == 2) s *= kk2_at(g, q);
+    } else if constexpr (KIND == 3) {
+      s = div2_at(g, q, a[m], b[m], c[m]);
+    } else if constexpr (KIND == 9) {
+      const Vec3 o = curl_at(g, q, a[m], b[m], c[m]);
+      s = cabs2(o.x) + cabs2(o.y) + cabs2(o.z);
+    } else if constexpr (KIND == 10) {
+      const double k2 = -kk2_at(g, q);
+      s = cabs2(c_scale(a[m], k2)) + cabs2(c_scale(b[m], k2)) + cabs2(c_scale(c[m], k2));
+    } else if constexpr (KIND == 11) {
+      const cplx A = a[m], B = b[m], Cc = c[m];
+      const Vec3 o = curl_at(g, q, A, B, Cc);
+      s = cre_dot(A, o.x) + cre_dot(B, o.y) + cre_dot(Cc, o.z);
+    } else if constexpr (KIND >= 6) {
       // scalars (pseudospec3D_phd.f90): 6 variance |a|^2, 7 kk2 |a|^2, 8 product Re(a d*)
-      s = kind == 8 ? cre_dot(a[m], d[m]) : cabs2(a[m]);
-      if (kind == 7) s *= kk2_at(g, q);
+      s = KIND == 8 ? cre_dot(a[m], d[m]) : cabs2(a[m]);
+      if constexpr (KIND == 7) s *= kk2_at(g, q);
     } else {
       // kind 4: count of modes outside tiny <= kn2 <= kmax holding a non-zero
       // value; kind 5: the same outside kn2 <= kmax only (a scalar whose mean,
       // kn2 < tiny, is carried)
       const double kn2 = kn2_of(g, q.i, q.j, q.k);
+      const bool kept = KIND == 4 ? (kn2 <= g.kmax && kn2 >= g.tiny) : kn2 <= g.kmax;
       const cplx A = a[m], B = b[m], Cc = c[m];
       const bool nz = A.x != 0.0 || A.y != 0.0 || B.x != 0.0 || B.y != 0.0 || Cc.x != 0.0 || Cc.y != 0.0;
-      const bool kept = kind == 4 ? (kn2 <= g.kmax && kn2 >= g.tiny) : kn2 <= g.kmax;
       acc += (!kept && nz) ? 1.0 : 0.0;
-      continue;
+      return;
     }
     acc += w * s * tmp;
-  }
+  });
   double r = block_sum(acc);
   if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
+// hdcheck's five sums (pseudospec3D_hd.f90:984-1105) in one pass over v =
+// (a, b, c) and the force (d, e, f): part[q * gridDim.x + block] for q =
+// <v^2>, <omega^2>, <v.f>, the helicity and <(div v)^2>.  Bound by the six
+// fields it reads (6 TB/s, 136 us at 256^3); the sums one by one read them
+// sixteen times and wrote the vorticity twice.
+__global__ __launch_bounds__(kBlock) void k_hdcheck(GridK g, const cplx *a, const cplx *b, const cplx *c,
+                                                    const cplx *d, const cplx *e, const cplx *f, double *part) {
+  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const double tmp = g.inv_n6;
+  for_modes(g, [&](const Idx &q, size_t m) {
+    const double w = (q.i == 0 ? 1.0 : 2.0) * tmp;
+    const cplx A = a[m], B = b[m], Cc = c[m];
+    const Vec3 o = curl_at(g, q, A, B, Cc);
+    acc[0] += w * (cabs2(A) + cabs2(B) + cabs2(Cc));
+    acc[1] += w * (cabs2(o.x) + cabs2(o.y) + cabs2(o.z));
+    acc[2] += w * (cre_dot(A, d[m]) + cre_dot(B, e[m]) + cre_dot(Cc, f[m]));
+    acc[3] += w * (cre_dot(A, o.x) + cre_dot(B, o.y) + cre_dot(Cc, o.z));
+    acc[4] += w * div2_at(g, q, A, B, Cc);
+  });
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+    const double r = block_sum(acc[q]);
+    if (threadIdx.x == 0) part[(size_t)q * gridDim.x + blockIdx.x] = r;
+  }
+}
+
+// row blockIdx.x of n partials each
 __global__ void k_sum_partials(const double *part, int n, double *out) {
   double acc = 0.0;
-  for (int q = threadIdx.x; q < n; q += blockDim.x) acc += part[q];
+  for (int q = threadIdx.x; q < n; q += blockDim.x) acc += part[(size_t)blockIdx.x * n + q];
   double r = block_sum(acc);
-  if (threadIdx.x == 0) *out = r;
+  if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
 // spectrumc, entrans, heltrans, crosspecc: shell kmn = int(sqrt(kk2)/Dkk +
 // off), bins 1..nb; off is .501 as a single-precision literal, except in
-// crosspecc (shift + .501 in working precision).  kind 0: |a|^2+|b|^2+|c|^2;
-// 1: Re(a d*) + Re(b e*) + Re(c f*); 2: kind 1 times kk2 (entrans, kin = 0).
-__global__ void k_spectrum(GridK g, int kind, double dkk, int nb, double off, const cplx *a, const cplx *b,
-                           const cplx *c, const cplx *d, const cplx *e, const cplx *f, double *part) {
+// crosspecc (shift + .501 in working precision).  The kinds of op_spectrum
+// (pseudo.h).  kind 7 fills two rows of nb bins, the energy and the helicity
+// of one read of (a, b, c), its curl formed at each mode.
+template <int KIND> constexpr int spectrum_rows() { return KIND == 7 ? 2 : 1; }
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_spectrum(GridK g, double dkk, int nb, double off, const cplx *a,
+                                                     const cplx *b, const cplx *c, const cplx *d, const cplx *e,
+                                                     const cplx *f, double *part) {
   extern __shared__ double bins[];
-  for (int q = threadIdx.x; q < nb; q += blockDim.x) bins[q] = 0.0;
+  constexpr int rows = spectrum_rows<KIND>();
+  for (int q = threadIdx.x; q < rows * nb; q += blockDim.x) bins[q] = 0.0;
   __syncthreads();
   const double tmp = g.inv_n6;
-  GRID_STRIDE(m, ncplx(g)) {
-    Idx q = decompose(m, g);
-    double kk2 = kk2_at(g, q);
-    int kmn = (int)(sqrt(kk2) / dkk + off);
+  for_modes(g, [&](const Idx &q, size_t m) {
+    const double kk2 = kk2_at(g, q);
+    const int kmn = (int)(sqrt(kk2) / dkk + off);
     if (kmn > 0 && kmn <= nb) {
       const double w = q.i == 0 ? 1.0 : 2.0;
       double s;
-      if (kind == 0) s = cabs2(a[m]) + cabs2(b[m]) + cabs2(c[m]);
-      else if (kind == 3) s = cabs2(a[m]);             // one scalar (spectrscc)
-      else if (kind == 4) s = cre_dot(a[m], d[m]);     // scalar transfer (sctrans)
-      else s = cre_dot(a[m], d[m]) + cre_dot(b[m], e[m]) + cre_dot(c[m], f[m]);
-      if (kind == 2) s = kk2 * s;
+      if constexpr (KIND == 0) {
+        s = cabs2(a[m]) + cabs2(b[m]) + cabs2(c[m]);
+      } else if constexpr (KIND == 3) {  // one scalar (spectrscc)
+        s = cabs2(a[m]);
+      } else if constexpr (KIND == 4) {  // scalar transfer (sctrans)
+        s = cre_dot(a[m], d[m]);
+      } else if constexpr (KIND == 5) {  // energy of the curl
+        const Vec3 o = curl_at(g, q, a[m], b[m], c[m]);
+        s = cabs2(o.x) + cabs2(o.y) + cabs2(o.z);
+      } else if constexpr (KIND == 6) {  // curl (a, b, c) against (d, e, f)
+        const Vec3 o = curl_at(g, q, a[m], b[m], c[m]);
+        s = cre_dot(o.x, d[m]) + cre_dot(o.y, e[m]) + cre_dot(o.z, f[m]);
+      } else if constexpr (KIND == 7 || KIND == 8) {  // (energy and) helicity
+        const cplx A = a[m], B = b[m], Cc = c[m];
+        const Vec3 o = curl_at(g, q, A, B, Cc);
+        s = cabs2(A) + cabs2(B) + cabs2(Cc);
+        const double h = cre_dot(A, o.x) + cre_dot(B, o.y) + cre_dot(Cc, o.z);
+        if constexpr (KIND == 7) atomicAdd(&bins[nb + kmn - 1], w * h * tmp);
+        else s = h;
+      } else {
+        s = cre_dot(a[m], d[m]) + cre_dot(b[m], e[m]) + cre_dot(c[m], f[m]);
+        if constexpr (KIND == 2) s = kk2 * s;
+      }
       atomicAdd(&bins[kmn - 1], w * s * tmp);
     }
-  }
+  });
   __syncthreads();
-  for (int q = threadIdx.x; q < nb; q += blockDim.x) part[(size_t)blockIdx.x * nb + q] = bins[q];
+  for (int q = threadIdx.x; q < rows * nb; q += blockDim.x) part[(size_t)blockIdx.x * rows * nb + q] = bins[q];
 }
 
-__global__ void k_spectrum_sum(const double *part, int nblk, int nb, double *out) {
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nb; q += gridDim.x * blockDim.x) {
-    double acc = 0.0;
-    for (int b = 0; b < nblk; ++b) acc += part[(size_t)b * nb + q];
+// Totals of nblk rows of nb partials, rows split over the block's kSumSeg
+// waves and added in a fixed order.  (One thread per bin over all rows was a
+// chain of 1024 loads: 238 us for any spectrum; this takes 6.)
+constexpr int kSumSeg = 16;
+__global__ __launch_bounds__(64 * kSumSeg) void k_spectrum_sum(const double *part, int nblk, int nb, double *out) {
+  __shared__ double sh[kSumSeg][64];
+  const int c = threadIdx.x % 64, seg = threadIdx.x / 64, q = blockIdx.x * 64 + c;
+  double acc = 0.0;
+  if (q < nb) {
+#pragma unroll 8
+    for (int b = seg; b < nblk; b += kSumSeg) acc += part[(size_t)b * nb + q];
+  }
+  sh[seg][c] = acc;
+  __syncthreads();
+  if (seg == 0 && q < nb) {
+    acc = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSumSeg; ++w) acc += sh[w][c];
     out[q] = acc;
   }
 }
@@ -488,54 +603,96 @@ __global__ void k_spectr1d(GridK g, int dir, double ldir, int nb, const cplx *a,
   for (int q = threadIdx.x; q < nb; q += blockDim.x) part[(size_t)blockIdx.x * nb + q] = bins[q];
 }
 
-// Axisymmetric spectra of pseudospec3D_rot.f90 about z.  bins 0: planes
+// Axisymmetric spectra of pseudospec3D_rot.f90 about z.  BINS 0: planes
 // kmn = int(|kz| Lz + 1) (specpara, entpara, heltpara); 1: cylinders
 // kmn = int(sqrt(kx^2 + ky^2)/Dkk + 1) (specperp, entperp, heltperp).
 // kind 0: |a|^2 + |b|^2 (xy) and |c|^2 (z); 1: Re(a d*) + Re(b e*) and
 // Re(c f*); 2: kind 1 times kk2.  Per block, three rows of nb bins: the total,
 // and the xy and z parts (every mode for planes, the kz = 0 plane only for
 // cylinders).
-__global__ void k_axispec(GridK g, int bins, int kind, int nb, double dkk, double lz, const cplx *a, const cplx *b,
-                          const cplx *c, const cplx *d, const cplx *e, const cplx *f, double *part) {
+// A thread keeps one kz and walks the lines, so a plane's sums stay in
+// registers until the end, and a line's modes, which share one cylinder, are
+// added across its lanes first; one atomic per mode and row had up to 64
+// lanes queue on one bin.
+struct HV {
+  double h, v;
+};
+GHX_DEV HV axis_terms(const GridK &g, int kind, const Idx &q, size_t m, const cplx *a, const cplx *b, const cplx *c,
+                      const cplx *d, const cplx *e, const cplx *f) {
+  const double w = (q.i == 0 ? 1.0 : 2.0) * g.inv_n6;
+  double h, v;
+  if (kind == 0) {
+    h = cabs2(a[m]) + cabs2(b[m]);
+    v = cabs2(c[m]);
+  } else if (kind == 3) {  // one field (spectpv)
+    h = cabs2(a[m]);
+    v = 0.0;
+  } else {
+    h = cre_dot(a[m], d[m]) + cre_dot(b[m], e[m]);
+    v = cre_dot(c[m], f[m]);
+    if (kind == 2) {
+      const double k2 = kk2_at(g, q);
+      h *= k2;
+      v *= k2;
+    }
+  }
+  return HV{w * h, w * v};
+}
+template <int BINS>
+__global__ __launch_bounds__(kBlock) void k_axispec(GridK g, int kind, int nb, double dkk, double lz, const cplx *a,
+                                                    const cplx *b, const cplx *c, const cplx *d, const cplx *e,
+                                                    const cplx *f, double *part) {
   extern __shared__ double bins3[];
   for (int q = threadIdx.x; q < 3 * nb; q += blockDim.x) bins3[q] = 0.0;
   __syncthreads();
-  const double tmp = g.inv_n6;
-  GRID_STRIDE(m, ncplx(g)) {
-    Idx q = decompose(m, g);
-    int kmn;
-    if (bins == 0) {
-      kmn = (int)(fabs(wavenum(q.k, g.nz, g.dkz)) * lz + 1);
-    } else {
-      const double kx = wavenum(q.i, g.nx, g.dkx), ky = wavenum(q.j, g.ny, g.dky);
-      kmn = (int)(sqrt(kx * kx + ky * ky) / dkk + 1);
-    }
-    if (kmn <= 0 || kmn > nb) continue;
-    const double w = (q.i == 0 ? 1.0 : 2.0) * tmp;
-    double h, v;
-    if (kind == 0) {
-      h = cabs2(a[m]) + cabs2(b[m]);
-      v = cabs2(c[m]);
-    } else if (kind == 3) {  // one field (spectpv)
-      h = cabs2(a[m]);
-      v = 0.0;
-    } else {
-      h = cre_dot(a[m], d[m]) + cre_dot(b[m], e[m]);
-      v = cre_dot(c[m], f[m]);
-      if (kind == 2) {
-        const double k2 = kk2_at(g, q);
-        h *= k2;
-        v *= k2;
+  const LineWalk w = line_walk(g);
+  const int k0 = threadIdx.x & (w.kl - 1), l0 = (int)blockIdx.x * w.lb + (threadIdx.x >> w.sh);
+  const int step = (int)gridDim.x * w.lb;
+  Idx q;
+  if constexpr (BINS == 0) {
+    for (q.k = k0; q.k < g.nz; q.k += w.kl) {
+      const int kmn = (int)(fabs(wavenum(q.k, g.nz, g.dkz)) * lz + 1);
+      if (kmn <= 0 || kmn > nb) continue;
+      double h = 0.0, v = 0.0;
+      for (int l = l0; l < w.nl; l += step) {
+        q.i = l / g.ny;
+        q.j = l - q.i * g.ny;
+        const HV t = axis_terms(g, kind, q, (size_t)l * g.nz + q.k, a, b, c, d, e, f);
+        h += t.h;
+        v += t.v;
       }
+      atomicAdd(&bins3[kmn - 1], h + v);
+      atomicAdd(&bins3[nb + kmn - 1], h);
+      atomicAdd(&bins3[2 * nb + kmn - 1], v);
     }
-    atomicAdd(&bins3[kmn - 1], w * (h + v));
-    if (bins == 0 || q.k == 0) {
-      atomicAdd(&bins3[nb + kmn - 1], w * h);
-      atomicAdd(&bins3[2 * nb + kmn - 1], w * v);
+  } else {
+    const int span = w.kl < 64 ? w.kl : 64;  // lanes of one wave on one line
+    // every lane of a wave walks the same number of lines (the last ones may
+    // be past the end), so that the sums across lanes see all of them
+    for (int base = (int)blockIdx.x * w.lb; base < w.nl; base += step) {
+      const int l = base + (threadIdx.x >> w.sh);
+      const bool in = l < w.nl;
+      q.i = in ? l / g.ny : 0;
+      q.j = in ? l - q.i * g.ny : 0;
+      const double kx = wavenum(q.i, g.nx, g.dkx), ky = wavenum(q.j, g.ny, g.dky);
+      const int kmn = (int)(sqrt(kx * kx + ky * ky) / dkk + 1);
+      const bool on = in && kmn > 0 && kmn <= nb;
+      double s = 0.0;
+      if (on)
+        for (q.k = k0; q.k < g.nz; q.k += w.kl) {
+          const HV t = axis_terms(g, kind, q, (size_t)l * g.nz + q.k, a, b, c, d, e, f);
+          s += t.h + t.v;
+          if (q.k == 0) {
+            atomicAdd(&bins3[nb + kmn - 1], t.h);
+            atomicAdd(&bins3[2 * nb + kmn - 1], t.v);
+          }
+        }
+      for (int o = span / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (on && (threadIdx.x & (span - 1)) == 0) atomicAdd(&bins3[kmn - 1], s);
     }
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < 3 * nb; q += blockDim.x) part[(size_t)blockIdx.x * 3 * nb + q] = bins3[q];
+  for (int p = threadIdx.x; p < 3 * nb; p += blockDim.x) part[(size_t)blockIdx.x * 3 * nb + p] = bins3[p];
 }
 
 // spec2D (pseudospec3D_rot.f90:1331-1629): E(kperp, kpara), kperp fastest,
@@ -733,19 +890,49 @@ hipError_t op_tg_real(const GridK &g, hipStream_t st, double *r1, double *r2, in
   LAUNCH(k_tg_real, nreal(g), st, g, r1, r2, kdn, kup);
 }
 
-size_t reduce_work_doubles() { return kRedBlocks + 8; }
+// blocks of a walk over the modes, at most `most`
+static unsigned walk_blocks(const GridK &g, int most) {
+  const LineWalk w = line_walk(g);
+  const int nb = (w.nl + w.lb - 1) / w.lb;
+  return (unsigned)(nb < most ? nb : most);
+}
+
+size_t reduce_work_doubles() { return 5 * kRedBlocks + 8; }
+
+static hipError_t to_host(double *out, const double *dev, size_t n, hipStream_t st) {
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  err = hipMemcpyAsync(out, dev, n * sizeof(double), hipMemcpyDeviceToHost, st);
+  if (err != hipSuccess) return err;
+  return hipStreamSynchronize(st);
+}
 
 hipError_t op_reduce(const GridK &g, hipStream_t st, int kind, const cplx *a, const cplx *b, const cplx *c,
                      const cplx *d, const cplx *e, const cplx *f, double *work, double *out) {
-  unsigned nb = nblocks(ncplx(g));
-  if (nb > (unsigned)kRedBlocks) nb = kRedBlocks;
-  hipLaunchKernelGGL(k_reduce, dim3(nb), dim3(kBlock), 0, st, g, kind, a, b, c, d, e, f, work);
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, st, work, (int)nb, work + kRedBlocks);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  err = hipMemcpyAsync(out, work + kRedBlocks, sizeof(double), hipMemcpyDeviceToHost, st);
-  if (err != hipSuccess) return err;
-  return hipStreamSynchronize(st);
+  const unsigned nb = walk_blocks(g, kRedBlocks);
+  switch (kind) {
+#define GHX_CASE(K)                                                                                      \
+  case K:                                                                                                \
+    hipLaunchKernelGGL(k_reduce<K>, dim3(nb), dim3(kBlock), 0, st, g, a, b, c, d, e, f, work); \
+    break;
+    GHX_CASE(0) GHX_CASE(1) GHX_CASE(2) GHX_CASE(3) GHX_CASE(4) GHX_CASE(5)
+    GHX_CASE(6) GHX_CASE(7) GHX_CASE(8) GHX_CASE(9) GHX_CASE(10) GHX_CASE(11)
+#undef GHX_CASE
+  default:
+    return hipErrorInvalidValue;
+  }
+  double *res = work + 5 * kRedBlocks;
+  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, st, work, (int)nb, res);
+  return to_host(out, res, 1, st);
+}
+
+hipError_t op_hdcheck(const GridK &g, hipStream_t st, const cplx *const *v, const cplx *const *f, double *work,
+                      double *out) {
+  const unsigned nb = walk_blocks(g, kRedBlocks);
+  hipLaunchKernelGGL(k_hdcheck, dim3(nb), dim3(kBlock), 0, st, g, v[0], v[1], v[2], f[0], f[1], f[2], work);
+  double *res = work + 5 * kRedBlocks;
+  hipLaunchKernelGGL(k_sum_partials, dim3(5), dim3(kBlock), 0, st, work, (int)nb, res);
+  return to_host(out, res, 5, st);
 }
 
 static unsigned spectrum_blocks(const GridK &g) {
@@ -754,19 +941,31 @@ static unsigned spectrum_blocks(const GridK &g) {
 }
 size_t spectrum_work_doubles(const GridK &g, int nb) { return (size_t)spectrum_blocks(g) * nb + nb; }
 
+static void sum_rows(hipStream_t st, const double *part, unsigned nblk, int nb, double *res) {
+  hipLaunchKernelGGL(k_spectrum_sum, dim3((nb + 63) / 64), dim3(64 * kSumSeg), 0, st, part, (int)nblk, nb, res);
+}
+
 hipError_t op_spectrum(const GridK &g, hipStream_t st, int kind, double dkk, int nb, const cplx *a, const cplx *b,
                        const cplx *c, const cplx *d, const cplx *e, const cplx *f, double *work, double *out,
                        double off) {
-  unsigned nblk = spectrum_blocks(g);
-  hipLaunchKernelGGL(k_spectrum, dim3(nblk), dim3(kBlock), nb * sizeof(double), st, g, kind, dkk, nb, off, a, b, c,
-                     d, e, f, work);
-  double *res = work + (size_t)nblk * nb;
-  hipLaunchKernelGGL(k_spectrum_sum, dim3((nb + kBlock - 1) / kBlock), dim3(kBlock), 0, st, work, (int)nblk, nb, res);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  err = hipMemcpyAsync(out, res, sizeof(double) * nb, hipMemcpyDeviceToHost, st);
-  if (err != hipSuccess) return err;
-  return hipStreamSynchronize(st);
+  const int rows = kind == 7 ? 2 : 1;
+  // no more blocks than spectrum_work_doubles counts, so that the work array
+  // (fixed in the call without allocation) holds their partials
+  const unsigned nblk = walk_blocks(g, (int)spectrum_blocks(g));
+  switch (kind) {
+#define GHX_CASE(K)                                                                                                \
+  case K:                                                                                                          \
+    hipLaunchKernelGGL(k_spectrum<K>, dim3(nblk), dim3(kBlock), rows * nb * sizeof(double), st, g, dkk, nb, off, a, \
+                       b, c, d, e, f, work);                                                                       \
+    break;
+    GHX_CASE(0) GHX_CASE(1) GHX_CASE(2) GHX_CASE(3) GHX_CASE(4) GHX_CASE(5) GHX_CASE(6) GHX_CASE(7) GHX_CASE(8)
+#undef GHX_CASE
+  default:
+    return hipErrorInvalidValue;
+  }
+  double *res = work + (size_t)nblk * rows * nb;
+  sum_rows(st, work, nblk, rows * nb, res);
+  return to_host(out, res, (size_t)rows * nb, st);
 }
 
 size_t axispec_work_doubles(const GridK &g, int nb) { return (size_t)spectrum_blocks(g) * 3 * nb + 3 * nb; }
@@ -774,17 +973,16 @@ size_t axispec_work_doubles(const GridK &g, int nb) { return (size_t)spectrum_bl
 hipError_t op_axispec(const GridK &g, hipStream_t st, int bins, int kind, int nb, double dkk, double lz,
                       const cplx *a, const cplx *b, const cplx *c, const cplx *d, const cplx *e, const cplx *f,
                       double *work, double *out) {
-  unsigned nblk = spectrum_blocks(g);
-  hipLaunchKernelGGL(k_axispec, dim3(nblk), dim3(kBlock), 3 * nb * sizeof(double), st, g, bins, kind, nb, dkk, lz, a,
-                     b, c, d, e, f, work);
+  const unsigned nblk = walk_blocks(g, (int)spectrum_blocks(g));
+  if (bins == 0)
+    hipLaunchKernelGGL(k_axispec<0>, dim3(nblk), dim3(kBlock), 3 * nb * sizeof(double), st, g, kind, nb, dkk, lz, a,
+                       b, c, d, e, f, work);
+  else
+    hipLaunchKernelGGL(k_axispec<1>, dim3(nblk), dim3(kBlock), 3 * nb * sizeof(double), st, g, kind, nb, dkk, lz, a,
+                       b, c, d, e, f, work);
   double *res = work + (size_t)nblk * 3 * nb;
-  hipLaunchKernelGGL(k_spectrum_sum, dim3((3 * nb + kBlock - 1) / kBlock), dim3(kBlock), 0, st, work, (int)nblk,
-                     3 * nb, res);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  err = hipMemcpyAsync(out, res, sizeof(double) * 3 * nb, hipMemcpyDeviceToHost, st);
-  if (err != hipSuccess) return err;
-  return hipStreamSynchronize(st);
+  sum_rows(st, work, nblk, 3 * nb, res);
+  return to_host(out, res, 3 * (size_t)nb, st);
 }
 
 hipError_t op_spec2d(const GridK &g, hipStream_t st, int kind, int np, int nzb, double dkk, double lz, const cplx *a,
@@ -830,12 +1028,15 @@ hipError_t op_spectr1d(const GridK &g, hipStream_t st, int dir, double ldir, int
   unsigned nblk = spectrum_blocks(g);
   hipLaunchKernelGGL(k_spectr1d, dim3(nblk), dim3(kBlock), nb * sizeof(double), st, g, dir, ldir, nb, a, work);
   double *res = work + (size_t)nblk * nb;
-  hipLaunchKernelGGL(k_spectrum_sum, dim3((nb + kBlock - 1) / kBlock), dim3(kBlock), 0, st, work, (int)nblk, nb, res);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  err = hipMemcpyAsync(out, res, sizeof(double) * nb, hipMemcpyDeviceToHost, st);
-  if (err != hipSuccess) return err;
-  return hipStreamSynchronize(st);
+  sum_rows(st, work, nblk, nb, res);
+  return to_host(out, res, (size_t)nb, st);
+}
+
+hipError_t op_max_sqrt(hipStream_t st, double *work, int n, double *out) {
+  hipLaunchKernelGGL(k_max_partials, dim3(1), dim3(kBlock), 0, st, work, n, work + n);
+  const hipError_t err = to_host(out, work + n, 1, st);
+  if (err == hipSuccess) *out = sqrt(*out);
+  return err;
 }
 
 hipError_t op_maxnorm(const GridK &g, hipStream_t st, const double *r1, const double *r2, const double *r3,
