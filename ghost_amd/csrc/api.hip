@@ -226,6 +226,12 @@ static GridK make_gridk(int nx, int ny, int nz, int arbsize, double Lx, double L
   double t = (double)nx * (double)ny * (double)nz;
   g.inv_n6 = 1.0 / (t * t);
   g.tiny = 0.0;
+  g.kxact = 0;
+  for (int q = 0; q < g.nxh; ++q) {
+    const double kx = (double)(q < nx / 2 ? q : q - nx);
+    if (g.rmp * (kx * kx) <= g.kmax) g.kxact = q + 1;
+  }
+  g.dirty = nullptr;
   return g;
 }
 
@@ -446,6 +452,7 @@ struct ghx_grid {
   double *rtmp = nullptr;   // real temporaries
   int rtmp_fields = 0;
   size_t nc = 0, nr = 0;
+  unsigned *dirty = nullptr;  // device word of the substeps on caller fields (GridK::dirty)
   double ps[3] = {1, 1, 1};  // pruned shares (rows, lines, modes), computed on first use
   bool ps_valid = false;
 };
@@ -485,6 +492,7 @@ extern "C" int ghx_grid_create(ghx_grid **grid, int nx, int ny, int nz, double L
   ghx_grid *g = new (std::nothrow) ghx_grid();
   if (!g) return set_err(GHX_ERR_NOMEM, "host allocation failed");
   int rc = plan_init(&g->plan, nx, ny, nz, GHX_FFTW_REAL_TO_COMPLEX);
+  if (!rc && hipMalloc(&g->dirty, 256) != hipSuccess) rc = set_err(GHX_ERR_NOMEM, "grid: device allocation");
   if (rc) { plan_release(&g->plan); delete g; return rc; }
   GridK k = make_gridk(nx, ny, nz, arbsize, Lx, Ly, Lz);
   // Dkk, nmax, tiny: main3D.fpp:905-909, 1728-1735
@@ -509,6 +517,7 @@ extern "C" int ghx_grid_destroy(ghx_grid *g) {
   if (g->work) (void)hipFree(g->work);
   if (g->ctmp) (void)hipFree(g->ctmp);
   if (g->rtmp) (void)hipFree(g->rtmp);
+  if (g->dirty) (void)hipFree(g->dirty);
   delete g;
   return GHX_OK;
 }
@@ -1503,11 +1512,13 @@ static PruneShares prune_shares(ghx_grid *g) {
 // Fused HD substep: q holds 9 Q-layout fields of scratch.
 // omegaz != 0: the rotating-frame step of include/roth_rkstep2.f90 (Coriolis
 // force added to the products in the last pass).
+// prune: 0, 1 or 2 as in fft_passes.h; dirty: the device word of prune = 2.
 static int hd_substep(ghx_grid *g, cplx *q, int o, double dt, double nu, const cplx *const *v, const cplx *const *c,
                       const cplx *const *f, const uint8_t *fline, cplx *const *out, int prune = 0,
-                      double omegaz = 0.0) {
+                      double omegaz = 0.0, const unsigned *dirty = nullptr) {
   const size_t nc = g->nc;
-  const FFTCtx &ctx = g->plan.ctx;
+  FFTCtx ctx = g->plan.ctx;
+  ctx.gk.dirty = dirty;
   Chain ch = chain_slots(q, ghx::slot_points(g->gk));
   FieldSet in, pq;
   for (int k = 0; k < 3; ++k) in.p[k] = const_cast<cplx *>(v[k]);
@@ -1515,7 +1526,7 @@ static int hd_substep(ghx_grid *g, cplx *q, int o, double dt, double nu, const c
   const double sc = (double)nc * sizeof(cplx);
   // Algorithmic traffic of each pass.  Pruned: fx = share of kx rows carrying
   // kept modes, fl = share of (kx,ky) lines, fm = share of kept modes.
-  const PruneShares ps = (prune && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
+  const PruneShares ps = (prune == 1 && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
   PROF(P_ZINV_CURL, (3 * ps.fm + 6 * ps.fl) * sc, ctx.stream, ghx::zinv(ctx, 1, 3, in, ch.q6, prune));
   PROF(P_YINV, (6 * ps.fl + 6 * ps.fx) * sc, ctx.stream, ghx::yinv(ctx, 6, ch.q6, ch.p6, prune));
   PROF(P_XCROSS, 9 * ps.fx * sc, ctx.stream, ghx::xcross(ctx, 0, pq, ch.p3, prune));
@@ -1532,29 +1543,49 @@ static int hd_substep(ghx_grid *g, cplx *q, int o, double dt, double nu, const c
   // alias) and the forcing on the kept modes, writes v_out on the kept modes
   // (on every mode without pruning)
   const int nvc = (const void *)c[0] == (const void *)v[0] ? 3 : 6;
-  PROF(P_ZFWD_RK_HD, (3 * ps.fl + nvc * ps.fm + 3 * (prune ? ps.fm : 1.0)) * sc, ctx.stream,
+  PROF(P_ZFWD_RK_HD, (3 * ps.fl + nvc * ps.fm + 3 * (prune == 1 ? ps.fm : 1.0)) * sc, ctx.stream,
        ghx::zfwd_rk_hd(ctx, ch.q3, rk, prune));
   return GHX_OK;
 }
 
 // lines (kx,ky) on which any of the fields is non-zero
+// (one wave per line, so that its lanes read neighbouring modes)
 __global__ void k_line_flags(const cplx *a, const cplx *b, const cplx *c, int nz, size_t nlines, uint8_t *flag) {
-  for (size_t l = (size_t)blockIdx.x * blockDim.x + threadIdx.x; l < nlines; l += (size_t)gridDim.x * blockDim.x) {
-    uint8_t nzf = 0;
+  const unsigned lane = threadIdx.x % 64, wpb = blockDim.x / 64;
+  for (size_t l = (size_t)blockIdx.x * wpb + threadIdx.x / 64; l < nlines; l += (size_t)gridDim.x * wpb) {
+    bool on = false;
     const size_t base = l * nz;
-    for (int k = 0; k < nz; ++k) {
+    for (int k = lane; k < nz; k += 64) {
       cplx x = a[base + k], y = b[base + k], z = c[base + k];
-      if (x.x != 0.0 || x.y != 0.0 || y.x != 0.0 || y.y != 0.0 || z.x != 0.0 || z.y != 0.0) nzf = 1;
+      on = on || x.x != 0.0 || x.y != 0.0 || y.x != 0.0 || y.y != 0.0 || z.x != 0.0 || z.y != 0.0;
     }
-    flag[l] = nzf;
+    const bool any = __ballot(on) != 0;
+    if (lane == 0) flag[l] = any;
   }
 }
 
 static int line_flags(ghx_grid *g, const cplx *a, const cplx *b, const cplx *c, uint8_t *flag) {
   size_t nl = (size_t)g->gk.nxh * g->gk.ny;
-  unsigned nb = (unsigned)((nl + 255) / 256);
+  unsigned nb = (unsigned)((nl + 3) / 4);
+  if (nb > 8192u) nb = 8192u;
   hipLaunchKernelGGL(k_line_flags, dim3(nb), dim3(256), 0, g->stream, a, b, c, g->gk.nz, nl, flag);
   HIPCHK(hipGetLastError());
+  return GHX_OK;
+}
+
+// The substeps on caller fields.  Nothing is known about their input, so a
+// kernel looks at the modes outside the dealias set first and leaves the answer
+// in a device word that the passes over the input read (no copy to the host);
+// GHOST's loops pass dealiased fields on every call but the first, and then the
+// z, y and x inverses skip what is zero.  The products are only used on the
+// kept modes, so the passes over them are pruned in either case.  Fields
+// from mean on may hold a mean (kn2 < tiny).  At 256 x 128 x 192 the look costs
+// 40 us and the passes go from 500 to 330 us.  (The forcing is read on the kept
+// modes of every line: marking the forced lines first read all of it, 120 us.)
+static int caller_prune() { return getenv("GHX_NO_PRUNE") ? 0 : 2; }
+static int caller_dirty(ghx_grid *g, const cplx *const *v, int nf, int mean, unsigned **dirty) {
+  HIPCHK(ghx::op_unkept(g->gk, g->stream, v, nf, mean, g->dirty));
+  *dirty = g->dirty;
   return GHX_OK;
 }
 
@@ -1569,15 +1600,10 @@ static int rkstep2(ghx_grid *g, int o, double dt, double nu, double omegaz, cons
     v[k] = C_(v_in[k]); c[k] = C_(C[k]); out[k] = M_(v_out[k]);
     ff[k] = f ? C_(f[k]) : nullptr;
   }
-  uint8_t *fl = nullptr;
-  if (f) {
-    // dense forcing: every line is read
-    size_t nl = (size_t)g->gk.nxh * g->gk.ny;
-    if ((rc = grid_work(g, (nl + 7) / 8 + 1))) return rc;
-    fl = (uint8_t *)g->work;
-    if ((rc = line_flags(g, ff[0], ff[1], ff[2], fl))) return rc;
-  }
-  return hd_substep(g, g->plan.q, o, dt, nu, v, c, f ? ff : nullptr, fl, out, 0, omegaz);
+  const cplx *vd[3] = {v[0], v[1], v[2]};
+  unsigned *dirty = nullptr;
+  if ((rc = caller_dirty(g, vd, 3, 3, &dirty))) return rc;
+  return hd_substep(g, g->plan.q, o, dt, nu, v, c, f ? ff : nullptr, nullptr, out, caller_prune(), omegaz, dirty);
 }
 
 extern "C" int ghx_hd_rkstep2(ghx_grid *g, int o, double dt, double nu, const void *const *v_in, const void *const *C,
@@ -1865,7 +1891,7 @@ static int hd_step_once(ghx_hd *s) {
     if (rc) return rc;
     s->clean = (n == 0.0);
   }
-  const int prune = s->clean && !getenv("GHX_NO_PRUNE") ? 1 : 0;
+  const int prune = getenv("GHX_NO_PRUNE") ? 0 : (s->clean ? 1 : 2);
   const cplx *fc[3] = {s->f[0], s->f[1], s->f[2]};
   const cplx *const *f = s->forced ? fc : nullptr;
   const cplx *v0[3] = {s->v[0], s->v[1], s->v[2]};
@@ -1882,7 +1908,7 @@ static int hd_step_once(ghx_hd *s) {
     const uint8_t *fl = s->fline;
     const cplx *fs[3];
     if (s->sgs || s->sgs_nuk) {  // the forcing of this substep is f + P(-div tau(vin)) - nu(k) kk2 vin
-      int rc = sgs_force(s, vin, fs, prune);
+      int rc = sgs_force(s, vin, fs, prune == 1 ? 1 : 0);
       if (rc) return rc;
       fo = fs;
       fl = s->sgs_fline;
@@ -1998,17 +2024,19 @@ extern "C" int ghx_mhd_touch(ghx_mhd *s) {
   return GHX_OK;
 }
 
-static int mhd_substep(ghx_mhd *s, int o, const cplx *const *vin, cplx *const *out, int prune) {
+static int mhd_substep(ghx_mhd *s, int o, const cplx *const *vin, cplx *const *out, int prune,
+                       const unsigned *dirty = nullptr) {
   ghx_grid *g = s->g;
   const size_t nc = g->nc, slot = ghx::slot_points(g->gk);
-  const FFTCtx &ctx = g->plan.ctx;
+  FFTCtx ctx = g->plan.ctx;
+  ctx.gk.dirty = dirty;
   // Q12 (slots 0-11) -> P12 (12-23) -> P9 (reuses 0-8) -> Q9 (reuses 12-20)
   FieldSet in, q12, p12, p9, q9, pq;
   for (int k = 0; k < 6; ++k) in.p[k] = const_cast<cplx *>(vin[k]);
   for (int k = 0; k < 12; ++k) { q12.p[k] = s->q + k * slot; p12.p[k] = s->q + (12 + k) * slot; }
   for (int k = 0; k < 9; ++k) { p9.p[k] = s->q + k * slot; q9.p[k] = s->q + (12 + k) * slot; }
   const double sc = (double)nc * sizeof(cplx);
-  const PruneShares ps = (prune && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
+  const PruneShares ps = (prune == 1 && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
   PROF(P_ZINV_MHD, (6 * ps.fm + 12 * ps.fl) * sc, ctx.stream, ghx::zinv(ctx, 2, 6, in, q12, prune));  // u w b j
   // the Y^-1 pass takes at most kMaxFields fields per launch
   PROF(P_YINV, (6 * ps.fl + 6 * ps.fx) * sc, ctx.stream, ghx::yinv(ctx, 6, q12, p12, prune));
@@ -2041,7 +2069,7 @@ static int mhd_substep(ghx_mhd *s, int o, const cplx *const *vin, cplx *const *o
   }
   rk.fline = s->forced ? s->fline : nullptr;
   const int nvc = vin[0] == s->s[0] ? 6 : 12;
-  PROF(P_ZFWD_RK_MHD, (9 * ps.fl + nvc * ps.fm + 6 * (prune ? ps.fm : 1.0)) * sc, ctx.stream,
+  PROF(P_ZFWD_RK_MHD, (9 * ps.fl + nvc * ps.fm + 6 * (prune == 1 ? ps.fm : 1.0)) * sc, ctx.stream,
        ghx::zfwd_rk_mhd(ctx, q9, rk, prune));
   return GHX_OK;
 }
@@ -2058,7 +2086,7 @@ extern "C" int ghx_mhd_step(ghx_mhd *s, int nsteps) {
       if (rc) return rc;
       s->clean = (a == 0.0 && b == 0.0);
     }
-    const int prune = s->clean && !getenv("GHX_NO_PRUNE") ? 1 : 0;
+    const int prune = getenv("GHX_NO_PRUNE") ? 0 : (s->clean ? 1 : 2);
     if (s->tr) {
       int rc = tracers_begin_step(s->tr);
       if (rc) return rc;
@@ -2194,7 +2222,7 @@ static int tracers_stage(ghx_tracers *t, cplx *q, const cplx *const *v, double d
     pp.p[c] = q + (3 + c) * slot;
   }
   const double sc = (double)g->nc * sizeof(cplx), sr = (double)g->nr * sizeof(double);
-  const PruneShares ps = (prune && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
+  const PruneShares ps = (prune == 1 && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
   PROF(P_ZINV_SPLINE, (3 * ps.fm + 3 * ps.fl) * sc, ctx.stream, ghx::zinv(ctx, 3, 3, in, qq, prune, t->spl));
   PROF(P_YINV_TRACER, (3 * ps.fl + 3 * ps.fx) * sc, ctx.stream, ghx::yinv(ctx, 3, qq, pp, prune));
   PROF(P_XINV_TRACER, 3 * (ps.fx * sc + sr), ctx.stream, ghx::xinv3i(ctx, pp, r3, prune));
@@ -2370,17 +2398,19 @@ extern "C" int ghx_bouss_set_tracers(ghx_bouss *s, ghx_tracers *t) {
 // include/bouss_rkstep2.f90:1-71 fused: one inverse chain for (v, th)
 // producing (u, w, grad th); w x u and -(u . grad th) in the x pass; one
 // forward chain ending in buoyancy, projection, heat current and the updates.
-static int bouss_substep(ghx_bouss *s, int o, const cplx *const *vin, cplx *const *out, int prune) {
+static int bouss_substep(ghx_bouss *s, int o, const cplx *const *vin, cplx *const *out, int prune,
+                         const unsigned *dirty = nullptr) {
   ghx_grid *g = s->g;
   const size_t nc = g->nc, slot = ghx::slot_points(g->gk);
-  const FFTCtx &ctx = g->plan.ctx;
+  FFTCtx ctx = g->plan.ctx;
+  ctx.gk.dirty = dirty;
   // Q9 (slots 0-8) -> P9 (9-17) -> P4 (reuses 0-3) -> Q4 (reuses 9-12)
   FieldSet in, q9, p9, pq, o3, pd, o1, p4, q4;
   for (int k = 0; k < 4; ++k) in.p[k] = const_cast<cplx *>(vin[k]);
   for (int k = 0; k < 9; ++k) { q9.p[k] = s->q + k * slot; p9.p[k] = s->q + (9 + k) * slot; }
   for (int k = 0; k < 4; ++k) { p4.p[k] = s->q + k * slot; q4.p[k] = s->q + (9 + k) * slot; }
   const double sc = (double)nc * sizeof(cplx);
-  const PruneShares ps = (prune && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
+  const PruneShares ps = (prune == 1 && g_prof.on) ? prune_shares(g) : PruneShares{1.0, 1.0, 1.0};
   PROF(P_ZINV_BOUSS, (4 * ps.fm + 9 * ps.fl) * sc, ctx.stream, ghx::zinv(ctx, 5, 4, in, q9, prune));
   PROF(P_YINV, (9 * ps.fl + 9 * ps.fx) * sc, ctx.stream, ghx::yinv(ctx, 9, q9, p9, prune));
   // w x u in GHOST's operand order (P = w, Q = u)
@@ -2402,7 +2432,7 @@ static int bouss_substep(ghx_bouss *s, int o, const cplx *const *vin, cplx *cons
   }
   rk.fline = s->forced ? s->fline : nullptr;
   const int nvc = vin[0] == s->s[0] ? 4 : 8;
-  PROF(P_ZFWD_RK_BOUSS, (4 * ps.fl + nvc * ps.fm + 4 * (prune ? ps.fm : 1.0)) * sc, ctx.stream,
+  PROF(P_ZFWD_RK_BOUSS, (4 * ps.fl + nvc * ps.fm + 4 * (prune == 1 ? ps.fm : 1.0)) * sc, ctx.stream,
        ghx::zfwd_rk_bouss(ctx, q4, rk, prune));
   return GHX_OK;
 }
@@ -2444,25 +2474,6 @@ extern "C" int ghx_bouss_ord3(ghx_grid *g, double dt, double xmom, const void *c
   return GHX_OK;
 }
 
-// Forcing-line flags for the stateless substeps below: the lines (kx, ky)
-// where any of the nf fields is non-zero, OR-ed, in g->work (2 nl bytes).
-static int stateless_flags(ghx_grid *g, const cplx *const *fa, int nf, uint8_t **flags) {
-  const size_t nl = (size_t)g->gk.nxh * g->gk.ny;
-  int rc = grid_work(g, (2 * nl + 7) / 8 + 1);
-  if (rc) return rc;
-  uint8_t *fl = (uint8_t *)g->work, *tmp = fl + nl;
-  for (int b = 0; b < nf; b += 3) {
-    const cplx *x = fa[b], *y = fa[b + 1 < nf ? b + 1 : b], *z = fa[b + 2 < nf ? b + 2 : b];
-    if ((rc = line_flags(g, x, y, z, b == 0 ? fl : tmp))) return rc;
-    if (b > 0) {
-      hipLaunchKernelGGL(k_or_flags, dim3((unsigned)((nl + 255) / 256)), dim3(256), 0, g->stream, fl, tmp, nl);
-      HIPCHK(hipGetLastError());
-    }
-  }
-  *flags = fl;
-  return GHX_OK;
-}
-
 // include/mhd_rkstep2.f90:4-65 for order index o on caller fields: vin, C
 // and vout hold (v_x, v_y, v_z, a_x, a_y, a_z); f (mechanical) and m
 // (electromotive) forcing, 3 fields each, both given or both NULL.  vout may
@@ -2480,13 +2491,11 @@ extern "C" int ghx_mhd_rkstep2(ghx_grid *g, int o, double dt, double nu, double 
   for (int k = 0; k < 6; ++k) { h.s[k] = M_(C[k]); vi[k] = C_(vin[k]); vo[k] = M_(vout[k]); }
   if (f) {
     for (int k = 0; k < 3; ++k) { h.f[k] = M_(f[k]); h.m[k] = M_(m[k]); }
-    const cplx *fa[6] = {h.f[0], h.f[1], h.f[2], h.m[0], h.m[1], h.m[2]};
-    if ((rc = stateless_flags(g, fa, 6, &h.fline))) return rc;
-    h.forced = true;
+    h.forced = true;  // without line flags: the kept modes of every line are read
   }
-  rc = mhd_substep(&h, o, vi, vo, 0);
-  h.fline = nullptr;  // g->work, not owned
-  return rc;
+  unsigned *dirty = nullptr;
+  if ((rc = caller_dirty(g, vi, 6, 6, &dirty))) return rc;
+  return mhd_substep(&h, o, vi, vo, caller_prune(), dirty);
 }
 
 // include/bouss_rkstep2.f90:1-71 (rotbouss_rkstep2.f90 with rot = 1: the
@@ -2509,13 +2518,11 @@ static int bouss_rkstep2_impl(ghx_grid *g, int o, double dt, double nu, double k
   for (int k = 0; k < 4; ++k) { h.s[k] = M_(C[k]); vi[k] = C_(vin[k]); vo[k] = M_(vout[k]); }
   if (f) {
     for (int k = 0; k < 4; ++k) h.f[k] = M_(f[k]);
-    const cplx *fa[4] = {h.f[0], h.f[1], h.f[2], h.f[3]};
-    if ((rc = stateless_flags(g, fa, 4, &h.fline))) return rc;
     h.forced = true;
   }
-  rc = bouss_substep(&h, o, vi, vo, 0);
-  h.fline = nullptr;
-  return rc;
+  unsigned *dirty = nullptr;
+  if ((rc = caller_dirty(g, vi, 4, 3, &dirty))) return rc;
+  return bouss_substep(&h, o, vi, vo, caller_prune(), dirty);
 }
 extern "C" int ghx_bouss_rkstep2(ghx_grid *g, int o, double dt, double nu, double kappa, double xmom, double xtemp,
                                  const void *const *vin, const void *const *C, const void *const *f,
@@ -2547,7 +2554,7 @@ extern "C" int ghx_bouss_step(ghx_bouss *s, int nsteps) {
       if (rc) return rc;
       s->clean = (a == 0.0 && b == 0.0);
     }
-    const int prune = s->clean && !getenv("GHX_NO_PRUNE") ? 1 : 0;
+    const int prune = getenv("GHX_NO_PRUNE") ? 0 : (s->clean ? 1 : 2);
     if (s->tr) {
       int rc = tracers_begin_step(s->tr);
       if (rc) return rc;

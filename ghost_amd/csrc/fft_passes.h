@@ -45,7 +45,7 @@ struct RKParams {
   const cplx *c[3];    // state at the start of the step
   cplx *out[3];        // updated state (may alias c or v element-wise)
   const cplx *f[3];    // forcing (may be null)
-  const uint8_t *fline;  // per (kx,ky) line: 1 if the forcing is non-zero there
+  const uint8_t *fline;  // per (kx,ky) line: 1 if the forcing is non-zero there (null: any line may be forced)
   size_t bstride = 0;       // elements between batch members (v, c, out, f)
   const double *nu_b = nullptr;  // per-member viscosity of a batched launch (else nu)
   double om2 = 0.0;  // 2 omegaz: Coriolis force of a frame rotating about z (0: none)
@@ -85,6 +85,7 @@ inline size_t slot_points(const GridK &g) { return (size_t)g.nz * g.ny * p_row(g
 // prune=1: the input is dealiased (zero outside tiny <= kn2 <= kmax): only
 // lines that carry kept modes are read and written (every pass below takes
 // the same flag; see the kernels for exactly what each one skips).
+// prune=2: outputs as with 1, inputs as GridK::dirty says (prune_input).
 // mode 3: nf fields in, nf out, each mode scaled by aux[kx] aux[nxh+ky]
 // aux[nxh+ny+kz] (the periodic cubic-spline prefilter of the tracers).
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune = 0,
@@ -117,7 +118,5 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
 // Z forward fused with the Boussinesq projection and update: in.p[0..2] =
 // products w x u, in.p[3] = -(u . grad th), Q layout.
 hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParams &rk, int prune = 0);
-// number of kx indices (from 0) whose kn2(kx,0,0) <= kmax
-int active_kx(const GridK &g);
 
 }  // namespace ghx

@@ -416,8 +416,9 @@ GHX_DEV void zinv_curl5(cplx (&ax)[E], cplx (&ay)[E], cplx (&az)[E], double kx, 
 
 template <int N, int MODE, typename Cfg = FFTCfg<N>>
 __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_, int nf, GridK g, const cplx *__restrict__ twt,
-                                             int prune, const double *__restrict__ aux) {
+                                             int prune_, const double *__restrict__ aux) {
   using F = LineFFT<N, +1, Cfg>;
+  const int prune = prune_input(g, prune_);
   constexpr int T = F::T, E = F::E;
   // store groups: the MHD and Boussinesq passes (MODE 2, 5) are at the
   // register limit and spill more with grouped reads; they store one point
@@ -715,6 +716,17 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
   // only lines inside the dealias disc are transformed and only kept modes
   // are read and written.
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
+  // prune == 2: the output buffers held something else, so the lines outside
+  // the dealias disc are zeroed here instead of being known to be zero
+  if (prune == 2 && j < g.ny && !((lmask >> lt) & 1u)) {
+    const size_t s0 = ((size_t)i * g.ny + j) * N;
+#pragma unroll 1
+    for (int m = 0; m < E; ++m) {
+      rk.out[0][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[1][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[2][s0 + t + T * m] = c_make(0.0, 0.0);
+    }
+  }
   if (lmask == 0u) return;  // uniform over the block
   const bool ok = j < g.ny && ((lmask >> lt) & 1u);
   const int stride = lds_line_stride(N);
@@ -746,7 +758,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
   if (!ok) return;
   const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j, g.ny, g.dky);
   const size_t sline = ((size_t)i * g.ny + j) * N;
-  const bool forced = rk.fline && rk.fline[(size_t)i * g.ny + j];
+  const bool forced = rk.f[0] && (!rk.fline || rk.fline[(size_t)i * g.ny + j]);
   const cplx z = c_make(0.0, 0.0);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -762,7 +774,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
       c_put<true>(&rk.out[0][s], rk_update(rk.c[0][s], rk.v[0][s], n0, forced ? rk.f[0][s] : z, kk2, rk.nu, rk.dt, rk.rmp));
       c_put<true>(&rk.out[1][s], rk_update(rk.c[1][s], rk.v[1][s], n1, forced ? rk.f[1][s] : z, kk2, rk.nu, rk.dt, rk.rmp));
       c_put<true>(&rk.out[2][s], rk_update(rk.c[2][s], rk.v[2][s], n2, forced ? rk.f[2][s] : z, kk2, rk.nu, rk.dt, rk.rmp));
-    } else if (!prune || kn2 < g.tiny) {
+    } else if (prune != 1 || kn2 < g.tiny) {
       // outside the kept modes; the k = 0 mode is written in pruned passes
       // too, since the next substep's inverse reads it from this output
       c_put<true>(&rk.out[0][s], z);
@@ -793,13 +805,25 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
   xcd_tile(bx, by);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
+  // prune == 2: the output buffers held something else, so the lines outside
+  // the dealias disc are zeroed here instead of being known to be zero
+  if (prune == 2 && j < g.ny && !((lmask >> lt) & 1u)) {
+    const size_t s0 = ((size_t)i * g.ny + j) * N;
+#pragma unroll 1
+    for (int m = 0; m < E; ++m) {
+      rk.out[0][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[1][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[2][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[3][s0 + t + T * m] = c_make(0.0, 0.0);
+    }
+  }
   if (lmask == 0u) return;  // uniform over the block
   const bool ok = j < g.ny && ((lmask >> lt) & 1u);
   const int stride = lds_line_stride(N);
   cplx *row = lds + lt * stride;
   const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j < g.ny ? j : 0, g.ny, g.dky);
   const size_t sline = ((size_t)i * g.ny + (ok ? j : 0)) * N;
-  const bool forced = ok && rk.fline && rk.fline[(size_t)i * g.ny + j];
+  const bool forced = ok && rk.f[0] && (!rk.fline || rk.fline[(size_t)i * g.ny + j]);
   const cplx z = c_make(0.0, 0.0);
   // v_z as the nonlinear term saw it, for the heat current: with ord = 1 the
   // update writes over the input (out == v) before the temperature is done.
@@ -831,7 +855,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
           rk.out[0][s] = rk_update(rk.c[0][s], rk.v[0][s], n0, forced ? rk.f[0][s] : z, kk2, rk.nu, rk.dt, rk.rmp);
           rk.out[1][s] = rk_update(rk.c[1][s], rk.v[1][s], n1, forced ? rk.f[1][s] : z, kk2, rk.nu, rk.dt, rk.rmp);
           rk.out[2][s] = rk_update(rk.c[2][s], rk.v[2][s], n2, forced ? rk.f[2][s] : z, kk2, rk.nu, rk.dt, rk.rmp);
-        } else if (!prune || kn2 < g.tiny) {
+        } else if (prune != 1 || kn2 < g.tiny) {
           rk.out[0][s] = z;
           rk.out[1][s] = z;
           rk.out[2][s] = z;
@@ -857,7 +881,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
                                rk.rmp);
     } else if (kn2 < g.tiny) {
       rk.out[3][s] = rk.c[3][s];
-    } else if (!prune) {
+    } else if (prune != 1) {
       rk.out[3][s] = z;
     }
   }
@@ -881,6 +905,17 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
   xcd_tile(bx, by);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
+  // prune == 2: the output buffers held something else, so the lines outside
+  // the dealias disc are zeroed here instead of being known to be zero
+  if (prune == 2 && j < g.ny && !((lmask >> lt) & 1u)) {
+    const size_t s0 = ((size_t)i * g.ny + j) * N;
+#pragma unroll 1
+    for (int m = 0; m < E; ++m) {
+      rk.out[(PART == 0 ? 0 : 3)][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[(PART == 0 ? 1 : 4)][s0 + t + T * m] = c_make(0.0, 0.0);
+      rk.out[(PART == 0 ? 2 : 5)][s0 + t + T * m] = c_make(0.0, 0.0);
+    }
+  }
   if (lmask == 0u) return;  // uniform over the block
   const bool ok = j < g.ny && ((lmask >> lt) & 1u);
   const int stride = lds_line_stride(N);
@@ -918,7 +953,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
   const double coef = PART == 0 ? rk.nu : rk.mu;
   const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j, g.ny, g.dky);
   const size_t sline = ((size_t)i * g.ny + j) * N;
-  const bool forced = rk.fline && rk.fline[(size_t)i * g.ny + j];
+  const bool forced = rk.f[c0] && (!rk.fline || rk.fline[(size_t)i * g.ny + j]);
   const cplx z = c_make(0.0, 0.0);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -940,7 +975,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
       upd(0, n0);
       upd(1, n1);
       upd(2, n2);
-    } else if (!prune || kn2 < g.tiny) {  // the k = 0 mode: as in k_zfwd_rk_hd
+    } else if (prune != 1 || kn2 < g.tiny) {  // the k = 0 mode: as in k_zfwd_rk_hd
       rk.out[c0][s] = z;
       rk.out[c0 + 1][s] = z;
       rk.out[c0 + 2][s] = z;
@@ -958,8 +993,9 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
 // ---------------------------------------------------------------------------
 template <int N, typename Cfg = FFTCfg<N>>
 __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf, GridK g, int nxp,
-                                             const cplx *__restrict__ twt, int kxlim, int prune) {
+                                             const cplx *__restrict__ twt, int prune_) {
   using F = LineFFT<N, +1, Cfg>;
+  const int prune = prune_input(g, prune_), kxlim = prune ? g.kxact : g.nxh;
   constexpr int T = F::T, E = F::E;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
@@ -1013,8 +1049,9 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
 
 template <int N, typename Cfg = FFTCfg<N>>
 __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf, GridK g, int nxp,
-                                             const cplx *__restrict__ twt, int kxlim, int prune) {
+                                             const cplx *__restrict__ twt, int prune) {
   using F = LineFFT<N, -1, Cfg>;
+  const int kxlim = prune ? g.kxact : g.nxh;
   constexpr int T = F::T, E = F::E;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
@@ -1548,7 +1585,8 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, i
 // (A_x, A_y), (A_z, B_x), (B_y, B_z); fields as k_xdot.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, GridK g, int nxp,
-                                              const cplx *__restrict__ twt, int kxlim) {
+                                              const cplx *__restrict__ twt, int prune) {
+  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfg<NX>;
   using FI = LineFFT<NX, +1>;
   using FF = LineFFT<NX, -1>;
@@ -1579,7 +1617,7 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
   for (int m = 0; m < E; ++m)
     z0[m] = c_make(((z0[m].x * z1[m].y + z0[m].y * z2[m].x) + z1[m].x * z2[m].y) * tmp, 0.0);
   FF::run(z0, buf, t, tw);
-  xpair_store1<NX, E, T>(z0, t, out.p[0] + off, kxlim);
+  xpair_store1<NX, E, T>(z0, t, out.p[0] + off, kxout);
 }
 
 // Fused X^-1 . (P x Q)/N^6 . X with two-for-one transforms: pairs (P_x, P_y),
@@ -1588,7 +1626,8 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
 // T <= 64 lanes.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
-                                                const cplx *__restrict__ twt, int kxlim) {
+                                                const cplx *__restrict__ twt, int prune) {
+  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfg<NX>;
   using FI = LineFFT<NX, +1>;
   using FF = LineFFT<NX, -1>;
@@ -1628,9 +1667,9 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
     z1[m] = c_make(oz, 0.0);
   }
   FF::run(z0, buf, t, tw);
-  xpair_store2<NX, E, T>(z0, buf, t, out.p[0] + off, out.p[1] + off, kxlim);
+  xpair_store2<NX, E, T>(z0, buf, t, out.p[0] + off, out.p[1] + off, kxout);
   FF::run(z1, buf, t, tw);
-  xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxlim);
+  xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxout);
 }
 
 // Fused X^-1 . (P x Q)/N^6 . X on P rows with GHOST's operand order
@@ -1642,7 +1681,8 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
 template <int N, int W, int SB>
 __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) void k_xcross(
     FieldSet in_, FieldSet out_, GridK g, int nxp, const cplx *__restrict__ twh, const cplx *__restrict__ twx,
-    int kxlim) {
+    int prune) {
+  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T, E = Cfg::E;
   extern __shared__ cplx lds[];
@@ -1654,7 +1694,7 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) 
   if constexpr (T <= 64) {
     if (!ok) return;
   }
-  const int lim = ok ? kxlim : 0;
+  const int lim = ok ? kxlim : 0, lout = ok ? kxout : 0;
   const size_t off = (size_t)(ok ? r : 0) * nxp;
   cplx *buf = lds + lt * lds_line_stride(N);
   const double tmp = g.inv_n6;
@@ -1696,7 +1736,7 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) 
       oz[m] = c_make((az[m].x - qx[m].x * py[m].x) * tmp, (az[m].y - qx[m].y * py[m].y) * tmp);
       az[m] = c_make(py[m].x * qz[m].x, py[m].y * qz[m].y);  // now P_y Q_z
     }
-    xrow_fwd<N, E, Cfg>(oz, buf, t, tw, out.p[2] + off, lim);
+    xrow_fwd<N, E, Cfg>(oz, buf, t, tw, out.p[2] + off, lout);
   }
   GHX_PHASE();
   {
@@ -1709,9 +1749,9 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) 
       oy[m] = c_make((pz[m].x * qx[m].x - ay[m].x) * tmp, (pz[m].y * qx[m].y - ay[m].y) * tmp);
     }
     GHX_PHASE();
-    xrow_fwd<N, E, Cfg>(ox, buf, t, tw, out.p[0] + off, lim);
+    xrow_fwd<N, E, Cfg>(ox, buf, t, tw, out.p[0] + off, lout);
     GHX_PHASE();
-    xrow_fwd<N, E, Cfg>(oy, buf, t, tw, out.p[1] + off, lim);
+    xrow_fwd<N, E, Cfg>(oy, buf, t, tw, out.p[1] + off, lout);
   }
 #undef GHX_PHASE
 }
@@ -1721,7 +1761,8 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) 
 // FFT[((A_x B_x + A_y B_y) + A_z B_z) tmp] with tmp = -1/N^6.
 template <int N>
 __global__ __launch_bounds__(kRowBound) void k_xdot(FieldSet in, FieldSet out, GridK g, int nxp,
-                                             const cplx *__restrict__ twh, const cplx *__restrict__ twx, int kxlim) {
+                                             const cplx *__restrict__ twh, const cplx *__restrict__ twx, int prune) {
+  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T, E = Cfg::E;
   extern __shared__ cplx lds[];
@@ -1733,7 +1774,7 @@ __global__ __launch_bounds__(kRowBound) void k_xdot(FieldSet in, FieldSet out, G
   if constexpr (T <= 64) {
     if (!ok) return;
   }
-  const int lim = ok ? kxlim : 0;
+  const int lim = ok ? kxlim : 0, lout = ok ? kxout : 0;
   const size_t off = (size_t)(ok ? r : 0) * nxp;
   cplx *buf = lds + lt * lds_line_stride(N);
   const double tmp = -g.inv_n6;
@@ -1757,7 +1798,7 @@ __global__ __launch_bounds__(kRowBound) void k_xdot(FieldSet in, FieldSet out, G
       else acc[m] = c_make((acc[m].x + p.x) * tmp, (acc[m].y + p.y) * tmp);
     }
   }
-  xrow_fwd<N, E, Cfg>(acc, buf, t, tw, out.p[0] + off, lim);
+  xrow_fwd<N, E, Cfg>(acc, buf, t, tw, out.p[0] + off, lout);
 }
 
 // ---------------------------------------------------------------------------
@@ -1765,17 +1806,6 @@ __global__ __launch_bounds__(kRowBound) void k_xdot(FieldSet in, FieldSet out, G
 // ---------------------------------------------------------------------------
 
 
-#if GHX_PART == 1
-int active_kx(const GridK &g) {
-  int n = 0;
-  for (int q = 0; q < g.nxh; ++q) {
-    double kx = (double)(q < g.nx / 2 ? q : q - g.nx);
-    if (g.rmp * (kx * kx) <= g.kmax) n = q + 1;
-  }
-  return n;
-}
-
-#endif
 
 #if GHX_PART == 2
 // 512-point z lines on the 16-points-per-lane schedule: 8-line tiles (128-byte
@@ -2003,8 +2033,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 #if GHX_PART == 1
 // the y passes on the four-points-per-lane schedule (FFTCtx::sched bit 1)
 template <int N>
-static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int kxlim,
-                               int prune) {
+static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
@@ -2015,32 +2044,31 @@ static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet
   if (inv) {
     allow_lds(k_yinv<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yinv<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, kxlim, prune);
+    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune);
   } else {
     allow_lds(k_yfwd<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yfwd<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, kxlim, prune);
+    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune);
   }
   return hipGetLastError();
 }
-static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int kxlim, int prune,
+static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune,
                   hipError_t *err) {
   if (!(c.sched & 2)) return false;
   switch (c.gk.ny) {
-  case 32: *err = launch_y_low<32>(c, inv, nf, in, out, kxlim, prune); return true;
-  case 64: *err = launch_y_low<64>(c, inv, nf, in, out, kxlim, prune); return true;
-  case 128: *err = launch_y_low<128>(c, inv, nf, in, out, kxlim, prune); return true;
-  case 256: *err = launch_y_low<256>(c, inv, nf, in, out, kxlim, prune); return true;
+  case 32: *err = launch_y_low<32>(c, inv, nf, in, out, prune); return true;
+  case 64: *err = launch_y_low<64>(c, inv, nf, in, out, prune); return true;
+  case 128: *err = launch_y_low<128>(c, inv, nf, in, out, prune); return true;
+  case 256: *err = launch_y_low<256>(c, inv, nf, in, out, prune); return true;
   default: return false;  // the same schedule either way, or the wide 512-point pass
   }
 }
 
 hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
   const int nxp = p_row(g);
   hipError_t lerr;
-  if (y_low(c, true, nf, in, out, kxlim, prune, &lerr)) return lerr;
+  if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;
   switch (g.ny) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
@@ -2056,14 +2084,14 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
       GHX_LAUNCH_CHECK((k_yinv<n_, FFTCfgWide<n_>>), s, kTileBound, TW, true);               \
       allow_lds(k_yinv<n_, FFTCfgWide<n_>>, lds);                                            \
       hipLaunchKernelGGL((k_yinv<n_, FFTCfgWide<n_>>), grid, dim3(L * TW), lds, c.stream, in, out, nf, g, nxp, \
-                         c.tw_y, kxlim, prune);                                              \
+                         c.tw_y, prune);                                              \
       break;                                                                                 \
     }                                                                                        \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, 8), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
     allow_lds(k_yinv<n_>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yinv<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, kxlim, prune); \
+    GHX_LAUNCH_CHECK((k_yinv<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2076,10 +2104,9 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
   const int nxp = p_row(g);
   hipError_t lerr;
-  if (y_low(c, false, nf, in, out, kxlim, prune, &lerr)) return lerr;
+  if (y_low(c, false, nf, in, out, prune, &lerr)) return lerr;
   switch (g.ny) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
@@ -2088,7 +2115,7 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
     allow_lds(k_yfwd<n_>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yfwd<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, kxlim, prune); \
+    GHX_LAUNCH_CHECK((k_yfwd<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2105,7 +2132,7 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out, int prune) {
   const GridK &g = c.gk;
   if (g.nx % 2) return hipErrorInvalidValue;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
+  const int kxlim = prune == 1 ? g.kxact : g.nxh;
   RealSet rs;
   for (int f = 0; f < nf; ++f) rs.p[f] = out[f];
   const long nrows = (long)g.nz * g.ny;
@@ -2147,7 +2174,7 @@ hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out,
 hipError_t xinv3i(const FFTCtx &c, const FieldSet &in, double *out, int prune) {
   const GridK &g = c.gk;
   if (g.nx % 2) return hipErrorInvalidValue;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
+  const int kxlim = prune == 1 ? g.kxact : g.nxh;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
   if (use_x2(g.nx)) {
@@ -2254,7 +2281,6 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
   (void)mode;
   const GridK &g = c.gk;
   if (g.nx % 2) return hipErrorInvalidValue;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
   if (use_x2(g.nx)) {
@@ -2265,7 +2291,7 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                                      \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xcross2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, kxlim);                                                                 \
+    GHX_LAUNCH_CHECK((k_xcross2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
@@ -2282,10 +2308,10 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);               \
     switch (tile_want("GHX_XV", 1)) {                                                       \
-    case 4: GHX_LAUNCH_CHECK((k_xcross<n_, 2, 1>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, 2, 1>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kxlim); break; \
+    case 4: GHX_LAUNCH_CHECK((k_xcross<n_, 2, 1>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, 2, 1>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); break; \
     /* 3 * 2^k rows: one wave per SIMD leaves the registers to hold the six */ \
     /* fields without scratch (7.5% faster on the ensemble's 48^3 and 96^3) */ \
-    default: GHX_LAUNCH_CHECK((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kxlim); break; \
+    default: GHX_LAUNCH_CHECK((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); break; \
     }                                                                                       \
     break;                                                                                  \
   }
@@ -2305,7 +2331,6 @@ namespace ghx {
 hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   if (g.nx % 2) return hipErrorInvalidValue;
-  const int kxlim = prune ? active_kx(g) : g.nxh;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
   if (use_x2(g.nx)) {
@@ -2316,7 +2341,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                                      \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xdot2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, kxlim);                                                                 \
+    GHX_LAUNCH_CHECK((k_xdot2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
@@ -2331,7 +2356,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                                      \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
-    GHX_LAUNCH_CHECK((k_xdot<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kxlim); \
+    GHX_LAUNCH_CHECK((k_xdot<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)

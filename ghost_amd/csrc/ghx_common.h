@@ -58,7 +58,19 @@ struct GridK {
   double rmp, rmq, rms;   // kn2 weights (1/n^2 when anisotropic, else 1)
   double kmax, tiny;
   double inv_n6;          // 1/(nx ny nz)^2
+  int kxact;              // number of kx indices (from 0) with kn2(kx,0,0) <= kmax
+  // prune == 2 (a substep on fields not known to be dealiased): a device word
+  // that is zero when the input turned out to be zero outside the kept modes
+  // (null: not looked at, taken as non-zero)
+  const unsigned *dirty;
 };
+
+// What a pass over the input of a substep skips: prune 0 nothing, 1 whatever
+// lies outside the dealias set, 2 that too if the dirty word allows it.
+// Passes over its output skip for 1 and 2 alike (only kept modes are used).
+GHX_DEV int prune_input(const GridK &g, int prune) {
+  return prune == 2 ? (g.dirty && *g.dirty == 0u ? 1 : 0) : prune;
+}
 
 // kn2 and kk2 exactly as GHOST forms them (no fused multiply-add, so the
 // dealias mask matches bit for bit): main3D.fpp:1764-1800.

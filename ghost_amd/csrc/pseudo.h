@@ -56,6 +56,10 @@ hipError_t op_tg_real(const GridK &g, hipStream_t st, double *r1, double *r2, in
 size_t reduce_work_doubles();
 hipError_t op_reduce(const GridK &g, hipStream_t st, int kind, const cplx *a, const cplx *b, const cplx *c,
                      const cplx *d, const cplx *e, const cplx *f, double *work, double *out);
+// *flag (device) = 0 if every one of the nf <= 6 fields is zero outside
+// tiny <= kn2 <= kmax, else non-zero; fields from `mean` on may be non-zero
+// below tiny.
+hipError_t op_unkept(const GridK &g, hipStream_t st, const cplx *const *v, int nf, int mean, unsigned *flag);
 // hdcheck's sums of v and the force f: out[5] host = <v^2>, <omega^2>, <v.f>,
 // helicity, <(div v)^2>; work as for op_reduce.
 hipError_t op_hdcheck(const GridK &g, hipStream_t st, const cplx *const *v, const cplx *const *f, double *work,

@@ -475,6 +475,26 @@ __global__ __launch_bounds__(kBlock) void k_reduce(GridK g, const cplx *a, const
   if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
+// Sets *flag where a field holds something outside the kept modes (op_unkept);
+// reads only those modes.
+struct V6 {
+  const cplx *p[6];
+};
+__global__ __launch_bounds__(kBlock) void k_unkept(GridK g, V6 v, int nf, int mean, unsigned *flag) {
+  bool on = false;
+  for_modes(g, [&](const Idx &q, size_t m) {
+    const double kn2 = kn2_of(g, q.i, q.j, q.k);
+    if (kn2 <= g.kmax && kn2 >= g.tiny) return;
+    const int n = kn2 < g.tiny ? mean : nf;
+    for (int f = 0; f < n; ++f) {
+      const cplx x = v.p[f][m];
+      on = on || x.x != 0.0 || x.y != 0.0;
+    }
+  });
+  if (__ballot(on) != 0 && threadIdx.x % 64 == 0) atomicOr(flag, 1u);
+}
+__global__ void k_clear_word(unsigned *p) { *p = 0u; }
+
 // hdcheck's five sums (pseudospec3D_hd.f90:984-1105) in one pass over v =
 // (a, b, c) and the force (d, e, f): part[q * gridDim.x + block] for q =
 // <v^2>, <omega^2>, <v.f>, the helicity and <(div v)^2>.  Bound by the six
@@ -933,6 +953,14 @@ hipError_t op_hdcheck(const GridK &g, hipStream_t st, const cplx *const *v, cons
   double *res = work + 5 * kRedBlocks;
   hipLaunchKernelGGL(k_sum_partials, dim3(5), dim3(kBlock), 0, st, work, (int)nb, res);
   return to_host(out, res, 5, st);
+}
+
+hipError_t op_unkept(const GridK &g, hipStream_t st, const cplx *const *v, int nf, int mean, unsigned *flag) {
+  V6 p;
+  for (int f = 0; f < 6; ++f) p.p[f] = f < nf ? v[f] : nullptr;
+  hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, st, flag);
+  hipLaunchKernelGGL(k_unkept, dim3(walk_blocks(g, kRedBlocks)), dim3(kBlock), 0, st, g, p, nf, mean, flag);
+  return hipGetLastError();
 }
 
 static unsigned spectrum_blocks(const GridK &g) {
