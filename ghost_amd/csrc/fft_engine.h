@@ -42,18 +42,18 @@ GHX_FFTCFG(10, 10, 2, 5, 2)
 GHX_FFTCFG(12, 12, 2, 3, 4)
 GHX_FFTCFG(16, 8, 2, 2, 8)
 GHX_FFTCFG(20, 20, 2, 5, 4)
-GHX_FFTCFG(24, 6, 4, 3, 2, 2, 2)
+GHX_FFTCFG(24, 6, 3, 6, 2, 2)
 GHX_FFTCFG(32, 8, 2, 4, 8)
 GHX_FFTCFG(40, 40, 2, 5, 8)
-GHX_FFTCFG(48, 6, 5, 3, 2, 2, 2, 2)
+GHX_FFTCFG(48, 6, 4, 6, 2, 2, 2)
 GHX_FFTCFG(64, 8, 2, 8, 8)
 GHX_FFTCFG(80, 40, 3, 5, 2, 8)
-GHX_FFTCFG(96, 6, 6, 3, 2, 2, 2, 2, 2)
+GHX_FFTCFG(96, 6, 5, 6, 2, 2, 2, 2)
 GHX_FFTCFG(128, 8, 3, 2, 8, 8)
 GHX_FFTCFG(160, 40, 3, 5, 4, 8)
-GHX_FFTCFG(192, 6, 7, 3, 2, 2, 2, 2, 2, 2)
+GHX_FFTCFG(192, 6, 6, 6, 2, 2, 2, 2, 2)
 GHX_FFTCFG(256, 8, 3, 4, 8, 8)
-GHX_FFTCFG(384, 6, 8, 3, 2, 2, 2, 2, 2, 2, 2)
+GHX_FFTCFG(384, 6, 7, 6, 2, 2, 2, 2, 2, 2)
 GHX_FFTCFG(512, 8, 3, 8, 8, 8)
 GHX_FFTCFG(768, 24, 4, 3, 4, 8, 8)
 GHX_FFTCFG(1024, 8, 4, 2, 8, 8, 8)
@@ -88,6 +88,28 @@ template <> struct FFTCfgWide<512> {
   static constexpr int T = 512 / 16;
   GHX_DEV static constexpr int radix(int) { return 8; }
 };
+
+// 12 points per lane for the 3 * 2^k lines: half the stages (and LDS
+// exchanges) of the 6-point schedules at twice the registers per field, for
+// passes that keep one field live (the y passes).  Those that hold three
+// fields spill on it or lose a wave per SIMD: measured at 192^3, the curl z
+// inverse 53 -> 75, the fused x pass 132 -> 157 us.  24 and 48 points gain
+// nothing (YInvCfg, YFwdCfg).
+template <int N> struct FFTCfgMid : FFTCfg<N> {};
+#define GHX_FFTCFGMID(N_, NS_, ...)                                     \
+  template <> struct FFTCfgMid<N_> {                                    \
+    static constexpr int E = 12;                                        \
+    static constexpr int NS = NS_;                                      \
+    static constexpr int T = N_ / 12;                                   \
+    GHX_DEV static constexpr int radix(int s) {                         \
+      constexpr int r[] = {__VA_ARGS__};                                \
+      return r[s];                                                      \
+    }                                                                   \
+  };
+GHX_FFTCFGMID(96, 3, 12, 4, 2)
+GHX_FFTCFGMID(192, 3, 12, 4, 4)
+GHX_FFTCFGMID(384, 4, 12, 4, 4, 2)
+#undef GHX_FFTCFGMID
 #undef GHX_FFTCFG
 
 // ---------------------------------------------------------------------------
@@ -137,6 +159,43 @@ template <int DIR> struct SmallDFT<5, DIR> {
     v[0] = c_add(v[0], c_add(t1, t2));
     v[1] = c_add(a1, b1); v[4] = c_sub(a1, b1);
     v[2] = c_add(a2, b2); v[3] = c_sub(a2, b2);
+  }
+};
+// 6 = 3 x 2 and 12 = 3 x 4 by the prime-factor (Good-Thomas) maps, which need
+// no twiddles between the factors: with n = 2a + 3b, k = 4c + 3d (mod 6),
+// nk = 2ac + 3bd; with n = 4a + 3b, k = 4c + 9d (mod 12), nk = 4ac + 3bd.
+template <int DIR> struct SmallDFT<6, DIR> {
+  GHX_DEV static void run(cplx *v) {
+    cplx x[2][3];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) x[b][a] = v[(2 * a + 3 * b) % 6];
+      SmallDFT<3, DIR>::run(x[b]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      v[(4 * c) % 6] = c_add(x[0][c], x[1][c]);
+      v[(4 * c + 3) % 6] = c_sub(x[0][c], x[1][c]);
+    }
+  }
+};
+template <int DIR> struct SmallDFT<12, DIR> {
+  GHX_DEV static void run(cplx *v) {
+    cplx x[4][3];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) x[b][a] = v[(4 * a + 3 * b) % 12];
+      SmallDFT<3, DIR>::run(x[b]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      cplx y[4] = {x[0][c], x[1][c], x[2][c], x[3][c]};
+      SmallDFT<4, DIR>::run(y);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[(4 * c + 9 * d) % 12] = y[d];
+    }
   }
 };
 template <int DIR> struct SmallDFT<8, DIR> {

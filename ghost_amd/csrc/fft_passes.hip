@@ -6,6 +6,8 @@
 // kz-contiguous spectral layout S.  The transposes are fused into the first
 // (load) or last (store) step of the x and z passes; global accesses are
 // either whole contiguous lines or L-point chunks along ky (L*16 bytes).
+#include <type_traits>
+
 #include "fft_engine.h"
 #include "fft_passes.h"
 
@@ -203,6 +205,10 @@ static bool use_x2(int nx) {
   if (env_switch("GHX_XC2", 1) != 1) return false;
   return x2_size(nx);
 }
+
+// Built-in tile width: `lines`, or as many more as fill a wavefront (a line of
+// few lanes would leave half or more of it idle: 4 lines of 8 lanes).
+static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
 
 template <typename K> static void allow_lds(K kern, size_t bytes) {
   if (bytes > 49152) (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -1083,16 +1089,20 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
       w[q] = inside ? x : c_make(0.0, 0.0);
     }
   };
+  constexpr bool prefetch = E <= 8;  // as in k_yinv
   cplx nxt[E];
-  tload(0, nxt);
+  if constexpr (prefetch) tload(0, nxt);
   for (int f = 0; f < nf; ++f) {
+    if constexpr (!prefetch) tload(f, nxt);
 #pragma unroll
     for (int q = 0; q < E; ++q) {
       const int idx = threadIdx.x + q * blockDim.x;
       lds[(idx % L) * stride + lds_pad(idx / L)] = nxt[q];
     }
     __syncthreads();
-    if (f + 1 < nf) tload(f + 1, nxt);
+    if constexpr (prefetch) {
+      if (f + 1 < nf) tload(f + 1, nxt);
+    }
     cplx v[E];
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = row[lds_pad(t + T * m)];
@@ -1426,7 +1436,7 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int kxlim) {
   using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1>;
+  using FI = LineFFT<NX, +1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1436,7 +1446,7 @@ __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, i
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp, roff = (size_t)r * NX;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx a[E], b[E], z[E];
   const int np = (nf + 1) / 2;
@@ -1466,7 +1476,7 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int kxlim) {
   using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1>;
+  using FI = LineFFT<NX, +1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1476,7 +1486,7 @@ __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out,
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx a[E], b[E], z0[E], z1[E];
   xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
@@ -1503,7 +1513,7 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part, GridK g, int nxp,
                                                       const cplx *__restrict__ twt, int kxlim) {
   using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1>;
+  using FI = LineFFT<NX, +1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1512,7 +1522,7 @@ __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part,
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
   const long nrows = (long)g.nz * g.ny, hop = (long)gridDim.x * rpb;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   double big = 0.0;
   long r = (long)blockIdx.x * rpb + lt;
@@ -1550,7 +1560,7 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt) {
   using Cfg = FFTCfg<NX>;
-  using FF = LineFFT<NX, -1>;
+  using FF = LineFFT<NX, -1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1560,7 +1570,7 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, i
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp, roff = (size_t)r * NX;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx z[E], nxt[E];
   const int np = (nf + 1) / 2;
@@ -1588,8 +1598,8 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
                                               const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1>;
-  using FF = LineFFT<NX, -1>;
+  using FI = LineFFT<NX, +1, Cfg>;
+  using FF = LineFFT<NX, -1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1600,7 +1610,7 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
   const size_t off = (size_t)r * nxp;
   cplx *buf = lds + lt * lds_line_stride(NX);
   const double tmp = -g.inv_n6;
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx a[E], b[E], z0[E], z1[E], z2[E];
   xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
@@ -1629,8 +1639,8 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
                                                 const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1>;
-  using FF = LineFFT<NX, -1>;
+  using FI = LineFFT<NX, +1, Cfg>;
+  using FF = LineFFT<NX, -1, Cfg>;
   constexpr int T = Cfg::T, E = Cfg::E;
   static_assert(T <= 64, "one row per wavefront or less");
   extern __shared__ cplx lds[];
@@ -1644,7 +1654,7 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
   const double tmp = g.inv_n6;
   const FieldView in = batch_view(in_, blockIdx.y);
   const FieldView out = batch_view(out_, blockIdx.y);
-  TwCache<NX> tw;
+  TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx a[E], b[E], z0[E], z1[E], z2[E];
   xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
@@ -1832,7 +1842,7 @@ static hipError_t launch_zinv_low(const FFTCtx &c, int nf, const FieldSet &in, c
   const GridK &g = c.gk;
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
-  const PassShape s = tile_shape(T, lds_line_stride(N), g.ny, tile_pick("GHX_LZ", c.tile_z, 4), max_lds());
+  const PassShape s = tile_shape(T, lds_line_stride(N), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds());
   const int L = s.lines;
   dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);
   allow_lds(k_zinv<N, 1, Cfg>, s.lds);
@@ -1863,7 +1873,7 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, mode == 0 || mode == 7 ? 8 : 4), max_lds()); \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, mode == 0 || mode == 7 ? 8 : 4)), max_lds()); \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
     if (mode == 0) {                                                                        \
@@ -1910,7 +1920,7 @@ hipError_t zfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", 8), max_lds());                                        \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 8)), max_lds());                                        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
     allow_lds(k_zfwd<n_>, lds);                                                             \
@@ -1946,7 +1956,7 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
   case n_: {                                                                                            \
     using Cfg = FFTCfgLow<n_>;                                                                          \
     constexpr int T = Cfg::T;                                                                           \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, 4), max_lds()); \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds()); \
     const int L = s.lines;                                                                              \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                                      \
     if (pf) {                                                                                           \
@@ -1970,7 +1980,7 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, 4), max_lds());         \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds());         \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
     allow_lds(k_zfwd_rk_hd<n_>, lds);                                                       \
@@ -1999,7 +2009,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
     if constexpr (FFTCfgLow<n_>::E != FFTCfg<n_>::E) if (low) {                              \
       using Cl = FFTCfgLow<n_>;                                                              \
       constexpr int T = Cl::T;                                                               \
-      const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", 4), max_lds()); \
+      const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds()); \
       const int L = s.lines; const size_t lds = s.lds;                                       \
       dim3 grid((g.ny + L - 1) / L, g.nxh);                                                  \
       allow_lds(k_zfwd_rk_mhd<n_, 0, Cl>, lds);                                              \
@@ -2011,7 +2021,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
       break;                                                                                 \
     }                                                                                        \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", 4), max_lds());                                        \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds());                                        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
     allow_lds(k_zfwd_rk_mhd<n_, 0>, lds);                                                   \
@@ -2031,6 +2041,14 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 #endif
 
 #if GHX_PART == 1
+// 12 points per lane for the long 3 * 2^k lines.  The lines below are latency,
+// not LDS: measured in one session, y inverse of six fields 100 -> 72 us at
+// 192^3 and 23 -> 20 at 96^3 but 14 -> 15 at 48^3; y forward of three
+// (without the prefetch, 8-line tiles) 47 -> 42 at 192^3 but 12 -> 13 at 96^3.
+template <int N>
+using YInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 96), FFTCfgMid<N>, FFTCfg<N>>::type;
+template <int N>
+using YFwdCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
 // the y passes on the four-points-per-lane schedule (FFTCtx::sched bit 1)
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
@@ -2038,7 +2056,7 @@ static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
   const int nxp = p_row(g);
-  const PassShape s = tile_shape(T, lds_line_stride(N), g.nxh, tile_pick("GHX_LY", c.tile_y, inv ? 8 : 4), max_lds());
+  const PassShape s = tile_shape(T, lds_line_stride(N), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, inv ? 8 : 4)), max_lds());
   const int L = s.lines;
   dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);
   if (inv) {
@@ -2072,7 +2090,8 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
   switch (g.ny) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
-    constexpr int T = FFTCfg<n_>::T;                                                        \
+    using Cfg = YInvCfg<n_>;                                                                \
+    constexpr int T = Cfg::T;                                                               \
     if constexpr (FFTCfgWide<n_>::E != FFTCfg<n_>::E)                                        \
     if (env_switch("GHX_YWIDE", 1) == 1 &&                                                   \
         wide_shape(FFTCfgWide<n_>::T, lds_line_stride(n_), g.nxh).lds <= max_lds()) {         \
@@ -2087,11 +2106,11 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
                          c.tw_y, prune);                                              \
       break;                                                                                 \
     }                                                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, 8), max_lds());        \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, 8)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
-    allow_lds(k_yinv<n_>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yinv<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
+    allow_lds(k_yinv<n_, Cfg>, lds);                                                             \
+    GHX_LAUNCH_CHECK((k_yinv<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2110,12 +2129,13 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
   switch (g.ny) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
-    constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, 4), max_lds());        \
+    using Cfg = YFwdCfg<n_>;                                                                \
+    constexpr int T = Cfg::T;                                                               \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, Cfg::E == 12 ? 8 : 4)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
-    allow_lds(k_yfwd<n_>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yfwd<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
+    allow_lds(k_yfwd<n_, Cfg>, lds);                                                             \
+    GHX_LAUNCH_CHECK((k_yfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2373,7 +2393,7 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_) + n_, g.ny, tile_want("GHX_LZ", 4), max_lds());              \
+    const PassShape s = tile_shape(T, lds_line_stride(n_) + n_, g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds());              \
     const int L = s.lines; const size_t lds = s.lds;                     \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
     allow_lds(k_zfwd_rk_bouss<n_>, lds);                                                    \
