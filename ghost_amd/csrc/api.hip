@@ -188,7 +188,8 @@ extern "C" int ghx_prof_read(int slot, const char **name, int *count, double *to
 struct ghx_plan {
   int nx, ny, nz, nxh, dir;
   FFTCtx ctx;
-  cplx *tw = nullptr;       // all twiddle tables
+  cplx *tw = nullptr;       // all twiddle tables, then the word below
+  unsigned *word = nullptr;  // device word of the substeps on caller fields (GridK::dirty)
   cplx *q = nullptr;        // Q scratch, q_fields fields
   int q_fields = 0;
   bool timing = false;
@@ -248,7 +249,8 @@ static int plan_init(ghx_plan *p, int nx, int ny, int nz, int dir) {
   fill_tw(h, nx / 2, nx);
   fill_tw(h, nx / 2 + nx, ny);
   fill_tw(h, nx / 2 + nx + ny, nz);
-  HIPCHK(hipMalloc(&p->tw, h.size() * sizeof(cplx)));
+  HIPCHK(hipMalloc(&p->tw, h.size() * sizeof(cplx) + 256));
+  p->word = reinterpret_cast<unsigned *>(p->tw + h.size());
   HIPCHK(hipMemcpy(p->tw, h.data(), h.size() * sizeof(cplx), hipMemcpyHostToDevice));
   p->ctx.gk = make_gridk(nx, ny, nz, 0, 1, 1, 1);
   p->ctx.tw_xh = p->tw;
@@ -452,7 +454,6 @@ struct ghx_grid {
   double *rtmp = nullptr;   // real temporaries
   int rtmp_fields = 0;
   size_t nc = 0, nr = 0;
-  unsigned *dirty = nullptr;  // device word of the substeps on caller fields (GridK::dirty)
   double ps[3] = {1, 1, 1};  // pruned shares (rows, lines, modes), computed on first use
   bool ps_valid = false;
 };
@@ -492,7 +493,6 @@ extern "C" int ghx_grid_create(ghx_grid **grid, int nx, int ny, int nz, double L
   ghx_grid *g = new (std::nothrow) ghx_grid();
   if (!g) return set_err(GHX_ERR_NOMEM, "host allocation failed");
   int rc = plan_init(&g->plan, nx, ny, nz, GHX_FFTW_REAL_TO_COMPLEX);
-  if (!rc && hipMalloc(&g->dirty, 256) != hipSuccess) rc = set_err(GHX_ERR_NOMEM, "grid: device allocation");
   if (rc) { plan_release(&g->plan); delete g; return rc; }
   GridK k = make_gridk(nx, ny, nz, arbsize, Lx, Ly, Lz);
   // Dkk, nmax, tiny: main3D.fpp:905-909, 1728-1735
@@ -517,7 +517,6 @@ extern "C" int ghx_grid_destroy(ghx_grid *g) {
   if (g->work) (void)hipFree(g->work);
   if (g->ctmp) (void)hipFree(g->ctmp);
   if (g->rtmp) (void)hipFree(g->rtmp);
-  if (g->dirty) (void)hipFree(g->dirty);
   delete g;
   return GHX_OK;
 }
@@ -1584,8 +1583,8 @@ static int line_flags(ghx_grid *g, const cplx *a, const cplx *b, const cplx *c, 
 // modes of every line: marking the forced lines first read all of it, 120 us.)
 static int caller_prune() { return getenv("GHX_NO_PRUNE") ? 0 : 2; }
 static int caller_dirty(ghx_grid *g, const cplx *const *v, int nf, int mean, unsigned **dirty) {
-  HIPCHK(ghx::op_unkept(g->gk, g->stream, v, nf, mean, g->dirty));
-  *dirty = g->dirty;
+  HIPCHK(ghx::op_unkept(g->gk, g->stream, v, nf, mean, g->plan.word));
+  *dirty = g->plan.word;
   return GHX_OK;
 }
 

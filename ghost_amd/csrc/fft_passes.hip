@@ -210,6 +210,17 @@ static bool use_x2(int nx) {
 // few lanes would leave half or more of it idle: 4 lines of 8 lanes).
 static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
 
+// Launches of up to this many kept lines (13 per CU; 96^3 has 3168, 128^3
+// 5504) leave the GPU waiting on the chain inside a block, so a block is given
+// one field or one component instead of all of them in turn.  Measured at
+// 32^3, 64^3, 96^3 and 128^3 (us, with ~3 of event overhead): six-field y
+// inverse 12.9 -> 7.3, 14.4 -> 9.7, 20.6 -> 13.3, 23.8 -> 27.7; curl z inverse
+// 11.8 -> 9.4, 12.9 -> 11.7, 17.8 -> 17.4, 20.9 -> 30.1; HD update 14.2 -> 8.8,
+// 15.9 -> 10.8, 16.6 -> 13.2, 23.3 -> 24.7.
+constexpr long kSmallLines = 3328;
+static bool small_z(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch <= kSmallLines; }
+static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= kSmallLines; }
+
 template <typename K> static void allow_lds(K kern, size_t bytes) {
   if (bytes > 49152) (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
@@ -595,6 +606,98 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
   }
 }
 
+// Z^-1 with one output field per block (blockIdx.z = member * outputs + field):
+// every field of the modes above from its inputs' modes and one transform.
+// For launches too small to fill the GPU, where the fields that a block works
+// through one after another are what a pass takes: 3 loads, 6 transforms and 6
+// tile stores in turn are 12 us at 32^3 to 64^3 whatever the tile, and one of
+// each is half of that.  Inputs are read again by each block that needs them
+// (cache hits at these sizes), and a curl costs a transform more.
+// What output o of a mode is: component c of the fields from f (kind 0 the
+// field itself, 1 its derivative along c, 2 their curl, 3 the curl of their
+// curl).
+struct ZOut {
+  int kind, f, c;
+};
+GHX_DEV ZOut zinv_output(int mode, int o) {
+  switch (mode) {
+  case 1: case 5: return o < 3 ? ZOut{0, o, 0} : o < 6 ? ZOut{2, 0, o - 3} : ZOut{1, 3, o - 6};
+  case 2: return o < 3 ? ZOut{0, o, 0} : o < 6 ? ZOut{2, 0, o - 3} : o < 9 ? ZOut{2, 3, o - 6} : ZOut{3, 3, o - 9};
+  case 4: return o < 3 ? ZOut{0, o, 0} : ZOut{1, 3, o - 3};
+  case 6: return ZOut{1, o / 3, o % 3};
+  case 7: return ZOut{2, 0, o};
+  default: return ZOut{0, o, 0};
+  }
+}
+
+template <int N, typename Cfg = FFTCfg<N>>
+__global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet out_, int mode, int nout, GridK g,
+                                                 const cplx *__restrict__ twt, int prune_,
+                                                 const double *__restrict__ aux) {
+  using F = LineFFT<N, +1, Cfg>;
+  constexpr int T = F::T, E = F::E;
+  const int prune = prune_input(g, prune_);
+  extern __shared__ cplx lds[];
+  const int L = blockDim.x / T;
+  const int lt = threadIdx.x / T, t = threadIdx.x % T;
+  const int member = blockIdx.z / nout, o = blockIdx.z - member * nout;
+  const ZOut w = zinv_output(mode, o);  // the same for the whole block
+  int bx, by;
+  xcd_tile(bx, by);
+  const int i = by, j0 = bx * L, j = j0 + lt;
+  const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
+  if (lmask == 0u) return;  // uniform over the block
+  TwCache<N, Cfg> tw;
+  tw.load(twt, t);
+  const bool ok = j < g.ny && ((lmask >> lt) & 1u);
+  const int stride = lds_line_stride(N);
+  cplx *row = lds + lt * stride;
+  const size_t sline = ((size_t)i * g.ny + (ok ? j : 0)) * N;
+  const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(ok ? j : 0, g.ny, g.dky);
+  // component q of the inputs' wavenumber, q mod 3
+  auto kq = [&](int q, int m) { return q == 0 ? kx : q == 1 ? ky : wavenum(t + T * m, g.nz, g.dkz); };
+  auto load = [&](cplx (&x)[E], int f) {
+    const cplx *p = in_.p[f] + (size_t)member * in_.bstride + sline;
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int k = t + T * m;
+      const bool need = ok && (!prune || kn2_of(g, i, j, k) <= g.kmax);
+      const cplx y = p[need ? k : 0];
+      x[m] = need ? y : c_make(0.0, 0.0);
+    }
+  };
+  const int c1 = w.c == 2 ? 0 : w.c + 1, c2 = w.c == 0 ? 2 : w.c - 1;  // c + 1, c + 2 mod 3
+  cplx v[E];
+  load(v, w.kind >= 2 ? w.f + c2 : w.f);
+  if (w.kind == 1) {
+    const double sc = mode == 6 ? 1.0 / ((double)g.nx * (double)g.ny * (double)g.nz) : 1.0;
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = c_scale(c_ik(kq(w.c, m), v[m]), sc);
+  } else if (w.kind >= 2) {
+    cplx x[E];
+    load(x, w.f + c1);
+    if (w.kind == 2) {  // i k_{c+1} a_{c+2} - i k_{c+2} a_{c+1}
+#pragma unroll
+      for (int m = 0; m < E; ++m) v[m] = c_sub(c_ik(kq(c1, m), v[m]), c_ik(kq(c2, m), x[m]));
+    } else {  // the same of b = curl a
+      cplx y[E];
+      load(y, w.f + w.c);
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        const double k0 = kq(w.c, m), k1 = kq(c1, m), k2 = kq(c2, m);
+        const cplx b2 = c_sub(c_ik(k0, x[m]), c_ik(k1, y[m])), b1 = c_sub(c_ik(k2, y[m]), c_ik(k0, v[m]));
+        v[m] = c_sub(c_ik(k1, b2), c_ik(k2, b1));
+      }
+    }
+  }
+  if (mode == 3) {
+    const double sxy = aux[i] * aux[g.nxh + (ok ? j : 0)];
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = c_scale(v[m], sxy * aux[g.nxh + g.ny + t + T * m]);
+  }
+  zinv_emit<N, E, Cfg>(v, lds, row, stride, L, t, tw, out_.p[o] + (size_t)member * out_.bstride, g, i, j0, lmask);
+}
+
 // ---------------------------------------------------------------------------
 // Z forward: Q -> S.  Block = (kx index i, ky chunk).  Transposed load.
 // ---------------------------------------------------------------------------
@@ -691,6 +794,169 @@ GHX_DEV cplx rk_update(cplx cc, cplx vv, cplx nl, cplx ff, double kk2, double nu
   double lx = -kk2 * vv.x, ly = -kk2 * vv.y;
   double sx = nu * lx + nl.x + ff.x, sy = nu * ly + nl.y + ff.y;
   return c_make(cc.x + dt * sx * rmp, cc.y + dt * sy * rmp);
+}
+
+// ---------------------------------------------------------------------------
+// Z forward fused with the projection and the RK update for small launches
+// (kSmallLines) and the Boussinesq update, one group of lanes per component: the block is G x L lines x T lanes, group c transforms its
+// component's tile and updates that component.  The tiles of all components
+// and the lanes' v and C are loaded together at the start, so a block waits
+// for memory once, and the transforms run side by side; the projection reads
+// the other components' modes from their LDS rows.  On large launches the
+// kernels below, which take the components in turn, are faster (HD 110
+// against 191 us at 256^3): three groups per line leave one block per CU,
+// whose loads, transforms and stores then do not overlap.
+// KIND 0: HD (include/hd_rkstep2.f90, roth_rkstep2.f90); 1: MHD, blockIdx.z
+// the part (0 velocity from fields 0..2 minus 3..5, 1 vector potential from
+// fields 6..8); 2: Boussinesq (include/bouss_rkstep2.f90:1-71), component 3
+// the temperature.
+// ---------------------------------------------------------------------------
+struct ZUpdate {
+  double dt, rmp, om2, xmom, xtemp;
+  double nu, mu;  // mu: of the vector potential or the temperature
+  const cplx *v[6], *c[6], *f[6];
+  cplx *out[6];
+  const uint8_t *fline;
+  size_t bstride;
+  const double *nu_b;
+};
+constexpr int zrk_groups(int KIND) { return KIND == 2 ? 4 : 3; }
+constexpr unsigned zrk_bound(int KIND) { return KIND == 2 ? 512 : 768; }
+
+template <int N, int KIND, typename Cfg = FFTCfg<N>>
+__global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, const cplx *__restrict__ twt,
+                                                         ZUpdate rk, int prune) {
+  using F = LineFFT<N, -1, Cfg>;
+  constexpr int T = F::T, E = F::E, G = zrk_groups(KIND);
+  extern __shared__ cplx lds[];
+  const int GL = blockDim.x / G, L = GL / T, lsh = 31 - __builtin_clz((unsigned)L);
+  // groups are whole waves except for the shortest lines (GL < 64)
+  int c = threadIdx.x / GL;
+  if (GL % 64 == 0) c = __builtin_amdgcn_readfirstlane(c);
+  const int tid = threadIdx.x - c * GL;
+  const int lt = tid / T, t = tid % T;
+  int bx, by;
+  xcd_tile(bx, by);
+  const int i = by, j0 = bx * L, j = j0 + lt;
+  const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
+  const bool inside = j < g.ny, on = (lmask >> lt) & 1u, ok = inside && on;
+  const int part = KIND == 1 ? (int)blockIdx.z : 0;
+  const size_t bo = KIND == 0 ? (size_t)blockIdx.z * rk.bstride : 0;
+  const int ci = KIND == 1 ? 3 * part + c : c;  // this group's component of the argument arrays
+  cplx *out = rk.out[ci] + bo;
+  const size_t sline = ((size_t)i * g.ny + (inside ? j : 0)) * N;
+  if (prune == 2 && inside && !on) {
+    // the output buffers held something else: lines outside the disc are zeroed
+#pragma unroll 1
+    for (int m = 0; m < E; ++m) out[sline + t + T * m] = c_make(0.0, 0.0);
+  }
+  if (lmask == 0u) return;  // uniform over the block
+  const int stride = lds_line_stride(N);
+  cplx *rows = lds + c * L * stride, *row = rows + lt * stride;
+  TwCache<N, Cfg> tw;
+  tw.load(twt, t);
+  // the tile of this component's product
+  cplx P[E];
+  {
+    const size_t qs = (size_t)g.nxh * g.ny, qb = (size_t)i * g.ny + j0;
+    const size_t io = KIND == 0 ? (size_t)blockIdx.z * in_.bstride : 0;
+    const cplx *a = in_.p[KIND == 1 && part ? 6 + c : c] + io;
+    const cplx *b = in_.p[KIND == 1 ? 3 + c : c];  // KIND 1, part 0
+    cplx w[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const int idx = tid + q * GL, l = idx & (L - 1);
+      const bool need = j0 + l < g.ny && ((lmask >> l) & 1u);
+      const size_t o = qb + (size_t)(idx >> lsh) * qs + (need ? l : 0);
+      cplx x = a[o];
+      if constexpr (KIND == 1) {
+        if (part == 0) x = c_sub(x, b[o]);
+      }
+      w[q] = need ? x : c_make(0.0, 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const int idx = tid + q * GL;
+      rows[(idx & (L - 1)) * stride + lds_pad(idx >> lsh)] = w[q];
+    }
+  }
+  const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(inside ? j : 0, g.ny, g.dky);
+  const cplx *vp = rk.v[ci] + bo, *cp = rk.c[ci] + bo;
+  cplx vv[E], cc[E];
+  auto kept = [&](int k) { return ok && kn2_of(g, i, j, k) <= g.kmax; };
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const int k = t + T * m;
+    const size_t s = sline + (kept(k) ? k : 0);
+    vv[m] = vp[s];
+    cc[m] = cp[s];  // a second hit in the cache where C is v
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < E; ++m) P[m] = row[lds_pad(t + T * m)];
+  line_sync<T>();  // a line's row is its own from here on
+  F::run(P, row, t, tw);
+  // the other field that this component's product needs: Coriolis v_y, v_x;
+  // buoyancy th; heat current v_z
+  if constexpr (KIND != 1) {
+    const bool rot = rk.om2 != 0.0;
+    const cplx *xp = rk.v[KIND == 2 || c < 2 ? c ^ 1 : 0];
+    const double xs = c == 0 ? -rk.om2 : c == 1 ? rk.om2 : KIND == 0 ? 0.0 : c == 2 ? rk.xmom : rk.xtemp;
+    if (KIND == 2 || rot) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        const int k = t + T * m;
+        const bool need = kept(k) && (c >= 2 ? KIND == 2 : rot);
+        const cplx x = xp[bo + sline + (need ? k : 0)];
+        if (need) P[m] = c_make(P[m].x + xs * x.x, P[m].y + xs * x.y);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < E; ++m) row[lds_pad(t + T * m)] = P[m];
+  // every lane has loaded what it reads of v before any lane stores (out may
+  // be v or C), and the other components' modes are in their rows
+  __syncthreads();
+  if (!ok) return;
+  const double nu = KIND == 0 ? (rk.nu_b ? rk.nu_b[blockIdx.z] : rk.nu) : (KIND == 1 ? part != 0 : c == 3) ? rk.mu : rk.nu;
+  const cplx *fp = rk.f[ci];
+  if (fp && rk.fline && !rk.fline[(size_t)i * g.ny + j]) fp = nullptr;
+  if (fp) fp += bo;
+  const cplx *row0 = lds + lt * stride, *row1 = row0 + L * stride, *row2 = row1 + L * stride;
+  const double kd = c == 0 ? kx : ky;
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const int k = t + T * m;
+    const size_t s = sline + k;
+    const double kz = wavenum(k, g.nz, g.dkz);
+    const double kn2 = kn2_of(g, i, j, k);
+    const cplx C = cc[m];
+    if (kn2 <= g.kmax && kn2 >= g.tiny) {
+      const double kk2 = g.anis ? kk2_of(g, kx, ky, kz) : kn2;
+      cplx n;
+      if (G == 4 && c == 3) {
+        n = P[m];
+      } else {
+        const cplx a = row0[lds_pad(k)], b = row1[lds_pad(k)], d = row2[lds_pad(k)];
+        const cplx dot = c_add(c_add(c_scale(a, kx), c_scale(b, ky)), c_scale(d, kz));
+        const double kc = c == 2 ? kz : kd;
+        const int plane = c == 0 ? i : c == 1 ? j : k;
+        n = c_make(-P[m].x, -P[m].y);
+        if (plane != 0) n = c_add(n, c_make(kc * dot.x / kk2, kc * dot.y / kk2));
+        // gauge3 is the exact negation of this projection
+        if (KIND == 1 && part != 0) n = c_make(-n.x, -n.y);
+      }
+      cplx ff = c_make(0.0, 0.0);
+      if (fp) ff = fp[s];
+      c_put<KIND == 0>(out + s, rk_update(C, vv[m], n, ff, kk2, nu, rk.dt, rk.rmp));
+    } else if (G == 4 && c == 3 && kn2 < g.tiny) {
+      out[s] = C;  // the mean of the temperature is carried
+    } else if (prune != 1 || kn2 < g.tiny) {
+      // outside the kept modes; the k = 0 mode is written in pruned passes
+      // too, since the next substep's inverse reads it from this output
+      out[s] = c_make(0.0, 0.0);
+    }
+  }
 }
 
 template <int N, typename Cfg = FFTCfg<N>, int PF = 0>
@@ -998,7 +1264,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
 // touched (kxlim < nx/2+1 when the fields are dealiased).
 // ---------------------------------------------------------------------------
 template <int N, typename Cfg = FFTCfg<N>>
-__global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf, GridK g, int nxp,
+__global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
                                              const cplx *__restrict__ twt, int prune_) {
   using F = LineFFT<N, +1, Cfg>;
   const int prune = prune_input(g, prune_), kxlim = prune ? g.kxact : g.nxh;
@@ -1008,8 +1274,12 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
   TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
   tw.load(twt, t);
-  const FieldView in = batch_view(in_, blockIdx.z);
-  const FieldView out = batch_view(out_, blockIdx.z);
+  // blockIdx.z: member and, where a launch is split over its fields, the
+  // block's first of nper fields
+  const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
+  const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
+  const FieldView in = batch_view(in_, member);
+  const FieldView out = batch_view(out_, member);
   int bx, by;
   xcd_tile(bx, by);
   const int z = by, kx0 = bx * L, kx = kx0 + lt;
@@ -1033,8 +1303,8 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
   // wider schedules have no registers for it and rely on a second block per CU
   constexpr bool prefetch = E <= 8;
   cplx nxt[prefetch ? E : 1];
-  if constexpr (prefetch) load(0, nxt);
-  for (int f = 0; f < nf; ++f) {
+  if constexpr (prefetch) load(f0, nxt);
+  for (int f = f0; f < nf; ++f) {
     cplx v[E];
     if constexpr (prefetch) {
 #pragma unroll
@@ -1054,7 +1324,7 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
 }
 
 template <int N, typename Cfg = FFTCfg<N>>
-__global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf, GridK g, int nxp,
+__global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
                                              const cplx *__restrict__ twt, int prune) {
   using F = LineFFT<N, -1, Cfg>;
   const int kxlim = prune ? g.kxact : g.nxh;
@@ -1064,8 +1334,12 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
   TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
   tw.load(twt, t);
-  const FieldView in = batch_view(in_, blockIdx.z);
-  const FieldView out = batch_view(out_, blockIdx.z);
+  // blockIdx.z: member and, where a launch is split over its fields, the
+  // block's first of nper fields
+  const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
+  const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
+  const FieldView in = batch_view(in_, member);
+  const FieldView out = batch_view(out_, member);
   int bx, by;
   xcd_tile(bx, by);
   const int z = by, kx0 = bx * L, kx = kx0 + lt;
@@ -1091,8 +1365,8 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
   };
   constexpr bool prefetch = E <= 8;  // as in k_yinv
   cplx nxt[E];
-  if constexpr (prefetch) tload(0, nxt);
-  for (int f = 0; f < nf; ++f) {
+  if constexpr (prefetch) tload(f0, nxt);
+  for (int f = f0; f < nf; ++f) {
     if constexpr (!prefetch) tload(f, nxt);
 #pragma unroll
     for (int q = 0; q < E; ++q) {
@@ -1851,10 +2125,37 @@ static hipError_t launch_zinv_low(const FFTCtx &c, int nf, const FieldSet &in, c
   return hipGetLastError();
 }
 
+static int zinv_outputs(int mode, int nf) {
+  switch (mode) {
+  case 1: case 4: return 6;
+  case 2: return 12;
+  case 5: case 6: return 9;
+  case 7: return 3;
+  default: return nf;
+  }
+}
+
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune,
                 const double *aux) {
   if (mode == 3 && !aux) return hipErrorInvalidValue;
   const GridK &g = c.gk;
+  if (small_z(c)) {
+    const int nout = zinv_outputs(mode, nf);
+    switch (g.nz) {
+#define GHX_CASE(n_)                                                                        \
+  case n_: {                                                                                \
+    constexpr int T = FFTCfg<n_>::T;                                                        \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds()); \
+    allow_lds(k_zinv_one<n_>, s.lds);                                                       \
+    GHX_LAUNCH_CHECK((k_zinv_one<n_>), s, kTileBound, T, true);                             \
+    hipLaunchKernelGGL((k_zinv_one<n_>), dim3((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch * nout), dim3(s.block), s.lds, c.stream, in, out, mode, nout, g, c.tw_z, prune, aux); \
+    return hipGetLastError();                                                               \
+  }
+      GHX_SIZES(GHX_CASE)
+#undef GHX_CASE
+    default: return hipErrorInvalidValue;
+    }
+  }
   if (mode == 1 && (c.sched & 1)) {
     switch (g.nz) {
     case 32: return launch_zinv_low<32>(c, nf, in, out, prune, aux);
@@ -1937,9 +2238,46 @@ hipError_t zfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 #endif
 
+// Launch of k_zrk: tiles of up to `want` lines, as many as G groups of T lanes
+// per line leave within the kernel's bound and the LDS of one block.
+static PassShape zrk_shape(int G, int T, unsigned bound, int rowslots, int nlines, int want, size_t ldsmax) {
+  int L = 1;
+  while (L * 2 <= want && L * 2 <= kMaxTile && L * 2 <= nlines && (unsigned)(G * L * 2 * T) <= bound &&
+         (size_t)G * L * 2 * rowslots * sizeof(cplx) <= ldsmax)
+    L *= 2;
+  return PassShape{L, (unsigned)(G * L * T), (size_t)G * L * rowslots * sizeof(cplx)};
+}
+template <int N, int KIND, typename Cfg>
+static hipError_t launch_zrk(const FFTCtx &c, const FieldSet &in, const ZUpdate &u, int prune, int nz) {
+  constexpr int T = Cfg::T, G = zrk_groups(KIND);
+  const GridK &g = c.gk;
+  const PassShape s = zrk_shape(G, T, zrk_bound(KIND), lds_line_stride(N), g.ny, tile_pick("GHX_LZ", c.tile_z, 4), max_lds());
+  const int L = s.lines;
+  allow_lds(k_zrk<N, KIND, Cfg>, s.lds);
+  GHX_LAUNCH_CHECK((k_zrk<N, KIND, Cfg>), s, zrk_bound(KIND), T, true);
+  hipLaunchKernelGGL((k_zrk<N, KIND, Cfg>), dim3((g.ny + L - 1) / L, g.nxh, nz), dim3(s.block), s.lds, c.stream, in, g,
+                     c.tw_z, u, prune);
+  return hipGetLastError();
+}
+
 #if GHX_PART == 4
 hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, int prune) {
   const GridK &g = c.gk;
+  if (small_z(c)) {
+    ZUpdate u{};
+    u.dt = rk.dt; u.rmp = rk.rmp; u.om2 = rk.om2; u.nu = rk.nu;
+    u.fline = rk.fline; u.bstride = rk.bstride; u.nu_b = rk.nu_b;
+    for (int k = 0; k < 3; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
+    switch (g.nz) {
+#define GHX_CASE(n_)                                                                        \
+  case n_:                                                                                  \
+    if constexpr (FFTCfgLow<n_>::E != FFTCfg<n_>::E) if (c.sched & 1) return launch_zrk<n_, 0, FFTCfgLow<n_>>(c, in, u, prune, c.batch); \
+    return launch_zrk<n_, 0, FFTCfg<n_>>(c, in, u, prune, c.batch);
+      GHX_SIZES(GHX_CASE)
+#undef GHX_CASE
+    default: return hipErrorInvalidValue;
+    }
+  }
   // 512-point lines take the four-points-per-lane schedule by default (128
   // lanes per line, four lines per 512-lane block): 124 registers per lane
   // against 224, two blocks per CU, so the update's loads of v and C overlap
@@ -2000,6 +2338,17 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
 #if GHX_PART == 5
 hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &rk, int prune) {
   const GridK &g = c.gk;
+  if (small_z(c)) {
+    ZUpdate u{};
+    u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.mu; u.fline = rk.fline;
+    for (int k = 0; k < 6; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
+    switch (g.nz) {
+#define GHX_CASE(n_) case n_: return launch_zrk<n_, 1, FFTCfg<n_>>(c, in, u, prune, 2);
+      GHX_SIZES(GHX_CASE)
+#undef GHX_CASE
+    default: return hipErrorInvalidValue;
+    }
+  }
   // the four-points-per-lane schedule where a size has one (GHX_ZLOW=0: the
   // default schedule)
   const bool low = env_switch("GHX_ZLOW", 1) == 1;
@@ -2053,20 +2402,21 @@ using YFwdCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N 
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
+  const int nper = small_y(c) ? 1 : nf;
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
   const int nxp = p_row(g);
   const PassShape s = tile_shape(T, lds_line_stride(N), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, inv ? 8 : 4)), max_lds());
   const int L = s.lines;
-  dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);
+  dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));
   if (inv) {
     allow_lds(k_yinv<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yinv<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune);
+    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune);
   } else {
     allow_lds(k_yfwd<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yfwd<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune);
+    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune);
   }
   return hipGetLastError();
 }
@@ -2084,6 +2434,12 @@ static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const F
 
 hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
+  // Long launches are split by field too, all tiles of one field before the
+  // next's: 6 fields 183 -> 172 us at 256^3, 650 -> 611 at 384^3, 9 fields 314
+  // -> 272 at 256^3, but 45 -> 46 us at 128 x 256 x 128 (5504 lines), 39 -> 40 at
+  // 192 x 128 x 128 (8320).  The 512-point wide pass loses 2%.
+  const long lines = (long)g.kxact * g.nz * c.batch;
+  const int nper = small_y(c) || (lines >= 10000 && g.ny != 512) ? 1 : nf;
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;
@@ -2099,18 +2455,18 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
       constexpr int TW = FFTCfgWide<n_>::T;                                                  \
       const PassShape s = wide_shape(TW, lds_line_stride(n_), g.nxh);                        \
       const int L = s.lines; const size_t lds = s.lds;                                       \
-      dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                         \
+      dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                         \
       GHX_LAUNCH_CHECK((k_yinv<n_, FFTCfgWide<n_>>), s, kTileBound, TW, true);               \
       allow_lds(k_yinv<n_, FFTCfgWide<n_>>, lds);                                            \
-      hipLaunchKernelGGL((k_yinv<n_, FFTCfgWide<n_>>), grid, dim3(L * TW), lds, c.stream, in, out, nf, g, nxp, \
+      hipLaunchKernelGGL((k_yinv<n_, FFTCfgWide<n_>>), grid, dim3(L * TW), lds, c.stream, in, out, nf, nper, g, nxp, \
                          c.tw_y, prune);                                              \
       break;                                                                                 \
     }                                                                                        \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, 8)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
-    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
+    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                          \
     allow_lds(k_yinv<n_, Cfg>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yinv<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
+    GHX_LAUNCH_CHECK((k_yinv<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2123,6 +2479,7 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
+  const int nper = small_y(c) ? 1 : nf;
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, false, nf, in, out, prune, &lerr)) return lerr;
@@ -2133,9 +2490,9 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
     constexpr int T = Cfg::T;                                                               \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, Cfg::E == 12 ? 8 : 4)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
-    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch);                                          \
+    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                          \
     allow_lds(k_yfwd<n_, Cfg>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, nxp, c.tw_y, prune); \
+    GHX_LAUNCH_CHECK((k_yfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2389,6 +2746,20 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
 
 hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParams &rk, int prune) {
   const GridK &g = c.gk;
+  // Beyond the small launches too on power-of-two lines of 32 to 256 points:
+  // 48 -> 32 us at 128^3, 249 -> 207 at 256^3 (but 37 -> 47 at 192 x 192 x 96)
+  if (small_z(c) || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) {
+    ZUpdate u{};
+    u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.kappa; u.om2 = rk.om2; u.xmom = rk.xmom; u.xtemp = rk.xtemp;
+    u.fline = rk.fline;
+    for (int k = 0; k < 4; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
+    switch (g.nz) {
+#define GHX_CASE(n_) case n_: return launch_zrk<n_, 2, FFTCfg<n_>>(c, in, u, prune, 1);
+      GHX_SIZES(GHX_CASE)
+#undef GHX_CASE
+    default: return hipErrorInvalidValue;
+    }
+  }
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
