@@ -206,6 +206,11 @@ static bool use_x2(int nx) {
   return x2_size(nx);
 }
 
+// z inverses of several fields: 8 lines (128-byte chunks of Q) while that is at
+// most 256 lanes, else 4 (measured, 4 against 8 lines: MHD 911 -> 802 us at
+// 512 x 512 x 256, 479 -> 395 at 512 x 512 x 128, 414 -> 350 at 384 x 384 x
+// 192, Boussinesq 147 -> 115 at 384 x 384 x 96, HD 434 -> 352 at 512 x 512 x
+// 256; but HD 394 -> 438 at 384^3, MHD 633 -> 648 at 256 x 256 x 512).
 // Built-in tile width: `lines`, or as many more as fill a wavefront (a line of
 // few lanes would leave half or more of it idle: 4 lines of 8 lanes).
 static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
@@ -2174,7 +2179,7 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, mode == 0 || mode == 7 ? 8 : 4)), max_lds()); \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, mode == 0 || mode == 7 || T <= 32 ? 8 : 4)), max_lds()); \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
     if (mode == 0) {                                                                        \
@@ -2251,7 +2256,10 @@ template <int N, int KIND, typename Cfg>
 static hipError_t launch_zrk(const FFTCtx &c, const FieldSet &in, const ZUpdate &u, int prune, int nz) {
   constexpr int T = Cfg::T, G = zrk_groups(KIND);
   const GridK &g = c.gk;
-  const PassShape s = zrk_shape(G, T, zrk_bound(KIND), lds_line_stride(N), g.ny, tile_pick("GHX_LZ", c.tile_z, 4), max_lds());
+  // up to 4 lines; the Boussinesq block at most 256 lanes (212 -> 177 us at
+  // 256^3 with 2 lines instead of 4)
+  const int want = KIND == 2 && G * T * 4 > 256 ? 2 : 4;
+  const PassShape s = zrk_shape(G, T, zrk_bound(KIND), lds_line_stride(N), g.ny, tile_pick("GHX_LZ", c.tile_z, want), max_lds());
   const int L = s.lines;
   allow_lds(k_zrk<N, KIND, Cfg>, s.lds);
   GHX_LAUNCH_CHECK((k_zrk<N, KIND, Cfg>), s, zrk_bound(KIND), T, true);
@@ -2350,7 +2358,8 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
     }
   }
   // the four-points-per-lane schedule where a size has one (GHX_ZLOW=0: the
-  // default schedule)
+  // default schedule); 8 lines to 256 lanes, else 4 (both parts together: 51 ->
+  // 46 us at 128^3, 113 -> 108 at 192^3, but 764 -> 814 at 512 x 512 x 256)
   const bool low = env_switch("GHX_ZLOW", 1) == 1;
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
@@ -2358,7 +2367,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
     if constexpr (FFTCfgLow<n_>::E != FFTCfg<n_>::E) if (low) {                              \
       using Cl = FFTCfgLow<n_>;                                                              \
       constexpr int T = Cl::T;                                                               \
-      const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds()); \
+      const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, T <= 32 ? 8 : 4)), max_lds()); \
       const int L = s.lines; const size_t lds = s.lds;                                       \
       dim3 grid((g.ny + L - 1) / L, g.nxh);                                                  \
       allow_lds(k_zfwd_rk_mhd<n_, 0, Cl>, lds);                                              \
@@ -2370,7 +2379,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
       break;                                                                                 \
     }                                                                                        \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds());                                        \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, T <= 32 ? 8 : 4)), max_lds());                                        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
     allow_lds(k_zfwd_rk_mhd<n_, 0>, lds);                                                   \
@@ -2760,11 +2769,12 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
     default: return hipErrorInvalidValue;
     }
   }
+  // 2 lines of 64 lanes and more (509 -> 455 us at 256 x 256 x 512)
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_) + n_, g.ny, tile_want("GHX_LZ", tile_default(T, 4)), max_lds());              \
+    const PassShape s = tile_shape(T, lds_line_stride(n_) + n_, g.ny, tile_want("GHX_LZ", T >= 64 ? 2 : tile_default(T, 4)), max_lds());              \
     const int L = s.lines; const size_t lds = s.lds;                     \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
     allow_lds(k_zfwd_rk_bouss<n_>, lds);                                                    \
