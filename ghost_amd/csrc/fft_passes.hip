@@ -739,19 +739,19 @@ GHX_DEV void zfwd_load_diff(cplx (&v)[E], cplx *lds, cplx *row, int stride, int 
   F::run(v, row, t, tw);
 }
 
-template <int N>
 // prune: only the kept modes of the output are wanted (the caller reads no
 // other), so only the dealias disc's lines are loaded (the y forward wrote no
 // others) and only their kept modes are written; the rest of `out` keeps
 // whatever it held.
+template <int N, typename Cfg = FFTCfg<N>>
 __global__ __launch_bounds__(kTileBound) void k_zfwd(FieldSet in, FieldSet out, int nf, GridK g, const cplx *__restrict__ twt,
                                              int prune) {
-  using F = LineFFT<N, -1>;
+  using F = LineFFT<N, -1, Cfg>;
   constexpr int T = F::T, E = F::E;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N> tw;  // stage twiddle roots of this lane, loaded once
+  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
   tw.load(twt, t);
   int bx, by;
   xcd_tile(bx, by);
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd(FieldSet in, FieldSet out, 
   const size_t sline = ((size_t)i * g.ny + (ok ? j : 0)) * N;
   for (int f = 0; f < nf; ++f) {
     cplx v[E];
-    zfwd_load<N, E>(v, lds, row, stride, L, t, tw, in.p[f], g, i, j0, lmask);
+    zfwd_load<N, E, Cfg>(v, lds, row, stride, L, t, tw, in.p[f], g, i, j0, lmask);
     if (ok) {
 #pragma unroll
       for (int m = 0; m < E; ++m) {
@@ -1709,8 +1709,7 @@ GHX_DEV void xpair_real(cplx (&z)[E], const double *sa, const double *sb, int t,
   for (int m = 0; m < E; ++m) z[m] = c_make(sa[t + T * m], sb ? sb[t + T * m] : 0.0);
 }
 
-// X^-1 of nf fields, two rows per transform (plain c2r; the last field of an
-// odd count goes alone).
+// X^-1 of nf fields (an even count), two rows per transform.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int kxlim) {
@@ -1728,25 +1727,84 @@ __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, i
   TwCache<NX, Cfg> tw;
   tw.load(twt, t);
   cplx a[E], b[E], z[E];
-  const int np = (nf + 1) / 2;
-  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[nf > 1 ? 1 : 0] + off, t, kxlim);
+  const int np = nf / 2;
+  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
   for (int p = 0; p < np; ++p) {
-    const bool two = 2 * p + 1 < nf;
-    xpair_make<NX, E, T>(z, a, b, t, kxlim, two);
-    if (p + 1 < np) {  // next pair in flight
-      const int fa = 2 * p + 2, fb = fa + 1 < nf ? fa + 1 : fa;
-      xpair_load<NX, E, T>(a, b, in.p[fa] + off, in.p[fb] + off, t, kxlim);
-    }
+    xpair_make<NX, E, T>(z, a, b, t, kxlim);
+    if (p + 1 < np)  // next pair in flight
+      xpair_load<NX, E, T>(a, b, in.p[2 * p + 2] + off, in.p[2 * p + 3] + off, t, kxlim);
     FI::run(z, buf, t, tw);
-    double *da = out.p[2 * p] + roff;
+    double *da = out.p[2 * p] + roff, *db = out.p[2 * p + 1] + roff;
 #pragma unroll
-    for (int m = 0; m < E; ++m) da[t + T * m] = z[m].x;
-    if (two) {
-      double *db = out.p[2 * p + 1] + roff;
-#pragma unroll
-      for (int m = 0; m < E; ++m) db[t + T * m] = z[m].y;
+    for (int m = 0; m < E; ++m) {
+      da[t + T * m] = z[m].x;
+      db[t + T * m] = z[m].y;
     }
   }
+}
+
+// One field's rows, paired with each other: rows 2p and 2p + 1 make one complex
+// line, so a lone field (or the last of an odd count) costs half a transform
+// per row; alone, with a zero imaginary part, it costs a whole one.  One field,
+// alone against paired: x inverse 519 -> 389 us at 512^3, 70 -> 53 at 256^3,
+// 429 -> 203 at 384^3, 55 -> 30 at 192^3; x forward 390 -> 192 at 384^3, 42 ->
+// 25 at 192^3, 10.7 -> 10.3 at 128^3, but 49 -> 52 at 256^3 and 397 -> 421 at
+// 512^3, which keep the lone form (pair_rows_fwd).  The last row of an odd
+// count goes alone.
+constexpr bool pair_rows_fwd(int nx) { return nx % 3 == 0 || nx <= 128; }
+template <int NX>
+__global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict__ in, double *__restrict__ out,
+                                                         long nrows, int nxp, const cplx *__restrict__ twt,
+                                                         int kxlim) {
+  using Cfg = FFTCfg<NX>;
+  using FI = LineFFT<NX, +1, Cfg>;
+  constexpr int T = Cfg::T, E = Cfg::E;
+  static_assert(T <= 64, "one line per wavefront or less");
+  extern __shared__ cplx lds[];
+  const int rpb = blockDim.x / T;
+  const int lt = threadIdx.x / T, t = threadIdx.x % T;
+  const long r = 2 * ((long)blockIdx.x * rpb + lt);
+  if (r >= nrows) return;
+  const bool two = r + 1 < nrows;
+  cplx *buf = lds + lt * lds_line_stride(NX);
+  TwCache<NX, Cfg> tw;
+  tw.load(twt, t);
+  const cplx *sa = in + (size_t)r * nxp;
+  cplx a[E], b[E], z[E];
+  xpair_load<NX, E, T>(a, b, sa, two ? sa + nxp : sa, t, kxlim);
+  xpair_make<NX, E, T>(z, a, b, t, kxlim, two);
+  FI::run(z, buf, t, tw);
+  double *da = out + (size_t)r * NX;
+#pragma unroll
+  for (int m = 0; m < E; ++m) da[t + T * m] = z[m].x;
+  if (two) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) da[NX + t + T * m] = z[m].y;
+  }
+}
+template <int NX>
+__global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restrict__ in, cplx *__restrict__ out,
+                                                         long nrows, int nxp, const cplx *__restrict__ twt) {
+  using Cfg = FFTCfg<NX>;
+  using FF = LineFFT<NX, -1, Cfg>;
+  constexpr int T = Cfg::T, E = Cfg::E;
+  static_assert(T <= 64, "one line per wavefront or less");
+  extern __shared__ cplx lds[];
+  const int rpb = blockDim.x / T;
+  const int lt = threadIdx.x / T, t = threadIdx.x % T;
+  const long r = 2 * ((long)blockIdx.x * rpb + lt);
+  if (r >= nrows) return;
+  const bool two = r + 1 < nrows;
+  cplx *buf = lds + lt * lds_line_stride(NX);
+  TwCache<NX, Cfg> tw;
+  tw.load(twt, t);
+  const double *sa = in + (size_t)r * NX;
+  cplx z[E];
+  xpair_real<E>(z, sa, two ? sa + NX : nullptr, t, T);
+  FF::run(z, buf, t, tw);
+  cplx *da = out + (size_t)r * nxp;
+  if (two) xpair_store2<NX, E, T>(z, buf, t, da, da + nxp, NX / 2 + 1);
+  else xpair_store1<NX, E, T>(z, t, da, NX / 2 + 1);
 }
 
 // X^-1 of three fields written interleaved (the tracer layout of k_xinv3i),
@@ -2140,6 +2198,10 @@ static int zinv_outputs(int mode, int nf) {
   }
 }
 
+// modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
+// (one field 287 -> 190 us at 384^3, 27.4 -> 26.0 at 192^3, the same at 96^3)
+template <int N>
+using ZInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune,
                 const double *aux) {
   if (mode == 3 && !aux) return hipErrorInvalidValue;
@@ -2175,17 +2237,38 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
   if (mode == 3 && g.nz == 512 && env_switch("GHX_ZWIDE", 1) != 0 &&
       wide_shape(FFTCfgWide<512>::T, lds_line_stride(512), g.ny).lds <= max_lds())
     return launch_zinv_wide<3>(c, nf, in, out, prune, aux);
+  if (mode == 0 || mode == 3) {
+    switch (g.nz) {
+#define GHX_CASE(n_)                                                                        \
+  case n_: {                                                                                \
+    using Cfg = ZInvCfg<n_>;                                                                \
+    constexpr int T = Cfg::T;                                                               \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 8)), max_lds()); \
+    const dim3 grid((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch);                        \
+    if (mode == 0) {                                                                        \
+      allow_lds((k_zinv<n_, 0, Cfg>), s.lds);                                               \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 0, Cfg>), s, kTileBound, T, true);                       \
+      hipLaunchKernelGGL((k_zinv<n_, 0, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+    } else {                                                                                \
+      allow_lds((k_zinv<n_, 3, Cfg>), s.lds);                                               \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 3, Cfg>), s, kTileBound, T, true);                       \
+      hipLaunchKernelGGL((k_zinv<n_, 3, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+    }                                                                                       \
+    return hipGetLastError();                                                               \
+  }
+      GHX_SIZES(GHX_CASE)
+#undef GHX_CASE
+    default: return hipErrorInvalidValue;
+    }
+  }
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, mode == 0 || mode == 7 || T <= 32 ? 8 : 4)), max_lds()); \
+    const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, mode == 7 || T <= 32 ? 8 : 4)), max_lds()); \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
-    if (mode == 0) {                                                                        \
-      allow_lds(k_zinv<n_, 0>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 0>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 0>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
-    } else if (mode == 1) {                                                                 \
+    if (mode == 1) {                                                                 \
       allow_lds(k_zinv<n_, 1>, lds);                                                        \
       GHX_LAUNCH_CHECK((k_zinv<n_, 1>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 1>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
     } else if (mode == 2) {                                                                 \
@@ -2203,9 +2286,6 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     } else if (mode == 7) {                                                                 \
       allow_lds(k_zinv<n_, 7>, lds);                                                        \
       GHX_LAUNCH_CHECK((k_zinv<n_, 7>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 7>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
-    } else {                                                                                \
-      allow_lds(k_zinv<n_, 3>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 3>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 3>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
     }                                                                                       \
     break;                                                                                  \
   }
@@ -2220,17 +2300,21 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
 #endif
 
 #if GHX_PART == 3
+// one field live, as ZInvCfg (one field 334 -> 260 us at 384^3)
+template <int N>
+using ZFwdCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
 hipError_t zfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
-    constexpr int T = FFTCfg<n_>::T;                                                        \
+    using Cfg = ZFwdCfg<n_>;                                                                \
+    constexpr int T = Cfg::T;                                                               \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 8)), max_lds());                                        \
     const int L = s.lines; const size_t lds = s.lds;                            \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
-    allow_lds(k_zfwd<n_>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_zfwd<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zfwd<n_>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune); \
+    allow_lds((k_zfwd<n_, Cfg>), lds);                                                             \
+    GHX_LAUNCH_CHECK((k_zfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2528,10 +2612,17 @@ hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out,
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                                      \
-    const int rpb = s.lines; const size_t lds = s.lds;                          \
-    const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xinv2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xinv2<n_>), gr, bl, lds, c.stream, in, rs, nf, g, nxp, c.tw_x, kxlim);                                                                 \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                       \
+    const int rpb = s.lines; const size_t lds = s.lds;                                      \
+    const dim3 bl(rpb * T);                                                                 \
+    if (nf > 1) { /* whole pairs of fields */                                               \
+      GHX_LAUNCH_CHECK((k_xinv2<n_>), s, kRowBound, T, false);                              \
+      hipLaunchKernelGGL((k_xinv2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, in, rs, nf & ~1, g, nxp, c.tw_x, kxlim); \
+    }                                                                                       \
+    if (nf & 1) { /* the last field's rows in pairs */                                      \
+      GHX_LAUNCH_CHECK((k_xinv_rows<n_>), s, kRowBound, T, false);                          \
+      hipLaunchKernelGGL((k_xinv_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, in.p[nf - 1], rs.p[nf - 1], nrows, nxp, c.tw_x, kxlim); \
+    }                                                                                       \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
@@ -2632,10 +2723,18 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                                      \
-    const int rpb = s.lines; const size_t lds = s.lds;                          \
-    const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xfwd2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xfwd2<n_>), gr, bl, lds, c.stream, rs, out, nf, g, nxp, c.tw_x);                                                                 \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                       \
+    const int rpb = s.lines; const size_t lds = s.lds;                                      \
+    const dim3 bl(rpb * T);                                                                 \
+    constexpr bool paired = pair_rows_fwd(n_);                                              \
+    if (nf > 1 || !paired) {                                                                \
+      GHX_LAUNCH_CHECK((k_xfwd2<n_>), s, kRowBound, T, false);                              \
+      hipLaunchKernelGGL((k_xfwd2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, rs, out, paired ? nf & ~1 : nf, g, nxp, c.tw_x); \
+    }                                                                                       \
+    if constexpr (paired) if (nf & 1) {                                                     \
+      GHX_LAUNCH_CHECK((k_xfwd_rows<n_>), s, kRowBound, T, false);                          \
+      hipLaunchKernelGGL((k_xfwd_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, rs.p[nf - 1], out.p[nf - 1], nrows, nxp, c.tw_x); \
+    }                                                                                       \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
