@@ -226,6 +226,16 @@ constexpr long kSmallLines = 3328;
 static bool small_z(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch <= kSmallLines; }
 static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= kSmallLines; }
 
+// Products of 192-point rows on 12 points per lane (k_xmul12) where their rows
+// give every CU a block of 16.  Measured (us, 6 -> 12 points): cross 22.2 -> 21.3
+// at 192 x 64 x 64, 47.9 -> 42.6 at 192 x 128 x 96, 125 -> 110 at 192^3, 467 -> 406
+// at 192 x 384 x 384, but 14.4 -> 18.1 at 192 x 32 x 32; dot 53.4 -> 51.2 at 192 x
+// 192 x 96, 99.5 -> 93.6 at 192^3.  Not the others: cross 24.5 -> 28.4 at 96^3 (8
+// lanes a row), 142 -> 142 and dot 115 -> 130 at 384 x 192 x 96 (spills).
+static bool use_xmul12(const GridK &g, int batch) {
+  return g.nx == 192 && use_x2(g.nx) && (long)g.nz * g.ny * batch >= 256 * 16;
+}
+
 template <typename K> static void allow_lds(K kern, size_t bytes) {
   if (bytes > 49152) (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
@@ -2019,6 +2029,69 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
   xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxout);
 }
 
+// k_xcross2 and k_xdot2 on 12 points per lane, two radix-12/16 stages for a
+// 192-point row instead of {6, 2..}: fewer LDS exchanges on the chain that
+// bounds them.  The three transformed pairs fill the registers (2 waves per
+// SIMD, as the 6-point kernels), so twiddles are read where they are used and
+// the scheduling barriers keep a pair's loads behind the transform before it.
+template <int NX, bool CROSS>
+__global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) void k_xmul12(
+    FieldSet in_, FieldSet out_, GridK g, int nxp, const cplx *__restrict__ twt, int prune) {
+  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
+  using Cfg = FFTCfgMid<NX>;
+  using FI = LineFFT<NX, +1, Cfg>;
+  using FF = LineFFT<NX, -1, Cfg>;
+  constexpr int T = Cfg::T, E = Cfg::E;
+  static_assert(T <= 64, "one row per wavefront or less");
+  extern __shared__ cplx lds[];
+  const int rpb = blockDim.x / T;
+  const int lt = threadIdx.x / T, t = threadIdx.x % T;
+  const long r = (long)blockIdx.x * rpb + lt;
+  if (r >= (long)g.nz * g.ny) return;  // whole lines only: wave-level syncs
+  const size_t off = (size_t)r * nxp;
+  cplx *buf = lds + lt * lds_line_stride(NX);
+  const FieldView in = batch_view(in_, blockIdx.y);
+  const FieldView out = batch_view(out_, blockIdx.y);
+  cplx z0[E], z1[E], z2[E];
+  auto inverse = [&](cplx (&z)[E], int fa, int fb) {
+    __builtin_amdgcn_sched_barrier(0);
+    cplx a[E], b[E];
+    xpair_load<NX, E, T>(a, b, in.p[fa] + off, in.p[fb] + off, t, kxlim);
+    xpair_make<NX, E, T>(z, a, b, t, kxlim);
+    __builtin_amdgcn_sched_barrier(0);
+    FI::run(z, buf, t, twt);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  inverse(z0, 0, 1);
+  inverse(z1, 2, 3);
+  inverse(z2, 4, 5);
+  if constexpr (CROSS) {
+    const double tmp = g.inv_n6;
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const double px = z0[m].x, py = z0[m].y, pz = z1[m].x, qx = z1[m].y, qy = z2[m].x, qz = z2[m].y;
+      const double ox = (py * qz - qy * pz) * tmp;
+      const double oy = (pz * qx - qz * px) * tmp;
+      const double oz = (px * qy - qx * py) * tmp;
+      z0[m] = c_make(ox, oy);
+      z1[m] = c_make(oz, 0.0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    FF::run(z0, buf, t, twt);
+    xpair_store2<NX, E, T>(z0, buf, t, out.p[0] + off, out.p[1] + off, kxout);
+    FF::run(z1, buf, t, twt);
+    xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxout);
+  } else {
+    const double tmp = -g.inv_n6;
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+      z0[m] = c_make(((z0[m].x * z1[m].y + z0[m].y * z2[m].x) + z1[m].x * z2[m].y) * tmp, 0.0);
+    __builtin_amdgcn_sched_barrier(0);
+    FF::run(z0, buf, t, twt);
+    xpair_store1<NX, E, T>(z0, t, out.p[0] + off, kxout);
+  }
+}
+
 // Fused X^-1 . (P x Q)/N^6 . X on P rows with GHOST's operand order
 // (pseudospec3D_hd.f90:377-389): out_x = (P_y Q_z - Q_y P_z) tmp,
 // out_y = (P_z Q_x - Q_z P_x) tmp, out_z = (P_x Q_y - Q_x P_y) tmp.
@@ -2768,6 +2841,14 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
   if (g.nx % 2) return hipErrorInvalidValue;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
+  if (use_xmul12(g, c.batch)) {
+    constexpr int T = FFTCfgMid<192>::T;
+    const PassShape s = row_shape(T, lds_line_stride(192), max_lds());
+    GHX_LAUNCH_CHECK((k_xmul12<192, true>), s, kRowBound, T, false);
+    hipLaunchKernelGGL((k_xmul12<192, true>), dim3((unsigned)((nrows + s.lines - 1) / s.lines), c.batch), dim3(s.block),
+                       s.lds, c.stream, in, out, g, nxp, c.tw_x, prune);
+    return hipGetLastError();
+  }
   if (use_x2(g.nx)) {
     switch (g.nx) {
 #define GHX_CASE(n_)                                                                        \
@@ -2818,6 +2899,14 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
   if (g.nx % 2) return hipErrorInvalidValue;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
+  if (use_xmul12(g, 1)) {
+    constexpr int T = FFTCfgMid<192>::T;
+    const PassShape s = row_shape(T, lds_line_stride(192), max_lds());
+    GHX_LAUNCH_CHECK((k_xmul12<192, false>), s, kRowBound, T, false);
+    hipLaunchKernelGGL((k_xmul12<192, false>), dim3((unsigned)((nrows + s.lines - 1) / s.lines), 1), dim3(s.block),
+                       s.lds, c.stream, in, out, g, nxp, c.tw_x, prune);
+    return hipGetLastError();
+  }
   if (use_x2(g.nx)) {
     switch (g.nx) {
 #define GHX_CASE(n_)                                                                        \
