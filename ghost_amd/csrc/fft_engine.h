@@ -342,3 +342,126 @@ template <int N, int DIR, typename Cfg = FFTCfg<N>> struct LineFFT {
     stages<0, 1, TwCache<N, Cfg>>(v, buf, t, tw);
   }
 };
+
+// ---------------------------------------------------------------------------
+// Lines of N = 3 * 2^k points (24 .. 384) in two or three stages of radix 6
+// and 8 or 4, instead of radix 6 and then 2, 2, ..: the lanes per stage differ.
+// The radix-6 stage uses all T = N / 6 lanes of the line with 6 points each,
+// the others A = N / 8 = 3/4 T of them with 8 points each, so a line takes one
+// or two LDS exchanges where the 6-point schedules take two to six.  The
+// inverse starts with radix 6, the forward ends with it: the wavenumber side
+// is held as x[t + T m] (m < 6) by every lane, the other side as x[t + A m]
+// (m < 8) by the lanes t < A, and a pass that does both needs no exchange to
+// get from one to the other.
+// ---------------------------------------------------------------------------
+template <int N> struct MixCfg;  // radices of the 8-point stages, in the inverse's order (1: no stage)
+template <> struct MixCfg<24> { static constexpr int R1 = 4, R2 = 1; };
+template <> struct MixCfg<48> { static constexpr int R1 = 8, R2 = 1; };
+template <> struct MixCfg<96> { static constexpr int R1 = 4, R2 = 4; };
+template <> struct MixCfg<192> { static constexpr int R1 = 8, R2 = 4; };
+template <> struct MixCfg<384> { static constexpr int R1 = 8, R2 = 8; };
+
+template <int N, int DIR> struct MixFFT {
+  using C = MixCfg<N>;
+  static constexpr int T = N / 6, A = N / 8;
+  static_assert(6 * C::R1 * C::R2 == N && T <= 64, "a line lives in one wavefront");
+
+  // the stage's roots of this lane, one per butterfly
+  template <int R, int Ns, int L, int E> GHX_DEV static void roots(cplx (&w)[E / R], const cplx *tw, int t) {
+#pragma unroll
+    for (int q = 0; q < E / R; ++q) w[q] = tw[((t + q * L) % Ns) * (N / (Ns * R))];
+  }
+  template <int R, bool TWIDDLE, int E> GHX_DEV static void butterflies(cplx (&v)[E], const cplx *w1) {
+    constexpr int Q = E / R;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      cplx u[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) u[r] = v[q + r * Q];
+      if constexpr (TWIDDLE) {
+        cplx w[R];
+        tw_powers<R>(DIR < 0 ? w1[q] : c_conj(w1[q]), w);
+#pragma unroll
+        for (int r = 1; r < R; ++r) u[r] = c_mul(u[r], w[r]);
+      }
+      SmallDFT<R, DIR>::run(u);
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q + r * Q] = u[r];
+    }
+  }
+  template <int R, int Ns, int L, int E> GHX_DEV static void put(const cplx (&v)[E], cplx *buf, int t) {
+    constexpr int Q = E / R;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = t + q * L, base = (j / Ns) * Ns * R + (j % Ns);
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf[lds_pad(base + r * Ns)] = v[q + r * Q];
+    }
+  }
+  template <int L, int E> GHX_DEV static void get(cplx (&v)[E], const cplx *buf, int t) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = buf[lds_pad(t + L * m)];
+  }
+
+  static constexpr int Q1 = 8 / C::R1, Q2 = 8 / C::R2;
+  struct Roots {
+    cplx a[Q1], b[C::R2 > 1 ? Q2 : 1];
+  };
+  // wavenumbers in (t + T m) -> samples out (t + A m, lanes t < A)
+  struct Inv {
+    Roots w;
+    GHX_DEV void load(const cplx *tw, int t) {
+      roots<C::R1, 6, A, 8>(w.a, tw, t);
+      if constexpr (C::R2 > 1) roots<C::R2, 6 * C::R1, A, 8>(w.b, tw, t);
+    }
+    GHX_DEV void run(cplx (&in)[6], cplx (&out)[8], cplx *buf, int t) const {
+      butterflies<6, false, 6>(in, nullptr);
+      put<6, 1, T, 6>(in, buf, t);
+      line_sync<T>();
+      if (t < A) {
+        get<A, 8>(out, buf, t);
+        butterflies<C::R1, true, 8>(out, w.a);
+      }
+      line_sync<T>();
+      if constexpr (C::R2 > 1) {
+        if (t < A) put<C::R1, 6, A, 8>(out, buf, t);
+        line_sync<T>();
+        if (t < A) {
+          get<A, 8>(out, buf, t);
+          butterflies<C::R2, true, 8>(out, w.b);
+        }
+        line_sync<T>();
+      }
+    }
+  };
+  // samples in (t + A m, lanes t < A) -> wavenumbers out (t + T m)
+  struct Fwd {
+    cplx b[C::R2 > 1 ? Q1 : 1], c[1];
+    GHX_DEV void load(const cplx *tw, int t) {
+      if constexpr (C::R2 > 1) roots<C::R1, C::R2, A, 8>(b, tw, t);
+      roots<6, N / 6, T, 6>(c, tw, t);
+    }
+    GHX_DEV void run(cplx (&in)[8], cplx (&out)[6], cplx *buf, int t) const {
+      if constexpr (C::R2 > 1) {
+        if (t < A) {
+          butterflies<C::R2, false, 8>(in, nullptr);
+          put<C::R2, 1, A, 8>(in, buf, t);
+        }
+        line_sync<T>();
+        if (t < A) {
+          get<A, 8>(in, buf, t);
+          butterflies<C::R1, true, 8>(in, b);
+        }
+        line_sync<T>();
+        if (t < A) put<C::R1, C::R2, A, 8>(in, buf, t);
+      } else if (t < A) {
+        butterflies<C::R1, false, 8>(in, nullptr);
+        put<C::R1, 1, A, 8>(in, buf, t);
+      }
+      line_sync<T>();
+      get<T, 6>(out, buf, t);
+      line_sync<T>();
+      butterflies<6, true, 6>(out, c);
+    }
+  };
+};

@@ -226,16 +226,6 @@ constexpr long kSmallLines = 3328;
 static bool small_z(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch <= kSmallLines; }
 static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= kSmallLines; }
 
-// Products of 192-point rows on 12 points per lane (k_xmul12) where their rows
-// give every CU a block of 16.  Measured (us, 6 -> 12 points): cross 22.2 -> 21.3
-// at 192 x 64 x 64, 47.9 -> 42.6 at 192 x 128 x 96, 125 -> 110 at 192^3, 467 -> 406
-// at 192 x 384 x 384, but 14.4 -> 18.1 at 192 x 32 x 32; dot 53.4 -> 51.2 at 192 x
-// 192 x 96, 99.5 -> 93.6 at 192^3.  Not the others: cross 24.5 -> 28.4 at 96^3 (8
-// lanes a row), 142 -> 142 and dot 115 -> 130 at 384 x 192 x 96 (spills).
-static bool use_xmul12(const GridK &g, int batch) {
-  return g.nx == 192 && use_x2(g.nx) && (long)g.nz * g.ny * batch >= 256 * 16;
-}
-
 template <typename K> static void allow_lds(K kern, size_t bytes) {
   if (bytes > 49152) (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
@@ -1719,14 +1709,52 @@ GHX_DEV void xpair_real(cplx (&z)[E], const double *sa, const double *sb, int t,
   for (int m = 0; m < E; ++m) z[m] = c_make(sa[t + T * m], sb ? sb[t + T * m] : 0.0);
 }
 
+// One lane's part of a row's transforms: KE points on the wavenumber side
+// (k = t + T m) and SE on the sample side (n = t + A m, in the lanes t < A).
+// Powers of two keep one layout; 3 * 2^k rows take the mixed stages (MixFFT),
+// whose passes the LDS exchanges bound less (6-point -> mixed, us): cross 1084
+// -> 743 at 384^3, 125 -> 98 at 192^3, 24.7 -> 21.6 at 96^3, 11.6 -> 9.8 at
+// 48^3, 10.5 -> 9.6 at 24^3; dot 116 -> 81 at 384 x 192 x 96; three
+// interleaved inverses 606 -> 446 at 384^3, 75 -> 63 at 192^3; one field's
+// inverse 200 -> 162 and forward 196 -> 170 at 384^3.
+template <int NX, bool MIX = (NX % 3 == 0)> struct XLine {
+  using Cfg = FFTCfg<NX>;
+  static constexpr int T = Cfg::T, A = T, KE = Cfg::E, SE = Cfg::E;
+  static_assert(T <= 64, "one row per wavefront or less");
+  TwCache<NX, Cfg> tw;
+  GHX_DEV void load_inv(const cplx *w, int t) { tw.load(w, t); }
+  GHX_DEV void load_fwd(const cplx *w, int t) { tw.load(w, t); }
+  GHX_DEV void load_fwd_too(const cplx *, int) {}  // after load_inv: the same roots
+  GHX_DEV static constexpr bool live(int) { return true; }
+  GHX_DEV void inv(cplx (&k)[KE], cplx (&x)[SE], cplx *buf, int t) const {
+#pragma unroll
+    for (int m = 0; m < SE; ++m) x[m] = k[m];
+    LineFFT<NX, +1, Cfg>::run(x, buf, t, tw);
+  }
+  GHX_DEV void fwd(cplx (&x)[SE], cplx (&k)[KE], cplx *buf, int t) const {
+#pragma unroll
+    for (int m = 0; m < KE; ++m) k[m] = x[m];
+    LineFFT<NX, -1, Cfg>::run(k, buf, t, tw);
+  }
+};
+template <int NX> struct XLine<NX, true> {
+  static constexpr int T = MixFFT<NX, +1>::T, A = MixFFT<NX, +1>::A, KE = 6, SE = 8;
+  typename MixFFT<NX, +1>::Inv wi;
+  typename MixFFT<NX, -1>::Fwd wf;
+  GHX_DEV void load_inv(const cplx *w, int t) { wi.load(w, t); }
+  GHX_DEV void load_fwd(const cplx *w, int t) { wf.load(w, t); }
+  GHX_DEV void load_fwd_too(const cplx *w, int t) { wf.load(w, t); }
+  GHX_DEV static bool live(int t) { return t < A; }
+  GHX_DEV void inv(cplx (&k)[6], cplx (&x)[8], cplx *buf, int t) const { wi.run(k, x, buf, t); }
+  GHX_DEV void fwd(cplx (&x)[8], cplx (&k)[6], cplx *buf, int t) const { wf.run(x, k, buf, t); }
+};
+
 // X^-1 of nf fields (an even count), two rows per transform.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int kxlim) {
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1734,21 +1762,23 @@ __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, i
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp, roff = (size_t)r * NX;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
-  cplx a[E], b[E], z[E];
+  X fft;
+  fft.load_inv(twt, t);
+  cplx a[KE], b[KE], z[KE], x[SE];
   const int np = nf / 2;
-  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
   for (int p = 0; p < np; ++p) {
-    xpair_make<NX, E, T>(z, a, b, t, kxlim);
+    xpair_make<NX, KE, T>(z, a, b, t, kxlim);
     if (p + 1 < np)  // next pair in flight
-      xpair_load<NX, E, T>(a, b, in.p[2 * p + 2] + off, in.p[2 * p + 3] + off, t, kxlim);
-    FI::run(z, buf, t, tw);
+      xpair_load<NX, KE, T>(a, b, in.p[2 * p + 2] + off, in.p[2 * p + 3] + off, t, kxlim);
+    fft.inv(z, x, buf, t);
     double *da = out.p[2 * p] + roff, *db = out.p[2 * p + 1] + roff;
+    if (X::live(t)) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) {
-      da[t + T * m] = z[m].x;
-      db[t + T * m] = z[m].y;
+      for (int m = 0; m < SE; ++m) {
+        da[t + A * m] = x[m].x;
+        db[t + A * m] = x[m].y;
+      }
     }
   }
 }
@@ -1766,10 +1796,8 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict__ in, double *__restrict__ out,
                                                          long nrows, int nxp, const cplx *__restrict__ twt,
                                                          int kxlim) {
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one line per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1777,28 +1805,27 @@ __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict_
   if (r >= nrows) return;
   const bool two = r + 1 < nrows;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
+  X fft;
+  fft.load_inv(twt, t);
   const cplx *sa = in + (size_t)r * nxp;
-  cplx a[E], b[E], z[E];
-  xpair_load<NX, E, T>(a, b, sa, two ? sa + nxp : sa, t, kxlim);
-  xpair_make<NX, E, T>(z, a, b, t, kxlim, two);
-  FI::run(z, buf, t, tw);
+  cplx a[KE], b[KE], z[KE], x[SE];
+  xpair_load<NX, KE, T>(a, b, sa, two ? sa + nxp : sa, t, kxlim);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim, two);
+  fft.inv(z, x, buf, t);
+  if (!X::live(t)) return;
   double *da = out + (size_t)r * NX;
 #pragma unroll
-  for (int m = 0; m < E; ++m) da[t + T * m] = z[m].x;
+  for (int m = 0; m < SE; ++m) da[t + A * m] = x[m].x;
   if (two) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) da[NX + t + T * m] = z[m].y;
+    for (int m = 0; m < SE; ++m) da[NX + t + A * m] = x[m].y;
   }
 }
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restrict__ in, cplx *__restrict__ out,
                                                          long nrows, int nxp, const cplx *__restrict__ twt) {
-  using Cfg = FFTCfg<NX>;
-  using FF = LineFFT<NX, -1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one line per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1806,15 +1833,15 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restric
   if (r >= nrows) return;
   const bool two = r + 1 < nrows;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
+  X fft;
+  fft.load_fwd(twt, t);
   const double *sa = in + (size_t)r * NX;
-  cplx z[E];
-  xpair_real<E>(z, sa, two ? sa + NX : nullptr, t, T);
-  FF::run(z, buf, t, tw);
+  cplx x[SE], z[KE];
+  if (X::live(t)) xpair_real<SE>(x, sa, two ? sa + NX : nullptr, t, A);
+  fft.fwd(x, z, buf, t);
   cplx *da = out + (size_t)r * nxp;
-  if (two) xpair_store2<NX, E, T>(z, buf, t, da, da + nxp, NX / 2 + 1);
-  else xpair_store1<NX, E, T>(z, t, da, NX / 2 + 1);
+  if (two) xpair_store2<NX, KE, T>(z, buf, t, da, da + nxp, NX / 2 + 1);
+  else xpair_store1<NX, KE, T>(z, t, da, NX / 2 + 1);
 }
 
 // X^-1 of three fields written interleaved (the tracer layout of k_xinv3i),
@@ -1822,10 +1849,8 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restric
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int kxlim) {
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1833,19 +1858,20 @@ __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out,
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
-  cplx a[E], b[E], z0[E], z1[E];
-  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
-  xpair_make<NX, E, T>(z0, a, b, t, kxlim);
-  xpair_load<NX, E, T>(a, b, in.p[2] + off, in.p[2] + off, t, kxlim);
-  FI::run(z0, buf, t, tw);
-  xpair_make<NX, E, T>(z1, a, b, t, kxlim, false);
-  FI::run(z1, buf, t, tw);
+  X fft;
+  fft.load_inv(twt, t);
+  cplx a[KE], b[KE], z[KE], z0[SE], z1[SE];
+  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[2] + off, in.p[2] + off, t, kxlim);
+  fft.inv(z, z0, buf, t);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim, false);
+  fft.inv(z, z1, buf, t);
+  if (!X::live(t)) return;
   double *dst = out + (size_t)r * NX * 3;
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int n = t + T * m;
+  for (int m = 0; m < SE; ++m) {
+    const int n = t + A * m;
     d_put<true>(dst + 3 * n + 0, z0[m].x);
     d_put<true>(dst + 3 * n + 1, z0[m].y);
     d_put<true>(dst + 3 * n + 2, z1[m].x);
@@ -1859,37 +1885,37 @@ __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out,
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part, GridK g, int nxp,
                                                       const cplx *__restrict__ twt, int kxlim) {
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   __shared__ double best[kRowBound / 64];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
   const long nrows = (long)g.nz * g.ny, hop = (long)gridDim.x * rpb;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
+  X fft;
+  fft.load_inv(twt, t);
   double big = 0.0;
   long r = (long)blockIdx.x * rpb + lt;
   if (r < nrows) {  // whole lines only: wave-level syncs inside
-    cplx a[E], b[E], z0[E], z1[E];
-    xpair_load<NX, E, T>(a, b, in.p[0] + (size_t)r * nxp, in.p[1] + (size_t)r * nxp, t, kxlim);
+    cplx a[KE], b[KE], z[KE], z0[SE], z1[SE];
+    xpair_load<NX, KE, T>(a, b, in.p[0] + (size_t)r * nxp, in.p[1] + (size_t)r * nxp, t, kxlim);
     for (; r < nrows; r += hop) {
       const size_t off = (size_t)r * nxp;
-      xpair_make<NX, E, T>(z0, a, b, t, kxlim);
-      xpair_load<NX, E, T>(a, b, in.p[2] + off, in.p[2] + off, t, kxlim);
-      FI::run(z0, buf, t, tw);
-      xpair_make<NX, E, T>(z1, a, b, t, kxlim, false);
+      xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+      xpair_load<NX, KE, T>(a, b, in.p[2] + off, in.p[2] + off, t, kxlim);
+      fft.inv(z, z0, buf, t);
+      xpair_make<NX, KE, T>(z, a, b, t, kxlim, false);
       if (r + hop < nrows) {
         const size_t no = (size_t)(r + hop) * nxp;
-        xpair_load<NX, E, T>(a, b, in.p[0] + no, in.p[1] + no, t, kxlim);
+        xpair_load<NX, KE, T>(a, b, in.p[0] + no, in.p[1] + no, t, kxlim);
       }
-      FI::run(z1, buf, t, tw);
+      fft.inv(z, z1, buf, t);
+      if (X::live(t)) {
 #pragma unroll
-      for (int m = 0; m < E; ++m)
-        big = fmax(big, z0[m].x * z0[m].x + z0[m].y * z0[m].y + z1[m].x * z1[m].x);
+        for (int m = 0; m < SE; ++m)
+          big = fmax(big, z0[m].x * z0[m].x + z0[m].y * z0[m].y + z1[m].x * z1[m].x);
+      }
     }
   }
   // (kRowBound lanes are whole waves; a narrower block leaves its missing lanes out)
@@ -1906,10 +1932,8 @@ __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part,
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt) {
-  using Cfg = FFTCfg<NX>;
-  using FF = LineFFT<NX, -1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1917,24 +1941,24 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, i
   if (r >= (long)g.nz * g.ny) return;
   const size_t off = (size_t)r * nxp, roff = (size_t)r * NX;
   cplx *buf = lds + lt * lds_line_stride(NX);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
-  cplx z[E], nxt[E];
+  X fft;
+  fft.load_fwd(twt, t);
+  cplx x[SE], nxt[SE], z[KE];
   const int np = (nf + 1) / 2;
-  xpair_real<E>(z, in.p[0] + roff, nf > 1 ? in.p[1] + roff : nullptr, t, T);
+  if (X::live(t)) xpair_real<SE>(x, in.p[0] + roff, nf > 1 ? in.p[1] + roff : nullptr, t, A);
   for (int p = 0; p < np; ++p) {
     const bool two = 2 * p + 1 < nf;
     if (p + 1 < np) {
       const int fa = 2 * p + 2;
-      xpair_real<E>(nxt, in.p[fa] + roff, fa + 1 < nf ? in.p[fa + 1] + roff : nullptr, t, T);
+      if (X::live(t)) xpair_real<SE>(nxt, in.p[fa] + roff, fa + 1 < nf ? in.p[fa + 1] + roff : nullptr, t, A);
     }
-    FF::run(z, buf, t, tw);
+    fft.fwd(x, z, buf, t);
     if (two)
-      xpair_store2<NX, E, T>(z, buf, t, out.p[2 * p] + off, out.p[2 * p + 1] + off, NX / 2 + 1);
+      xpair_store2<NX, KE, T>(z, buf, t, out.p[2 * p] + off, out.p[2 * p + 1] + off, NX / 2 + 1);
     else
-      xpair_store1<NX, E, T>(z, t, out.p[2 * p] + off, NX / 2 + 1);
+      xpair_store1<NX, KE, T>(z, t, out.p[2 * p] + off, NX / 2 + 1);
 #pragma unroll
-    for (int m = 0; m < E; ++m) z[m] = nxt[m];
+    for (int m = 0; m < SE; ++m) x[m] = nxt[m];
   }
 }
 
@@ -1944,11 +1968,8 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  using FF = LineFFT<NX, -1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1957,24 +1978,27 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
   const size_t off = (size_t)r * nxp;
   cplx *buf = lds + lt * lds_line_stride(NX);
   const double tmp = -g.inv_n6;
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
-  cplx a[E], b[E], z0[E], z1[E], z2[E];
-  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
-  xpair_make<NX, E, T>(z0, a, b, t, kxlim);
-  xpair_load<NX, E, T>(a, b, in.p[2] + off, in.p[3] + off, t, kxlim);
-  FI::run(z0, buf, t, tw);
-  xpair_make<NX, E, T>(z1, a, b, t, kxlim);
-  xpair_load<NX, E, T>(a, b, in.p[4] + off, in.p[5] + off, t, kxlim);
-  FI::run(z1, buf, t, tw);
-  xpair_make<NX, E, T>(z2, a, b, t, kxlim);
-  FI::run(z2, buf, t, tw);
+  X fft;
+  fft.load_inv(twt, t);
+  cplx a[KE], b[KE], z[KE], z0[SE], z1[SE], z2[SE];
+  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[2] + off, in.p[3] + off, t, kxlim);
+  fft.inv(z, z0, buf, t);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[4] + off, in.p[5] + off, t, kxlim);
+  fft.inv(z, z1, buf, t);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  fft.inv(z, z2, buf, t);
   // samples: A_x = z0.x, A_y = z0.y, A_z = z1.x, B_x = z1.y, B_y = z2.x, B_z = z2.y
+  fft.load_fwd_too(twt, t);
+  if (X::live(t)) {
 #pragma unroll
-  for (int m = 0; m < E; ++m)
-    z0[m] = c_make(((z0[m].x * z1[m].y + z0[m].y * z2[m].x) + z1[m].x * z2[m].y) * tmp, 0.0);
-  FF::run(z0, buf, t, tw);
-  xpair_store1<NX, E, T>(z0, t, out.p[0] + off, kxout);
+    for (int m = 0; m < SE; ++m)
+      z0[m] = c_make(((z0[m].x * z1[m].y + z0[m].y * z2[m].x) + z1[m].x * z2[m].y) * tmp, 0.0);
+  }
+  fft.fwd(z0, z, buf, t);
+  xpair_store1<NX, KE, T>(z, t, out.p[0] + off, kxout);
 }
 
 // Fused X^-1 . (P x Q)/N^6 . X with two-for-one transforms: pairs (P_x, P_y),
@@ -1985,11 +2009,8 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
-  using Cfg = FFTCfg<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  using FF = LineFFT<NX, -1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
+  using X = XLine<NX>;
+  constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -2001,74 +2022,23 @@ __global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet ou
   const double tmp = g.inv_n6;
   const FieldView in = batch_view(in_, blockIdx.y);
   const FieldView out = batch_view(out_, blockIdx.y);
-  TwCache<NX, Cfg> tw;
-  tw.load(twt, t);
-  cplx a[E], b[E], z0[E], z1[E], z2[E];
-  xpair_load<NX, E, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
-  xpair_make<NX, E, T>(z0, a, b, t, kxlim);
-  xpair_load<NX, E, T>(a, b, in.p[2] + off, in.p[3] + off, t, kxlim);
-  FI::run(z0, buf, t, tw);
-  xpair_make<NX, E, T>(z1, a, b, t, kxlim);
-  xpair_load<NX, E, T>(a, b, in.p[4] + off, in.p[5] + off, t, kxlim);
-  FI::run(z1, buf, t, tw);
-  xpair_make<NX, E, T>(z2, a, b, t, kxlim);
-  FI::run(z2, buf, t, tw);
+  X fft;
+  fft.load_inv(twt, t);
+  cplx a[KE], b[KE], z[KE], z0[SE], z1[SE], z2[SE];
+  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[2] + off, in.p[3] + off, t, kxlim);
+  fft.inv(z, z0, buf, t);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  xpair_load<NX, KE, T>(a, b, in.p[4] + off, in.p[5] + off, t, kxlim);
+  fft.inv(z, z1, buf, t);
+  xpair_make<NX, KE, T>(z, a, b, t, kxlim);
+  fft.inv(z, z2, buf, t);
   // samples: P_x = z0.x, P_y = z0.y, P_z = z1.x, Q_x = z1.y, Q_y = z2.x, Q_z = z2.y
+  fft.load_fwd_too(twt, t);
+  if (X::live(t)) {
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const double px = z0[m].x, py = z0[m].y, pz = z1[m].x, qx = z1[m].y, qy = z2[m].x, qz = z2[m].y;
-    const double ox = (py * qz - qy * pz) * tmp;
-    const double oy = (pz * qx - qz * px) * tmp;
-    const double oz = (px * qy - qx * py) * tmp;
-    z0[m] = c_make(ox, oy);
-    z1[m] = c_make(oz, 0.0);
-  }
-  FF::run(z0, buf, t, tw);
-  xpair_store2<NX, E, T>(z0, buf, t, out.p[0] + off, out.p[1] + off, kxout);
-  FF::run(z1, buf, t, tw);
-  xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxout);
-}
-
-// k_xcross2 and k_xdot2 on 12 points per lane, two radix-12/16 stages for a
-// 192-point row instead of {6, 2..}: fewer LDS exchanges on the chain that
-// bounds them.  The three transformed pairs fill the registers (2 waves per
-// SIMD, as the 6-point kernels), so twiddles are read where they are used and
-// the scheduling barriers keep a pair's loads behind the transform before it.
-template <int NX, bool CROSS>
-__global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) void k_xmul12(
-    FieldSet in_, FieldSet out_, GridK g, int nxp, const cplx *__restrict__ twt, int prune) {
-  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
-  using Cfg = FFTCfgMid<NX>;
-  using FI = LineFFT<NX, +1, Cfg>;
-  using FF = LineFFT<NX, -1, Cfg>;
-  constexpr int T = Cfg::T, E = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
-  extern __shared__ cplx lds[];
-  const int rpb = blockDim.x / T;
-  const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  const long r = (long)blockIdx.x * rpb + lt;
-  if (r >= (long)g.nz * g.ny) return;  // whole lines only: wave-level syncs
-  const size_t off = (size_t)r * nxp;
-  cplx *buf = lds + lt * lds_line_stride(NX);
-  const FieldView in = batch_view(in_, blockIdx.y);
-  const FieldView out = batch_view(out_, blockIdx.y);
-  cplx z0[E], z1[E], z2[E];
-  auto inverse = [&](cplx (&z)[E], int fa, int fb) {
-    __builtin_amdgcn_sched_barrier(0);
-    cplx a[E], b[E];
-    xpair_load<NX, E, T>(a, b, in.p[fa] + off, in.p[fb] + off, t, kxlim);
-    xpair_make<NX, E, T>(z, a, b, t, kxlim);
-    __builtin_amdgcn_sched_barrier(0);
-    FI::run(z, buf, t, twt);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  inverse(z0, 0, 1);
-  inverse(z1, 2, 3);
-  inverse(z2, 4, 5);
-  if constexpr (CROSS) {
-    const double tmp = g.inv_n6;
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
+    for (int m = 0; m < SE; ++m) {
       const double px = z0[m].x, py = z0[m].y, pz = z1[m].x, qx = z1[m].y, qy = z2[m].x, qz = z2[m].y;
       const double ox = (py * qz - qy * pz) * tmp;
       const double oy = (pz * qx - qz * px) * tmp;
@@ -2076,20 +2046,11 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) 
       z0[m] = c_make(ox, oy);
       z1[m] = c_make(oz, 0.0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    FF::run(z0, buf, t, twt);
-    xpair_store2<NX, E, T>(z0, buf, t, out.p[0] + off, out.p[1] + off, kxout);
-    FF::run(z1, buf, t, twt);
-    xpair_store1<NX, E, T>(z1, t, out.p[2] + off, kxout);
-  } else {
-    const double tmp = -g.inv_n6;
-#pragma unroll
-    for (int m = 0; m < E; ++m)
-      z0[m] = c_make(((z0[m].x * z1[m].y + z0[m].y * z2[m].x) + z1[m].x * z2[m].y) * tmp, 0.0);
-    __builtin_amdgcn_sched_barrier(0);
-    FF::run(z0, buf, t, twt);
-    xpair_store1<NX, E, T>(z0, t, out.p[0] + off, kxout);
   }
+  fft.fwd(z0, z, buf, t);
+  xpair_store2<NX, KE, T>(z, buf, t, out.p[0] + off, out.p[1] + off, kxout);
+  fft.fwd(z1, z, buf, t);
+  xpair_store1<NX, KE, T>(z, t, out.p[2] + off, kxout);
 }
 
 // Fused X^-1 . (P x Q)/N^6 . X on P rows with GHOST's operand order
@@ -2841,14 +2802,6 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
   if (g.nx % 2) return hipErrorInvalidValue;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
-  if (use_xmul12(g, c.batch)) {
-    constexpr int T = FFTCfgMid<192>::T;
-    const PassShape s = row_shape(T, lds_line_stride(192), max_lds());
-    GHX_LAUNCH_CHECK((k_xmul12<192, true>), s, kRowBound, T, false);
-    hipLaunchKernelGGL((k_xmul12<192, true>), dim3((unsigned)((nrows + s.lines - 1) / s.lines), c.batch), dim3(s.block),
-                       s.lds, c.stream, in, out, g, nxp, c.tw_x, prune);
-    return hipGetLastError();
-  }
   if (use_x2(g.nx)) {
     switch (g.nx) {
 #define GHX_CASE(n_)                                                                        \
@@ -2899,14 +2852,6 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
   if (g.nx % 2) return hipErrorInvalidValue;
   const long nrows = (long)g.nz * g.ny;
   const int nxp = p_row(g);
-  if (use_xmul12(g, 1)) {
-    constexpr int T = FFTCfgMid<192>::T;
-    const PassShape s = row_shape(T, lds_line_stride(192), max_lds());
-    GHX_LAUNCH_CHECK((k_xmul12<192, false>), s, kRowBound, T, false);
-    hipLaunchKernelGGL((k_xmul12<192, false>), dim3((unsigned)((nrows + s.lines - 1) / s.lines), 1), dim3(s.block),
-                       s.lds, c.stream, in, out, g, nxp, c.tw_x, prune);
-    return hipGetLastError();
-  }
   if (use_x2(g.nx)) {
     switch (g.nx) {
 #define GHX_CASE(n_)                                                                        \

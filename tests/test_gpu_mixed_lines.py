@@ -1,6 +1,9 @@
-"""Products of 192-point rows take 12 points per lane from 4096 rows on and 6
-below: one RK2 step of each solver on both sides of the line, rotating and
-forced or not, against the oracle, relative L2 1e-12."""
+"""Lines of 3 * 2^k points (24 .. 384) in radix-6, 8 and 4 stages, along each
+axis and next to axes that fill neither a wavefront nor a tile: one RK2 step of
+each solver with the tracers' velocities and the extrema, against the oracle,
+relative L2 1e-12 (the transforms of one to three fields alone are in
+test_gpu_row_pairs)."""
+import numpy as np
 import pytest
 
 from test_gpu_parity import grids, rel, to_gpu, to_np
@@ -8,20 +11,36 @@ from test_gpu_small_launch import state
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(192, 64, 64), (192, 48, 64), (192, 32, 128), (192, 24, 192)]
+LENGTHS = [24, 48, 96, 192, 384]
+SHAPES = [(n, 24, 16) for n in LENGTHS] + [(24, n, 16) for n in LENGTHS] + [(16, 24, n) for n in LENGTHS] + [
+    (192, 48, 64), (96, 96, 48), (48, 192, 96), (24, 64, 384)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
 def test_hd(gpu, shape):
+    from ghost_amd.lagpart import GPart
     from ghost_amd.solvers import HDSolver
     g, og = grids(shape)
     v = state(og, 3, 301)
-    s = HDSolver(g, dt=1e-3, nu=4e-3, ord=2)
+    s = HDSolver(g, dt=1e-3, nu=4e-3, ord=1)
     s.set_velocity([to_gpu(x) for x in v])
-    og.hd_step(v, 1e-3, 4e-3, ord=2)
+    p = GPart(g, 40)
+    rng = np.random.default_rng(302)
+    pos = [rng.uniform(0.0, n, 40) for n in shape]
+    p.set_positions(*[to_gpu(x) for x in pos])
+    s.set_tracers(p)
+    og.hd_step(v, 1e-3, 4e-3, ord=1)
     s.step(1)
     for got, want in zip(s.velocity(), v):
         assert rel(to_np(got), want) < 1e-12
+    ref = [x.copy() for x in pos]
+    og.tracer_stage(v, ref, [x.copy() for x in pos], 1e-3, 1.0, ghost_solve=False)
+    for x, want, n in zip(p.positions(), ref, shape):
+        d = np.mod(to_np(x) - want + n / 2, n) - n / 2
+        assert np.max(np.abs(d)) < 1e-10
+    V = [to_gpu(x) for x in v]
+    for kin in (0, 1):
+        assert g.maxabs(*V, kin) == pytest.approx(og.maxabs(*v, kin), rel=1e-12)
 
 
 @pytest.mark.parametrize("shape", SHAPES)
