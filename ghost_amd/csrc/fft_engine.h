@@ -89,12 +89,9 @@ template <> struct FFTCfgWide<512> {
   GHX_DEV static constexpr int radix(int) { return 8; }
 };
 
-// 12 points per lane for the 3 * 2^k lines: half the stages (and LDS
-// exchanges) of the 6-point schedules at twice the registers per field, for
-// passes that keep one field live (the y passes).  Those that hold three
-// fields spill on it or lose a wave per SIMD: measured at 192^3, the curl z
-// inverse 53 -> 75, the fused x pass 132 -> 157 us.  24 and 48 points gain
-// nothing (YInvCfg, YFwdCfg).
+// 12 points per lane for the 3 * 2^k lines, for passes that keep one field live
+// and wait on memory more than on their exchanges (the y passes, the one-field
+// z inverses).  The others take the mixed stages (MixFFT).
 template <int N> struct FFTCfgMid : FFTCfg<N> {};
 #define GHX_FFTCFGMID(N_, NS_, ...)                                     \
   template <> struct FFTCfgMid<N_> {                                    \
@@ -352,7 +349,13 @@ template <int N, int DIR, typename Cfg = FFTCfg<N>> struct LineFFT {
 // inverse starts with radix 6, the forward ends with it: the wavenumber side
 // is held as x[t + T m] (m < 6) by every lane, the other side as x[t + A m]
 // (m < 8) by the lanes t < A, and a pass that does both needs no exchange to
-// get from one to the other.
+// get from one to the other.  Measured, 6-point schedule -> mixed stages, us: X
+// cross 1084 -> 743 at 384^3, 125 -> 98 at 192^3, 24.7 -> 21.6 at 96^3, 11.6 ->
+// 9.8 at 48^3, 10.5 -> 9.6 at 24^3; X dot 116 -> 81 at 384 x 192 x 96; three
+// interleaved x inverses 606 -> 446 at 384^3; one field's x inverse 200 -> 162,
+// x forward 196 -> 170 and z forward 266 -> 238 at 384^3; curl z inverse 391 ->
+// 325 at 384^3, 54 -> 46 at 192^3; MHD z inverse 97 -> 83, HD update 52 -> 47 at
+// 192^3, 57 -> 32 at 96 x 96 x 384.
 // ---------------------------------------------------------------------------
 template <int N> struct MixCfg;  // radices of the 8-point stages, in the inverse's order (1: no stage)
 template <> struct MixCfg<24> { static constexpr int R1 = 4, R2 = 1; };
@@ -464,4 +467,67 @@ template <int N, int DIR> struct MixFFT {
       butterflies<6, true, 6>(out, c);
     }
   };
+};
+
+// One lane's part of a line's transforms in either direction, with KE points
+// on the wavenumber side (k = t + T m, every lane) and SE on the sample side
+// (n = t + A m, in the lanes with live(t)): LineFFT of a schedule Cfg, one
+// layout on both sides, or MixFFT for FFTCfgMix.
+constexpr bool mix_length(int n) { return n == 24 || n == 48 || n == 96 || n == 192 || n == 384; }
+template <int N, bool = mix_length(N)> struct FFTCfgMix : FFTCfg<N> {};
+template <int N> struct FFTCfgMix<N, true> {
+  static constexpr int E = 6, T = N / 6;
+};
+
+template <int N, typename Cfg = FFTCfg<N>> struct Line {
+  static constexpr int T = Cfg::T, A = T, KE = Cfg::E, SE = Cfg::E;
+  TwCache<N, Cfg> tw;
+  GHX_DEV void load_inv(const cplx *w, int t) { tw.load(w, t); }
+  GHX_DEV void load_fwd(const cplx *w, int t) { tw.load(w, t); }
+  GHX_DEV void load_fwd_too(const cplx *, int) {}  // after load_inv: the same roots
+  GHX_DEV static constexpr bool live(int) { return true; }
+  GHX_DEV void inv(cplx (&k)[KE], cplx (&x)[SE], cplx *buf, int t) const {
+#pragma unroll
+    for (int m = 0; m < SE; ++m) x[m] = k[m];
+    LineFFT<N, +1, Cfg>::run(x, buf, t, tw);
+  }
+  GHX_DEV void fwd(cplx (&x)[SE], cplx (&k)[KE], cplx *buf, int t) const {
+#pragma unroll
+    for (int m = 0; m < KE; ++m) k[m] = x[m];
+    LineFFT<N, -1, Cfg>::run(k, buf, t, tw);
+  }
+  // samples to and from the line's LDS row
+  GHX_DEV static void put(const cplx (&x)[SE], cplx *row, int t) {
+#pragma unroll
+    for (int m = 0; m < SE; ++m) row[lds_pad(t + T * m)] = x[m];
+  }
+  GHX_DEV static void get(cplx (&x)[SE], const cplx *row, int t) {
+#pragma unroll
+    for (int m = 0; m < SE; ++m) x[m] = row[lds_pad(t + T * m)];
+  }
+};
+template <int N> struct Line<N, FFTCfgMix<N, true>> {
+  using I = MixFFT<N, +1>;
+  using F = MixFFT<N, -1>;
+  static constexpr int T = I::T, A = I::A, KE = 6, SE = 8;
+  typename I::Inv wi;
+  typename F::Fwd wf;
+  GHX_DEV void load_inv(const cplx *w, int t) { wi.load(w, t); }
+  GHX_DEV void load_fwd(const cplx *w, int t) { wf.load(w, t); }
+  GHX_DEV void load_fwd_too(const cplx *w, int t) { wf.load(w, t); }
+  GHX_DEV static bool live(int t) { return t < A; }
+  GHX_DEV void inv(cplx (&k)[6], cplx (&x)[8], cplx *buf, int t) const { wi.run(k, x, buf, t); }
+  GHX_DEV void fwd(cplx (&x)[8], cplx (&k)[6], cplx *buf, int t) const { wf.run(x, k, buf, t); }
+  GHX_DEV static void put(const cplx (&x)[8], cplx *row, int t) {
+    if (t < A) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) row[lds_pad(t + A * m)] = x[m];
+    }
+  }
+  GHX_DEV static void get(cplx (&x)[8], const cplx *row, int t) {
+    if (t < A) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) x[m] = row[lds_pad(t + A * m)];
+    }
+  }
 };

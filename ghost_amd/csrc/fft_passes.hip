@@ -370,14 +370,12 @@ GHX_DEV unsigned tile_lines_active(const GridK &g, int i, int j0, int L) {
 // ---------------------------------------------------------------------------
 // Z^-1: S -> Q.  Block = (kx index i, ky chunk j0..j0+L-1).
 // ---------------------------------------------------------------------------
-// The store half of zinv_emit: the transformed line v (natural order, lane t
-// holding points t + T m) into the block's LDS rows, then the tile to Q.
-template <int N, int E, typename Cfg = FFTCfg<N>, int GW = 0>
-GHX_DEV void zinv_store(const cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, cplx *dst,
+// The store half of zinv_emit: the transformed line v (samples as Line holds
+// them) into the block's LDS rows, then the tile to Q.
+template <int N, int E, typename Cfg = FFTCfgMix<N>, int GW = 0>
+GHX_DEV void zinv_store(const cplx (&v)[Line<N, Cfg>::SE], cplx *lds, cplx *row, int stride, int L, int t, cplx *dst,
                         const GridK &g, int i, int j0, unsigned lmask) {
-  constexpr int T = LineFFT<N, +1, Cfg>::T;
-#pragma unroll
-  for (int m = 0; m < E; ++m) row[lds_pad(t + T * m)] = v[m];
+  Line<N, Cfg>::put(v, row, t);
   __syncthreads();
   const int ny = g.ny;
   tile_store_rows<E, false, GW>(lds, stride, L, dst + (size_t)i * ny + j0, (size_t)g.nxh * ny,
@@ -385,11 +383,17 @@ GHX_DEV void zinv_store(const cplx (&v)[E], cplx *lds, cplx *row, int stride, in
   __syncthreads();
 }
 
-template <int N, int E, typename Cfg = FFTCfg<N>, int GW = 0>
-GHX_DEV void zinv_emit(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, const TwCache<N, Cfg> &tw,
+template <int N, int E, typename Cfg = FFTCfgMix<N>, int GW = 0>
+GHX_DEV void zinv_emit(const Line<N, Cfg> &fft, cplx (&v)[E], cplx (&x)[Line<N, Cfg>::SE], cplx *lds, cplx *row,
+                       int stride, int L, int t, cplx *dst, const GridK &g, int i, int j0, unsigned lmask) {
+  fft.inv(v, x, row, t);
+  zinv_store<N, E, Cfg, GW>(x, lds, row, stride, L, t, dst, g, i, j0, lmask);
+}
+template <int N, int E, typename Cfg = FFTCfgMix<N>, int GW = 0>
+GHX_DEV void zinv_emit(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, const Line<N, Cfg> &fft,
                        cplx *dst, const GridK &g, int i, int j0, unsigned lmask) {
-  LineFFT<N, +1, Cfg>::run(v, row, t, tw);
-  zinv_store<N, E, Cfg, GW>(v, lds, row, stride, L, t, dst, g, i, j0, lmask);
+  cplx x[Line<N, Cfg>::SE];
+  zinv_emit<N, E, Cfg, GW>(fft, v, x, lds, row, stride, L, t, dst, g, i, j0, lmask);
 }
 
 // A vector field's z inverse and its curl's with five transforms instead of
@@ -399,49 +403,53 @@ GHX_DEV void zinv_emit(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, in
 //   curl_x = i ky Z^-1(a_z) - Z^-1(i kz a_y)
 //   curl_y = Z^-1(i kz a_x) - i kx Z^-1(a_z)
 //   curl_z = i kx Z^-1(a_y) - i ky Z^-1(a_x)
-// ax, ay, az (the spectral lines, lane t holding points t + T m) are
-// transformed in place; the six results go to o[0..2] (a) and o[3..5] (curl a).
+// ax, ay, az are the spectral lines (lane t holding points t + T m); the six
+// results go to o[0..2] (a) and o[3..5] (curl a).
 template <int N, int E, typename Cfg, int GW = 0>
 GHX_DEV void zinv_curl5(cplx (&ax)[E], cplx (&ay)[E], cplx (&az)[E], double kx, double ky, cplx *lds, cplx *row,
-                        int stride, int L, int t, const TwCache<N, Cfg> &tw, cplx *const *o, const GridK &g, int i,
+                        int stride, int L, int t, const Line<N, Cfg> &fft, cplx *const *o, const GridK &g, int i,
                         int j0, unsigned lmask) {
-  using F = LineFFT<N, +1, Cfg>;
-  constexpr int T = F::T;
-  zinv_emit<N, E, Cfg, GW>(az, lds, row, stride, L, t, tw, o[2], g, i, j0, lmask);  // az := Z^-1(a_z)
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, SE = F::SE;
+  cplx zx[SE], zy[SE], zz[SE];  // Z^-1 of the three
+  zinv_emit<N, E, Cfg, GW>(fft, az, zz, lds, row, stride, L, t, o[2], g, i, j0, lmask);
   {
-    cplx w[E];
+    cplx w[E], x[SE];
 #pragma unroll
     for (int m = 0; m < E; ++m) w[m] = c_ik(wavenum(t + T * m, g.nz, g.dkz), ay[m]);
-    F::run(w, row, t, tw);
+    fft.inv(w, x, row, t);
+    if (F::live(t)) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) w[m] = c_sub(c_ik(ky, az[m]), w[m]);
-    zinv_store<N, E, Cfg, GW>(w, lds, row, stride, L, t, o[3], g, i, j0, lmask);
+      for (int m = 0; m < SE; ++m) x[m] = c_sub(c_ik(ky, zz[m]), x[m]);
+    }
+    zinv_store<N, E, Cfg, GW>(x, lds, row, stride, L, t, o[3], g, i, j0, lmask);
   }
   {
-    cplx w[E];
+    cplx w[E], x[SE];
 #pragma unroll
     for (int m = 0; m < E; ++m) w[m] = c_ik(wavenum(t + T * m, g.nz, g.dkz), ax[m]);
-    F::run(w, row, t, tw);
+    fft.inv(w, x, row, t);
+    if (F::live(t)) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) w[m] = c_sub(w[m], c_ik(kx, az[m]));
-    zinv_store<N, E, Cfg, GW>(w, lds, row, stride, L, t, o[4], g, i, j0, lmask);
+      for (int m = 0; m < SE; ++m) x[m] = c_sub(x[m], c_ik(kx, zz[m]));
+    }
+    zinv_store<N, E, Cfg, GW>(x, lds, row, stride, L, t, o[4], g, i, j0, lmask);
   }
-  zinv_emit<N, E, Cfg, GW>(ax, lds, row, stride, L, t, tw, o[0], g, i, j0, lmask);  // ax := Z^-1(a_x)
-  zinv_emit<N, E, Cfg, GW>(ay, lds, row, stride, L, t, tw, o[1], g, i, j0, lmask);  // ay := Z^-1(a_y)
-  {
-    cplx w[E];
+  zinv_emit<N, E, Cfg, GW>(fft, ax, zx, lds, row, stride, L, t, o[0], g, i, j0, lmask);
+  zinv_emit<N, E, Cfg, GW>(fft, ay, zy, lds, row, stride, L, t, o[1], g, i, j0, lmask);
+  if (F::live(t)) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) w[m] = c_sub(c_ik(kx, ay[m]), c_ik(ky, ax[m]));
-    zinv_store<N, E, Cfg, GW>(w, lds, row, stride, L, t, o[5], g, i, j0, lmask);
+    for (int m = 0; m < SE; ++m) zx[m] = c_sub(c_ik(kx, zy[m]), c_ik(ky, zx[m]));
   }
+  zinv_store<N, E, Cfg, GW>(zx, lds, row, stride, L, t, o[5], g, i, j0, lmask);
 }
 
-template <int N, int MODE, typename Cfg = FFTCfg<N>>
+template <int N, int MODE, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_, int nf, GridK g, const cplx *__restrict__ twt,
                                              int prune_, const double *__restrict__ aux) {
-  using F = LineFFT<N, +1, Cfg>;
+  using F = Line<N, Cfg>;
   const int prune = prune_input(g, prune_);
-  constexpr int T = F::T, E = F::E;
+  constexpr int T = F::T, E = F::KE;
   // store groups: the MHD and Boussinesq passes (MODE 2, 5) are at the
   // register limit and spill more with grouped reads; they store one point
   // per trip.  The curl pass takes all 8 points of a lane in one group
@@ -450,8 +458,8 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_inv(twt, t);
   const FieldView in = batch_view(in_, blockIdx.z);
   const FieldView out = batch_view(out_, blockIdx.z);
   int bx, by;
@@ -486,7 +494,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
         v[m] = load(in.p[f], t + T * m);
         if constexpr (MODE == 3) v[m] = c_scale(v[m], sxy * aux[g.nxh + g.ny + t + T * m]);
       }
-      zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, tw, out.p[f], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, fft, out.p[f], g, i, j0, lmask);
     }
   } else if constexpr (MODE == 1) {
     // v -> (v, curl v)
@@ -499,7 +507,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
       vz[m] = load(in.p[2], t + T * m);
     }
     cplx *const o[6] = {out.p[0], out.p[1], out.p[2], out.p[3], out.p[4], out.p[5]};
-    zinv_curl5<N, E, Cfg, SG>(vx, vy, vz, kx, ky, lds, row, stride, L, t, tw, o, g, i, j0, lmask);
+    zinv_curl5<N, E, Cfg, SG>(vx, vy, vz, kx, ky, lds, row, stride, L, t, fft, o, g, i, j0, lmask);
   } else if constexpr (MODE == 2) {
     // (v, A) -> (v, curl v, b = curl A, curl b)
     const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j, g.ny, g.dky);
@@ -512,7 +520,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
         vz[m] = load(in.p[2], t + T * m);
       }
       cplx *const o[6] = {out.p[0], out.p[1], out.p[2], out.p[3], out.p[4], out.p[5]};
-      zinv_curl5<N, E, Cfg, SG>(vx, vy, vz, kx, ky, lds, row, stride, L, t, tw, o, g, i, j0, lmask);
+      zinv_curl5<N, E, Cfg, SG>(vx, vy, vz, kx, ky, lds, row, stride, L, t, fft, o, g, i, j0, lmask);
     }
     // b = curl A per mode (rotor3), then b and curl b
     cplx bx[E], by[E], bz[E];
@@ -525,7 +533,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
       bz[m] = c_sub(c_ik(kx, ay), c_ik(ky, ax));
     }
     cplx *const o[6] = {out.p[6], out.p[7], out.p[8], out.p[9], out.p[10], out.p[11]};
-    zinv_curl5<N, E, Cfg, SG>(bx, by, bz, kx, ky, lds, row, stride, L, t, tw, o, g, i, j0, lmask);
+    zinv_curl5<N, E, Cfg, SG>(bx, by, bz, kx, ky, lds, row, stride, L, t, fft, o, g, i, j0, lmask);
   } else if constexpr (MODE == 6) {
     // velocity gradients: v -> d v_i / d x_j for i, j = 1..3 (out.p[3 i + j],
     // i major), derivk3 (pseudospec3D_hd.f90:22-88) scaled by 1/(nx ny nz)
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
           const double kd = dir == 0 ? kx : (dir == 1 ? ky : wavenum(t + T * m, g.nz, g.dkz));
           v[m] = c_scale(c_ik(kd, u[c][m]), sc);
         }
-        zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, tw, out.p[3 * c + dir], g, i, j0, lmask);
+        zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, fft, out.p[3 * c + dir], g, i, j0, lmask);
       }
   } else if constexpr (MODE == 7) {
     // v -> curl v, rotor3's components formed at each mode
@@ -566,11 +574,10 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
                : c == 1 ? c_sub(c_ik(kz, u[0][m]), c_ik(kx, u[2][m]))
                         : c_sub(c_ik(kx, u[1][m]), c_ik(ky, u[0][m]));
       }
-      zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, tw, out.p[c], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(v, lds, row, stride, L, t, fft, out.p[c], g, i, j0, lmask);
     }
   } else {
     // MODE 4: (a, b, c, d) -> (a, b, c, grad d).  MODE 5: (v, th) -> (v, curl v, grad th).
-    using F = LineFFT<N, +1, Cfg>;
     const double kx = wavenum(i, g.nx, g.dkx), ky = wavenum(j, g.ny, g.dky);
     cplx ux[E], uy[E], uz[E];
 #pragma unroll
@@ -581,11 +588,11 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
     }
     if constexpr (MODE == 5) {
       cplx *const o[6] = {out.p[0], out.p[1], out.p[2], out.p[3], out.p[4], out.p[5]};
-      zinv_curl5<N, E, Cfg, SG>(ux, uy, uz, kx, ky, lds, row, stride, L, t, tw, o, g, i, j0, lmask);
+      zinv_curl5<N, E, Cfg, SG>(ux, uy, uz, kx, ky, lds, row, stride, L, t, fft, o, g, i, j0, lmask);
     } else {
-      zinv_emit<N, E, Cfg, SG>(ux, lds, row, stride, L, t, tw, out.p[0], g, i, j0, lmask);
-      zinv_emit<N, E, Cfg, SG>(uy, lds, row, stride, L, t, tw, out.p[1], g, i, j0, lmask);
-      zinv_emit<N, E, Cfg, SG>(uz, lds, row, stride, L, t, tw, out.p[2], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(ux, lds, row, stride, L, t, fft, out.p[0], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(uy, lds, row, stride, L, t, fft, out.p[1], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(uz, lds, row, stride, L, t, fft, out.p[2], g, i, j0, lmask);
     }
     // derivk3 (pseudospec3D_hd.f90:22-88) of the scalar along x, y, z:
     // Z^-1(i kx d) = i kx Z^-1(d) and likewise for ky, so two transforms
@@ -597,15 +604,18 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
       cplx w[E];
 #pragma unroll
       for (int m = 0; m < E; ++m) w[m] = c_ik(wavenum(t + T * m, g.nz, g.dkz), d[m]);
-      zinv_emit<N, E, Cfg, SG>(w, lds, row, stride, L, t, tw, out.p[base + 2], g, i, j0, lmask);
+      zinv_emit<N, E, Cfg, SG>(w, lds, row, stride, L, t, fft, out.p[base + 2], g, i, j0, lmask);
     }
-    F::run(d, row, t, tw);
+    cplx x[F::SE];
+    fft.inv(d, x, row, t);
 #pragma unroll
     for (int dir = 0; dir < 2; ++dir) {
-      cplx w[E];
+      cplx w[F::SE];
       const double kd = dir == 0 ? kx : ky;
+      if (F::live(t)) {
 #pragma unroll
-      for (int m = 0; m < E; ++m) w[m] = c_ik(kd, d[m]);
+        for (int m = 0; m < F::SE; ++m) w[m] = c_ik(kd, x[m]);
+      }
       zinv_store<N, E, Cfg, SG>(w, lds, row, stride, L, t, out.p[base + dir], g, i, j0, lmask);
     }
   }
@@ -635,12 +645,12 @@ GHX_DEV ZOut zinv_output(int mode, int o) {
   }
 }
 
-template <int N, typename Cfg = FFTCfg<N>>
+template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet out_, int mode, int nout, GridK g,
                                                  const cplx *__restrict__ twt, int prune_,
                                                  const double *__restrict__ aux) {
-  using F = LineFFT<N, +1, Cfg>;
-  constexpr int T = F::T, E = F::E;
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE;
   const int prune = prune_input(g, prune_);
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
@@ -652,8 +662,8 @@ __global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet 
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   if (lmask == 0u) return;  // uniform over the block
-  TwCache<N, Cfg> tw;
-  tw.load(twt, t);
+  F fft;
+  fft.load_inv(twt, t);
   const bool ok = j < g.ny && ((lmask >> lt) & 1u);
   const int stride = lds_line_stride(N);
   cplx *row = lds + lt * stride;
@@ -700,59 +710,37 @@ __global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet 
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = c_scale(v[m], sxy * aux[g.nxh + g.ny + t + T * m]);
   }
-  zinv_emit<N, E, Cfg>(v, lds, row, stride, L, t, tw, out_.p[o] + (size_t)member * out_.bstride, g, i, j0, lmask);
+  zinv_emit<N, E, Cfg>(v, lds, row, stride, L, t, fft, out_.p[o] + (size_t)member * out_.bstride, g, i, j0, lmask);
 }
 
 // ---------------------------------------------------------------------------
 // Z forward: Q -> S.  Block = (kx index i, ky chunk).  Transposed load.
 // ---------------------------------------------------------------------------
-template <int N, int E, typename Cfg = FFTCfg<N>>
-GHX_DEV void zfwd_load(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, const TwCache<N, Cfg> &tw,
+template <int N, int E, typename Cfg = FFTCfgMix<N>>
+GHX_DEV void zfwd_load(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, const Line<N, Cfg> &fft,
                        const cplx *src, const GridK &g, int i, int j0, unsigned lmask = ~0u) {
-  using F = LineFFT<N, -1, Cfg>;
-  constexpr int T = F::T;
   tile_load_q<E>(lds, stride, L, src, (size_t)g.nxh * g.ny, (size_t)i * g.ny, j0, g.ny, lmask);
   __syncthreads();
-#pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = row[lds_pad(t + T * m)];
+  cplx x[Line<N, Cfg>::SE];
+  fft.get(x, row, t);
   __syncthreads();
-  F::run(v, row, t, tw);
-}
-
-// The transform of a difference of two Q fields, FFT(a - b) = FFT(a) - FFT(b):
-// the lines are subtracted before one transform.
-template <int N, int E>
-GHX_DEV void zfwd_load_diff(cplx (&v)[E], cplx *lds, cplx *row, int stride, int L, int t, const TwCache<N> &tw,
-                            const cplx *srca, const cplx *srcb, const GridK &g, int i, int j0, unsigned lmask) {
-  using F = LineFFT<N, -1>;
-  constexpr int T = F::T;
-  tile_load_q<E>(lds, stride, L, srca, (size_t)g.nxh * g.ny, (size_t)i * g.ny, j0, g.ny, lmask);
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = row[lds_pad(t + T * m)];
-  __syncthreads();
-  tile_load_q<E>(lds, stride, L, srcb, (size_t)g.nxh * g.ny, (size_t)i * g.ny, j0, g.ny, lmask);
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = c_sub(v[m], row[lds_pad(t + T * m)]);
-  __syncthreads();
-  F::run(v, row, t, tw);
+  fft.fwd(x, v, row, t);
 }
 
 // prune: only the kept modes of the output are wanted (the caller reads no
 // other), so only the dealias disc's lines are loaded (the y forward wrote no
 // others) and only their kept modes are written; the rest of `out` keeps
 // whatever it held.
-template <int N, typename Cfg = FFTCfg<N>>
+template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zfwd(FieldSet in, FieldSet out, int nf, GridK g, const cplx *__restrict__ twt,
                                              int prune) {
-  using F = LineFFT<N, -1, Cfg>;
-  constexpr int T = F::T, E = F::E;
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_fwd(twt, t);
   int bx, by;
   xcd_tile(bx, by);
   const int i = by, j0 = bx * L, j = j0 + lt;
@@ -764,7 +752,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd(FieldSet in, FieldSet out, 
   const size_t sline = ((size_t)i * g.ny + (ok ? j : 0)) * N;
   for (int f = 0; f < nf; ++f) {
     cplx v[E];
-    zfwd_load<N, E, Cfg>(v, lds, row, stride, L, t, tw, in.p[f], g, i, j0, lmask);
+    zfwd_load<N, E, Cfg>(v, lds, row, stride, L, t, fft, in.p[f], g, i, j0, lmask);
     if (ok) {
 #pragma unroll
       for (int m = 0; m < E; ++m) {
@@ -828,11 +816,11 @@ struct ZUpdate {
 constexpr int zrk_groups(int KIND) { return KIND == 2 ? 4 : 3; }
 constexpr unsigned zrk_bound(int KIND) { return KIND == 2 ? 512 : 768; }
 
-template <int N, int KIND, typename Cfg = FFTCfg<N>>
+template <int N, int KIND, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, const cplx *__restrict__ twt,
                                                          ZUpdate rk, int prune) {
-  using F = LineFFT<N, -1, Cfg>;
-  constexpr int T = F::T, E = F::E, G = zrk_groups(KIND);
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE, G = zrk_groups(KIND);
   extern __shared__ cplx lds[];
   const int GL = blockDim.x / G, L = GL / T, lsh = 31 - __builtin_clz((unsigned)L);
   // groups are whole waves except for the shortest lines (GL < 64)
@@ -858,8 +846,8 @@ __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, 
   if (lmask == 0u) return;  // uniform over the block
   const int stride = lds_line_stride(N);
   cplx *rows = lds + c * L * stride, *row = rows + lt * stride;
-  TwCache<N, Cfg> tw;
-  tw.load(twt, t);
+  F fft;
+  fft.load_fwd(twt, t);
   // the tile of this component's product
   cplx P[E];
   {
@@ -897,10 +885,10 @@ __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, 
     cc[m] = cp[s];  // a second hit in the cache where C is v
   }
   __syncthreads();
-#pragma unroll
-  for (int m = 0; m < E; ++m) P[m] = row[lds_pad(t + T * m)];
+  cplx x[F::SE];
+  fft.get(x, row, t);
   line_sync<T>();  // a line's row is its own from here on
-  F::run(P, row, t, tw);
+  fft.fwd(x, P, row, t);
   // the other field that this component's product needs: Coriolis v_y, v_x;
   // buoyancy th; heat current v_z
   if constexpr (KIND != 1) {
@@ -964,16 +952,16 @@ __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, 
   }
 }
 
-template <int N, typename Cfg = FFTCfg<N>, int PF = 0>
+template <int N, typename Cfg = FFTCfgMix<N>, int PF = 0>
 __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g, const cplx *__restrict__ twt, RKParams rk,
                                                    int prune) {
-  using F = LineFFT<N, -1, Cfg>;
-  constexpr int T = F::T, E = F::E;
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_fwd(twt, t);
   const FieldView in = batch_view(in_, blockIdx.z);
   if (blockIdx.z && rk.bstride) {
     const size_t o = (size_t)blockIdx.z * rk.bstride;
@@ -1018,17 +1006,17 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
     for (int f = 0; f < 3; ++f) {
       tile_put_q<E>(lds, stride, L, w);
       __syncthreads();
-#pragma unroll
-      for (int m = 0; m < E; ++m) P[f][m] = row[lds_pad(t + T * m)];
+      cplx x[F::SE];
+      fft.get(x, row, t);
       __syncthreads();
       if (f < 2) tile_fetch_q<E>(w, L, in.p[f + 1], qs, qb, j0, g.ny, lmask);
-      F::run(P[f], row, t, tw);
+      fft.fwd(x, P[f], row, t);
       __syncthreads();
     }
   } else {
 #pragma unroll
     for (int f = 0; f < 3; ++f) {
-      zfwd_load<N, E, Cfg>(P[f], lds, row, stride, L, t, tw, in.p[f], g, i, j0, lmask);
+      zfwd_load<N, E, Cfg>(P[f], lds, row, stride, L, t, fft, in.p[f], g, i, j0, lmask);
       __syncthreads();
     }
   }
@@ -1068,16 +1056,16 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
 // the z product, nonlhd3 projection, heat current xtemp v_z added to the
 // advection, then the updates of v (nu) and th (kappa).  The k = 0 mode keeps
 // the step-start mean of th; v is zero there and outside the dealias set.
-template <int N>
+template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK g, const cplx *__restrict__ twt,
                                                       BoussRKParams rk, int prune) {
-  using F = LineFFT<N, -1>;
-  constexpr int T = F::T, E = F::E;
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_fwd(twt, t);
   int bx, by;
   xcd_tile(bx, by);
   const int i = by, j0 = bx * L, j = j0 + lt;
@@ -1110,7 +1098,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
     cplx P[3][E];
 #pragma unroll
     for (int f = 0; f < 3; ++f) {
-      zfwd_load<N, E>(P[f], lds, row, stride, L, t, tw, in.p[f], g, i, j0, lmask);
+      zfwd_load<N, E, Cfg>(P[f], lds, row, stride, L, t, fft, in.p[f], g, i, j0, lmask);
       __syncthreads();
     }
     if (ok) {
@@ -1142,7 +1130,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
     }
   }
   cplx A[E];
-  zfwd_load<N, E>(A, lds, row, stride, L, t, tw, in.p[3], g, i, j0, lmask);
+  zfwd_load<N, E, Cfg>(A, lds, row, stride, L, t, fft, in.p[3], g, i, j0, lmask);
   if (!ok) return;
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -1168,16 +1156,16 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
 // (w x u, j x b) (PART 0) and gauge3 (:230-336) for the potential from u x b
 // (PART 1).  The two parts are separate launches so that each keeps its
 // fields in registers.
-template <int N, int PART, typename Cfg = FFTCfg<N>>
+template <int N, int PART, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g, const cplx *__restrict__ twt, MHDRKParams rk,
                                                     int prune) {
-  using F = LineFFT<N, -1, Cfg>;
-  constexpr int T = F::T, E = F::E;
+  using F = Line<N, Cfg>;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_fwd(twt, t);
   int bx, by;
   xcd_tile(bx, by);
   const int i = by, j0 = bx * L, j = j0 + lt;
@@ -1218,11 +1206,11 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
     }
     tile_put_q<E>(lds, stride, L, wa);
     __syncthreads();
-#pragma unroll
-    for (int m = 0; m < E; ++m) D[f][m] = row[lds_pad(t + T * m)];
+    cplx x[F::SE];
+    fft.get(x, row, t);
     __syncthreads();
     if (f < 2) fetch(f + 1);
-    F::run(D[f], row, t, tw);
+    fft.fwd(x, D[f], row, t);
     __syncthreads();
   }
   if (!ok) return;
@@ -1268,17 +1256,17 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
 // an LDS tile with L-point (L*16-byte) chunks along kx.  Only kx < kxlim is
 // touched (kxlim < nx/2+1 when the fields are dealiased).
 // ---------------------------------------------------------------------------
-template <int N, typename Cfg = FFTCfg<N>>
+template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
                                              const cplx *__restrict__ twt, int prune_) {
-  using F = LineFFT<N, +1, Cfg>;
+  using F = Line<N, Cfg>;
   const int prune = prune_input(g, prune_), kxlim = prune ? g.kxact : g.nxh;
-  constexpr int T = F::T, E = F::E;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_inv(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
   // block's first of nper fields
   const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
@@ -1318,9 +1306,9 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
     } else {
       load(f, v);
     }
-    F::run(v, row, t, tw);
-#pragma unroll
-    for (int m = 0; m < E; ++m) row[lds_pad(t + T * m)] = v[m];
+    cplx x[F::SE];
+    fft.inv(v, x, row, t);
+    F::put(x, row, t);
     __syncthreads();
     tile_store_rows<E, true>(lds, stride, L, out.p[f] + (size_t)z * g.ny * nxp + kx0, (size_t)nxp,
                        [=](int l) { return kx0 + l < kxlim; });
@@ -1328,17 +1316,17 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
   }
 }
 
-template <int N, typename Cfg = FFTCfg<N>>
+template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
                                              const cplx *__restrict__ twt, int prune) {
-  using F = LineFFT<N, -1, Cfg>;
+  using F = Line<N, Cfg>;
   const int kxlim = prune ? g.kxact : g.nxh;
-  constexpr int T = F::T, E = F::E;
+  constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
-  TwCache<N, Cfg> tw;  // stage twiddle roots of this lane, loaded once
-  tw.load(twt, t);
+  F fft;  // with this lane's stage roots, loaded once
+  fft.load_fwd(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
   // block's first of nper fields
   const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
@@ -1382,11 +1370,10 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
     if constexpr (prefetch) {
       if (f + 1 < nf) tload(f + 1, nxt);
     }
-    cplx v[E];
-#pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = row[lds_pad(t + T * m)];
+    cplx v[E], x[F::SE];
+    F::get(x, row, t);
     __syncthreads();
-    F::run(v, row, t, tw);
+    fft.fwd(x, v, row, t);
     if (ok) {
       cplx *dst = out.p[f] + ((size_t)z * g.nxh + kx) * N;
 #pragma unroll
@@ -1709,51 +1696,12 @@ GHX_DEV void xpair_real(cplx (&z)[E], const double *sa, const double *sb, int t,
   for (int m = 0; m < E; ++m) z[m] = c_make(sa[t + T * m], sb ? sb[t + T * m] : 0.0);
 }
 
-// One lane's part of a row's transforms: KE points on the wavenumber side
-// (k = t + T m) and SE on the sample side (n = t + A m, in the lanes t < A).
-// Powers of two keep one layout; 3 * 2^k rows take the mixed stages (MixFFT),
-// whose passes the LDS exchanges bound less (6-point -> mixed, us): cross 1084
-// -> 743 at 384^3, 125 -> 98 at 192^3, 24.7 -> 21.6 at 96^3, 11.6 -> 9.8 at
-// 48^3, 10.5 -> 9.6 at 24^3; dot 116 -> 81 at 384 x 192 x 96; three
-// interleaved inverses 606 -> 446 at 384^3, 75 -> 63 at 192^3; one field's
-// inverse 200 -> 162 and forward 196 -> 170 at 384^3.
-template <int NX, bool MIX = (NX % 3 == 0)> struct XLine {
-  using Cfg = FFTCfg<NX>;
-  static constexpr int T = Cfg::T, A = T, KE = Cfg::E, SE = Cfg::E;
-  static_assert(T <= 64, "one row per wavefront or less");
-  TwCache<NX, Cfg> tw;
-  GHX_DEV void load_inv(const cplx *w, int t) { tw.load(w, t); }
-  GHX_DEV void load_fwd(const cplx *w, int t) { tw.load(w, t); }
-  GHX_DEV void load_fwd_too(const cplx *, int) {}  // after load_inv: the same roots
-  GHX_DEV static constexpr bool live(int) { return true; }
-  GHX_DEV void inv(cplx (&k)[KE], cplx (&x)[SE], cplx *buf, int t) const {
-#pragma unroll
-    for (int m = 0; m < SE; ++m) x[m] = k[m];
-    LineFFT<NX, +1, Cfg>::run(x, buf, t, tw);
-  }
-  GHX_DEV void fwd(cplx (&x)[SE], cplx (&k)[KE], cplx *buf, int t) const {
-#pragma unroll
-    for (int m = 0; m < KE; ++m) k[m] = x[m];
-    LineFFT<NX, -1, Cfg>::run(k, buf, t, tw);
-  }
-};
-template <int NX> struct XLine<NX, true> {
-  static constexpr int T = MixFFT<NX, +1>::T, A = MixFFT<NX, +1>::A, KE = 6, SE = 8;
-  typename MixFFT<NX, +1>::Inv wi;
-  typename MixFFT<NX, -1>::Fwd wf;
-  GHX_DEV void load_inv(const cplx *w, int t) { wi.load(w, t); }
-  GHX_DEV void load_fwd(const cplx *w, int t) { wf.load(w, t); }
-  GHX_DEV void load_fwd_too(const cplx *w, int t) { wf.load(w, t); }
-  GHX_DEV static bool live(int t) { return t < A; }
-  GHX_DEV void inv(cplx (&k)[6], cplx (&x)[8], cplx *buf, int t) const { wi.run(k, x, buf, t); }
-  GHX_DEV void fwd(cplx (&x)[8], cplx (&k)[6], cplx *buf, int t) const { wf.run(x, k, buf, t); }
-};
-
 // X^-1 of nf fields (an even count), two rows per transform.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int kxlim) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -1796,7 +1744,8 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict__ in, double *__restrict__ out,
                                                          long nrows, int nxp, const cplx *__restrict__ twt,
                                                          int kxlim) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -1824,7 +1773,8 @@ __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict_
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restrict__ in, cplx *__restrict__ out,
                                                          long nrows, int nxp, const cplx *__restrict__ twt) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -1849,7 +1799,8 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd_rows(const double *__restric
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int kxlim) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -1885,7 +1836,8 @@ __global__ __launch_bounds__(kRowBound) void k_xinv3i2(FieldSet in, double *out,
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part, GridK g, int nxp,
                                                       const cplx *__restrict__ twt, int kxlim) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   __shared__ double best[kRowBound / 64];
@@ -1932,7 +1884,8 @@ __global__ __launch_bounds__(kRowBound) void k_xnorm2(FieldSet in, double *part,
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt) {
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -1968,7 +1921,8 @@ template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -2004,12 +1958,15 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
 // Fused X^-1 . (P x Q)/N^6 . X with two-for-one transforms: pairs (P_x, P_y),
 // (P_z, Q_x), (Q_y, Q_z) inverse, (out_x, out_y) and out_z forward.  Same
 // fields, products and operand order as k_xcross.  One row per line of
-// T <= 64 lanes.
+// T <= 64 lanes.  384-point rows ask for a third wave per SIMD (168 registers,
+// 6 in scratch: 743 -> 685 us at 384^3); at 192 and 96 points that spills 15
+// and 11 and loses (98 -> 127 us at 192^3, 21.6 -> 25.9 at 96^3).
 template <int NX>
-__global__ __launch_bounds__(kRowBound) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
+__global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(NX == 384 ? 3 : 2))) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
-  using X = XLine<NX>;
+  using X = Line<NX, FFTCfgMix<NX>>;
+  static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
   const int rpb = blockDim.x / T;
@@ -2232,10 +2189,11 @@ static int zinv_outputs(int mode, int nf) {
   }
 }
 
-// modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
-// (one field 287 -> 190 us at 384^3, 27.4 -> 26.0 at 192^3, the same at 96^3)
+// Modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
+// (the spline pass 27 us against 30 on the mixed stages at 192^3, 153 against
+// 217 at 384^3); the mixed stages below.
 template <int N>
-using ZInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
+using ZInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfgMix<N>>::type;
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune,
                 const double *aux) {
   if (mode == 3 && !aux) return hipErrorInvalidValue;
@@ -2334,15 +2292,12 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
 #endif
 
 #if GHX_PART == 3
-// one field live, as ZInvCfg (one field 334 -> 260 us at 384^3)
-template <int N>
-using ZFwdCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
 hipError_t zfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
-    using Cfg = ZFwdCfg<n_>;                                                                \
+    using Cfg = FFTCfgMix<n_>;                                                              \
     constexpr int T = Cfg::T;                                                               \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_want("GHX_LZ", tile_default(T, 8)), max_lds());                                        \
     const int L = s.lines; const size_t lds = s.lds;                            \
@@ -2398,7 +2353,7 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
 #define GHX_CASE(n_)                                                                        \
   case n_:                                                                                  \
     if constexpr (FFTCfgLow<n_>::E != FFTCfg<n_>::E) if (c.sched & 1) return launch_zrk<n_, 0, FFTCfgLow<n_>>(c, in, u, prune, c.batch); \
-    return launch_zrk<n_, 0, FFTCfg<n_>>(c, in, u, prune, c.batch);
+    return launch_zrk<n_, 0, FFTCfgMix<n_>>(c, in, u, prune, c.batch);
       GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
@@ -2469,7 +2424,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
     u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.mu; u.fline = rk.fline;
     for (int k = 0; k < 6; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
     switch (g.nz) {
-#define GHX_CASE(n_) case n_: return launch_zrk<n_, 1, FFTCfg<n_>>(c, in, u, prune, 2);
+#define GHX_CASE(n_) case n_: return launch_zrk<n_, 1, FFTCfgMix<n_>>(c, in, u, prune, 2);
       GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
@@ -2517,14 +2472,17 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 #endif
 
 #if GHX_PART == 1
-// 12 points per lane for the long 3 * 2^k lines.  The lines below are latency,
-// not LDS: measured in one session, y inverse of six fields 100 -> 72 us at
-// 192^3 and 23 -> 20 at 96^3 but 14 -> 15 at 48^3; y forward of three
-// (without the prefetch, 8-line tiles) 47 -> 42 at 192^3 but 12 -> 13 at 96^3.
+// Schedules of the 3 * 2^k lines.  The y inverse is bound by its stores from 96
+// points on and takes 12 points per lane (six fields: mixed stages 100 against
+// 70 us at 192^3, 17.6 against 13.4 at 96^3); so does the y forward from 192 on
+// (45 against 43 us at 192^3), and keeps 6 at 96 (mixed 13.7 against 12.6 for
+// four fields, 12 points 13 against 12).  Shorter lines take the mixed stages
+// (9.0 -> 8.3 us at 48^3).
 template <int N>
-using YInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 96), FFTCfgMid<N>, FFTCfg<N>>::type;
-template <int N>
-using YFwdCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfg<N>>::type;
+using YInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E, FFTCfgMid<N>, FFTCfgMix<N>>::type;
+template <int N> struct YFwd { using Cfg = YInvCfg<N>; };
+template <> struct YFwd<96> { using Cfg = FFTCfg<96>; };
+template <int N> using YFwdCfg = typename YFwd<N>::Cfg;
 // the y passes on the four-points-per-lane schedule (FFTCtx::sched bit 1)
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
@@ -2846,6 +2804,11 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
 }  // namespace ghx
 
 #if GHX_PART == 8
+// The Boussinesq update on 192-point lines spills on the mixed stages (70 -> 84
+// us at 192^3) and keeps 6 points per lane; 384 and 96 points gain (64 -> 50 us
+// at 96 x 96 x 384, 15 -> 14 at 96^3).
+template <int N>
+using ZBoussCfg = typename std::conditional<N == 192, FFTCfg<N>, FFTCfgMix<N>>::type;
 namespace ghx {
 hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
@@ -2896,7 +2859,7 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
     u.fline = rk.fline;
     for (int k = 0; k < 4; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
     switch (g.nz) {
-#define GHX_CASE(n_) case n_: return launch_zrk<n_, 2, FFTCfg<n_>>(c, in, u, prune, 1);
+#define GHX_CASE(n_) case n_: return launch_zrk<n_, 2, FFTCfgMix<n_>>(c, in, u, prune, 1);
       GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
@@ -2910,8 +2873,9 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
     const PassShape s = tile_shape(T, lds_line_stride(n_) + n_, g.ny, tile_want("GHX_LZ", T >= 64 ? 2 : tile_default(T, 4)), max_lds());              \
     const int L = s.lines; const size_t lds = s.lds;                     \
     dim3 grid((g.ny + L - 1) / L, g.nxh);                                                   \
-    allow_lds(k_zfwd_rk_bouss<n_>, lds);                                                    \
-    GHX_LAUNCH_CHECK((k_zfwd_rk_bouss<n_>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zfwd_rk_bouss<n_>), grid, dim3(L * T), lds, c.stream, in, g, c.tw_z, rk, prune); \
+    using Cfg = ZBoussCfg<n_>;                                                              \
+    allow_lds((k_zfwd_rk_bouss<n_, Cfg>), lds);                                                    \
+    GHX_LAUNCH_CHECK((k_zfwd_rk_bouss<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zfwd_rk_bouss<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, g, c.tw_z, rk, prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
