@@ -1696,7 +1696,7 @@ GHX_DEV void xpair_real(cplx (&z)[E], const double *sa, const double *sb, int t,
   for (int m = 0; m < E; ++m) z[m] = c_make(sa[t + T * m], sb ? sb[t + T * m] : 0.0);
 }
 
-// X^-1 of nf fields (an even count), two rows per transform.
+// X^-1 of nf fields, two rows per transform (the last of an odd count alone).
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, int nf, GridK g, int nxp,
                                               const cplx *__restrict__ twt, int kxlim) {
@@ -1713,32 +1713,38 @@ __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, i
   X fft;
   fft.load_inv(twt, t);
   cplx a[KE], b[KE], z[KE], x[SE];
-  const int np = nf / 2;
-  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[1] + off, t, kxlim);
+  const int np = (nf + 1) / 2, last = nf - 1;
+  xpair_load<NX, KE, T>(a, b, in.p[0] + off, in.p[last ? 1 : 0] + off, t, kxlim);
   for (int p = 0; p < np; ++p) {
-    xpair_make<NX, KE, T>(z, a, b, t, kxlim);
-    if (p + 1 < np)  // next pair in flight
-      xpair_load<NX, KE, T>(a, b, in.p[2 * p + 2] + off, in.p[2 * p + 3] + off, t, kxlim);
+    const bool two = 2 * p < last;
+    xpair_make<NX, KE, T>(z, a, b, t, kxlim, two);
+    if (p + 1 < np) {  // next pair in flight
+      const int fa = 2 * p + 2;
+      xpair_load<NX, KE, T>(a, b, in.p[fa] + off, in.p[fa < last ? fa + 1 : fa] + off, t, kxlim);
+    }
     fft.inv(z, x, buf, t);
-    double *da = out.p[2 * p] + roff, *db = out.p[2 * p + 1] + roff;
     if (X::live(t)) {
+      double *da = out.p[2 * p] + roff;
 #pragma unroll
-      for (int m = 0; m < SE; ++m) {
-        da[t + A * m] = x[m].x;
-        db[t + A * m] = x[m].y;
+      for (int m = 0; m < SE; ++m) da[t + A * m] = x[m].x;
+      if (two) {
+        double *db = out.p[2 * p + 1] + roff;
+#pragma unroll
+        for (int m = 0; m < SE; ++m) db[t + A * m] = x[m].y;
       }
     }
   }
 }
 
-// One field's rows, paired with each other: rows 2p and 2p + 1 make one complex
-// line, so a lone field (or the last of an odd count) costs half a transform
-// per row; alone, with a zero imaginary part, it costs a whole one.  One field,
-// alone against paired: x inverse 519 -> 389 us at 512^3, 70 -> 53 at 256^3,
-// 429 -> 203 at 384^3, 55 -> 30 at 192^3; x forward 390 -> 192 at 384^3, 42 ->
-// 25 at 192^3, 10.7 -> 10.3 at 128^3, but 49 -> 52 at 256^3 and 397 -> 421 at
-// 512^3, which keep the lone form (pair_rows_fwd).  The last row of an odd
-// count goes alone.
+// A lone field's rows, paired with each other: rows 2p and 2p + 1 make one
+// complex line, half a transform per row; alone, with a zero imaginary part, a
+// row costs a whole one.  One field, alone against paired: x inverse 519 -> 389
+// us at 512^3, 70 -> 53 at 256^3, 429 -> 203 at 384^3, 55 -> 30 at 192^3 (6-point
+// schedule); x forward 390 -> 192 at 384^3, 42 -> 25 at 192^3, 10.7 -> 10.3 at
+// 128^3, but 49 -> 52 at 256^3 and 397 -> 421 at 512^3, which keep the lone form
+// (pair_rows_fwd).  The last of an odd count stays in its launch: as one of its
+// own 26.1 against 24.6 us for three inverses at 128^3, 79 against 74 at 192^3,
+// 565 against 563 at 512 x 512 x 256.  The last row of an odd count goes alone.
 constexpr bool pair_rows_fwd(int nx) { return nx % 3 == 0 || nx <= 128; }
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict__ in, double *__restrict__ out,
@@ -2607,13 +2613,12 @@ hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out,
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                       \
     const int rpb = s.lines; const size_t lds = s.lds;                                      \
     const dim3 bl(rpb * T);                                                                 \
-    if (nf > 1) { /* whole pairs of fields */                                               \
+    if (nf > 1) { /* pairs of fields, the last of an odd count alone */                     \
       GHX_LAUNCH_CHECK((k_xinv2<n_>), s, kRowBound, T, false);                              \
-      hipLaunchKernelGGL((k_xinv2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, in, rs, nf & ~1, g, nxp, c.tw_x, kxlim); \
-    }                                                                                       \
-    if (nf & 1) { /* the last field's rows in pairs */                                      \
+      hipLaunchKernelGGL((k_xinv2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, in, rs, nf, g, nxp, c.tw_x, kxlim); \
+    } else { /* a lone field's rows in pairs */                                             \
       GHX_LAUNCH_CHECK((k_xinv_rows<n_>), s, kRowBound, T, false);                          \
-      hipLaunchKernelGGL((k_xinv_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, in.p[nf - 1], rs.p[nf - 1], nrows, nxp, c.tw_x, kxlim); \
+      hipLaunchKernelGGL((k_xinv_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, in.p[0], rs.p[0], nrows, nxp, c.tw_x, kxlim); \
     }                                                                                       \
     return hipGetLastError();                                                               \
   }
@@ -2718,14 +2723,14 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                       \
     const int rpb = s.lines; const size_t lds = s.lds;                                      \
     const dim3 bl(rpb * T);                                                                 \
-    constexpr bool paired = pair_rows_fwd(n_);                                              \
-    if (nf > 1 || !paired) {                                                                \
-      GHX_LAUNCH_CHECK((k_xfwd2<n_>), s, kRowBound, T, false);                              \
-      hipLaunchKernelGGL((k_xfwd2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, rs, out, paired ? nf & ~1 : nf, g, nxp, c.tw_x); \
-    }                                                                                       \
-    if constexpr (paired) if (nf & 1) {                                                     \
+    bool paired = false;                                                                    \
+    if constexpr (pair_rows_fwd(n_)) paired = nf == 1;                                      \
+    if (paired) {                                                                           \
       GHX_LAUNCH_CHECK((k_xfwd_rows<n_>), s, kRowBound, T, false);                          \
-      hipLaunchKernelGGL((k_xfwd_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, rs.p[nf - 1], out.p[nf - 1], nrows, nxp, c.tw_x); \
+      hipLaunchKernelGGL((k_xfwd_rows<n_>), dim3((unsigned)((nrows + 2 * rpb - 1) / (2 * rpb))), bl, lds, c.stream, rs.p[0], out.p[0], nrows, nxp, c.tw_x); \
+    } else {                                                                                \
+      GHX_LAUNCH_CHECK((k_xfwd2<n_>), s, kRowBound, T, false);                              \
+      hipLaunchKernelGGL((k_xfwd2<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), bl, lds, c.stream, rs, out, nf, g, nxp, c.tw_x); \
     }                                                                                       \
     return hipGetLastError();                                                               \
   }
