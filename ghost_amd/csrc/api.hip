@@ -2596,7 +2596,7 @@ struct EnsGroup {
   ghx_grid *g = nullptr;
   std::vector<int> members;
   cplx *mem = nullptr;    // v [member][3][nc], v1 [member][3][nc], scratch [member][12][slot]
-  double *nu = nullptr;   // per-member viscosity (device)
+  double *nu = nullptr;   // per-member viscosity (device), then a word for the check of the states
   size_t nc = 0, slot = 0;
   int tz = 0, ty = 0;     // tile widths of the z and y passes (0: built-in)
   int sched = 0;          // radix schedules of the z and y passes (FFTCtx::sched)
@@ -2679,7 +2679,7 @@ extern "C" int ghx_ensemble_create(ghx_ensemble **out, int nmembers, const int *
     G.slot = ghx::slot_points(G.g->gk);
     (void)prune_shares(G.g);
     he = hipMalloc(&G.mem, (cnt * 6 * G.nc + cnt * 12 * G.slot) * sizeof(cplx));
-    if (he == hipSuccess) he = hipMalloc(&G.nu, cnt * sizeof(double));
+    if (he == hipSuccess) he = hipMalloc(&G.nu, (cnt + 1) * sizeof(double));
     std::vector<double> h(cnt);
     for (size_t b = 0; b < cnt; ++b) h[b] = nu[G.members[b]];
     if (he == hipSuccess) he = hipMemcpy(G.nu, h.data(), cnt * sizeof(double), hipMemcpyHostToDevice);
@@ -2821,16 +2821,33 @@ static int ens_capture(ghx_ensemble *e) {
 }
 
 // The members' states are dealiased once checked; every step keeps them so.
-static int ens_check_clean(ghx_ensemble *e, EnsGroup &G) {
-  bool clean = true;
-  for (size_t b = 0; b < G.members.size() && clean; ++b) {
-    const cplx *v = G.v() + b * 3 * G.nc;
-    double n = 0;
-    int rc = count_unkept(G.g, v, v + G.nc, v + 2 * G.nc, &n);
-    if (rc) return rc;
-    clean = (n == 0.0);
+// Groups whose fields were handed out since are checked together, with one wait
+// (each member by itself waits for the GPU members times); only if one of them
+// holds something outside the kept modes are they told apart.
+static int ens_check_clean(ghx_ensemble *e) {
+  bool asked = false;
+  for (EnsGroup &G : e->groups) asked = asked || !G.clean;
+  if (!asked) return GHX_OK;
+  EnsGroup &G0 = e->groups[0];
+  unsigned *word = reinterpret_cast<unsigned *>(G0.nu + G0.members.size()), any = 1;
+  HIPCHK(ghx::op_clear_word(e->stream, word));
+  for (EnsGroup &G : e->groups)
+    if (!G.clean)
+      HIPCHK(ghx::op_unkept_run(G.g->gk, e->stream, G.v(), G.nc, 3 * (int)G.members.size(), word));
+  HIPCHK(hipMemcpyAsync(&any, word, sizeof(any), hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
+  for (EnsGroup &G : e->groups) {
+    if (G.clean) continue;
+    bool clean = true;
+    for (size_t b = 0; any && b < G.members.size() && clean; ++b) {
+      const cplx *v = G.v() + b * 3 * G.nc;
+      double n = 0;
+      int rc = count_unkept(G.g, v, v + G.nc, v + 2 * G.nc, &n);
+      if (rc) return rc;
+      clean = (n == 0.0);
+    }
+    G.clean = clean;
   }
-  G.clean = clean;
   return GHX_OK;
 }
 
@@ -2838,27 +2855,24 @@ extern "C" int ghx_ensemble_step(ghx_ensemble *e, int nsteps) {
   ARGCHK(e && nsteps >= 0, "bad ensemble_step arguments");
   const bool allow_prune = !getenv("GHX_NO_PRUNE");
   for (int s = 0; s < nsteps; ++s) {
+    // the captured step holds buffers and schedules, not values: it outlives
+    // writes to the states, and a state that is not clean takes the eager step
+    int rc = ens_check_clean(e);
+    if (rc) return rc;
     bool all_clean = true;
-    for (EnsGroup &G : e->groups) {
-      if (!G.clean) {
-        ens_drop_graph(e);
-        int rc = ens_check_clean(e, G);
-        if (rc) return rc;
-      }
-      all_clean = all_clean && G.clean;
-    }
+    for (EnsGroup &G : e->groups) all_clean = all_clean && G.clean;
     if (e->use_graph && all_clean && allow_prune) {
       if (!e->exec) {
         const bool prof_was = g_prof.on;
         g_prof.on = false;  // no profiler events inside the graph
-        const int rc = ens_capture(e);
+        rc = ens_capture(e);
         g_prof.on = prof_was;
         if (rc) return rc;
       }
       HIPCHK(hipGraphLaunch(e->exec, e->stream));
     } else {
       for (EnsGroup &G : e->groups) {
-        int rc = ens_step_group(e, G, G.clean && allow_prune ? 1 : 0);
+        rc = ens_step_group(e, G, G.clean && allow_prune ? 1 : 0);
         if (rc) return rc;
       }
     }
@@ -2893,7 +2907,7 @@ extern "C" int ghx_ensemble_autotune(ghx_ensemble *e, int steps, int *tz_out, in
   int rc = GHX_OK;
   for (size_t gi = 0; gi < e->groups.size() && !rc; ++gi) {
     EnsGroup &G = e->groups[gi];
-    if (!G.clean && (rc = ens_check_clean(e, G))) break;
+    if (!G.clean && (rc = ens_check_clean(e))) break;
     const size_t bytes = G.members.size() * 3 * G.nc * sizeof(cplx);
     cplx *save = nullptr;
     hipError_t he = hipMalloc(&save, bytes);

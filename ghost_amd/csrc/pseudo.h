@@ -60,6 +60,9 @@ hipError_t op_reduce(const GridK &g, hipStream_t st, int kind, const cplx *a, co
 // tiny <= kn2 <= kmax, else non-zero; fields from `mean` on may be non-zero
 // below tiny.
 hipError_t op_unkept(const GridK &g, hipStream_t st, const cplx *const *v, int nf, int mean, unsigned *flag);
+// the same for nf fields `stride` points apart, into a flag that op_clear_word has cleared
+hipError_t op_unkept_run(const GridK &g, hipStream_t st, const cplx *v, size_t stride, int nf, unsigned *flag);
+hipError_t op_clear_word(hipStream_t st, unsigned *word);
 // hdcheck's sums of v and the force f: out[5] host = <v^2>, <omega^2>, <v.f>,
 // helicity, <(div v)^2>; work as for op_reduce.
 hipError_t op_hdcheck(const GridK &g, hipStream_t st, const cplx *const *v, const cplx *const *f, double *work,

@@ -501,6 +501,20 @@ __global__ __launch_bounds__(kBlock) void k_unkept(GridK g, V6 v, int nf, int me
   });
   if (__ballot(on) != 0 && threadIdx.x % 64 == 0) atomicOr(flag, 1u);
 }
+
+// The same for consecutive fields of one grid, one blockIdx.y each, all their
+// modes outside tiny <= kn2 <= kmax; *flag is not cleared here.
+__global__ __launch_bounds__(kBlock) void k_unkept_run(GridK g, const cplx *v, size_t stride, unsigned *flag) {
+  bool on = false;
+  const cplx *p = v + blockIdx.y * stride;
+  for_modes(g, [&](const Idx &q, size_t m) {
+    const double kn2 = kn2_of(g, q.i, q.j, q.k);
+    if (kn2 <= g.kmax && kn2 >= g.tiny) return;
+    const cplx x = p[m];
+    on = on || x.x != 0.0 || x.y != 0.0;
+  });
+  if (__ballot(on) != 0 && threadIdx.x % 64 == 0) atomicOr(flag, 1u);
+}
 __global__ void k_clear_word(unsigned *p) { *p = 0u; }
 
 // hdcheck's five sums (pseudospec3D_hd.f90:984-1105) in one pass over v =
@@ -962,6 +976,14 @@ hipError_t op_unkept(const GridK &g, hipStream_t st, const cplx *const *v, int n
   for (int f = 0; f < 6; ++f) p.p[f] = f < nf ? v[f] : nullptr;
   hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, st, flag);
   hipLaunchKernelGGL(k_unkept, dim3(walk_blocks(g, kRedBlocks)), dim3(kBlock), 0, st, g, p, nf, mean, flag);
+  return hipGetLastError();
+}
+hipError_t op_clear_word(hipStream_t st, unsigned *word) {
+  hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, st, word);
+  return hipGetLastError();
+}
+hipError_t op_unkept_run(const GridK &g, hipStream_t st, const cplx *v, size_t stride, int nf, unsigned *flag) {
+  hipLaunchKernelGGL(k_unkept_run, dim3(walk_blocks(g, 256), nf), dim3(kBlock), 0, st, g, v, stride, flag);
   return hipGetLastError();
 }
 
