@@ -10,6 +10,7 @@
 // Transform convention (FFTW's, which GHOST uses): DIR = -1 forward,
 // DIR = +1 inverse, both unnormalised.
 #pragma once
+#include <type_traits>
 #include "ghx_common.h"
 
 // LDS padding: one spare slot every 8 complex points keeps the stride-R
@@ -472,12 +473,13 @@ template <int N, int DIR> struct MixFFT {
 // One lane's part of a line's transforms in either direction, with KE points
 // on the wavenumber side (k = t + T m, every lane) and SE on the sample side
 // (n = t + A m, in the lanes with live(t)): LineFFT of a schedule Cfg, one
-// layout on both sides, or MixFFT for FFTCfgMix.
+// layout on both sides, or MixFFT for FFTCfgMixed.
 constexpr bool mix_length(int n) { return n == 24 || n == 48 || n == 96 || n == 192 || n == 384; }
-template <int N, bool = mix_length(N)> struct FFTCfgMix : FFTCfg<N> {};
-template <int N> struct FFTCfgMix<N, true> {
+template <int N> struct FFTCfgMixed {
   static constexpr int E = 6, T = N / 6;
 };
+template <int N>
+using FFTCfgMix = typename std::conditional<mix_length(N), FFTCfgMixed<N>, FFTCfg<N>>::type;
 
 template <int N, typename Cfg = FFTCfg<N>> struct Line {
   static constexpr int T = Cfg::T, A = T, KE = Cfg::E, SE = Cfg::E;
@@ -506,7 +508,7 @@ template <int N, typename Cfg = FFTCfg<N>> struct Line {
     for (int m = 0; m < SE; ++m) x[m] = row[lds_pad(t + T * m)];
   }
 };
-template <int N> struct Line<N, FFTCfgMix<N, true>> {
+template <int N> struct Line<N, FFTCfgMixed<N>> {
   using I = MixFFT<N, +1>;
   using F = MixFFT<N, -1>;
   static constexpr int T = I::T, A = I::A, KE = 6, SE = 8;
