@@ -90,8 +90,15 @@ static PassShape wide_shape(int TW, int rowslots, int nlines) {
 }
 // Rows per block of an x pass: kRowBound lanes, fewer rows when their LDS
 // lines would not fit (the kernels read the row count from blockDim.x / T).
-static PassShape row_shape(int T, int rowslots, size_t ldsmax) {
-  int r = (int)kRowBound / T;
+// Rows synchronise by wavefront, so launches of up to 9 wavefronts per CU go
+// out one wavefront per block, which spreads them over all CUs (16 rows of 64
+// points per wavefront otherwise leave half of them idle at 64^3).  Measured,
+// blocks of 256 -> 64 lanes, us: X cross 11.2 -> 8.4 at 32^3, 11.4 -> 10.6 at
+// 64^3, 12.6 -> 11.8 at 128 x 64 x 32, 23.1 -> 22.1 at 384 x 48 x 48, tracers'
+// inverse 14.2 -> 12.0 at 96^3 (2304 wavefronts); the same at 128^3 (4096).
+static PassShape row_shape(int T, int rowslots, size_t ldsmax, long rows = 1L << 30) {
+  const int lanes = rows * T <= 64 * 2304L ? 64 : (int)kRowBound;
+  int r = lanes / T;
   if (r < 1) r = 1;
   while (r > 1 && (size_t)r * rowslots * sizeof(cplx) > ldsmax) r >>= 1;
   return PassShape{r, (unsigned)(r * T), (size_t)r * rowslots * sizeof(cplx)};
@@ -2612,7 +2619,7 @@ hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out,
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                                      \
     const dim3 bl(rpb * T);                                                                 \
     if (nf > 1) { /* pairs of fields, the last of an odd count alone */                     \
@@ -2634,7 +2641,7 @@ hipError_t xinv(const FFTCtx &c, int nf, const FieldSet &in, double *const *out,
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     GHX_LAUNCH_CHECK((k_xinv<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xinv<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, rs, nf, g, nxp, c.tw_xh, c.tw_x, kxlim); \
     break;                                                                                  \
@@ -2658,7 +2665,7 @@ hipError_t xinv3i(const FFTCtx &c, const FieldSet &in, double *out, int prune) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
     GHX_LAUNCH_CHECK((k_xinv3i2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xinv3i2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, kxlim);                                                                 \
@@ -2674,7 +2681,7 @@ hipError_t xinv3i(const FFTCtx &c, const FieldSet &in, double *out, int prune) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     GHX_LAUNCH_CHECK((k_xinv3i<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xinv3i<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kxlim); \
     break;                                                                                  \
@@ -2722,7 +2729,7 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                                      \
     const dim3 bl(rpb * T);                                                                 \
     bool paired = false;                                                                    \
@@ -2746,7 +2753,7 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     GHX_LAUNCH_CHECK((k_xfwd<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xfwd<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, rs, out, nf, g, nxp, c.tw_xh, c.tw_x); \
     break;                                                                                  \
@@ -2772,7 +2779,7 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                              \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows * c.batch);                              \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);                      \
     GHX_LAUNCH_CHECK((k_xcross2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
@@ -2788,7 +2795,7 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                              \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows * c.batch);                              \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);               \
     switch (tile_want("GHX_XV", 1)) {                                                       \
@@ -2827,7 +2834,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfg<n_>::T;                                                        \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
     GHX_LAUNCH_CHECK((k_xdot2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
@@ -2843,7 +2850,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
-    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds());                                        \
+    const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     GHX_LAUNCH_CHECK((k_xdot<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); \
     break;                                                                                  \
