@@ -340,8 +340,12 @@ static int do_r2c(ghx_plan *p, int nf, const double *const *in, void *const *out
   }
   const double sc = (double)nc * sizeof(cplx), sr = (double)p->nx * p->ny * p->nz * sizeof(double);
   timer_begin(p);
-  PROF(P_XFWD, nf * (sr + sc), p->ctx.stream, ghx::xfwd(p->ctx, nf, in, pp));
-  PROF(P_YFWD, nf * 2 * sc, p->ctx.stream, ghx::yfwd(p->ctx, nf, pp, q, prune));
+  if (ghx::xyplane(p->ctx)) {
+    PROF(P_XFWD, nf * (sr + sc), p->ctx.stream, ghx::xyplane_fwd(p->ctx, nf, in, q));
+  } else {
+    PROF(P_XFWD, nf * (sr + sc), p->ctx.stream, ghx::xfwd(p->ctx, nf, in, pp));
+    PROF(P_YFWD, nf * 2 * sc, p->ctx.stream, ghx::yfwd(p->ctx, nf, pp, q, prune));
+  }
   PROF(P_ZFWD, nf * 2 * sc, p->ctx.stream, ghx::zfwd(p->ctx, nf, q, o, prune));
   timer_end(p);
   return GHX_OK;
@@ -362,8 +366,12 @@ static int do_c2r(ghx_plan *p, int nf, const void *const *in, double *const *out
   const double sc = (double)nc * sizeof(cplx), sr = (double)p->nx * p->ny * p->nz * sizeof(double);
   timer_begin(p);
   PROF(P_ZINV, nf * 2 * sc, p->ctx.stream, ghx::zinv(p->ctx, 0, nf, i, q));
-  PROF(P_YINV, nf * 2 * sc, p->ctx.stream, ghx::yinv(p->ctx, nf, q, pp));
-  PROF(P_XINV, nf * (sr + sc), p->ctx.stream, ghx::xinv(p->ctx, nf, pp, out));
+  if (ghx::xyplane(p->ctx)) {
+    PROF(P_XINV, nf * (sr + sc), p->ctx.stream, ghx::xyplane_inv(p->ctx, nf, q, out));
+  } else {
+    PROF(P_YINV, nf * 2 * sc, p->ctx.stream, ghx::yinv(p->ctx, nf, q, pp));
+    PROF(P_XINV, nf * (sr + sc), p->ctx.stream, ghx::xinv(p->ctx, nf, pp, out));
+  }
   timer_end(p);
   return GHX_OK;
 }
@@ -1736,8 +1744,12 @@ static int velocity_gradients(ghx_grid *g, const void *const *v, double *const *
     pp.p[f] = p->q + (9 + f) * slot;
   }
   HIPCHK(ghx::zinv(p->ctx, 6, 9, in, q, prune, nullptr));
-  HIPCHK(ghx::yinv(p->ctx, 9, q, pp, prune));
-  HIPCHK(ghx::xinv(p->ctx, 9, pp, grad9, prune));
+  if (ghx::xyplane(p->ctx)) {
+    HIPCHK(ghx::xyplane_inv(p->ctx, 9, q, grad9, prune));
+  } else {
+    HIPCHK(ghx::yinv(p->ctx, 9, q, pp, prune));
+    HIPCHK(ghx::xinv(p->ctx, 9, pp, grad9, prune));
+  }
   return GHX_OK;
 }
 

@@ -105,6 +105,11 @@ constexpr int kNormBlocks = 4096;
 hipError_t xnormmax(const FFTCtx &c, const FieldSet &in, double *part, int *nblk);
 // X forward: real rows -> P.
 hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &out);
+// X and Y of small planes in one launch, R <-> Q (k_xyplane): whether the grid's
+// sizes take it, and the two directions (prune as in yinv, 0 or 1).
+bool xyplane(const FFTCtx &c);
+hipError_t xyplane_fwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &q);
+hipError_t xyplane_inv(const FFTCtx &c, int nf, const FieldSet &q, double *const *out, int prune = 0);
 // Fused X^-1 . cross product . X on P rows: in.p[0..2] = A, in.p[3..5] = B
 // -> out.p[0..2] = FFT[(A x B)/N^6] in GHOST's operand order.
 hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet &out, int prune = 0);

@@ -2767,6 +2767,162 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
 }
 #endif
 
+#if GHX_PART == 9
+// ---------------------------------------------------------------------------
+// Small planes: X and Y of one field's (x, y) plane in one block, the plane held
+// in LDS between them (one line of y per kx), so the P array is neither written
+// nor read and a launch of three goes.  Rows go in pairs of the field's own (NY
+// is even).  Sides of 24 to 64 points: at most 76 KB of LDS, two blocks per CU;
+// 96 x 96 points would leave one.  Whole transforms, separate passes -> planes,
+// r2c and c2r, us: 13.2 -> 9.1 and 9.9 -> 9.2 at 32^3, 13.0 -> 10.8 and 11.9 ->
+// 10.5 at 64^3, 23.2 -> 16.0 and 21.7 -> 14.9 at 64 x 64 x 256; of several
+// fields 22.5 -> 14.7 and 15.7 -> 9.5 (6 of 32^3), 72.9 -> 52.2 and 63.7 -> 42.9
+// (3 of 64 x 64 x 512).  prune (inverse): as in k_yinv, q holds data on the
+// dealias set's lines only; the forward writes every line.
+// ---------------------------------------------------------------------------
+template <int NX, int NY, bool FWD>
+__global__ __launch_bounds__(kRowBound) void k_xyplane(RealSet re, FieldSet q, GridK g, const cplx *__restrict__ twx,
+                                                       const cplx *__restrict__ twy, int prune) {
+  using X = Line<NX, FFTCfgMix<NX>>;
+  using Y = Line<NY, FFTCfgMix<NY>>;
+  static_assert(X::T <= 64 && Y::T <= 64 && NY % 2 == 0, "lines within a wavefront, rows in pairs");
+  constexpr int H = NX / 2 + 1, SX = lds_line_stride(NX), SY = lds_line_stride(NY);
+  constexpr int LX = (int)kRowBound / X::T, LY = (int)kRowBound / Y::T;
+  extern __shared__ cplx lds[];
+  cplx *plane = lds + LX * SX;  // H lines of SY points
+  const int z = blockIdx.x;
+  double *real = re.p[blockIdx.y] + (size_t)z * NY * NX;
+  cplx *spec = q.p[blockIdx.y] + (size_t)z * H * NY;
+  auto rows = [&]() {
+    const int t = threadIdx.x % X::T;
+    cplx *buf = lds + (threadIdx.x / X::T) * SX;
+    X fft;
+    if constexpr (FWD) fft.load_fwd(twx, t);
+    else fft.load_inv(twx, t);
+    for (int p = threadIdx.x / X::T; p < NY / 2; p += LX) {
+      double *r0 = real + (size_t)(2 * p) * NX, *r1 = r0 + NX;
+      cplx x[X::SE], k[X::KE];
+      if constexpr (FWD) {
+        if (X::live(t)) xpair_real<X::SE>(x, r0, r1, t, X::A);
+        fft.fwd(x, k, buf, t);
+#pragma unroll
+        for (int m = 0; m < X::KE; ++m) buf[lds_pad(t + X::T * m)] = k[m];
+        line_sync<X::T>();
+#pragma unroll
+        for (int m = 0; m <= X::KE / 2; ++m) {
+          const int i = t + X::T * m;
+          if (i < H) {
+            const cplx c = c_conj(buf[lds_pad((NX - i) % NX)]);
+            const cplx d = c_sub(k[m], c);
+            plane[i * SY + lds_pad(2 * p)] = c_scale(c_add(k[m], c), 0.5);
+            plane[i * SY + lds_pad(2 * p + 1)] = c_make(0.5 * d.y, -0.5 * d.x);
+          }
+        }
+        line_sync<X::T>();
+      } else {
+        cplx a[X::KE], b[X::KE];
+#pragma unroll
+        for (int m = 0; m < X::KE; ++m) {
+          const int i = t + X::T * m, c = i < H ? i : NX - i;
+          a[m] = plane[c * SY + lds_pad(2 * p)];
+          b[m] = plane[c * SY + lds_pad(2 * p + 1)];
+        }
+        xpair_make<NX, X::KE, X::T>(k, a, b, t, H);
+        fft.inv(k, x, buf, t);
+        if (X::live(t)) {
+#pragma unroll
+          for (int m = 0; m < X::SE; ++m) {
+            r0[t + X::A * m] = x[m].x;
+            r1[t + X::A * m] = x[m].y;
+          }
+        }
+      }
+    }
+  };
+  auto lines = [&]() {
+    const int t = threadIdx.x % Y::T;
+    Y fft;
+    if constexpr (FWD) fft.load_fwd(twy, t);
+    else fft.load_inv(twy, t);
+    for (int i = threadIdx.x / Y::T; i < H; i += LY) {
+      cplx *row = plane + i * SY, *s = spec + (size_t)i * NY;
+      cplx x[Y::SE], k[Y::KE];
+      if constexpr (FWD) {
+        Y::get(x, row, t);
+        line_sync<Y::T>();
+        fft.fwd(x, k, row, t);
+#pragma unroll
+        for (int m = 0; m < Y::KE; ++m) s[t + Y::T * m] = k[m];
+      } else {
+#pragma unroll
+        for (int m = 0; m < Y::KE; ++m) {
+          const int j = t + Y::T * m;
+          const bool need = !prune || kn2_of(g, i, j, 0) <= g.kmax;
+          const cplx v = s[need ? j : 0];
+          k[m] = need ? v : c_make(0.0, 0.0);
+        }
+        fft.inv(k, x, row, t);
+        Y::put(x, row, t);
+      }
+    }
+  };
+  if constexpr (FWD) rows();
+  else lines();
+  __syncthreads();
+  if constexpr (FWD) lines();
+  else rows();
+}
+
+#define GHX_PLANE_SIZES(X) X(24) X(32) X(48) X(64)
+template <int NX, int NY, bool FWD>
+static hipError_t launch_xyplane(const FFTCtx &c, int nf, const RealSet &re, const FieldSet &q, int prune) {
+  constexpr int LX = (int)kRowBound / Line<NX, FFTCfgMix<NX>>::T;
+  const PassShape s{LX, kRowBound, ((size_t)LX * lds_line_stride(NX) + (size_t)(NX / 2 + 1) * lds_line_stride(NY)) * sizeof(cplx)};
+  allow_lds(k_xyplane<NX, NY, FWD>, s.lds);
+  GHX_LAUNCH_CHECK((k_xyplane<NX, NY, FWD>), s, kRowBound, 1, false);
+  hipLaunchKernelGGL((k_xyplane<NX, NY, FWD>), dim3(c.gk.nz, nf), dim3(s.block), s.lds, c.stream, re, q, c.gk, c.tw_x, c.tw_y, prune);
+  return hipGetLastError();
+}
+template <int NX, bool FWD>
+static hipError_t plane_y(const FFTCtx &c, int nf, const RealSet &re, const FieldSet &q, int prune) {
+  switch (c.gk.ny) {
+#define GHX_CASE(n_) case n_: return launch_xyplane<NX, n_, FWD>(c, nf, re, q, prune);
+    GHX_PLANE_SIZES(GHX_CASE)
+#undef GHX_CASE
+  default: return hipErrorInvalidValue;
+  }
+}
+template <bool FWD>
+static hipError_t plane_x(const FFTCtx &c, int nf, const RealSet &re, const FieldSet &q, int prune) {
+  switch (c.gk.nx) {
+#define GHX_CASE(n_) case n_: return plane_y<n_, FWD>(c, nf, re, q, prune);
+    GHX_PLANE_SIZES(GHX_CASE)
+#undef GHX_CASE
+  default: return hipErrorInvalidValue;
+  }
+}
+static bool plane_size(int n) {
+  switch (n) {
+#define GHX_CASE(n_) case n_:
+    GHX_PLANE_SIZES(GHX_CASE)
+#undef GHX_CASE
+    return true;
+  default: return false;
+  }
+}
+bool xyplane(const FFTCtx &c) { return plane_size(c.gk.nx) && plane_size(c.gk.ny) && use_x2(c.gk.nx); }
+hipError_t xyplane_fwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &q) {
+  RealSet rs;
+  for (int f = 0; f < nf; ++f) rs.p[f] = const_cast<double *>(in[f]);
+  return plane_x<true>(c, nf, rs, q, 0);
+}
+hipError_t xyplane_inv(const FFTCtx &c, int nf, const FieldSet &q, double *const *out, int prune) {
+  RealSet rs;
+  for (int f = 0; f < nf; ++f) rs.p[f] = out[f];
+  return plane_x<false>(c, nf, rs, q, prune);
+}
+#endif
+
 #if GHX_PART == 7
 hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet &out, int prune) {
   (void)mode;
