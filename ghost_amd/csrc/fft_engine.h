@@ -228,6 +228,34 @@ template <int R> GHX_DEV void tw_powers(cplx w1, cplx *w) {
   if constexpr (R > 7) w[7] = c_mul(w[4], w[3]);
 }
 
+// The same with more of the powers read, for the lines of 3 * 2^k points: w1 and
+// w3 for radix 8, w1 and w2 for radix 4, w1 to w3 for radix 6, so that no power
+// is further than two products from correctly rounded roots.  RMS relative error
+// of one line of random points in units of 1e-16, radix-3 and radix-2 stages
+// with every twiddle from the table | one root and the tree above | these: the
+// mixed stages' inverse 1.55 | 1.80 | 1.50 (24 points), 1.70 | 2.40 | 1.63 (48),
+// 1.86 | 2.17 | 1.84 (96), 2.01 | 2.73 | 1.90 (192), 2.13 | 3.22 | 2.12 (384);
+// their forward 1.55 | 2.31 | 1.41, 1.70 | 2.11 | 1.60, 1.86 | 2.29 | 1.69, 2.01
+// | 2.77 | 1.92, 2.13 | 3.09 | 2.09; 12 points per lane 1.86 | 1.87 | 1.69 (96),
+// 2.01 | 2.13 | 1.84 (192), 2.13 | 2.26 | 1.99 (384).  (w3 of radix 4 read as
+// well costs a wave per SIMD: MHD z inverse 23.7 -> 26.5 us at 96^3.)
+template <int R> constexpr int tw_nroots() { return R == 6 ? 3 : R == 4 || R == 8 ? 2 : 1; }
+template <int R> constexpr int tw_power(int r) { return R == 8 && r == 1 ? 3 : r + 1; }  // of the r-th root read
+template <int R> GHX_DEV void tw_powers(const cplx (&p)[tw_nroots<R>()], cplx *w) {
+  static_assert(R == 2 || R == 4 || R == 6 || R == 8, "the radices of the 3 * 2^k lines");
+  w[1] = p[0];
+  if constexpr (R == 4) w[2] = p[1], w[3] = c_mul(p[0], p[1]);
+  if constexpr (R == 6) w[2] = p[1], w[3] = p[2], w[4] = c_mul(p[1], p[1]), w[5] = c_mul(p[1], p[2]);
+  if constexpr (R == 8) {
+    w[2] = c_mul(p[0], p[0]);
+    w[3] = p[1];
+    w[4] = c_mul(p[0], p[1]);
+    w[5] = c_mul(w[2], p[1]);
+    w[6] = c_mul(p[1], p[1]);
+    w[7] = c_mul(w[4], p[1]);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Synchronisation of one line's LDS exchange.  A line of T <= 64 lanes lives
 // inside one wavefront (T is a power of two and blocks are whole lines), so
@@ -250,9 +278,12 @@ template <int T> GHX_DEV void line_sync() {
 // lane for every stage of one schedule in registers, loaded once, for kernels
 // that run many transforms of the same length per lane.
 // ---------------------------------------------------------------------------
+// A butterfly reads one root, on the lines of 3 * 2^k points tw_nroots of them.
+template <int N, int R> constexpr int line_nroots() { return N % 3 == 0 && N >= 24 ? tw_nroots<R>() : 1; }
+template <int N, int R> constexpr int line_power(int r) { return line_nroots<N, R>() > 1 ? tw_power<R>(r) : 1; }
 struct TwTable {
   const cplx *p;
-  template <int S> GHX_DEV cplx root(int, int idx) const { return p[idx]; }
+  template <int S> GHX_DEV cplx root(int, int r, int idx) const { (void)r; return p[idx]; }
 };
 
 template <int N, typename Cfg = FFTCfg<N>> struct TwCache {
@@ -260,17 +291,21 @@ template <int N, typename Cfg = FFTCfg<N>> struct TwCache {
   cplx w[NS > 0 ? NS : 1][E];
   template <int S, int Ns> GHX_DEV void fill(const cplx *tw, int t) {
     if constexpr (S < NS) {
-      constexpr int R = Cfg::radix(S), Q = E / R;
+      constexpr int R = Cfg::radix(S), Q = E / R, M = line_nroots<N, R>();
       if constexpr (Ns > 1) {
         constexpr int tws = N / (Ns * R);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) w[S][q] = tw[((t + q * T) % Ns) * tws];
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int r = 0; r < M; ++r) w[S][q * M + r] = tw[((t + q * T) % Ns) * line_power<N, R>(r) * tws];
       }
       fill<S + 1, Ns * R>(tw, t);
     }
   }
   GHX_DEV void load(const cplx *tw, int t) { fill<0, 1>(tw, t); }
-  template <int S> GHX_DEV cplx root(int q, int) const { return w[S][q]; }
+  template <int S> GHX_DEV cplx root(int q, int r, int) const {
+    return w[S][q * line_nroots<N, Cfg::radix(S)>() + r];
+  }
 };
 
 // ---------------------------------------------------------------------------
@@ -302,8 +337,15 @@ template <int N, int DIR, typename Cfg = FFTCfg<N>> struct LineFFT {
           const int k = j % Ns;
           constexpr int tws = N / (Ns * R);
           cplx w[R];
-          const cplx w1 = tw.template root<S>(q, k * tws);
-          tw_powers<R>(DIR < 0 ? w1 : c_conj(w1), w);
+          constexpr int M = line_nroots<N, R>();
+          cplx p[M];
+#pragma unroll
+          for (int r = 0; r < M; ++r) {
+            const cplx x = tw.template root<S>(q, r, k * line_power<N, R>(r) * tws);
+            p[r] = DIR < 0 ? x : c_conj(x);
+          }
+          if constexpr (M > 1) tw_powers<R>(p, w);
+          else tw_powers<R>(p[0], w);
 #pragma unroll
           for (int r = 1; r < R; ++r) u[r] = c_mul(u[r], w[r]);
         }
@@ -351,9 +393,9 @@ template <int N, int DIR, typename Cfg = FFTCfg<N>> struct LineFFT {
 // is held as x[t + T m] (m < 6) by every lane, the other side as x[t + A m]
 // (m < 8) by the lanes t < A, and a pass that does both needs no exchange to
 // get from one to the other.  Measured, 6-point schedule -> mixed stages, us: X
-// cross 1084 -> 743 at 384^3, 125 -> 98 at 192^3, 24.7 -> 21.6 at 96^3, 11.6 ->
-// 9.8 at 48^3, 10.5 -> 9.6 at 24^3; X dot 116 -> 81 at 384 x 192 x 96; three
-// interleaved x inverses 606 -> 446 at 384^3; one field's x inverse 200 -> 162,
+// cross 1084 -> 729 at 384^3, 125 -> 100 at 192^3, 24.7 -> 21.6 at 96^3, 11.6 ->
+// 9.0 at 48^3, 10.5 -> 8.2 at 24^3; X dot 116 -> 88 at 384 x 192 x 96; three
+// interleaved x inverses 606 -> 440 at 384^3; one field's x inverse 200 -> 163,
 // x forward 196 -> 170 and z forward 266 -> 238 at 384^3; curl z inverse 391 ->
 // 325 at 384^3, 54 -> 46 at 192^3; MHD z inverse 97 -> 83, HD update 52 -> 47 at
 // 192^3, 57 -> 32 at 96 x 96 x 384.
@@ -370,12 +412,17 @@ template <int N, int DIR> struct MixFFT {
   static constexpr int T = N / 6, A = N / 8;
   static_assert(6 * C::R1 * C::R2 == N && T <= 64, "a line lives in one wavefront");
 
-  // the stage's roots of this lane, one per butterfly
-  template <int R, int Ns, int L, int E> GHX_DEV static void roots(cplx (&w)[E / R], const cplx *tw, int t) {
+  // the stage's roots of this lane, tw_nroots of each butterfly
+  template <int R, int E> struct Stage {
+    cplx w[E / R][tw_nroots<R>()];
+    template <int Ns, int L> GHX_DEV void load(const cplx *tw, int t) {
 #pragma unroll
-    for (int q = 0; q < E / R; ++q) w[q] = tw[((t + q * L) % Ns) * (N / (Ns * R))];
-  }
-  template <int R, bool TWIDDLE, int E> GHX_DEV static void butterflies(cplx (&v)[E], const cplx *w1) {
+      for (int q = 0; q < E / R; ++q)
+#pragma unroll
+        for (int r = 0; r < tw_nroots<R>(); ++r) w[q][r] = tw[((t + q * L) % Ns) * tw_power<R>(r) * (N / (Ns * R))];
+    }
+  };
+  template <int R, bool TWIDDLE, int E> GHX_DEV static void butterflies(cplx (&v)[E], const Stage<R, E> *st) {
     constexpr int Q = E / R;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -383,8 +430,10 @@ template <int N, int DIR> struct MixFFT {
 #pragma unroll
       for (int r = 0; r < R; ++r) u[r] = v[q + r * Q];
       if constexpr (TWIDDLE) {
-        cplx w[R];
-        tw_powers<R>(DIR < 0 ? w1[q] : c_conj(w1[q]), w);
+        cplx w[R], p[tw_nroots<R>()];
+#pragma unroll
+        for (int r = 0; r < tw_nroots<R>(); ++r) p[r] = DIR < 0 ? st->w[q][r] : c_conj(st->w[q][r]);
+        tw_powers<R>(p, w);
 #pragma unroll
         for (int r = 1; r < R; ++r) u[r] = c_mul(u[r], w[r]);
       }
@@ -407,16 +456,14 @@ template <int N, int DIR> struct MixFFT {
     for (int m = 0; m < E; ++m) v[m] = buf[lds_pad(t + L * m)];
   }
 
-  static constexpr int Q1 = 8 / C::R1, Q2 = 8 / C::R2;
-  struct Roots {
-    cplx a[Q1], b[C::R2 > 1 ? Q2 : 1];
-  };
+  struct None {};
   // wavenumbers in (t + T m) -> samples out (t + A m, lanes t < A)
   struct Inv {
-    Roots w;
+    Stage<C::R1, 8> a;
+    typename std::conditional<(C::R2 > 1), Stage<C::R2, 8>, None>::type b;
     GHX_DEV void load(const cplx *tw, int t) {
-      roots<C::R1, 6, A, 8>(w.a, tw, t);
-      if constexpr (C::R2 > 1) roots<C::R2, 6 * C::R1, A, 8>(w.b, tw, t);
+      a.template load<6, A>(tw, t);
+      if constexpr (C::R2 > 1) b.template load<6 * C::R1, A>(tw, t);
     }
     GHX_DEV void run(cplx (&in)[6], cplx (&out)[8], cplx *buf, int t) const {
       butterflies<6, false, 6>(in, nullptr);
@@ -424,7 +471,7 @@ template <int N, int DIR> struct MixFFT {
       line_sync<T>();
       if (t < A) {
         get<A, 8>(out, buf, t);
-        butterflies<C::R1, true, 8>(out, w.a);
+        butterflies<C::R1, true, 8>(out, &a);
       }
       line_sync<T>();
       if constexpr (C::R2 > 1) {
@@ -432,7 +479,7 @@ template <int N, int DIR> struct MixFFT {
         line_sync<T>();
         if (t < A) {
           get<A, 8>(out, buf, t);
-          butterflies<C::R2, true, 8>(out, w.b);
+          butterflies<C::R2, true, 8>(out, &b);
         }
         line_sync<T>();
       }
@@ -440,10 +487,11 @@ template <int N, int DIR> struct MixFFT {
   };
   // samples in (t + A m, lanes t < A) -> wavenumbers out (t + T m)
   struct Fwd {
-    cplx b[C::R2 > 1 ? Q1 : 1], c[1];
+    typename std::conditional<(C::R2 > 1), Stage<C::R1, 8>, None>::type b;
+    Stage<6, 6> c;
     GHX_DEV void load(const cplx *tw, int t) {
-      if constexpr (C::R2 > 1) roots<C::R1, C::R2, A, 8>(b, tw, t);
-      roots<6, N / 6, T, 6>(c, tw, t);
+      if constexpr (C::R2 > 1) b.template load<C::R2, A>(tw, t);
+      c.template load<N / 6, T>(tw, t);
     }
     GHX_DEV void run(cplx (&in)[8], cplx (&out)[6], cplx *buf, int t) const {
       if constexpr (C::R2 > 1) {
@@ -454,7 +502,7 @@ template <int N, int DIR> struct MixFFT {
         line_sync<T>();
         if (t < A) {
           get<A, 8>(in, buf, t);
-          butterflies<C::R1, true, 8>(in, b);
+          butterflies<C::R1, true, 8>(in, &b);
         }
         line_sync<T>();
         if (t < A) put<C::R1, C::R2, A, 8>(in, buf, t);
@@ -465,7 +513,7 @@ template <int N, int DIR> struct MixFFT {
       line_sync<T>();
       get<T, 6>(out, buf, t);
       line_sync<T>();
-      butterflies<6, true, 6>(out, c);
+      butterflies<6, true, 6>(out, &c);
     }
   };
 };

@@ -1973,11 +1973,10 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
 // Fused X^-1 . (P x Q)/N^6 . X with two-for-one transforms: pairs (P_x, P_y),
 // (P_z, Q_x), (Q_y, Q_z) inverse, (out_x, out_y) and out_z forward.  Same
 // fields, products and operand order as k_xcross.  One row per line of
-// T <= 64 lanes.  384-point rows ask for a third wave per SIMD (168 registers,
-// 6 in scratch: 743 -> 685 us at 384^3); at 192 and 96 points that spills 15
-// and 11 and loses (98 -> 127 us at 192^3, 21.6 -> 25.9 at 96^3).
+// T <= 64 lanes.  Two waves per SIMD: a third would put registers of the 3 *
+// 2^k rows into scratch, 20 of them and 726 -> 1072 us at 384^3.
 template <int NX>
-__global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(NX == 384 ? 3 : 2))) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
+__global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
                                                 const cplx *__restrict__ twt, int prune) {
   const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
   using X = Line<NX, FFTCfgMix<NX>>;
