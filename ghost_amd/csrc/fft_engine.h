@@ -239,22 +239,37 @@ template <int R> GHX_DEV void tw_powers(cplx w1, cplx *w) {
 // | 2.77 | 1.92, 2.13 | 3.09 | 2.09; 12 points per lane 1.86 | 1.87 | 1.69 (96),
 // 2.01 | 2.13 | 1.84 (192), 2.13 | 2.26 | 1.99 (384).  (w3 of radix 4 read as
 // well costs a wave per SIMD: MHD z inverse 23.7 -> 26.5 us at 96^3.)
-template <int R> constexpr int tw_nroots() { return R == 6 ? 3 : R == 4 || R == 8 ? 2 : 1; }
-template <int R> constexpr int tw_power(int r) { return R == 8 && r == 1 ? 3 : r + 1; }  // of the r-th root read
-template <int R> GHX_DEV void tw_powers(const cplx (&p)[tw_nroots<R>()], cplx *w) {
-  static_assert(R == 2 || R == 4 || R == 6 || R == 8, "the radices of the 3 * 2^k lines");
+// FULL: every power read, for passes with registers to spare.
+template <int R, bool FULL = false> constexpr int tw_nroots() { return FULL ? R - 1 : R == 6 ? 3 : R == 4 || R == 8 ? 2 : 1; }
+// the power that the r-th root read is
+template <int R, bool FULL = false> constexpr int tw_power(int r) { return !FULL && R == 8 && r == 1 ? 3 : r + 1; }
+template <int R, int M> GHX_DEV void tw_powers(const cplx (&p)[M], cplx *w) {
   w[1] = p[0];
-  if constexpr (R == 4) w[2] = p[1], w[3] = c_mul(p[0], p[1]);
-  if constexpr (R == 6) w[2] = p[1], w[3] = p[2], w[4] = c_mul(p[1], p[1]), w[5] = c_mul(p[1], p[2]);
-  if constexpr (R == 8) {
-    w[2] = c_mul(p[0], p[0]);
-    w[3] = p[1];
-    w[4] = c_mul(p[0], p[1]);
-    w[5] = c_mul(w[2], p[1]);
-    w[6] = c_mul(p[1], p[1]);
-    w[7] = c_mul(w[4], p[1]);
+  if constexpr (M == R - 1) {
+#pragma unroll
+    for (int r = 2; r < R; ++r) w[r] = p[r - 1];
+  } else if constexpr (M == 1) {
+    tw_powers<R>(p[0], w);
+  } else {
+    static_assert(M == tw_nroots<R>(), "the roots of the 3 * 2^k lines");
+    if constexpr (R == 4) w[2] = p[1], w[3] = c_mul(p[0], p[1]);
+    if constexpr (R == 6) w[2] = p[1], w[3] = p[2], w[4] = c_mul(p[1], p[1]), w[5] = c_mul(p[1], p[2]);
+    if constexpr (R == 8) {
+      w[2] = c_mul(p[0], p[0]);
+      w[3] = p[1];
+      w[4] = c_mul(p[0], p[1]);
+      w[5] = c_mul(w[2], p[1]);
+      w[6] = c_mul(p[1], p[1]);
+      w[7] = c_mul(w[4], p[1]);
+    }
   }
 }
+
+// A schedule Cfg whose stages read more roots than its length asks for: the
+// tw_nroots of the 3 * 2^k lines, or with FULL every power.
+template <typename Cfg, bool FULL> struct FFTCfgRoots : Cfg {};
+template <typename Cfg> struct cfg_roots { static constexpr int value = 0; };
+template <typename Cfg, bool FULL> struct cfg_roots<FFTCfgRoots<Cfg, FULL>> { static constexpr int value = FULL ? 2 : 1; };
 
 // ---------------------------------------------------------------------------
 // Synchronisation of one line's LDS exchange.  A line of T <= 64 lanes lives
@@ -278,9 +293,13 @@ template <int T> GHX_DEV void line_sync() {
 // lane for every stage of one schedule in registers, loaded once, for kernels
 // that run many transforms of the same length per lane.
 // ---------------------------------------------------------------------------
-// A butterfly reads one root, on the lines of 3 * 2^k points tw_nroots of them.
-template <int N, int R> constexpr int line_nroots() { return N % 3 == 0 && N >= 24 ? tw_nroots<R>() : 1; }
-template <int N, int R> constexpr int line_power(int r) { return line_nroots<N, R>() > 1 ? tw_power<R>(r) : 1; }
+// A butterfly reads one root, more on the lines of 3 * 2^k points and on FFTCfgRoots.
+template <int N, int R, typename Cfg> constexpr int line_nroots() {
+  return (N % 3 == 0 && N >= 24) || cfg_roots<Cfg>::value > 0 ? tw_nroots<R, cfg_roots<Cfg>::value == 2>() : 1;
+}
+template <int N, int R, typename Cfg> constexpr int line_power(int r) {
+  return line_nroots<N, R, Cfg>() > 1 ? tw_power<R, cfg_roots<Cfg>::value == 2>(r) : 1;
+}
 struct TwTable {
   const cplx *p;
   template <int S> GHX_DEV cplx root(int, int r, int idx) const { (void)r; return p[idx]; }
@@ -291,20 +310,20 @@ template <int N, typename Cfg = FFTCfg<N>> struct TwCache {
   cplx w[NS > 0 ? NS : 1][E];
   template <int S, int Ns> GHX_DEV void fill(const cplx *tw, int t) {
     if constexpr (S < NS) {
-      constexpr int R = Cfg::radix(S), Q = E / R, M = line_nroots<N, R>();
+      constexpr int R = Cfg::radix(S), Q = E / R, M = line_nroots<N, R, Cfg>();
       if constexpr (Ns > 1) {
         constexpr int tws = N / (Ns * R);
 #pragma unroll
         for (int q = 0; q < Q; ++q)
 #pragma unroll
-          for (int r = 0; r < M; ++r) w[S][q * M + r] = tw[((t + q * T) % Ns) * line_power<N, R>(r) * tws];
+          for (int r = 0; r < M; ++r) w[S][q * M + r] = tw[((t + q * T) % Ns) * line_power<N, R, Cfg>(r) * tws];
       }
       fill<S + 1, Ns * R>(tw, t);
     }
   }
   GHX_DEV void load(const cplx *tw, int t) { fill<0, 1>(tw, t); }
   template <int S> GHX_DEV cplx root(int q, int r, int) const {
-    return w[S][q * line_nroots<N, Cfg::radix(S)>() + r];
+    return w[S][q * line_nroots<N, Cfg::radix(S), Cfg>() + r];
   }
 };
 
@@ -337,15 +356,14 @@ template <int N, int DIR, typename Cfg = FFTCfg<N>> struct LineFFT {
           const int k = j % Ns;
           constexpr int tws = N / (Ns * R);
           cplx w[R];
-          constexpr int M = line_nroots<N, R>();
+          constexpr int M = line_nroots<N, R, Cfg>();
           cplx p[M];
 #pragma unroll
           for (int r = 0; r < M; ++r) {
-            const cplx x = tw.template root<S>(q, r, k * line_power<N, R>(r) * tws);
+            const cplx x = tw.template root<S>(q, r, k * line_power<N, R, Cfg>(r) * tws);
             p[r] = DIR < 0 ? x : c_conj(x);
           }
-          if constexpr (M > 1) tw_powers<R>(p, w);
-          else tw_powers<R>(p[0], w);
+          tw_powers<R, M>(p, w);
 #pragma unroll
           for (int r = 1; r < R; ++r) u[r] = c_mul(u[r], w[r]);
         }
@@ -407,19 +425,19 @@ template <> struct MixCfg<96> { static constexpr int R1 = 4, R2 = 4; };
 template <> struct MixCfg<192> { static constexpr int R1 = 8, R2 = 4; };
 template <> struct MixCfg<384> { static constexpr int R1 = 8, R2 = 8; };
 
-template <int N, int DIR> struct MixFFT {
+template <int N, int DIR, bool FULL = false> struct MixFFT {
   using C = MixCfg<N>;
   static constexpr int T = N / 6, A = N / 8;
   static_assert(6 * C::R1 * C::R2 == N && T <= 64, "a line lives in one wavefront");
 
   // the stage's roots of this lane, tw_nroots of each butterfly
   template <int R, int E> struct Stage {
-    cplx w[E / R][tw_nroots<R>()];
+    cplx w[E / R][tw_nroots<R, FULL>()];
     template <int Ns, int L> GHX_DEV void load(const cplx *tw, int t) {
 #pragma unroll
       for (int q = 0; q < E / R; ++q)
 #pragma unroll
-        for (int r = 0; r < tw_nroots<R>(); ++r) w[q][r] = tw[((t + q * L) % Ns) * tw_power<R>(r) * (N / (Ns * R))];
+        for (int r = 0; r < tw_nroots<R, FULL>(); ++r) w[q][r] = tw[((t + q * L) % Ns) * tw_power<R, FULL>(r) * (N / (Ns * R))];
     }
   };
   template <int R, bool TWIDDLE, int E> GHX_DEV static void butterflies(cplx (&v)[E], const Stage<R, E> *st) {
@@ -430,10 +448,10 @@ template <int N, int DIR> struct MixFFT {
 #pragma unroll
       for (int r = 0; r < R; ++r) u[r] = v[q + r * Q];
       if constexpr (TWIDDLE) {
-        cplx w[R], p[tw_nroots<R>()];
+        cplx w[R], p[tw_nroots<R, FULL>()];
 #pragma unroll
-        for (int r = 0; r < tw_nroots<R>(); ++r) p[r] = DIR < 0 ? st->w[q][r] : c_conj(st->w[q][r]);
-        tw_powers<R>(p, w);
+        for (int r = 0; r < tw_nroots<R, FULL>(); ++r) p[r] = DIR < 0 ? st->w[q][r] : c_conj(st->w[q][r]);
+        tw_powers<R, tw_nroots<R, FULL>()>(p, w);
 #pragma unroll
         for (int r = 1; r < R; ++r) u[r] = c_mul(u[r], w[r]);
       }
@@ -556,9 +574,9 @@ template <int N, typename Cfg = FFTCfg<N>> struct Line {
     for (int m = 0; m < SE; ++m) x[m] = row[lds_pad(t + T * m)];
   }
 };
-template <int N> struct Line<N, FFTCfgMixed<N>> {
-  using I = MixFFT<N, +1>;
-  using F = MixFFT<N, -1>;
+template <int N, bool FULL> struct MixLine {
+  using I = MixFFT<N, +1, FULL>;
+  using F = MixFFT<N, -1, FULL>;
   static constexpr int T = I::T, A = I::A, KE = 6, SE = 8;
   typename I::Inv wi;
   typename F::Fwd wf;
@@ -581,3 +599,5 @@ template <int N> struct Line<N, FFTCfgMixed<N>> {
     }
   }
 };
+template <int N> struct Line<N, FFTCfgMixed<N>> : MixLine<N, false> {};
+template <int N, bool FULL> struct Line<N, FFTCfgRoots<FFTCfgMixed<N>, FULL>> : MixLine<N, FULL> {};

@@ -1662,6 +1662,70 @@ GHX_DEV void xpair_make(cplx (&z)[E], const cplx (&A)[E], const cplx (&B)[E], in
   }
 }
 
+// Two rows of one field in one line, each at its own scale.  A row transformed
+// alone has a rounding error relative to itself; in a line with a larger one it
+// would take the larger one's, and a zero row would come out as noise.  So both
+// are brought to order one by powers of two (exact) before they are combined,
+// and back after the transform (RowScale::out).  A zero row comes out zero; a
+// row that holds Inf or NaN is left out of the line and comes out NaN.
+struct RowScale {
+  double in, out;
+};
+// exponent of the row's largest component, times two, with the lowest bit set
+// unless the row is zero
+template <int E> GHX_DEV unsigned row_key(const cplx (&A)[E]) {
+  unsigned hi = 0, lo = 0;
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const unsigned long long x = __builtin_bit_cast(unsigned long long, A[m].x);
+    const unsigned long long y = __builtin_bit_cast(unsigned long long, A[m].y);
+    const unsigned hx = (unsigned)(x >> 32) & 0x7fffffffu, hy = (unsigned)(y >> 32) & 0x7fffffffu;
+    hi = hi > hx ? hi : hx;
+    hi = hi > hy ? hi : hy;
+    lo |= (unsigned)x | (unsigned)y;
+  }
+  return (hi >> 20) * 2u + ((hi | lo) != 0u ? 1u : 0u);
+}
+GHX_DEV RowScale row_scale(unsigned key) {
+  unsigned e = key >> 1;
+  if (e == 2047u) return RowScale{0.0, __builtin_nan("")};
+  if (key == 0u) return RowScale{0.0, 0.0};
+  e = e < 1u ? 1u : e > 2045u ? 2045u : e;
+  return RowScale{__builtin_bit_cast(double, (unsigned long long)(2046u - e) << 52),
+                  __builtin_bit_cast(double, (unsigned long long)e << 52)};
+}
+// z = A sa.in + i B sb.in, A and B masked as in xpair_make
+template <int NX, int E, int T>
+GHX_DEV void xpair_make_scaled(cplx (&z)[E], cplx (&A)[E], cplx (&B)[E], int t, int kxlim, bool hasb, RowScale &sa,
+                               RowScale &sb) {
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const int k = t + T * m;
+    const int kk = k <= NX / 2 ? k : NX - k;
+    const bool live = kk < kxlim, lb = live && hasb;
+    const bool realpt = (kk == 0) || (kk == NX / 2);
+    const double s = k > NX / 2 ? -1.0 : 1.0;  // upper half: conjugate
+    A[m] = c_make(live ? A[m].x : 0.0, live && !realpt ? s * A[m].y : 0.0);
+    B[m] = c_make(lb ? B[m].x : 0.0, lb && !realpt ? s * B[m].y : 0.0);
+  }
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 key = {(unsigned short)row_key<E>(A), (unsigned short)row_key<E>(B)};
+#pragma unroll
+  for (int o = T / 2; o > 0; o >>= 1)
+    key = __builtin_elementwise_max(key, __builtin_bit_cast(us2, __shfl_xor(__builtin_bit_cast(int, key), o, 64)));
+  sa = row_scale(key.x);
+  sb = row_scale(key.y);
+  if ((key.x >> 1) == 2047u || (key.y >> 1) == 2047u) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      if ((key.x >> 1) == 2047u) A[m] = c_make(0.0, 0.0);
+      if ((key.y >> 1) == 2047u) B[m] = c_make(0.0, 0.0);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < E; ++m) z[m] = c_make(A[m].x * sa.in - B[m].y * sb.in, A[m].y * sa.in + B[m].x * sb.in);
+}
+
 // Z = forward transform of x_a + i x_b in natural order (z[m] = Z[t + T m]);
 // stores A[k], B[k] for k < kxlim (k <= NX/2) to the rows da, db.  The
 // mirrored Z[NX-k] come through the line's LDS buffer.
@@ -1754,12 +1818,17 @@ __global__ __launch_bounds__(kRowBound) void k_xinv2(FieldSet in, RealSet out, i
 // (pair_rows_fwd).  The last of an odd count stays in its launch: as one of its
 // own 26.1 against 24.6 us for three inverses at 128^3, 79 against 74 at 192^3,
 // 565 against 563 at 512 x 512 x 256.  The last row of an odd count goes alone.
+// The inverse brings each row to its own scale (xpair_make_scaled) and reads
+// two roots per radix-8 stage, since a row alone drops the imaginary half of
+// its rounding error: c2r alone | paired with one root | as here, 1e-16: 4.63 |
+// 4.94 | 4.54 at 128^3, 4.14 | 4.62 | 3.88 at 512 x 64 x 32.  Neither shows in
+// the times (c2r of 512^3 1157 -> 1156 us); reading every power does (1180).
 constexpr bool pair_rows_fwd(int nx) { return nx % 3 == 0 || nx <= 128; }
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict__ in, double *__restrict__ out,
                                                          long nrows, int nxp, const cplx *__restrict__ twt,
                                                          int kxlim) {
-  using X = Line<NX, FFTCfgMix<NX>>;
+  using X = Line<NX, FFTCfgRoots<FFTCfgMix<NX>, false>>;
   static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, A = X::A, KE = X::KE, SE = X::SE;
   extern __shared__ cplx lds[];
@@ -1774,15 +1843,16 @@ __global__ __launch_bounds__(kRowBound) void k_xinv_rows(const cplx *__restrict_
   const cplx *sa = in + (size_t)r * nxp;
   cplx a[KE], b[KE], z[KE], x[SE];
   xpair_load<NX, KE, T>(a, b, sa, two ? sa + nxp : sa, t, kxlim);
-  xpair_make<NX, KE, T>(z, a, b, t, kxlim, two);
+  RowScale ra, rb;
+  xpair_make_scaled<NX, KE, T>(z, a, b, t, kxlim, two, ra, rb);
   fft.inv(z, x, buf, t);
   if (!X::live(t)) return;
   double *da = out + (size_t)r * NX;
 #pragma unroll
-  for (int m = 0; m < SE; ++m) da[t + A * m] = x[m].x;
+  for (int m = 0; m < SE; ++m) da[t + A * m] = x[m].x * ra.out;
   if (two) {
 #pragma unroll
-    for (int m = 0; m < SE; ++m) da[NX + t + A * m] = x[m].y;
+    for (int m = 0; m < SE; ++m) da[NX + t + A * m] = x[m].y * rb.out;
   }
 }
 template <int NX>
@@ -2777,13 +2847,15 @@ hipError_t xfwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet
 // 10.5 at 64^3, 23.2 -> 16.0 and 21.7 -> 14.9 at 64 x 64 x 256; of several
 // fields 22.5 -> 14.7 and 15.7 -> 9.5 (6 of 32^3), 72.9 -> 52.2 and 63.7 -> 42.9
 // (3 of 64 x 64 x 512).  prune (inverse): as in k_yinv, q holds data on the
-// dealias set's lines only; the forward writes every line.
+// dealias set's lines only; the forward writes every line.  Rows at their own
+// scale as in k_xinv_rows, and every twiddle power read: c2r 10.3 -> 10.6 us,
+// r2c 9.95 -> 9.8 at 64^3, errors 4.29 -> 3.41e-16 and 4.36 -> 3.40e-16.
 // ---------------------------------------------------------------------------
 template <int NX, int NY, bool FWD>
 __global__ __launch_bounds__(kRowBound) void k_xyplane(RealSet re, FieldSet q, GridK g, const cplx *__restrict__ twx,
                                                        const cplx *__restrict__ twy, int prune) {
-  using X = Line<NX, FFTCfgMix<NX>>;
-  using Y = Line<NY, FFTCfgMix<NY>>;
+  using X = Line<NX, FFTCfgRoots<FFTCfgMix<NX>, true>>;
+  using Y = Line<NY, FFTCfgRoots<FFTCfgMix<NY>, true>>;
   static_assert(X::T <= 64 && Y::T <= 64 && NY % 2 == 0, "lines within a wavefront, rows in pairs");
   constexpr int H = NX / 2 + 1, SX = lds_line_stride(NX), SY = lds_line_stride(NY);
   constexpr int LX = (int)kRowBound / X::T, LY = (int)kRowBound / Y::T;
@@ -2826,13 +2898,14 @@ __global__ __launch_bounds__(kRowBound) void k_xyplane(RealSet re, FieldSet q, G
           a[m] = plane[c * SY + lds_pad(2 * p)];
           b[m] = plane[c * SY + lds_pad(2 * p + 1)];
         }
-        xpair_make<NX, X::KE, X::T>(k, a, b, t, H);
+        RowScale ra, rb;
+        xpair_make_scaled<NX, X::KE, X::T>(k, a, b, t, H, true, ra, rb);
         fft.inv(k, x, buf, t);
         if (X::live(t)) {
 #pragma unroll
           for (int m = 0; m < X::SE; ++m) {
-            r0[t + X::A * m] = x[m].x;
-            r1[t + X::A * m] = x[m].y;
+            r0[t + X::A * m] = x[m].x * ra.out;
+            r1[t + X::A * m] = x[m].y * rb.out;
           }
         }
       }
