@@ -11,10 +11,10 @@
 #include "fft_engine.h"
 #include "fft_passes.h"
 
-// The launchers are split into parts (GHX_PART=1..8) so the build compiles
+// The launchers are split into parts (GHX_PART=1..9) so the build compiles
 // them in parallel; each part instantiates only the kernels it launches.
 #ifndef GHX_PART
-#error "compile with -DGHX_PART=1..8"
+#error "compile with -DGHX_PART=1..9"
 #endif
 
 namespace ghx {
@@ -104,6 +104,57 @@ static PassShape row_shape(int T, int rowslots, size_t ldsmax, long rows = 1L <<
   return PassShape{r, (unsigned)(r * T), (size_t)r * rowslots * sizeof(cplx)};
 }
 
+constexpr int zrk_groups(int KIND) { return KIND == 2 ? 4 : 3; }
+constexpr unsigned zrk_bound(int KIND) { return KIND == 2 ? 512 : 768; }
+// Launch of k_zrk (KIND 0 HD, 1 MHD, 2 Boussinesq; one group of lanes per
+// component): tiles of up to `want` lines, as many as G groups of T lanes per
+// line leave within the kernel's bound and the LDS of one block.
+static PassShape zrk_shape(int G, int T, unsigned bound, int rowslots, int nlines, int want, size_t ldsmax) {
+  int L = 1;
+  while (L * 2 <= want && L * 2 <= kMaxTile && L * 2 <= nlines && (unsigned)(G * L * 2 * T) <= bound &&
+         (size_t)G * L * 2 * rowslots * sizeof(cplx) <= ldsmax)
+    L *= 2;
+  return PassShape{L, (unsigned)(G * L * T), (size_t)G * L * rowslots * sizeof(cplx)};
+}
+// The small planes' kernel (k_xyplane): kRowBound lanes, a padded x line for
+// every T of them and the plane's nx / 2 + 1 y lines.
+#define GHX_PLANE_SIZES(X) X(24) X(32) X(48) X(64)
+static bool plane_size(int n) {
+  switch (n) {
+#define GHX_CASE(n_) case n_:
+    GHX_PLANE_SIZES(GHX_CASE)
+#undef GHX_CASE
+    return true;
+  default:
+    return false;
+  }
+}
+static constexpr PassShape plane_shape(int nx, int ny, int Tx) {
+  const int rows = (int)kRowBound / Tx;
+  return PassShape{rows, kRowBound, ((size_t)rows * lds_line_stride(nx) + (size_t)(nx / 2 + 1) * lds_line_stride(ny)) * sizeof(cplx)};
+}
+
+// Modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
+// (the spline pass 27 us against 30 on the mixed stages at 192^3, 153 against
+// 217 at 384^3); the mixed stages below.
+template <int N>
+using ZInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfgMix<N>>::type;
+// Schedules of the 3 * 2^k lines.  The y inverse is bound by its stores from 96
+// points on and takes 12 points per lane (six fields: mixed stages 100 against
+// 70 us at 192^3, 17.6 against 13.4 at 96^3); so does the y forward from 192 on
+// (45 against 43 us at 192^3), and keeps 6 at 96 (mixed 13.7 against 12.6 for
+// four fields, 12 points 13 against 12).  Shorter lines take the mixed stages
+// (9.0 -> 8.3 us at 48^3).
+template <int N>
+using YInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E, FFTCfgMid<N>, FFTCfgMix<N>>::type;
+template <int N> struct YFwd { using Cfg = YInvCfg<N>; };
+template <> struct YFwd<96> { using Cfg = FFTCfg<96>; };
+template <int N> using YFwdCfg = typename YFwd<N>::Cfg;
+// The Boussinesq update on 192-point lines spills on the mixed stages (70 -> 84
+// us at 192^3) and keeps 6 points per lane; 384 and 96 points gain (64 -> 50 us
+// at 96 x 96 x 384, 15 -> 14 at 96^3).
+template <int N>
+using ZBoussCfg = typename std::conditional<N == 192, FFTCfg<N>, FFTCfgMix<N>>::type;
 // Refuses, before it is issued, a launch that its kernel was not built for:
 // more lanes than its __launch_bounds__ or than the code object's maximum
 // work-group size, a block that is not whole lines of T lanes, a tile wider
@@ -147,22 +198,33 @@ static bool x2_size(int nx) {
 }
 
 #if GHX_PART == 1
-// The launch shape a pass of line length n takes (kind 0: z and y tile
-// passes; 1: the Boussinesq z forward, whose LDS rows hold n more points; 2:
-// the wide y inverse; 3: two-for-one x passes, n = nx; 4: half-length x
-// passes, n = nx/2), for `nlines` lines along the tiled axis, a requested
-// tile width `want` (as the GHX_LZ/GHX_LY knobs and the autotuner give it)
-// and a device LDS limit; then the check the launchers apply.  Host-only.
+// The launch shape a pass of line length n takes for `nlines` lines along the
+// tiled axis, a requested tile width `want` (as the GHX_LZ/GHX_LY knobs and the
+// autotuner give it) and a device LDS limit; then the check the launchers
+// apply.  Host-only.  Kinds: 0 z and y tile passes on the default schedule; 1
+// the Boussinesq z forward, whose LDS rows hold n more points; 2 the wide y
+// inverse; 3 two-for-one x passes (n = nx) and 4 half-length x passes (n =
+// nx/2) in full blocks; 5, 6, 7 the grouped HD, MHD and Boussinesq updates; 8
+// the small planes' kernel (n = nx, nlines = ny); 10 and 11 the x passes of 3
+// and 4 for nlines rows; 12 the y inverse, 13 the y forward and 14 the z
+// inverse of separate fields on their own schedules.
 extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                               long long *lds, int *lanes) {
   int T = 0, rows = 0;
   switch (n) {
 #define GHX_CASE(n_)                                                                   \
   case n_:                                                                             \
-    if (kind == 0 || kind == 1) T = FFTCfg<n_>::T, rows = lds_line_stride(n_) + (kind == 1 ? n_ : 0); \
-    if (kind == 2 && FFTCfgWide<n_>::E != FFTCfg<n_>::E) T = FFTCfgWide<n_>::T, rows = lds_line_stride(n_); \
-    if (kind == 3 && x2_size(n_)) T = FFTCfg<n_>::T, rows = lds_line_stride(n_);      \
-    if (kind == 4) T = FFTCfgLow<n_>::T, rows = lds_line_stride(n_);                 \
+    rows = lds_line_stride(n_);                                                        \
+    if (kind == 0) T = FFTCfg<n_>::T;                                                  \
+    if (kind == 1) T = FFTCfg<n_>::T, rows += n_;                                      \
+    if (kind == 2 && FFTCfgWide<n_>::E != FFTCfg<n_>::E) T = FFTCfgWide<n_>::T;        \
+    if ((kind == 3 || kind == 10) && x2_size(n_)) T = FFTCfg<n_>::T;                   \
+    if (kind == 4 || kind == 11) T = FFTCfgLow<n_>::T;                                 \
+    if (kind >= 5 && kind <= 7) T = FFTCfgMix<n_>::T;                                  \
+    if (kind == 8 && plane_size(n_) && plane_size(nlines)) T = FFTCfgMix<n_>::T;       \
+    if (kind == 12) T = YInvCfg<n_>::T;                                                \
+    if (kind == 13) T = YFwdCfg<n_>::T;                                                \
+    if (kind == 14) T = ZInvCfg<n_>::T;                                                \
     break;
     GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
@@ -172,16 +234,24 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
   if (T <= 0 || nlines < 1 || ldsmax <= 0) return -1;
   PassShape s;
   unsigned bound = kTileBound;
-  if (kind == 0 || kind == 1) s = tile_shape(T, rows, nlines, want, (size_t)ldsmax);
-  else if (kind == 2) s = wide_shape(T, rows, nlines);
-  else s = row_shape(T, rows, (size_t)ldsmax), bound = kRowBound;
+  switch (kind) {
+  case 2: s = wide_shape(T, rows, nlines); break;
+  case 3: case 4: s = row_shape(T, rows, (size_t)ldsmax), bound = kRowBound; break;
+  case 5: case 6: case 7:
+    bound = zrk_bound(kind - 5);
+    s = zrk_shape(zrk_groups(kind - 5), T, bound, rows, nlines, want, (size_t)ldsmax);
+    break;
+  case 8: s = plane_shape(n, nlines, T), bound = kRowBound; break;
+  case 10: case 11: s = row_shape(T, rows, (size_t)ldsmax, nlines), bound = kRowBound; break;
+  default: s = tile_shape(T, rows, nlines, want, (size_t)ldsmax); break;
+  }
   if (lines) *lines = s.lines;
   if (block) *block = (int)s.block;
   if (lds) *lds = (long long)s.lds;
   if (lanes) *lanes = T;
-  const bool tile = kind <= 2;
+  const bool tile = kind <= 2 || (kind >= 5 && kind <= 7) || kind >= 12;
   if (s.block < 1 || s.block > bound || s.block % (unsigned)T || s.lds > (size_t)ldsmax) return -2;
-  if (tile && (s.lines > kMaxTile || (s.lines & (s.lines - 1)))) return -2;
+  if (tile && (s.lines < 1 || s.lines > kMaxTile || (s.lines & (s.lines - 1)))) return -2;
   return 0;
 }
 #endif
@@ -822,8 +892,6 @@ struct ZUpdate {
   size_t bstride;
   const double *nu_b;
 };
-constexpr int zrk_groups(int KIND) { return KIND == 2 ? 4 : 3; }
-constexpr unsigned zrk_bound(int KIND) { return KIND == 2 ? 512 : 768; }
 
 template <int N, int KIND, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, const cplx *__restrict__ twt,
@@ -2273,11 +2341,6 @@ static int zinv_outputs(int mode, int nf) {
   }
 }
 
-// Modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
-// (the spline pass 27 us against 30 on the mixed stages at 192^3, 153 against
-// 217 at 384^3); the mixed stages below.
-template <int N>
-using ZInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E && (N >= 192), FFTCfgMid<N>, FFTCfgMix<N>>::type;
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune,
                 const double *aux) {
   if (mode == 3 && !aux) return hipErrorInvalidValue;
@@ -2400,15 +2463,6 @@ hipError_t zfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 #endif
 
-// Launch of k_zrk: tiles of up to `want` lines, as many as G groups of T lanes
-// per line leave within the kernel's bound and the LDS of one block.
-static PassShape zrk_shape(int G, int T, unsigned bound, int rowslots, int nlines, int want, size_t ldsmax) {
-  int L = 1;
-  while (L * 2 <= want && L * 2 <= kMaxTile && L * 2 <= nlines && (unsigned)(G * L * 2 * T) <= bound &&
-         (size_t)G * L * 2 * rowslots * sizeof(cplx) <= ldsmax)
-    L *= 2;
-  return PassShape{L, (unsigned)(G * L * T), (size_t)G * L * rowslots * sizeof(cplx)};
-}
 template <int N, int KIND, typename Cfg>
 static hipError_t launch_zrk(const FFTCtx &c, const FieldSet &in, const ZUpdate &u, int prune, int nz) {
   constexpr int T = Cfg::T, G = zrk_groups(KIND);
@@ -2556,17 +2610,6 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 #endif
 
 #if GHX_PART == 1
-// Schedules of the 3 * 2^k lines.  The y inverse is bound by its stores from 96
-// points on and takes 12 points per lane (six fields: mixed stages 100 against
-// 70 us at 192^3, 17.6 against 13.4 at 96^3); so does the y forward from 192 on
-// (45 against 43 us at 192^3), and keeps 6 at 96 (mixed 13.7 against 12.6 for
-// four fields, 12 points 13 against 12).  Shorter lines take the mixed stages
-// (9.0 -> 8.3 us at 48^3).
-template <int N>
-using YInvCfg = typename std::conditional<FFTCfgMid<N>::E != FFTCfg<N>::E, FFTCfgMid<N>, FFTCfgMix<N>>::type;
-template <int N> struct YFwd { using Cfg = YInvCfg<N>; };
-template <> struct YFwd<96> { using Cfg = FFTCfg<96>; };
-template <int N> using YFwdCfg = typename YFwd<N>::Cfg;
 // the y passes on the four-points-per-lane schedule (FFTCtx::sched bit 1)
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
@@ -2945,11 +2988,9 @@ __global__ __launch_bounds__(kRowBound) void k_xyplane(RealSet re, FieldSet q, G
   else rows();
 }
 
-#define GHX_PLANE_SIZES(X) X(24) X(32) X(48) X(64)
 template <int NX, int NY, bool FWD>
 static hipError_t launch_xyplane(const FFTCtx &c, int nf, const RealSet &re, const FieldSet &q, int prune) {
-  constexpr int LX = (int)kRowBound / Line<NX, FFTCfgMix<NX>>::T;
-  const PassShape s{LX, kRowBound, ((size_t)LX * lds_line_stride(NX) + (size_t)(NX / 2 + 1) * lds_line_stride(NY)) * sizeof(cplx)};
+  constexpr PassShape s = plane_shape(NX, NY, FFTCfgMix<NX>::T);
   allow_lds(k_xyplane<NX, NY, FWD>, s.lds);
   GHX_LAUNCH_CHECK((k_xyplane<NX, NY, FWD>), s, kRowBound, 1, false);
   hipLaunchKernelGGL((k_xyplane<NX, NY, FWD>), dim3(c.gk.nz, nf), dim3(s.block), s.lds, c.stream, re, q, c.gk, c.tw_x, c.tw_y, prune);
@@ -2971,15 +3012,6 @@ static hipError_t plane_x(const FFTCtx &c, int nf, const RealSet &re, const Fiel
     GHX_PLANE_SIZES(GHX_CASE)
 #undef GHX_CASE
   default: return hipErrorInvalidValue;
-  }
-}
-static bool plane_size(int n) {
-  switch (n) {
-#define GHX_CASE(n_) case n_:
-    GHX_PLANE_SIZES(GHX_CASE)
-#undef GHX_CASE
-    return true;
-  default: return false;
   }
 }
 bool xyplane(const FFTCtx &c) { return plane_size(c.gk.nx) && plane_size(c.gk.ny) && use_x2(c.gk.nx); }
@@ -3046,11 +3078,6 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
 }  // namespace ghx
 
 #if GHX_PART == 8
-// The Boussinesq update on 192-point lines spills on the mixed stages (70 -> 84
-// us at 192^3) and keeps 6 points per lane; 384 and 96 points gain (64 -> 50 us
-// at 96 x 96 x 384, 15 -> 14 at 96^3).
-template <int N>
-using ZBoussCfg = typename std::conditional<N == 192, FFTCfg<N>, FFTCfgMix<N>>::type;
 namespace ghx {
 hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;

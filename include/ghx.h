@@ -511,7 +511,10 @@ int ghx_stream_probe(int kind, void *dst, const void *src, size_t bytes, int blo
 
 /* Launch shape of an FFT pass (no counterpart in GHOST; host-only, no GPU
  * needed): kind 0 z/y tile passes, 1 Boussinesq z forward, 2 wide y inverse,
- * 3 two-for-one x passes (n = nx), 4 half-length x passes (n = nx/2); for a
+ * 3 two-for-one x passes (n = nx), 4 half-length x passes (n = nx/2), 5, 6, 7
+ * the grouped HD, MHD and Boussinesq updates, 8 the small planes' kernel (n =
+ * nx, nlines = ny), 10 and 11 the x passes of 3 and 4 for nlines rows, 12 the
+ * y inverse, 13 the y forward, 14 the z inverse of separate fields; for a
  * line length n, nlines lines along the tiled axis, a requested tile width
  * and an LDS limit in bytes.  Returns 0 when the shape passes the check every
  * launcher applies before it launches (lanes within the kernel's launch

@@ -1,0 +1,64 @@
+"""Launch shapes of the grouped updates, the small planes, the x passes by row
+count and the y and z passes on schedules of their own, as in
+test_launch_shapes: computed on the host by the functions the launchers call,
+for every line length, tile request and both LDS limits."""
+import pytest
+
+from test_launch_shapes import LIMITS, ROW_BOUND, SIZES, TILE_BOUND, WANTS, X2, shape
+
+ROWS = [1, 2, 63, 64, 65, 2303, 2304, 2305, 4607, 4608, 4609, 9215, 9216, 9217, 18432, 18433, 147456, 147457, 1 << 20]
+
+
+@pytest.mark.parametrize("kind,groups,bound", [(5, 3, 768), (6, 3, 768), (7, 4, 512)])
+def test_grouped_updates(kind, groups, bound):
+    for n in SIZES:
+        for nlines in (1, 2, 3, 5, 8, 17, 33, 1024):
+            for want in WANTS:
+                for limit in LIMITS:
+                    rc, L, block, lds, T = shape(kind, n, nlines, want, limit)
+                    one = groups * (n + n // 8 + 1) * 16  # one line of every component
+                    assert rc == (0 if one <= limit else -2), (kind, n, nlines, want, limit)
+                    assert L >= 1 and L & (L - 1) == 0 and L <= 32
+                    assert L <= max(1, nlines) and (want < 2 or L <= want)
+                    assert block == groups * L * T <= bound and lds == L * one
+
+
+def test_small_planes():
+    for nx in SIZES:
+        for ny in SIZES:
+            rc, rows, block, lds, T = shape(8, nx, ny, 0, 163840)
+            if nx not in (24, 32, 48, 64) or ny not in (24, 32, 48, 64):
+                assert rc == -1
+                continue
+            assert rc == 0 and block == ROW_BOUND == rows * T
+            assert lds == (rows * (nx + nx // 8 + 1) + (nx // 2 + 1) * (ny + ny // 8 + 1)) * 16 <= 163840
+            assert shape(8, nx, ny, 0, 65536)[0] == (0 if lds <= 65536 else -2)
+    assert shape(8, 64, 64, 0, 65536)[0] == -2  # 76 KB: the separate passes run there
+
+
+@pytest.mark.parametrize("kind", [10, 11])
+def test_row_passes_by_row_count(kind):
+    for n in SIZES:
+        for rows in ROWS:
+            for limit in LIMITS:
+                rc, R, block, lds, T = shape(kind, n, rows, 0, limit)
+                if kind == 10 and n not in X2:
+                    assert rc == -1
+                    continue
+                assert rc == 0 and R >= 1 and block == R * T <= ROW_BOUND
+                assert lds == R * (n + n // 8 + 1) * 16 <= limit
+                # up to 2304 wavefronts in blocks of one, then whole blocks
+                assert block == max(T, 64 if rows * T <= 64 * 2304 else ROW_BOUND)
+
+
+@pytest.mark.parametrize("kind,lanes", [(12, {96: 8, 192: 16, 384: 32}), (13, {192: 16, 384: 32}),
+                                        (14, {192: 16, 384: 32})])
+def test_passes_on_other_schedules(kind, lanes):
+    for n in SIZES:
+        for nlines in (1, 3, 8, 33, 1024):
+            for want in WANTS:
+                for limit in LIMITS:
+                    rc, L, block, lds, T = shape(kind, n, nlines, want, limit)
+                    assert rc == 0 and T == lanes.get(n, shape(0, n, nlines, want, limit)[4])
+                    assert L >= 1 and L & (L - 1) == 0 and L <= min(32, max(1, nlines))
+                    assert block == L * T <= TILE_BOUND and lds == L * (n + n // 8 + 1) * 16 <= limit
