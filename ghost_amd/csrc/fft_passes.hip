@@ -129,10 +129,18 @@ static bool plane_size(int n) {
     return false;
   }
 }
-static constexpr PassShape plane_shape(int nx, int ny, int Tx) {
+static constexpr PassShape plane_shape(int nx, int ny) {
+  const int Tx = nx % 3 == 0 ? nx / 6 : nx / 8;
   const int rows = (int)kRowBound / Tx;
   return PassShape{rows, kRowBound, ((size_t)rows * lds_line_stride(nx) + (size_t)(nx / 2 + 1) * lds_line_stride(ny)) * sizeof(cplx)};
 }
+
+// Whether a device gives the LDS of these launches; where it does not, the
+// separate x and y passes and the updates that take one component after another run.
+// (gfx950's 160 KiB hold them all; 64 KiB refuse planes of 64 x 48 and 64 x 64
+// points and the Boussinesq update of 1024-point lines.)
+static bool takes_plane(int nx, int ny, size_t ldsmax) { return plane_shape(nx, ny).lds <= ldsmax; }
+static bool takes_zrk(int G, int rowslots, size_t ldsmax) { return (size_t)G * rowslots * sizeof(cplx) <= ldsmax; }
 
 // Modes 0 and 3 hold one field: 12 points per lane for the long 3 * 2^k lines
 // (the spline pass 27 us against 30 on the mixed stages at 192^3, 153 against
@@ -207,7 +215,8 @@ static bool x2_size(int nx) {
 // nx/2) in full blocks; 5, 6, 7 the grouped HD, MHD and Boussinesq updates; 8
 // the small planes' kernel (n = nx, nlines = ny); 10 and 11 the x passes of 3
 // and 4 for nlines rows; 12 the y inverse, 13 the y forward and 14 the z
-// inverse of separate fields on their own schedules.
+// inverse of separate fields on their own schedules.  Kinds 5 to 8 give -3 where
+// the launcher takes the other kernels.
 extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                               long long *lds, int *lanes) {
   int T = 0, rows = 0;
@@ -238,10 +247,13 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
   case 2: s = wide_shape(T, rows, nlines); break;
   case 3: case 4: s = row_shape(T, rows, (size_t)ldsmax), bound = kRowBound; break;
   case 5: case 6: case 7:
+    if (!takes_zrk(zrk_groups(kind - 5), rows, (size_t)ldsmax)) return -3;
     bound = zrk_bound(kind - 5);
     s = zrk_shape(zrk_groups(kind - 5), T, bound, rows, nlines, want, (size_t)ldsmax);
     break;
-  case 8: s = plane_shape(n, nlines, T), bound = kRowBound; break;
+  case 8:
+    if (!takes_plane(n, nlines, (size_t)ldsmax)) return -3;
+    s = plane_shape(n, nlines), bound = kRowBound; break;
   case 10: case 11: s = row_shape(T, rows, (size_t)ldsmax, nlines), bound = kRowBound; break;
   default: s = tile_shape(T, rows, nlines, want, (size_t)ldsmax); break;
   }
@@ -2482,7 +2494,7 @@ static hipError_t launch_zrk(const FFTCtx &c, const FieldSet &in, const ZUpdate 
 #if GHX_PART == 4
 hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, int prune) {
   const GridK &g = c.gk;
-  if (small_z(c)) {
+  if (small_z(c) && takes_zrk(zrk_groups(0), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.om2 = rk.om2; u.nu = rk.nu;
     u.fline = rk.fline; u.bstride = rk.bstride; u.nu_b = rk.nu_b;
@@ -2557,7 +2569,7 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
 #if GHX_PART == 5
 hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &rk, int prune) {
   const GridK &g = c.gk;
-  if (small_z(c)) {
+  if (small_z(c) && takes_zrk(zrk_groups(1), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.mu; u.fline = rk.fline;
     for (int k = 0; k < 6; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
@@ -2990,7 +3002,8 @@ __global__ __launch_bounds__(kRowBound) void k_xyplane(RealSet re, FieldSet q, G
 
 template <int NX, int NY, bool FWD>
 static hipError_t launch_xyplane(const FFTCtx &c, int nf, const RealSet &re, const FieldSet &q, int prune) {
-  constexpr PassShape s = plane_shape(NX, NY, FFTCfgMix<NX>::T);
+  constexpr PassShape s = plane_shape(NX, NY);
+  static_assert(s.lines * Line<NX, FFTCfgMix<NX>>::T == (int)kRowBound, "a line of every T lanes");
   allow_lds(k_xyplane<NX, NY, FWD>, s.lds);
   GHX_LAUNCH_CHECK((k_xyplane<NX, NY, FWD>), s, kRowBound, 1, false);
   hipLaunchKernelGGL((k_xyplane<NX, NY, FWD>), dim3(c.gk.nz, nf), dim3(s.block), s.lds, c.stream, re, q, c.gk, c.tw_x, c.tw_y, prune);
@@ -3014,7 +3027,10 @@ static hipError_t plane_x(const FFTCtx &c, int nf, const RealSet &re, const Fiel
   default: return hipErrorInvalidValue;
   }
 }
-bool xyplane(const FFTCtx &c) { return plane_size(c.gk.nx) && plane_size(c.gk.ny) && use_x2(c.gk.nx); }
+bool xyplane(const FFTCtx &c) {
+  return plane_size(c.gk.nx) && plane_size(c.gk.ny) && use_x2(c.gk.nx) &&
+         takes_plane(c.gk.nx, c.gk.ny, max_lds());
+}
 hipError_t xyplane_fwd(const FFTCtx &c, int nf, const double *const *in, const FieldSet &q) {
   RealSet rs;
   for (int f = 0; f < nf; ++f) rs.p[f] = const_cast<double *>(in[f]);
@@ -3122,7 +3138,8 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
   const GridK &g = c.gk;
   // Beyond the small launches too on power-of-two lines of 32 to 256 points:
   // 48 -> 32 us at 128^3, 249 -> 207 at 256^3 (but 37 -> 47 at 192 x 192 x 96)
-  if (small_z(c) || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) {
+  if ((small_z(c) || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) &&
+      takes_zrk(zrk_groups(2), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.kappa; u.om2 = rk.om2; u.xmom = rk.xmom; u.xtemp = rk.xtemp;
     u.fline = rk.fline;

@@ -520,7 +520,8 @@ int ghx_stream_probe(int kind, void *dst, const void *src, size_t bytes, int blo
  * launcher applies before it launches (lanes within the kernel's launch
  * bounds, whole lines, tile widths a power of two up to 32, LDS within the
  * limit), -2 when it would be refused, -1 for a size or kind without a
- * kernel. */
+ * kernel, -3 (kinds 5 to 8) when the limit makes the launcher take other
+ * kernels instead. */
 int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                    long long *lds, int *lanes);
 
