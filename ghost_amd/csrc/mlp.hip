@@ -22,6 +22,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <new>
 #include <string>
@@ -417,9 +418,14 @@ DEV float row16_sum(float x) {
 }
 
 constexpr int TRAIN_TILE = 4 * 16 * NH + 2 * 16 * 16;  // bf16 values of one wave's transposes
-constexpr size_t TRAIN_LDS = WAVES * (NPAR + 1) * sizeof(float);
-static_assert(TRAIN_LDS >= LPAR * sizeof(float), "and, before them, the parameters");
-static_assert(TRAIN_LDS >= WAVES * TRAIN_TILE * sizeof(__bf16), "the sums' LDS also holds the transposes");
+// LDS of the training kernel with the gradient sums of SUMS waves in it at once
+// (the same memory holds the parameters first, then the transposes).  All four
+// take 84 KB; where a device gives a block less, two at a time take 42 KB and a
+// step 1.2 us more (10 steps at a batch of 65536: 414 -> 423 us).
+constexpr size_t train_lds_bytes(int sums) { return sums * (NPAR + 1) * sizeof(float); }
+static_assert(train_lds_bytes(2) <= 48 * 1024, "two waves' sums fit the LDS that every device gives a block");
+static_assert(train_lds_bytes(2) >= LPAR * sizeof(float), "and, before them, the parameters");
+static_assert(train_lds_bytes(2) >= WAVES * TRAIN_TILE * sizeof(__bf16), "the sums' LDS also holds the transposes");
 struct Perm {
   unsigned long long mul, add, base;
 };
@@ -430,11 +436,13 @@ struct Perm {
 // 3.5 us per tile and wave, most of it the activations' VALU work (43 us with
 // the weights gathered from global memory by each wave, the samples loaded
 // when their tile starts and the sums over lanes through the permute unit).
+template <int SUMS>
 __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X, const float *__restrict__ T,
                                                      long long n, long long batch, Perm pm,
                                                      const float *__restrict__ P, double *__restrict__ partial) {
   // the waves' transpose tiles, then (same memory) their gradient sums
   extern __shared__ __align__(16) char train_lds[];
+  static_assert(WAVES % SUMS == 0, "the waves take turns in whole groups");
   const int l = threadIdx.x & 63, c = l & 15, q = l >> 4, wv = threadIdx.x >> 6;
   __bf16 *Tdz2 = reinterpret_cast<__bf16 *>(train_lds) + wv * TRAIN_TILE, *Th1 = Tdz2 + 16 * NH, *Tdz1 = Th1 + 16 * NH, *Th2 = Tdz1 + 16 * NH;
   __bf16 *Tx = Th2 + 16 * NH, *Tdy = Tx + 256;
@@ -598,45 +606,61 @@ __global__ __launch_bounds__(BLOCK) void k_mlp_train(const float *__restrict__ X
   loss = row16_sum(loss);
   loss += __shfl_xor(loss, 16);
   loss += __shfl_xor(loss, 32);
-  __syncthreads();  // every wave is done with its transposes
+  // the waves' sums, SUMS of them in LDS at a time, added in wave order
   float *sums = reinterpret_cast<float *>(train_lds);
-  float *out = sums + wv * (NPAR + 1);
+  constexpr int PER = (NPAR + BLOCK) / BLOCK;  // elements per thread
+  double tot[PER];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int u = 0; u < PER; ++u) tot[u] = 0.0;
+  auto put = [&](float *out) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * mb + 4 * q + r;
-      if (c < NI) out[OW1 + row * NI + c] = gW1[mb][r];
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) out[OW2 + row * NH + 16 * nb + c] = gW2[mb][nb][r];
-    }
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = 4 * q + r;
-      if (j < NO) out[OW3 + j * NH + 16 * nb + c] = gW3[nb][r];
-    }
-  if (c == 0) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        out[OB1 + 16 * b + 4 * q + r] = gb1[b][r];
-        out[OB2 + 16 * b + 4 * q + r] = gb2[b][r];
+        const int row = 16 * mb + 4 * q + r;
+        if (c < NI) out[OW1 + row * NI + c] = gW1[mb][r];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) out[OW2 + row * NH + 16 * nb + c] = gW2[mb][nb][r];
       }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (4 * q + r < NO) out[OB3 + 4 * q + r] = gb3[r];
-  }
-  if (l == 0) out[NPAR] = loss / ((float)batch * (float)NO);
-  __syncthreads();
-  double *prow = partial + (size_t)blockIdx.x * (NPAR + 1);
-  for (int k = threadIdx.x; k <= NPAR; k += BLOCK) {
-    double s = 0.0;
+    for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) s += (double)sums[w * (NPAR + 1) + k];
-    prow[k] = s;
+      for (int r = 0; r < 4; ++r) {
+        const int j = 4 * q + r;
+        if (j < NO) out[OW3 + j * NH + 16 * nb + c] = gW3[nb][r];
+      }
+    if (c == 0) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          out[OB1 + 16 * b + 4 * q + r] = gb1[b][r];
+          out[OB2 + 16 * b + 4 * q + r] = gb2[b][r];
+        }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * q + r < NO) out[OB3 + 4 * q + r] = gb3[r];
+    }
+    if (l == 0) out[NPAR] = loss / ((float)batch * (float)NO);
+  };
+#pragma unroll
+  for (int w0 = 0; w0 < WAVES; w0 += SUMS) {
+    __syncthreads();  // the transposes, or the sums before, are done with
+    if (wv >= w0 && wv < w0 + SUMS) put(sums + (wv - w0) * (NPAR + 1));
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int k = (int)threadIdx.x + u * BLOCK;
+      if (k > NPAR) break;
+#pragma unroll
+      for (int w = 0; w < SUMS; ++w) tot[u] += (double)sums[w * (NPAR + 1) + k];
+    }
+  }
+  double *prow = partial + (size_t)blockIdx.x * (NPAR + 1);
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int k = (int)threadIdx.x + u * BLOCK;
+    if (k <= NPAR) prow[k] = tot[u];
   }
 }
 
@@ -765,12 +789,30 @@ uint64_t next_prime_above(uint64_t n) {
 
 }  // namespace
 
+// Whether the device gives the training kernel all its waves' sums at once
+// (GHX_TRAIN_WIDE=0: as if not).
+static bool train_wide() {
+  const char *e = getenv("GHX_TRAIN_WIDE");
+  if (e && *e == '0') return false;
+  int dev = 0, most = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      (size_t)most < train_lds_bytes(WAVES))
+    return false;
+  if (hipFuncSetAttribute((const void *)k_mlp_train<WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)train_lds_bytes(WAVES)) == hipSuccess)
+    return true;
+  (void)hipGetLastError();  // the narrow kernel runs instead
+  return false;
+}
+
 struct ghx_mlp {
   float *P = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
   double *partial = nullptr;  // GRID rows of NPAR + 1
   float *losses = nullptr;    // per-step losses of a training call, loss_cap entries
   long long loss_cap = 0;
   double *mom = nullptr;
+  bool wide = false;          // the training kernel may have all its waves' sums in LDS
   Norm norm;
   long long step = 0;
   hipStream_t stream = nullptr;
@@ -823,7 +865,7 @@ extern "C" int ghx_mlp_create(ghx_mlp **mp, unsigned long long seed) {
   m->m1 = m->P + (NPAR + 1);
   m->m2 = m->m1 + (NPAR + 1);
   m->grad = m->m2 + (NPAR + 1);
-  MHIP(hipFuncSetAttribute((const void *)k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TRAIN_LDS));
+  m->wide = train_wide();
   MHIP(hipMemset(m->P, 0, 4 * (NPAR + 1) * sizeof(float)));
   MHIP(hipMemcpy(m->P, h.data(), NPAR * sizeof(float), hipMemcpyHostToDevice));
   *mp = m;
@@ -939,7 +981,12 @@ static int grad_batch(ghx_mlp *m, long long n, const float *X, const float *T, l
   // wave per SIMD); a small batch leaves no empty rows to add
   const long long tiles = (batch + 15) / 16, need = (tiles + WAVES - 1) / WAVES;
   const int nblk = (int)(need < GRID ? need : GRID);
-  hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(BLOCK), TRAIN_LDS, m->stream, X, T, n, batch, pm, m->P, m->partial);
+  if (m->wide)
+    hipLaunchKernelGGL(k_mlp_train<WAVES>, dim3(nblk), dim3(BLOCK), train_lds_bytes(WAVES), m->stream, X, T, n, batch,
+                       pm, m->P, m->partial);
+  else
+    hipLaunchKernelGGL(k_mlp_train<2>, dim3(nblk), dim3(BLOCK), train_lds_bytes(2), m->stream, X, T, n, batch, pm,
+                       m->P, m->partial);
   MHIP(hipGetLastError());
   hipLaunchKernelGGL(k_mlp_reduce, dim3((NPAR + RCOL) / RCOL), dim3(RCOL * RSEG), 0, m->stream, m->partial, nblk,
                      m->grad, ad ? 1 : 0, ad ? *ad : AdamStep{});
