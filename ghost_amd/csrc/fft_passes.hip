@@ -116,6 +116,15 @@ static PassShape zrk_shape(int G, int T, unsigned bound, int rowslots, int nline
     L *= 2;
   return PassShape{L, (unsigned)(G * L * T), (size_t)G * L * rowslots * sizeof(cplx)};
 }
+// The schedules of the grouped updates are those of the large launches' updates,
+// so that a run's rounding does not hang on its size: four points per lane for
+// MHD where a length has that schedule and for HD's 512-point lines (and others
+// on request, FFTCtx::sched), 64 and 512 points 1.84 and 2.52e-16 of rounding a
+// line against 2.52 and 3.42 on the default schedule.
+template <int N> constexpr bool has_low() { return FFTCfgLow<N>::E != FFTCfg<N>::E; }
+template <int N, int KIND>
+using ZrkCfg = typename std::conditional<has_low<N>() && (KIND == 1 || (KIND == 0 && N == 512)), FFTCfgLow<N>, FFTCfgMix<N>>::type;
+
 // The small planes' kernel (k_xyplane): kRowBound lanes, a padded x line for
 // every T of them and the plane's nx / 2 + 1 y lines.
 #define GHX_PLANE_SIZES(X) X(24) X(32) X(48) X(64)
@@ -229,7 +238,9 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
     if (kind == 2 && FFTCfgWide<n_>::E != FFTCfg<n_>::E) T = FFTCfgWide<n_>::T;        \
     if ((kind == 3 || kind == 10) && x2_size(n_)) T = FFTCfg<n_>::T;                   \
     if (kind == 4 || kind == 11) T = FFTCfgLow<n_>::T;                                 \
-    if (kind >= 5 && kind <= 7) T = FFTCfgMix<n_>::T;                                  \
+    if (kind == 5) T = ZrkCfg<n_, 0>::T;                                               \
+    if (kind == 6) T = ZrkCfg<n_, 1>::T;                                               \
+    if (kind == 7) T = ZrkCfg<n_, 2>::T;                                               \
     if (kind == 8 && plane_size(n_) && plane_size(nlines)) T = FFTCfgMix<n_>::T;       \
     if (kind == 12) T = YInvCfg<n_>::T;                                                \
     if (kind == 13) T = YFwdCfg<n_>::T;                                                \
@@ -2360,16 +2371,21 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
   if (small_z(c)) {
     const int nout = zinv_outputs(mode, nf);
     switch (g.nz) {
-#define GHX_CASE(n_)                                                                        \
-  case n_: {                                                                                \
-    constexpr int T = FFTCfg<n_>::T;                                                        \
+#define GHX_ONE(n_, Cfg_)                                                                    \
+  {                                                                                         \
+    constexpr int T = Cfg_::T;                                                              \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds()); \
-    allow_lds(k_zinv_one<n_>, s.lds);                                                       \
-    GHX_LAUNCH_CHECK((k_zinv_one<n_>), s, kTileBound, T, true);                             \
-    hipLaunchKernelGGL((k_zinv_one<n_>), dim3((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch * nout), dim3(s.block), s.lds, c.stream, in, out, mode, nout, g, c.tw_z, prune, aux); \
+    allow_lds((k_zinv_one<n_, Cfg_>), s.lds);                                               \
+    GHX_LAUNCH_CHECK((k_zinv_one<n_, Cfg_>), s, kTileBound, T, true);                       \
+    hipLaunchKernelGGL((k_zinv_one<n_, Cfg_>), dim3((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch * nout), dim3(s.block), s.lds, c.stream, in, out, mode, nout, g, c.tw_z, prune, aux); \
     return hipGetLastError();                                                               \
   }
+#define GHX_CASE(n_)                                                                        \
+  case n_:                                                                                  \
+    if constexpr (has_low<n_>()) if (mode == 1 && (c.sched & 1)) GHX_ONE(n_, FFTCfgLow<n_>) \
+    GHX_ONE(n_, FFTCfgMix<n_>)
       GHX_SIZES(GHX_CASE)
+#undef GHX_ONE
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
     }
@@ -2494,6 +2510,12 @@ static hipError_t launch_zrk(const FFTCtx &c, const FieldSet &in, const ZUpdate 
 #if GHX_PART == 4
 hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, int prune) {
   const GridK &g = c.gk;
+  // 512-point lines take the four-points-per-lane schedule by default (128
+  // lanes per line, four lines per 512-lane block): 124 registers per lane
+  // against 224, two blocks per CU, so the update's loads of v and C overlap
+  // more (0.71 -> 0.70 ms at 512^3; GHX_ZLOW=0 selects the default schedule).
+  // Other sizes take it on request (FFTCtx::sched bit 0).
+  const bool low = (c.sched & 1) || (g.nz == 512 && env_switch("GHX_ZLOW", 1) == 1);
   if (small_z(c) && takes_zrk(zrk_groups(0), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.om2 = rk.om2; u.nu = rk.nu;
@@ -2502,19 +2524,13 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
     switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_:                                                                                  \
-    if constexpr (FFTCfgLow<n_>::E != FFTCfg<n_>::E) if (c.sched & 1) return launch_zrk<n_, 0, FFTCfgLow<n_>>(c, in, u, prune, c.batch); \
+    if constexpr (has_low<n_>()) if (low) return launch_zrk<n_, 0, FFTCfgLow<n_>>(c, in, u, prune, c.batch); \
     return launch_zrk<n_, 0, FFTCfgMix<n_>>(c, in, u, prune, c.batch);
       GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
     }
   }
-  // 512-point lines take the four-points-per-lane schedule by default (128
-  // lanes per line, four lines per 512-lane block): 124 registers per lane
-  // against 224, two blocks per CU, so the update's loads of v and C overlap
-  // more (0.71 -> 0.70 ms at 512^3; GHX_ZLOW=0 selects the default schedule).
-  // Other sizes take it on request (FFTCtx::sched bit 0).
-  const bool low = (c.sched & 1) || (g.nz == 512 && env_switch("GHX_ZLOW", 1) == 1);
   // On the four-points-per-lane schedule the next field's Q tile is loaded
   // while this one is transformed (138 registers against 124; 0.698 -> 0.671
   // ms at 512^3; GHX_ZPF=0 loads one tile at a time)
@@ -2569,12 +2585,16 @@ hipError_t zfwd_rk_hd(const FFTCtx &c, const FieldSet &in, const RKParams &rk, i
 #if GHX_PART == 5
 hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &rk, int prune) {
   const GridK &g = c.gk;
+  const bool low = env_switch("GHX_ZLOW", 1) == 1;
   if (small_z(c) && takes_zrk(zrk_groups(1), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.mu; u.fline = rk.fline;
     for (int k = 0; k < 6; ++k) { u.v[k] = rk.v[k]; u.c[k] = rk.c[k]; u.f[k] = rk.f[k]; u.out[k] = rk.out[k]; }
     switch (g.nz) {
-#define GHX_CASE(n_) case n_: return launch_zrk<n_, 1, FFTCfgMix<n_>>(c, in, u, prune, 2);
+#define GHX_CASE(n_)                                                                        \
+  case n_:                                                                                  \
+    if constexpr (has_low<n_>()) if (low) return launch_zrk<n_, 1, FFTCfgLow<n_>>(c, in, u, prune, 2); \
+    return launch_zrk<n_, 1, FFTCfgMix<n_>>(c, in, u, prune, 2);
       GHX_SIZES(GHX_CASE)
 #undef GHX_CASE
     default: return hipErrorInvalidValue;
@@ -2583,7 +2603,6 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
   // the four-points-per-lane schedule where a size has one (GHX_ZLOW=0: the
   // default schedule); 8 lines to 256 lanes, else 4 (both parts together: 51 ->
   // 46 us at 128^3, 113 -> 108 at 192^3, but 764 -> 814 at 512 x 512 x 256)
-  const bool low = env_switch("GHX_ZLOW", 1) == 1;
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \

@@ -66,3 +66,14 @@ def test_passes_on_other_schedules(kind, lanes):
                     assert rc == 0 and T == lanes.get(n, shape(0, n, nlines, want, limit)[4])
                     assert L >= 1 and L & (L - 1) == 0 and L <= min(32, max(1, nlines))
                     assert block == L * T <= TILE_BOUND and lds == L * (n + n // 8 + 1) * 16 <= limit
+
+
+def test_updates_keep_the_large_launches_schedule():
+    """Four points per lane for MHD on 32 to 512 points and HD on 512, as the
+    updates that take one component after another; else the default schedule."""
+    for n in SIZES:
+        low = n in (32, 64, 128, 256, 512)
+        default = shape(0, n, 8, 1, 163840)[4]
+        assert shape(5, n, 8, 1, 163840)[4] == (128 if n == 512 else default)
+        assert shape(6, n, 8, 1, 163840)[4] == (n // 4 if low else default)
+        assert shape(7, n, 8, 1, 163840)[4] == default
