@@ -172,6 +172,36 @@ template <int N> using YFwdCfg = typename YFwd<N>::Cfg;
 // at 96 x 96 x 384, 15 -> 14 at 96^3).
 template <int N>
 using ZBoussCfg = typename std::conditional<N == 192, FFTCfg<N>, FFTCfgMix<N>>::type;
+// Launches of up to this many kept lines (13 per CU; 96^3 has 3168, 128^3
+// 5504) leave the GPU waiting on the chain inside a block, so a block is given
+// one field or one component instead of all of them in turn.  Measured at
+// 32^3, 64^3, 96^3 and 128^3 (us, with ~3 of event overhead): six-field y
+// inverse 12.9 -> 7.3, 14.4 -> 9.7, 20.6 -> 13.3, 23.8 -> 27.7; curl z inverse
+// 11.8 -> 9.4, 12.9 -> 11.7, 17.8 -> 17.4, 20.9 -> 30.1; HD update 14.2 -> 8.8,
+// 15.9 -> 10.8, 16.6 -> 13.2, 23.3 -> 24.7.
+// Long z lines turn earlier: what one field per block reads and transforms
+// again grows with the line.  All fields in turn | one per block, curl and
+// update: 256 points, 704 lines 17.5 | 15.0 and 20.4 | 15.0, 1408 lines 18.7 |
+// 22.1 and 22.2 | 24.0; 384 points, 704 lines 18.5 | 17.8, 1408 23.7 | 26.5; 512
+// points, 352 lines 17.9 | 15.8, 704 18.9 | 22.4, 3168 28.2 | 50.2; 1024 points,
+// 352 lines 33.0 | 30.2, 704 35.0 | 46.7.  (192 points: 18.3 | 17.4 at 1408 lines,
+// 23.1 | 21.5 at 3168, but 23.5 | 25.7 at 2752; whole steps of HD, MHD and
+// Boussinesq gain or lose up to 7% either way and keep the limit.)  So beyond
+// 192 points the limit is a volume, and never below 384 lines, which leave CUs
+// without a tile.  Fields that are only transformed, and a curl alone, read
+// little twice and keep kSmallLines at any length (c2r of 64 x 32 x 512 16.4 |
+// 15.1, diagnostics of 64 x 64 x 1024 444 | 419).
+constexpr long kSmallLines = 3328;
+static constexpr long small_z_lines(int nz) {
+  const long v = 1408L * 192 / nz;
+  return nz <= 192 ? kSmallLines : v > 384 ? v : 384;
+}
+// The y passes read nothing twice; the lines of 384 points (six fields in turn |
+// one per block 38.3 | 25.5 at 1408 lines, 45.0 | 52.9 at 3168) and of 1024
+// (30.9 | 26.6 at 352, 33.5 | 40.3 at 704) turn earlier all the same, 512 and
+// less not below 3328 (52.3 | 54.9 at 3168 of 512).
+static constexpr long small_y_lines(int ny) { return ny > 512 ? 512 : ny == 384 ? 2112 : kSmallLines; }
+
 // Refuses, before it is issued, a launch that its kernel was not built for:
 // more lanes than its __launch_bounds__ or than the code object's maximum
 // work-group size, a block that is not whole lines of T lanes, a tile wider
@@ -224,7 +254,9 @@ static bool x2_size(int nx) {
 // nx/2) in full blocks; 5, 6, 7 the grouped HD, MHD and Boussinesq updates; 8
 // the small planes' kernel (n = nx, nlines = ny); 10 and 11 the x passes of 3
 // and 4 for nlines rows; 12 the y inverse, 13 the y forward and 14 the z
-// inverse of separate fields on their own schedules.  Kinds 5 to 8 give -3 where
+// inverse of separate fields on their own schedules; 15 and 16: *lines is the
+// number of kept lines up to which a z or y launch takes one field per block
+// (nothing else is set).  Kinds 5 to 8 give -3 where
 // the launcher takes the other kernels.
 extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                               long long *lds, int *lanes) {
@@ -250,6 +282,10 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
 #undef GHX_CASE
   default:
     break;
+  }
+  if ((kind == 15 || kind == 16) && rows > 0 && lines) {
+    *lines = (int)(kind == 15 ? small_z_lines(n) : small_y_lines(n));
+    return 0;
   }
   if (T <= 0 || nlines < 1 || ldsmax <= 0) return -1;
   PassShape s;
@@ -317,16 +353,9 @@ static bool use_x2(int nx) {
 // few lanes would leave half or more of it idle: 4 lines of 8 lanes).
 static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
 
-// Launches of up to this many kept lines (13 per CU; 96^3 has 3168, 128^3
-// 5504) leave the GPU waiting on the chain inside a block, so a block is given
-// one field or one component instead of all of them in turn.  Measured at
-// 32^3, 64^3, 96^3 and 128^3 (us, with ~3 of event overhead): six-field y
-// inverse 12.9 -> 7.3, 14.4 -> 9.7, 20.6 -> 13.3, 23.8 -> 27.7; curl z inverse
-// 11.8 -> 9.4, 12.9 -> 11.7, 17.8 -> 17.4, 20.9 -> 30.1; HD update 14.2 -> 8.8,
-// 15.9 -> 10.8, 16.6 -> 13.2, 23.3 -> 24.7.
-constexpr long kSmallLines = 3328;
-static bool small_z(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch <= kSmallLines; }
-static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= kSmallLines; }
+static long z_lines(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch; }
+static bool small_z(const FFTCtx &c) { return z_lines(c) <= small_z_lines(c.gk.nz); }
+static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= small_y_lines(c.gk.ny); }
 
 template <typename K> static void allow_lds(K kern, size_t bytes) {
   if (bytes > 49152) (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -1369,7 +1398,12 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
   fft.load_inv(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
   // block's first of nper fields
-  const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
+  int member = blockIdx.z, f0 = 0;
+  if (nper < nf_) {
+    const int parts = (nf_ + nper - 1) / nper;
+    member = blockIdx.z / parts;
+    f0 = ((int)blockIdx.z - member * parts) * nper;
+  }
   const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
   const FieldView in = batch_view(in_, member);
   const FieldView out = batch_view(out_, member);
@@ -1429,7 +1463,12 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
   fft.load_fwd(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
   // block's first of nper fields
-  const int parts = (nf_ + nper - 1) / nper, member = blockIdx.z / parts, f0 = ((int)blockIdx.z - member * parts) * nper;
+  int member = blockIdx.z, f0 = 0;
+  if (nper < nf_) {
+    const int parts = (nf_ + nper - 1) / nper;
+    member = blockIdx.z / parts;
+    f0 = ((int)blockIdx.z - member * parts) * nper;
+  }
   const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
   const FieldView in = batch_view(in_, member);
   const FieldView out = batch_view(out_, member);
@@ -2368,7 +2407,7 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
                 const double *aux) {
   if (mode == 3 && !aux) return hipErrorInvalidValue;
   const GridK &g = c.gk;
-  if (small_z(c)) {
+  if (mode == 0 || mode == 3 || mode == 7 ? z_lines(c) <= kSmallLines : small_z(c)) {
     const int nout = zinv_outputs(mode, nf);
     switch (g.nz) {
 #define GHX_ONE(n_, Cfg_)                                                                    \
@@ -3155,9 +3194,11 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
 
 hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParams &rk, int prune) {
   const GridK &g = c.gk;
-  // Beyond the small launches too on power-of-two lines of 32 to 256 points:
-  // 48 -> 32 us at 128^3, 249 -> 207 at 256^3 (but 37 -> 47 at 192 x 192 x 96)
-  if ((small_z(c) || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) &&
+  // Up to kSmallLines at any length (63 against 78 us for 2112 lines of 512
+  // points, 115 against 196 of 1024), and beyond on power-of-two lines of 32 to
+  // 256 points: 48 -> 32 us at 128^3, 249 -> 207 at 256^3 (but 37 -> 47 at 192 x
+  // 192 x 96)
+  if ((z_lines(c) <= kSmallLines || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) &&
       takes_zrk(zrk_groups(2), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};
     u.dt = rk.dt; u.rmp = rk.rmp; u.nu = rk.nu; u.mu = rk.kappa; u.om2 = rk.om2; u.xmom = rk.xmom; u.xtemp = rk.xtemp;

@@ -77,3 +77,13 @@ def test_updates_keep_the_large_launches_schedule():
         assert shape(5, n, 8, 1, 163840)[4] == (128 if n == 512 else default)
         assert shape(6, n, 8, 1, 163840)[4] == (n // 4 if low else default)
         assert shape(7, n, 8, 1, 163840)[4] == default
+
+
+def test_one_field_per_block_ends_earlier_on_long_lines():
+    """Up to 192 points one limit, beyond a volume of lines (5 to 40% slower
+    above it at 256 to 1024 points), never below a tile for most CUs."""
+    for n in SIZES:
+        z, y = shape(15, n, 1, 0, 163840), shape(16, n, 1, 0, 163840)
+        assert z[0] == y[0] == 0
+        assert z[1] == (3328 if n <= 192 else max(384, 1408 * 192 // n))
+        assert y[1] == {384: 2112, 1024: 512}.get(n, 3328)
