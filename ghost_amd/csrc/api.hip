@@ -189,7 +189,7 @@ struct ghx_plan {
   int nx, ny, nz, nxh, dir;
   FFTCtx ctx;
   cplx *tw = nullptr;       // all twiddle tables, then the word below
-  unsigned *word = nullptr;  // device word of the substeps on caller fields (GridK::dirty)
+  unsigned *word = nullptr;  // device word of the substeps on caller fields (FFTCtx::dirty)
   cplx *q = nullptr;        // Q scratch, q_fields fields
   int q_fields = 0;
   bool timing = false;
@@ -232,7 +232,6 @@ static GridK make_gridk(int nx, int ny, int nz, int arbsize, double Lx, double L
     const double kx = (double)(q < nx / 2 ? q : q - nx);
     if (g.rmp * (kx * kx) <= g.kmax) g.kxact = q + 1;
   }
-  g.dirty = nullptr;
   return g;
 }
 
@@ -1525,7 +1524,7 @@ static int hd_substep(ghx_grid *g, cplx *q, int o, double dt, double nu, const c
                       double omegaz = 0.0, const unsigned *dirty = nullptr) {
   const size_t nc = g->nc;
   FFTCtx ctx = g->plan.ctx;
-  ctx.gk.dirty = dirty;
+  ctx.dirty = dirty;
   Chain ch = chain_slots(q, ghx::slot_points(g->gk));
   FieldSet in, pq;
   for (int k = 0; k < 3; ++k) in.p[k] = const_cast<cplx *>(v[k]);
@@ -2040,7 +2039,7 @@ static int mhd_substep(ghx_mhd *s, int o, const cplx *const *vin, cplx *const *o
   ghx_grid *g = s->g;
   const size_t nc = g->nc, slot = ghx::slot_points(g->gk);
   FFTCtx ctx = g->plan.ctx;
-  ctx.gk.dirty = dirty;
+  ctx.dirty = dirty;
   // Q12 (slots 0-11) -> P12 (12-23) -> P9 (reuses 0-8) -> Q9 (reuses 12-20)
   FieldSet in, q12, p12, p9, q9, pq;
   for (int k = 0; k < 6; ++k) in.p[k] = const_cast<cplx *>(vin[k]);
@@ -2414,7 +2413,7 @@ static int bouss_substep(ghx_bouss *s, int o, const cplx *const *vin, cplx *cons
   ghx_grid *g = s->g;
   const size_t nc = g->nc, slot = ghx::slot_points(g->gk);
   FFTCtx ctx = g->plan.ctx;
-  ctx.gk.dirty = dirty;
+  ctx.dirty = dirty;
   // Q9 (slots 0-8) -> P9 (9-17) -> P4 (reuses 0-3) -> Q4 (reuses 9-12)
   FieldSet in, q9, p9, pq, o3, pd, o1, p4, q4;
   for (int k = 0; k < 4; ++k) in.p[k] = const_cast<cplx *>(vin[k]);

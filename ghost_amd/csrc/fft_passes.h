@@ -30,6 +30,9 @@ struct FFTCtx {
   // inverse, forward update), bit 1 the y passes, on four points per lane
   // (FFTCfgLow) where that differs from the default schedule
   int sched = 0;
+  // prune == 2: a device word that is zero when the input turned out to be zero
+  // outside the kept modes (null: not looked at, taken as non-zero)
+  const unsigned *dirty = nullptr;
 };
 
 constexpr int kMaxFields = 12;
@@ -85,7 +88,7 @@ inline size_t slot_points(const GridK &g) { return (size_t)g.nz * g.ny * p_row(g
 // prune=1: the input is dealiased (zero outside tiny <= kn2 <= kmax): only
 // lines that carry kept modes are read and written (every pass below takes
 // the same flag; see the kernels for exactly what each one skips).
-// prune=2: outputs as with 1, inputs as GridK::dirty says (prune_input).
+// prune=2: outputs as with 1, inputs as FFTCtx::dirty says.
 // mode 3: nf fields in, nf out, each mode scaled by aux[kx] aux[nxh+ky]
 // aux[nxh+ny+kz] (the periodic cubic-spline prefilter of the tracers).
 hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const FieldSet &out, int prune = 0,

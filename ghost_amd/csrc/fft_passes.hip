@@ -353,6 +353,14 @@ static bool use_x2(int nx) {
 // few lanes would leave half or more of it idle: 4 lines of 8 lanes).
 static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
 
+// What a launch passes for its input's pruning (prune_input): the flag and the
+// device word that may clear it.
+static int prune_in(const FFTCtx &c, int prune) { return prune == 2 ? (c.dirty ? 1 : 0) : prune; }
+static const unsigned *prune_word(const FFTCtx &c, int prune) { return prune == 2 ? c.dirty : nullptr; }
+// kx below which a pass reads its input (unless the word says more) and writes its output
+static int kx_in(const FFTCtx &c, int prune) { return prune_in(c, prune) ? c.gk.kxact : c.gk.nxh; }
+static int kx_out(const FFTCtx &c, int prune) { return prune ? c.gk.kxact : c.gk.nxh; }
+
 static long z_lines(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.ny * c.batch; }
 static bool small_z(const FFTCtx &c) { return z_lines(c) <= small_z_lines(c.gk.nz); }
 static bool small_y(const FFTCtx &c) { return (long)c.gk.kxact * c.gk.nz * c.batch <= small_y_lines(c.gk.ny); }
@@ -577,9 +585,9 @@ GHX_DEV void zinv_curl5(cplx (&ax)[E], cplx (&ay)[E], cplx (&az)[E], double kx, 
 
 template <int N, int MODE, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_, int nf, GridK g, const cplx *__restrict__ twt,
-                                             int prune_, const double *__restrict__ aux) {
+                                             int prune_, const unsigned *dirty, const double *__restrict__ aux) {
   using F = Line<N, Cfg>;
-  const int prune = prune_input(g, prune_);
+  const int prune = prune_input(prune_, dirty);
   constexpr int T = F::T, E = F::KE;
   // store groups: the MHD and Boussinesq passes (MODE 2, 5) are at the
   // register limit and spill more with grouped reads; they store one point
@@ -778,11 +786,11 @@ GHX_DEV ZOut zinv_output(int mode, int o) {
 
 template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet out_, int mode, int nout, GridK g,
-                                                 const cplx *__restrict__ twt, int prune_,
+                                                 const cplx *__restrict__ twt, int prune_, const unsigned *dirty,
                                                  const double *__restrict__ aux) {
   using F = Line<N, Cfg>;
   constexpr int T = F::T, E = F::KE;
-  const int prune = prune_input(g, prune_);
+  const int prune = prune_input(prune_, dirty);
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
   const int lt = threadIdx.x / T, t = threadIdx.x % T;
@@ -1385,11 +1393,21 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
 // an LDS tile with L-point (L*16-byte) chunks along kx.  Only kx < kxlim is
 // touched (kxlim < nx/2+1 when the fields are dealiased).
 // ---------------------------------------------------------------------------
+// A y launch split over its fields has parts = nf blocks per tile and member,
+// one field each; else parts = 1.  inv divides blockIdx.z by parts without a
+// division or a branch ahead of the kernel's other argument reads (exact up to
+// 65535 for up to kMaxFields parts).
+struct YSplit {
+  int parts;
+  unsigned inv;
+};
+static inline YSplit ysplit(int parts) { return YSplit{parts, (unsigned)(((1ull << 31) + parts - 1) / parts)}; }
+
 template <int N, typename Cfg = FFTCfgMix<N>>
-__global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
-                                             const cplx *__restrict__ twt, int prune_) {
+__global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf_, YSplit sp, GridK g, int nxp,
+                                             const cplx *__restrict__ twt, int kxlim, int prune, const unsigned *dirty) {
   using F = Line<N, Cfg>;
-  const int prune = prune_input(g, prune_), kxlim = prune ? g.kxact : g.nxh;
+  if (dirty && *dirty != 0u) prune = 0, kxlim = g.nxh;  // (as prune_input)
   constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
@@ -1397,14 +1415,9 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
   F fft;  // with this lane's stage roots, loaded once
   fft.load_inv(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
-  // block's first of nper fields
-  int member = blockIdx.z, f0 = 0;
-  if (nper < nf_) {
-    const int parts = (nf_ + nper - 1) / nper;
-    member = blockIdx.z / parts;
-    f0 = ((int)blockIdx.z - member * parts) * nper;
-  }
-  const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
+  // block's field (ysplit)
+  const int member = __umulhi(2u * blockIdx.z, sp.inv), f0 = (int)blockIdx.z - member * sp.parts;
+  const int nf = sp.parts > 1 ? f0 + 1 : nf_;
   const FieldView in = batch_view(in_, member);
   const FieldView out = batch_view(out_, member);
   int bx, by;
@@ -1451,10 +1464,9 @@ __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_
 }
 
 template <int N, typename Cfg = FFTCfgMix<N>>
-__global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf_, int nper, GridK g, int nxp,
-                                             const cplx *__restrict__ twt, int prune) {
+__global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_, int nf_, YSplit sp, GridK g, int nxp,
+                                             const cplx *__restrict__ twt, int kxlim, int prune) {
   using F = Line<N, Cfg>;
-  const int kxlim = prune ? g.kxact : g.nxh;
   constexpr int T = F::T, E = F::KE;
   extern __shared__ cplx lds[];
   const int L = blockDim.x / T;
@@ -1462,14 +1474,9 @@ __global__ __launch_bounds__(kTileBound) void k_yfwd(FieldSet in_, FieldSet out_
   F fft;  // with this lane's stage roots, loaded once
   fft.load_fwd(twt, t);
   // blockIdx.z: member and, where a launch is split over its fields, the
-  // block's first of nper fields
-  int member = blockIdx.z, f0 = 0;
-  if (nper < nf_) {
-    const int parts = (nf_ + nper - 1) / nper;
-    member = blockIdx.z / parts;
-    f0 = ((int)blockIdx.z - member * parts) * nper;
-  }
-  const int nf = f0 + nper < nf_ ? f0 + nper : nf_;
+  // block's field (ysplit)
+  const int member = __umulhi(2u * blockIdx.z, sp.inv), f0 = (int)blockIdx.z - member * sp.parts;
+  const int nf = sp.parts > 1 ? f0 + 1 : nf_;
   const FieldView in = batch_view(in_, member);
   const FieldView out = batch_view(out_, member);
   int bx, by;
@@ -2134,8 +2141,8 @@ __global__ __launch_bounds__(kRowBound) void k_xfwd2(RealSet in, FieldSet out, i
 // (A_x, A_y), (A_z, B_x), (B_y, B_z); fields as k_xdot.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, GridK g, int nxp,
-                                              const cplx *__restrict__ twt, int prune) {
-  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
+                                              const cplx *__restrict__ twt, int kxin, int kxout, const unsigned *dirty) {
+  const int kxlim = dirty && *dirty != 0u ? g.nxh : kxin;  // (as prune_input)
   using X = Line<NX, FFTCfgMix<NX>>;
   static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, KE = X::KE, SE = X::SE;
@@ -2177,8 +2184,8 @@ __global__ __launch_bounds__(kRowBound) void k_xdot2(FieldSet in, FieldSet out, 
 // 2^k rows into scratch, 20 of them and 726 -> 1072 us at 384^3.
 template <int NX>
 __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) void k_xcross2(FieldSet in_, FieldSet out_, GridK g, int nxp,
-                                                const cplx *__restrict__ twt, int prune) {
-  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
+                                                const cplx *__restrict__ twt, int kxin, int kxout, const unsigned *dirty) {
+  const int kxlim = dirty && *dirty != 0u ? g.nxh : kxin;  // (as prune_input)
   using X = Line<NX, FFTCfgMix<NX>>;
   static_assert(X::T <= 64, "one row per wavefront or less");
   constexpr int T = X::T, KE = X::KE, SE = X::SE;
@@ -2233,8 +2240,8 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(2))) 
 template <int N, int W, int SB>
 __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) void k_xcross(
     FieldSet in_, FieldSet out_, GridK g, int nxp, const cplx *__restrict__ twh, const cplx *__restrict__ twx,
-    int prune) {
-  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
+    int kxin, int kxout, const unsigned *dirty) {
+  const int kxlim = dirty && *dirty != 0u ? g.nxh : kxin;  // (as prune_input)
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T, E = Cfg::E;
   extern __shared__ cplx lds[];
@@ -2313,8 +2320,8 @@ __global__ __launch_bounds__(kRowBound) __attribute__((amdgpu_waves_per_eu(W))) 
 // FFT[((A_x B_x + A_y B_y) + A_z B_z) tmp] with tmp = -1/N^6.
 template <int N>
 __global__ __launch_bounds__(kRowBound) void k_xdot(FieldSet in, FieldSet out, GridK g, int nxp,
-                                             const cplx *__restrict__ twh, const cplx *__restrict__ twx, int prune) {
-  const int kxlim = prune_input(g, prune) ? g.kxact : g.nxh, kxout = prune ? g.kxact : g.nxh;
+                                             const cplx *__restrict__ twh, const cplx *__restrict__ twx, int kxin, int kxout, const unsigned *dirty) {
+  const int kxlim = dirty && *dirty != 0u ? g.nxh : kxin;  // (as prune_input)
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T, E = Cfg::E;
   extern __shared__ cplx lds[];
@@ -2373,7 +2380,7 @@ static hipError_t launch_zinv_wide(const FFTCtx &c, int nf, const FieldSet &in, 
   dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);
   allow_lds(k_zinv<512, MODE, Cfg>, s.lds);
   GHX_LAUNCH_CHECK((k_zinv<512, MODE, Cfg>), s, kTileBound, T, true);
-  hipLaunchKernelGGL((k_zinv<512, MODE, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux);
+  hipLaunchKernelGGL((k_zinv<512, MODE, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux);
   return hipGetLastError();
 }
 
@@ -2389,7 +2396,7 @@ static hipError_t launch_zinv_low(const FFTCtx &c, int nf, const FieldSet &in, c
   dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);
   allow_lds(k_zinv<N, 1, Cfg>, s.lds);
   GHX_LAUNCH_CHECK((k_zinv<N, 1, Cfg>), s, kTileBound, T, true);
-  hipLaunchKernelGGL((k_zinv<N, 1, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux);
+  hipLaunchKernelGGL((k_zinv<N, 1, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux);
   return hipGetLastError();
 }
 
@@ -2416,7 +2423,7 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.ny, tile_pick("GHX_LZ", c.tile_z, tile_default(T, 4)), max_lds()); \
     allow_lds((k_zinv_one<n_, Cfg_>), s.lds);                                               \
     GHX_LAUNCH_CHECK((k_zinv_one<n_, Cfg_>), s, kTileBound, T, true);                       \
-    hipLaunchKernelGGL((k_zinv_one<n_, Cfg_>), dim3((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch * nout), dim3(s.block), s.lds, c.stream, in, out, mode, nout, g, c.tw_z, prune, aux); \
+    hipLaunchKernelGGL((k_zinv_one<n_, Cfg_>), dim3((g.ny + s.lines - 1) / s.lines, g.nxh, c.batch * nout), dim3(s.block), s.lds, c.stream, in, out, mode, nout, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     return hipGetLastError();                                                               \
   }
 #define GHX_CASE(n_)                                                                        \
@@ -2454,11 +2461,11 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     if (mode == 0) {                                                                        \
       allow_lds((k_zinv<n_, 0, Cfg>), s.lds);                                               \
       GHX_LAUNCH_CHECK((k_zinv<n_, 0, Cfg>), s, kTileBound, T, true);                       \
-      hipLaunchKernelGGL((k_zinv<n_, 0, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      hipLaunchKernelGGL((k_zinv<n_, 0, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else {                                                                                \
       allow_lds((k_zinv<n_, 3, Cfg>), s.lds);                                               \
       GHX_LAUNCH_CHECK((k_zinv<n_, 3, Cfg>), s, kTileBound, T, true);                       \
-      hipLaunchKernelGGL((k_zinv<n_, 3, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      hipLaunchKernelGGL((k_zinv<n_, 3, Cfg>), grid, dim3(s.block), s.lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     }                                                                                       \
     return hipGetLastError();                                                               \
   }
@@ -2476,22 +2483,22 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     dim3 grid((g.ny + L - 1) / L, g.nxh, c.batch);                                          \
     if (mode == 1) {                                                                 \
       allow_lds(k_zinv<n_, 1>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 1>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 1>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 1>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 1>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else if (mode == 2) {                                                                 \
       allow_lds(k_zinv<n_, 2>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 2>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 2>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 2>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 2>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else if (mode == 4) {                                                                 \
       allow_lds(k_zinv<n_, 4>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 4>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 4>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 4>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 4>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else if (mode == 5) {                                                                 \
       allow_lds(k_zinv<n_, 5>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 5>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 5>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 5>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 5>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else if (mode == 6) {                                                                 \
       allow_lds(k_zinv<n_, 6>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 6>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 6>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 6>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 6>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     } else if (mode == 7) {                                                                 \
       allow_lds(k_zinv<n_, 7>, lds);                                                        \
-      GHX_LAUNCH_CHECK((k_zinv<n_, 7>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 7>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune, aux); \
+      GHX_LAUNCH_CHECK((k_zinv<n_, 7>), s, kTileBound, T, true); hipLaunchKernelGGL((k_zinv<n_, 7>), grid, dim3(L * T), lds, c.stream, in, out, nf, g, c.tw_z, prune_in(c, prune), prune_word(c, prune), aux); \
     }                                                                                       \
     break;                                                                                  \
   }
@@ -2684,21 +2691,21 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const int nper = small_y(c) ? 1 : nf;
+  const YSplit sp = ysplit(small_y(c) ? nf : 1);
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
   const int nxp = p_row(g);
   const PassShape s = tile_shape(T, lds_line_stride(N), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, inv ? 8 : 4)), max_lds());
   const int L = s.lines;
-  dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));
+  dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * sp.parts);
   if (inv) {
     allow_lds(k_yinv<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yinv<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune);
+    hipLaunchKernelGGL((k_yinv<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, sp, g, nxp, c.tw_y, kx_in(c, prune), prune_in(c, prune), prune_word(c, prune));
   } else {
     allow_lds(k_yfwd<N, Cfg>, s.lds);
     GHX_LAUNCH_CHECK((k_yfwd<N, Cfg>), s, kTileBound, T, true);
-    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune);
+    hipLaunchKernelGGL((k_yfwd<N, Cfg>), grid, dim3(L * T), s.lds, c.stream, in, out, nf, sp, g, nxp, c.tw_y, kx_out(c, prune), prune);
   }
   return hipGetLastError();
 }
@@ -2721,7 +2728,7 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
   // -> 272 at 256^3, but 45 -> 46 us at 128 x 256 x 128 (5504 lines), 39 -> 40 at
   // 192 x 128 x 128 (8320).  The 512-point wide pass loses 2%.
   const long lines = (long)g.kxact * g.nz * c.batch;
-  const int nper = small_y(c) || (lines >= 10000 && g.ny != 512) ? 1 : nf;
+  const YSplit sp = ysplit(small_y(c) || (lines >= 10000 && g.ny != 512) ? nf : 1);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;
@@ -2737,18 +2744,18 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
       constexpr int TW = FFTCfgWide<n_>::T;                                                  \
       const PassShape s = wide_shape(TW, lds_line_stride(n_), g.nxh);                        \
       const int L = s.lines; const size_t lds = s.lds;                                       \
-      dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                         \
+      dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * sp.parts);                                         \
       GHX_LAUNCH_CHECK((k_yinv<n_, FFTCfgWide<n_>>), s, kTileBound, TW, true);               \
       allow_lds(k_yinv<n_, FFTCfgWide<n_>>, lds);                                            \
-      hipLaunchKernelGGL((k_yinv<n_, FFTCfgWide<n_>>), grid, dim3(L * TW), lds, c.stream, in, out, nf, nper, g, nxp, \
-                         c.tw_y, prune);                                              \
+      hipLaunchKernelGGL((k_yinv<n_, FFTCfgWide<n_>>), grid, dim3(L * TW), lds, c.stream, in, out, nf, sp, g, nxp, \
+                         c.tw_y, kx_in(c, prune), prune_in(c, prune), prune_word(c, prune));                                              \
       break;                                                                                 \
     }                                                                                        \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, 8)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
-    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                          \
+    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * sp.parts);                                          \
     allow_lds(k_yinv<n_, Cfg>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yinv<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune); \
+    GHX_LAUNCH_CHECK((k_yinv<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yinv<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, sp, g, nxp, c.tw_y, kx_in(c, prune), prune_in(c, prune), prune_word(c, prune)); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -2761,7 +2768,7 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const int nper = small_y(c) ? 1 : nf;
+  const YSplit sp = ysplit(small_y(c) ? nf : 1);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, false, nf, in, out, prune, &lerr)) return lerr;
@@ -2772,9 +2779,9 @@ hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
     constexpr int T = Cfg::T;                                                               \
     const PassShape s = tile_shape(T, lds_line_stride(n_), g.nxh, tile_pick("GHX_LY", c.tile_y, tile_default(T, Cfg::E == 12 ? 8 : 4)), max_lds());        \
     const int L = s.lines; const size_t lds = s.lds;                            \
-    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * ((nf + nper - 1) / nper));                                          \
+    dim3 grid((g.nxh + L - 1) / L, g.nz, c.batch * sp.parts);                                          \
     allow_lds(k_yfwd<n_, Cfg>, lds);                                                             \
-    GHX_LAUNCH_CHECK((k_yfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, nper, g, nxp, c.tw_y, prune); \
+    GHX_LAUNCH_CHECK((k_yfwd<n_, Cfg>), s, kTileBound, T, true); hipLaunchKernelGGL((k_yfwd<n_, Cfg>), grid, dim3(L * T), lds, c.stream, in, out, nf, sp, g, nxp, c.tw_y, kx_out(c, prune), prune); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)
@@ -3116,7 +3123,7 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows * c.batch);                              \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xcross2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
+    GHX_LAUNCH_CHECK((k_xcross2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, kx_in(c, prune), kx_out(c, prune), prune_word(c, prune));                                                                 \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
@@ -3133,10 +3140,10 @@ hipError_t xcross(const FFTCtx &c, int mode, const FieldSet &in, const FieldSet 
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb), c.batch), bl(rpb * T);               \
     switch (tile_want("GHX_XV", 1)) {                                                       \
-    case 4: GHX_LAUNCH_CHECK((k_xcross<n_, 2, 1>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, 2, 1>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); break; \
+    case 4: GHX_LAUNCH_CHECK((k_xcross<n_, 2, 1>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, 2, 1>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kx_in(c, prune), kx_out(c, prune), prune_word(c, prune)); break; \
     /* 3 * 2^k rows: one wave per SIMD leaves the registers to hold the six */ \
     /* fields without scratch (7.5% faster on the ensemble's 48^3 and 96^3) */ \
-    default: GHX_LAUNCH_CHECK((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); break; \
+    default: GHX_LAUNCH_CHECK((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xcross<n_, (n_ % 3 == 0) ? 1 : 2, 0>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kx_in(c, prune), kx_out(c, prune), prune_word(c, prune)); break; \
     }                                                                                       \
     break;                                                                                  \
   }
@@ -3166,7 +3173,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
     const dim3 gr((unsigned)((nrows + rpb - 1) / rpb)), bl(rpb * T);                      \
-    GHX_LAUNCH_CHECK((k_xdot2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, prune);                                                                 \
+    GHX_LAUNCH_CHECK((k_xdot2<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot2<n_>), gr, bl, lds, c.stream, in, out, g, nxp, c.tw_x, kx_in(c, prune), kx_out(c, prune), prune_word(c, prune));                                                                 \
     return hipGetLastError();                                                               \
   }
       GHX_X2_SIZES(GHX_CASE)
@@ -3181,7 +3188,7 @@ hipError_t xdot(const FFTCtx &c, const FieldSet &in, const FieldSet &out, int pr
     constexpr int T = FFTCfgLow<n_>::T;                                                     \
     const PassShape s = row_shape(T, lds_line_stride(n_), max_lds(), nrows);                                        \
     const int rpb = s.lines; const size_t lds = s.lds;                          \
-    GHX_LAUNCH_CHECK((k_xdot<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, prune); \
+    GHX_LAUNCH_CHECK((k_xdot<n_>), s, kRowBound, T, false); hipLaunchKernelGGL((k_xdot<n_>), dim3((unsigned)((nrows + rpb - 1) / rpb)), dim3(rpb * T), lds, c.stream, in, out, g, nxp, c.tw_xh, c.tw_x, kx_in(c, prune), kx_out(c, prune), prune_word(c, prune)); \
     break;                                                                                  \
   }
     GHX_SIZES(GHX_CASE)

@@ -54,23 +54,23 @@ GHX_DEV double wavenum(int q, int n, double dk) {
 struct GridK {
   int nx, ny, nz, nxh;
   int anis;
+  int kxact;              // number of kx indices (from 0) with kn2(kx,0,0) <= kmax
   double dkx, dky, dkz;   // box factors 1/L (1 when not an arbitrary box)
   double rmp, rmq, rms;   // kn2 weights (1/n^2 when anisotropic, else 1)
   double kmax, tiny;
   double inv_n6;          // 1/(nx ny nz)^2
-  int kxact;              // number of kx indices (from 0) with kn2(kx,0,0) <= kmax
-  // prune == 2 (a substep on fields not known to be dealiased): a device word
-  // that is zero when the input turned out to be zero outside the kept modes
-  // (null: not looked at, taken as non-zero)
-  const unsigned *dirty;
 };
 
+// Kernel arguments are read from host memory, a cache line at a time, and each
+// further round of such reads is half a microsecond of a launch: what every
+// kernel carries stays at 96 bytes (112 cost the x inverse of 128^3 0.6 of 21.4
+// us), and pruning comes as plain arguments.
+static_assert(sizeof(GridK) == 96, "the grid constants of every kernel");
+
 // What a pass over the input of a substep skips: prune 0 nothing, 1 whatever
-// lies outside the dealias set, 2 that too if the dirty word allows it.
-// Passes over its output skip for 1 and 2 alike (only kept modes are used).
-GHX_DEV int prune_input(const GridK &g, int prune) {
-  return prune == 2 ? (g.dirty && *g.dirty == 0u ? 1 : 0) : prune;
-}
+// lies outside the dealias set, unless the device word dirty (may be null) says
+// that the input holds something there.
+GHX_DEV int prune_input(int prune, const unsigned *dirty) { return dirty && *dirty != 0u ? 0 : prune; }
 
 // kn2 and kk2 exactly as GHOST forms them (no fused multiply-add, so the
 // dealias mask matches bit for bit): main3D.fpp:1764-1800.
