@@ -202,6 +202,7 @@ def _declare(L):
         "ghx_stream_probe": (_I, [_I, _P, _P, C.c_size_t, _I, _P]),
         "ghx_pass_shape": (_I, [_I, _I, _I, _I, C.c_longlong, C.POINTER(_I), C.POINTER(_I),
                                 C.POINTER(C.c_longlong), C.POINTER(_I)]),
+        "ghx_tile_order": (_I, [_I, _I, _I, C.POINTER(_I)]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(L, name)

@@ -375,7 +375,16 @@ template <typename K> static void allow_lds(K kern, size_t bytes) {
 // line shares its lines with the neighbouring tile along the chunked axis, so
 // within each group of 16 linear ids the two ids that land on the same XCD
 // (b and b+8) are given neighbouring tiles.  Tiles stay spread over the XCDs
-// in their natural order, which keeps pruned passes load-balanced.
+// in their natural order, which keeps pruned passes load-balanced, but for rows
+// of 16, 32, .. tiles (128, 256, .. ky): there a tile would meet the same XCD in
+// every row, and the tiles that pruning empties (the middle third of ky) are
+// the same in every row, so two XCDs would idle while two have half as much
+// again.  So in the pruned z passes each such row starts one XCD further than
+// the last (spread).  us without | with: curl z inverse 119.9 | 81.6 at 256^3, 33.6
+// | 24.5 at 128 x 256 x 128, 355 | 293 at 512 x 512 x 256; MHD update 291 | 202 at
+// 256^3.  (Without pruning, and in the y passes, whose rows are of other lengths
+// and pass all XCDs by themselves, it only costs: one field's z inverse of 64 x
+// 64 x 512 14.8 | 17.2, y inverses up to a third.)
 // ---------------------------------------------------------------------------
 // Member b of a batched launch: every field pointer moves by b * bstride.
 // The view reads the pointers from the kernel arguments on each use and adds
@@ -391,13 +400,24 @@ struct FieldView {
 };
 GHX_DEV FieldView batch_view(const FieldSet &fs, unsigned b) { return FieldView{FieldRef{fs, (size_t)b * fs.bstride}}; }
 
-GHX_DEV void xcd_tile(int &bx, int &by) {
-  const int nb = gridDim.x * gridDim.y;
-  int b = blockIdx.y * gridDim.x + blockIdx.x;
-  if (b < (nb & ~15)) b = (b & ~15) | ((b & 7) << 1) | ((b >> 3) & 1);
+// tile of linear id b among rows of gx tiles, nb in all
+__host__ __device__ inline int xcd_order(int b, int row, int gx, int nb, bool spread) {
+  if (b >= (nb & ~15)) return b;
+  if (spread && (gx & 15) == 0) b = (b & ~7) | ((b + row) & 7);
+  return (b & ~15) | ((b & 7) << 1) | ((b >> 3) & 1);
+}
+GHX_DEV void xcd_tile(int &bx, int &by, bool spread = false) {
+  const int b = xcd_order(blockIdx.y * gridDim.x + blockIdx.x, blockIdx.y, gridDim.x, gridDim.x * gridDim.y, spread);
   bx = b % gridDim.x;
   by = b / gridDim.x;
 }
+#if GHX_PART == 1
+extern "C" int ghx_tile_order(int gx, int rows, int spread, int *tile) {
+  if (gx < 1 || rows < 1 || !tile) return -1;
+  for (int b = 0; b < gx * rows; ++b) tile[b] = xcd_order(b, b / gx, gx, gx * rows, spread != 0);
+  return 0;
+}
+#endif
 
 // ---------------------------------------------------------------------------
 // Tile helpers (block = L lines x T lanes; line lt = threadIdx.x / T)
@@ -602,7 +622,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv(FieldSet in_, FieldSet out_
   const FieldView in = batch_view(in_, blockIdx.z);
   const FieldView out = batch_view(out_, blockIdx.z);
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   // prune: the input is dealiased, so only lines inside the dealias disc
   // carry data; only their kept modes are read and only they are written.
@@ -797,7 +817,7 @@ __global__ __launch_bounds__(kTileBound) void k_zinv_one(FieldSet in_, FieldSet 
   const int member = blockIdx.z / nout, o = blockIdx.z - member * nout;
   const ZOut w = zinv_output(mode, o);  // the same for the whole block
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   if (lmask == 0u) return;  // uniform over the block
@@ -881,7 +901,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd(FieldSet in, FieldSet out, 
   F fft;  // with this lane's stage roots, loaded once
   fft.load_fwd(twt, t);
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   if (lmask == 0u) return;  // uniform over the block
@@ -966,7 +986,7 @@ __global__ __launch_bounds__(zrk_bound(KIND)) void k_zrk(FieldSet in_, GridK g, 
   const int tid = threadIdx.x - c * GL;
   const int lt = tid / T, t = tid % T;
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   const bool inside = j < g.ny, on = (lmask >> lt) & 1u, ok = inside && on;
@@ -1112,7 +1132,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_hd(FieldSet in_, GridK g
   }
   if (rk.nu_b) rk.nu = rk.nu_b[blockIdx.z];
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   // prune: all state buffers are dealiased (zero outside the kept modes), so
   // only lines inside the dealias disc are transformed and only kept modes
@@ -1204,7 +1224,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_bouss(FieldSet in, GridK
   F fft;  // with this lane's stage roots, loaded once
   fft.load_fwd(twt, t);
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   // prune == 2: the output buffers held something else, so the lines outside
@@ -1304,7 +1324,7 @@ __global__ __launch_bounds__(kTileBound) void k_zfwd_rk_mhd(FieldSet in, GridK g
   F fft;  // with this lane's stage roots, loaded once
   fft.load_fwd(twt, t);
   int bx, by;
-  xcd_tile(bx, by);
+  xcd_tile(bx, by, prune != 0);
   const int i = by, j0 = bx * L, j = j0 + lt;
   const unsigned lmask = prune ? tile_lines_active(g, i, j0, L) : ~0u;
   // prune == 2: the output buffers held something else, so the lines outside

@@ -526,6 +526,11 @@ int ghx_stream_probe(int kind, void *dst, const void *src, size_t bytes, int blo
 int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                    long long *lds, int *lanes);
 
+/* The tile that each block of a z or y pass takes, by the block's linear id, for
+ * `rows` rows of gx tiles (host-only): tile[0 .. gx * rows).  spread: 1 as in
+ * the pruned z passes. */
+int ghx_tile_order(int gx, int rows, int spread, int *tile);
+
 #ifdef __cplusplus
 }
 #endif
