@@ -202,6 +202,20 @@ static constexpr long small_z_lines(int nz) {
 // less not below 3328 (52.3 | 54.9 at 3168 of 512).
 static constexpr long small_y_lines(int ny) { return ny > 512 ? 512 : ny == 384 ? 2112 : kSmallLines; }
 
+// Long y inverses are split by field too, all tiles of one field before the
+// next's, where that was measured to gain.  All fields in turn | split, us: up to
+// 96 points 41.1 | 39.1 (6 fields of 256 x 64 x 256), 49.9 | 43.4 (256 x 96 x 192);
+// 192 points 113.9 | 110.7 (9 fields of 192^3), 71.1 | 71.2 (6), 40.4 | 40.6 (3); six
+// and more fields of 256 and 384 points on long launches 179.8 | 171.6 (256^3),
+// 650 | 611 (384^3), but 77.8 | 80.5 (256 x 256 x 128), 215.9 | 249.4 (512 x 384 x
+// 96), and three 74.5 | 83.5 (256^3), 145.8 | 166.2 (384 x 384 x 192); not 128
+// points (78.7 | 82.1 for 256 x 128 x 256), 512 (2%) or 1024 (the same).  45 | 46
+// us at 128 x 256 x 128 (5504 lines), 39 | 40 at 192 x 128 x 128 (8320).
+static constexpr bool long_y(int ny, int nf, long lines) {
+  if (ny <= 96 || ny == 192) return lines >= 10000;
+  return (ny == 256 || ny == 384) && nf >= 6 && lines >= 20000;
+}
+
 // Refuses, before it is issued, a launch that its kernel was not built for:
 // more lanes than its __launch_bounds__ or than the code object's maximum
 // work-group size, a block that is not whole lines of T lanes, a tile wider
@@ -255,8 +269,9 @@ static bool x2_size(int nx) {
 // the small planes' kernel (n = nx, nlines = ny); 10 and 11 the x passes of 3
 // and 4 for nlines rows; 12 the y inverse, 13 the y forward and 14 the z
 // inverse of separate fields on their own schedules; 15 and 16: *lines is the
-// number of kept lines up to which a z or y launch takes one field per block
-// (nothing else is set).  Kinds 5 to 8 give -3 where
+// number of kept lines up to which a z or y launch takes one field per block; 17:
+// *lines is 1 where a y inverse of want fields and nlines kept lines beyond that
+// takes one too (nothing else is set).  Kinds 5 to 8 give -3 where
 // the launcher takes the other kernels.
 extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                               long long *lds, int *lanes) {
@@ -285,6 +300,10 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
   }
   if ((kind == 15 || kind == 16) && rows > 0 && lines) {
     *lines = (int)(kind == 15 ? small_z_lines(n) : small_y_lines(n));
+    return 0;
+  }
+  if (kind == 17 && rows > 0 && lines) {
+    *lines = long_y(n, want, nlines) ? 1 : 0;
     return 0;
   }
   if (T <= 0 || nlines < 1 || ldsmax <= 0) return -1;
@@ -2743,12 +2762,8 @@ static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const F
 
 hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  // Long launches are split by field too, all tiles of one field before the
-  // next's: 6 fields 183 -> 172 us at 256^3, 650 -> 611 at 384^3, 9 fields 314
-  // -> 272 at 256^3, but 45 -> 46 us at 128 x 256 x 128 (5504 lines), 39 -> 40 at
-  // 192 x 128 x 128 (8320).  The 512-point wide pass loses 2%.
   const long lines = (long)g.kxact * g.nz * c.batch;
-  const YSplit sp = ysplit(small_y(c) || (lines >= 10000 && g.ny != 512) ? nf : 1);
+  const YSplit sp = ysplit(small_y(c) || long_y(g.ny, nf, lines) ? nf : 1);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;

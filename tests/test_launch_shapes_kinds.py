@@ -87,3 +87,12 @@ def test_one_field_per_block_ends_earlier_on_long_lines():
         assert z[0] == y[0] == 0
         assert z[1] == (3328 if n <= 192 else max(384, 1408 * 192 // n))
         assert y[1] == {384: 2112, 1024: 512}.get(n, 3328)
+
+
+def test_long_y_inverses_split_where_it_gains():
+    for n in SIZES:
+        for nf in (1, 3, 6, 9):
+            for lines in (3329, 9999, 10000, 11008, 16416, 19999, 20000, 22016, 49536):
+                want = lines >= 10000 and (n <= 96 or n == 192 or
+                                           (n in (256, 384) and nf >= 6 and lines >= 20000))
+                assert shape(17, n, lines, nf, 163840)[:2] == (0, int(want))
