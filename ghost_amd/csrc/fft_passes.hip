@@ -1440,7 +1440,13 @@ struct YSplit {
   int parts;
   unsigned inv;
 };
-static inline YSplit ysplit(int parts) { return YSplit{parts, (unsigned)(((1ull << 31) + parts - 1) / parts)}; }
+// (whole fields where the members' fields would be more blocks than a grid's z
+// extent holds: 10923 members of six fields)
+constexpr long kGridZ = 65535;
+static inline YSplit ysplit(bool split, int nf, int batch) {
+  const int parts = split && (long)nf * batch <= kGridZ ? nf : 1;
+  return YSplit{parts, (unsigned)(((1ull << 31) + parts - 1) / parts)};
+}
 
 template <int N, typename Cfg = FFTCfgMix<N>>
 __global__ __launch_bounds__(kTileBound) void k_yinv(FieldSet in_, FieldSet out_, int nf_, YSplit sp, GridK g, int nxp,
@@ -2730,7 +2736,7 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
 template <int N>
 static hipError_t launch_y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const YSplit sp = ysplit(small_y(c) ? nf : 1);
+  const YSplit sp = ysplit(small_y(c), nf, c.batch);
   using Cfg = FFTCfgLow<N>;
   constexpr int T = Cfg::T;
   const int nxp = p_row(g);
@@ -2763,7 +2769,7 @@ static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const F
 hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   const long lines = (long)g.kxact * g.nz * c.batch;
-  const YSplit sp = ysplit(small_y(c) || long_y(g.ny, nf, lines) ? nf : 1);
+  const YSplit sp = ysplit(small_y(c) || long_y(g.ny, nf, lines), nf, c.batch);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;
@@ -2803,7 +2809,7 @@ hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out
 
 hipError_t yfwd(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
-  const YSplit sp = ysplit(small_y(c) ? nf : 1);
+  const YSplit sp = ysplit(small_y(c), nf, c.batch);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, false, nf, in, out, prune, &lerr)) return lerr;

@@ -983,7 +983,10 @@ hipError_t op_clear_word(hipStream_t st, unsigned *word) {
   return hipGetLastError();
 }
 hipError_t op_unkept_run(const GridK &g, hipStream_t st, const cplx *v, size_t stride, int nf, unsigned *flag) {
-  hipLaunchKernelGGL(k_unkept_run, dim3(walk_blocks(g, 256), nf), dim3(kBlock), 0, st, g, v, stride, flag);
+  constexpr int most = 65535;  // a grid's y extent
+  for (int f = 0; f < nf; f += most)
+    hipLaunchKernelGGL(k_unkept_run, dim3(walk_blocks(g, 256), nf - f < most ? nf - f : most), dim3(kBlock), 0, st, g,
+                       v + (size_t)f * stride, stride, flag);
   return hipGetLastError();
 }
 
