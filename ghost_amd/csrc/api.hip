@@ -95,12 +95,13 @@ extern "C" int ghx_sync(void) {
 namespace {
 enum ProfSlot {
   P_ZINV, P_ZINV_CURL, P_ZINV_MHD, P_YINV, P_YFWD, P_XINV, P_XFWD, P_XCROSS, P_ZFWD, P_ZFWD_RK_HD, P_ZFWD_RK_MHD,
-  P_ZINV_SPLINE, P_TRACER_STAGE, P_ZINV_BOUSS, P_XDOT, P_ZFWD_RK_BOUSS, P_YINV_TRACER, P_XINV_TRACER, P_NSLOTS
+  P_ZINV_SPLINE, P_TRACER_STAGE, P_ZINV_BOUSS, P_XDOT, P_ZFWD_RK_BOUSS, P_YINV_TRACER, P_XINV_TRACER,
+  P_XYPLANE_FWD, P_XYPLANE_INV, P_NSLOTS
 };
 const char *kProfNames[P_NSLOTS] = {"zinv", "zinv_curl", "zinv_mhd", "ypass_inv", "ypass_fwd", "xinv",
                                     "xfwd", "xcross", "zfwd", "zfwd_rk_hd", "zfwd_rk_mhd", "zinv_spline",
                                     "tracer_stage", "zinv_bouss", "xdot", "zfwd_rk_bouss", "ypass_inv_tracer",
-                                    "xinv_tracer"};
+                                    "xinv_tracer", "xyplane_fwd", "xyplane_inv"};
 struct ProfRec {
   int slot;
   double bytes;
@@ -340,7 +341,7 @@ static int do_r2c(ghx_plan *p, int nf, const double *const *in, void *const *out
   const double sc = (double)nc * sizeof(cplx), sr = (double)p->nx * p->ny * p->nz * sizeof(double);
   timer_begin(p);
   if (ghx::xyplane(p->ctx)) {
-    PROF(P_XFWD, nf * (sr + sc), p->ctx.stream, ghx::xyplane_fwd(p->ctx, nf, in, q));
+    PROF(P_XYPLANE_FWD, nf * (sr + sc), p->ctx.stream, ghx::xyplane_fwd(p->ctx, nf, in, q));
   } else {
     PROF(P_XFWD, nf * (sr + sc), p->ctx.stream, ghx::xfwd(p->ctx, nf, in, pp));
     PROF(P_YFWD, nf * 2 * sc, p->ctx.stream, ghx::yfwd(p->ctx, nf, pp, q, prune));
@@ -366,7 +367,7 @@ static int do_c2r(ghx_plan *p, int nf, const void *const *in, double *const *out
   timer_begin(p);
   PROF(P_ZINV, nf * 2 * sc, p->ctx.stream, ghx::zinv(p->ctx, 0, nf, i, q));
   if (ghx::xyplane(p->ctx)) {
-    PROF(P_XINV, nf * (sr + sc), p->ctx.stream, ghx::xyplane_inv(p->ctx, nf, q, out));
+    PROF(P_XYPLANE_INV, nf * (sr + sc), p->ctx.stream, ghx::xyplane_inv(p->ctx, nf, q, out));
   } else {
     PROF(P_YINV, nf * 2 * sc, p->ctx.stream, ghx::yinv(p->ctx, nf, q, pp));
     PROF(P_XINV, nf * (sr + sc), p->ctx.stream, ghx::xinv(p->ctx, nf, pp, out));
