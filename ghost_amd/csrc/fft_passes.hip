@@ -210,8 +210,11 @@ static constexpr long small_y_lines(int ny) { return ny > 512 ? 512 : ny == 384 
 // 650 | 611 (384^3), but 77.8 | 80.5 (256 x 256 x 128), 215.9 | 249.4 (512 x 384 x
 // 96), and three 74.5 | 83.5 (256^3), 145.8 | 166.2 (384 x 384 x 192); not 128
 // points (78.7 | 82.1 for 256 x 128 x 256), 512 (2%) or 1024 (the same).  45 | 46
-// us at 128 x 256 x 128 (5504 lines), 39 | 40 at 192 x 128 x 128 (8320).
-static constexpr bool long_y(int ny, int nf, long lines) {
+// us at 128 x 256 x 128 (5504 lines), 39 | 40 at 192 x 128 x 128 (8320).  Without
+// pruning three fields gain too: 172 | 166 (256^3), 286 | 269 (384 x 384 x 192), 71 |
+// 68 (256 x 256 x 128).
+static constexpr bool long_y(int ny, int nf, long lines, bool pruned) {
+  if (!pruned) return lines >= 10000 && ny != 512;
   if (ny <= 96 || ny == 192) return lines >= 10000;
   return (ny == 256 || ny == 384) && nf >= 6 && lines >= 20000;
 }
@@ -269,9 +272,9 @@ static bool x2_size(int nx) {
 // the small planes' kernel (n = nx, nlines = ny); 10 and 11 the x passes of 3
 // and 4 for nlines rows; 12 the y inverse, 13 the y forward and 14 the z
 // inverse of separate fields on their own schedules; 15 and 16: *lines is the
-// number of kept lines up to which a z or y launch takes one field per block; 17:
-// *lines is 1 where a y inverse of want fields and nlines kept lines beyond that
-// takes one too (nothing else is set).  Kinds 5 to 8 give -3 where
+// number of kept lines up to which a z or y launch takes one field per block; 17
+// and 18: *lines is 1 where a pruned or whole y inverse of want fields and nlines
+// kept lines beyond that takes one too (nothing else is set).  Kinds 5 to 8 give -3 where
 // the launcher takes the other kernels.
 extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long ldsmax, int *lines, int *block,
                               long long *lds, int *lanes) {
@@ -302,8 +305,8 @@ extern "C" int ghx_pass_shape(int kind, int n, int nlines, int want, long long l
     *lines = (int)(kind == 15 ? small_z_lines(n) : small_y_lines(n));
     return 0;
   }
-  if (kind == 17 && rows > 0 && lines) {
-    *lines = long_y(n, want, nlines) ? 1 : 0;
+  if ((kind == 17 || kind == 18) && rows > 0 && lines) {
+    *lines = long_y(n, want, nlines, kind == 17) ? 1 : 0;
     return 0;
   }
   if (T <= 0 || nlines < 1 || ldsmax <= 0) return -1;
@@ -2769,7 +2772,7 @@ static bool y_low(const FFTCtx &c, bool inv, int nf, const FieldSet &in, const F
 hipError_t yinv(const FFTCtx &c, int nf, const FieldSet &in, const FieldSet &out, int prune) {
   const GridK &g = c.gk;
   const long lines = (long)g.kxact * g.nz * c.batch;
-  const YSplit sp = ysplit(small_y(c) || long_y(g.ny, nf, lines), nf, c.batch);
+  const YSplit sp = ysplit(small_y(c) || long_y(g.ny, nf, lines, prune != 0), nf, c.batch);
   const int nxp = p_row(g);
   hipError_t lerr;
   if (y_low(c, true, nf, in, out, prune, &lerr)) return lerr;

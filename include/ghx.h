@@ -516,8 +516,8 @@ int ghx_stream_probe(int kind, void *dst, const void *src, size_t bytes, int blo
  * nx, nlines = ny), 10 and 11 the x passes of 3 and 4 for nlines rows, 12 the
  * y inverse, 13 the y forward, 14 the z inverse of separate fields, 15 and 16
  * the kept lines up to which a z or y launch takes one field per block, 17
- * whether a y inverse of `want` fields and nlines kept lines beyond takes one
- * too (*lines 0 or 1); for a
+ * and 18 whether a pruned or whole y inverse of `want` fields and nlines kept
+ * lines beyond takes one too (*lines 0 or 1); for a
  * line length n, nlines lines along the tiled axis, a requested tile width
  * and an LDS limit in bytes.  Returns 0 when the shape passes the check every
  * launcher applies before it launches (lanes within the kernel's launch

@@ -96,3 +96,4 @@ def test_long_y_inverses_split_where_it_gains():
                 want = lines >= 10000 and (n <= 96 or n == 192 or
                                            (n in (256, 384) and nf >= 6 and lines >= 20000))
                 assert shape(17, n, lines, nf, 163840)[:2] == (0, int(want))
+                assert shape(18, n, lines, nf, 163840)[:2] == (0, int(lines >= 10000 and n != 512))
