@@ -91,8 +91,8 @@ static PassShape wide_shape(int TW, int rowslots, int nlines) {
 // Rows per block of an x pass: kRowBound lanes, fewer rows when their LDS
 // lines would not fit (the kernels read the row count from blockDim.x / T).
 // Rows synchronise by wavefront, so launches of up to 9 wavefronts per CU go
-// out one wavefront per block, which spreads them over all CUs (16 rows of 64
-// points per wavefront otherwise leave half of them idle at 64^3).  Measured,
+// out one wavefront per block, which spreads them over all CUs (blocks of 32 rows
+// of 64 points otherwise leave half of them idle at 64^3).  Measured,
 // blocks of 256 -> 64 lanes, us: X cross 11.2 -> 8.4 at 32^3, 11.4 -> 10.6 at
 // 64^3, 12.6 -> 11.8 at 128 x 64 x 32, 23.1 -> 22.1 at 384 x 48 x 48, tracers'
 // inverse 14.2 -> 12.0 at 96^3 (2304 wavefronts); the same at 128^3 (4096).
@@ -366,11 +366,6 @@ static bool use_x2(int nx) {
   return x2_size(nx);
 }
 
-// z inverses of several fields: 8 lines (128-byte chunks of Q) while that is at
-// most 256 lanes, else 4 (measured, 4 against 8 lines: MHD 911 -> 802 us at
-// 512 x 512 x 256, 479 -> 395 at 512 x 512 x 128, 414 -> 350 at 384 x 384 x
-// 192, Boussinesq 147 -> 115 at 384 x 384 x 96, HD 434 -> 352 at 512 x 512 x
-// 256; but HD 394 -> 438 at 384^3, MHD 633 -> 648 at 256 x 256 x 512).
 // Built-in tile width: `lines`, or as many more as fill a wavefront (a line of
 // few lanes would leave half or more of it idle: 4 lines of 8 lanes).
 static constexpr int tile_default(int T, int lines) { return lines * T >= 64 ? lines : 64 / T; }
@@ -2522,6 +2517,12 @@ hipError_t zinv(const FFTCtx &c, int mode, int nf, const FieldSet &in, const Fie
     default: return hipErrorInvalidValue;
     }
   }
+  // Several fields: 8 lines (128-byte chunks of Q) while that is at most 256
+  // lanes, else 4; the curl alone 8.  4 against 8 lines, us: curl 95.7 | 81.6 at
+  // 256^3, 282 | 236 at 512 x 512 x 192, 166 | 137 at 384 x 384 x 192, MHD 299 | 256 at
+  // 256 x 384 x 256, Boussinesq 127 | 107 at 384 x 384 x 96 (but 22.6 | 24.1 for the
+  // curl at 128 x 128 x 192, 40.3 | 42.2 at 192^3); of 64 lanes HD 394 | 438 at 384^3,
+  // MHD 633 | 648 at 256 x 256 x 512; the curl alone 225 | 181 at 256^3.
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
@@ -2695,8 +2696,9 @@ hipError_t zfwd_rk_mhd(const FFTCtx &c, const FieldSet &in, const MHDRKParams &r
     }
   }
   // the four-points-per-lane schedule where a size has one (GHX_ZLOW=0: the
-  // default schedule); 8 lines to 256 lanes, else 4 (both parts together: 51 ->
-  // 46 us at 128^3, 113 -> 108 at 192^3, but 764 -> 814 at 512 x 512 x 256)
+  // default schedule); 8 lines to 256 lanes, else 4 (both parts together, 4 | 8
+  // lines: 103 | 87 us at 384 x 384 x 48, 53 | 52 at 256 x 256 x 48, from 96 points on
+  // within 5% either way; of 64 lanes 764 | 814 at 512 x 512 x 256)
   switch (g.nz) {
 #define GHX_CASE(n_)                                                                        \
   case n_: {                                                                                \
@@ -3247,8 +3249,8 @@ hipError_t zfwd_rk_bouss(const FFTCtx &c, const FieldSet &in, const BoussRKParam
   const GridK &g = c.gk;
   // Up to kSmallLines at any length (63 against 78 us for 2112 lines of 512
   // points, 115 against 196 of 1024), and beyond on power-of-two lines of 32 to
-  // 256 points: 48 -> 32 us at 128^3, 249 -> 207 at 256^3 (but 37 -> 47 at 192 x
-  // 192 x 96)
+  // 256 points: 48 -> 26 us at 128^3, 207 -> 169 at 256^3, 113 -> 83 at 256 x 256 x 128
+  // (but 37 -> 47 at 192 x 192 x 96)
   if ((z_lines(c) <= kSmallLines || (g.nz >= 32 && g.nz <= 256 && (g.nz & (g.nz - 1)) == 0)) &&
       takes_zrk(zrk_groups(2), lds_line_stride(g.nz), max_lds())) {
     ZUpdate u{};

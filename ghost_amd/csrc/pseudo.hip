@@ -604,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void k_spectrum(GridK g, double dkk, int nb
 
 // Totals of nblk rows of nb partials, rows split over the block's kSumSeg
 // waves and added in a fixed order.  (One thread per bin over all rows was a
-// chain of 1024 loads: 238 us for any spectrum; this takes 6.)
+// chain of 1024 loads: 238 us for any spectrum; this takes 11.)
 constexpr int kSumSeg = 16;
 __global__ __launch_bounds__(64 * kSumSeg) void k_spectrum_sum(const double *part, int nblk, int nb, double *out) {
   __shared__ double sh[kSumSeg][64];

@@ -265,7 +265,9 @@ int ghx_hd_fields(ghx_hd *s, void **v, void **f);
 /* call after writing v through those pointers.  The next step checks whether
  * v is zero outside the dealias set (tiny <= kn2 <= kmax); while it is, the
  * passes skip every line that carries no kept mode (exact zeros in, discarded
- * values out), otherwise the first step runs the full transforms. */
+ * values out); otherwise the first step's inverses read every mode, and its
+ * passes over the products, of which only kept modes are used, skip them all
+ * the same. */
 int ghx_hd_touch(ghx_hd *s);
 /* call after writing f: records which (kx,ky) lines carry forcing, or 0 for none */
 int ghx_hd_set_forcing(ghx_hd *s, int enabled);
