@@ -316,7 +316,7 @@ typedef struct ghx_bouss ghx_bouss;
  * already multiplied by bvfreq (main3D.fpp:973-974).  ord 1 to 3; ord = 3
  * without rotation adds the correction of bouss_rkstep2.f90:73-145 after the
  * last substep (the state then keeps modes outside the dealias set, as
- * GHOST's does, and the next step runs unpruned).  With xmom = xtemp = 0
+ * GHOST's does, and the next step's inverses run unpruned).  With xmom = xtemp = 0
  * th is a passive scalar: the PHD solver (include/phd_rkstep{1,2}.f90). */
 int ghx_bouss_create(ghx_bouss **s, ghx_grid *g, int ord, double dt, double nu, double kappa, double xmom,
                      double xtemp);
